@@ -20,6 +20,9 @@ int elf_gemm_dw_group(int n, const elf_dw_problem* problems, int K, float scale,
 	static_assert(sizeof(elf_dw_problem) == sizeof(elf::DwProblem) && offsetof(elf_dw_problem, acc) == offsetof(elf::DwProblem, acc) &&
 	                  offsetof(elf_dw_problem, N) == offsetof(elf::DwProblem, N),
 	              "elf_dw_problem and elf::DwProblem differ");
+	// (the launcher also takes sizes that are multiples of 64; this entry point refuses them, as its header says)
+	for (int i = 0; problems && i < n && i < 16; i++)
+		ELF_REQUIRE(problems[i].M % 256 == 0 && problems[i].N % 256 == 0, "elf_gemm_dw_group: problem %d (M=%d N=%d) needs M, N multiples of 256", i, problems[i].M, problems[i].N);
 	return elf::gemm_dw_group(n, reinterpret_cast<const elf::DwProblem*>(problems), K, scale, (hipStream_t)stream);
 }
 

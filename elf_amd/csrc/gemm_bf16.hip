@@ -1,18 +1,13 @@
-// bf16 MFMA GEMM for gfx950 (CDNA4): C[M,N] (+)= sum_k A(m,k) * B(n,k), fp32 accumulation.
+// Dispatch of the bf16 GEMM: C[M,N] (+)= sum_k A(m,k) * B(n,k), fp32 accumulation.
 //
-// The three contractions of a linear layer under the split backward map onto one kernel:
+// The three contractions of a linear layer under the split backward:
 //   forward  Y  = X  . W^T   A = X  [M,K] k-contiguous ("R"), B = W  [N,K] k-contiguous ("R")
 //   dX       dX = dY . W     A = dY [M,K] k-contiguous ("R"), B = W  [K,N] n-contiguous ("T")
 //   dW       dW += dY^T . X  A = dY [K,M] m-contiguous ("T"), B = X  [K,N] n-contiguous ("T")
 // (reference semantics: elf/zb_utils.py:20 forward, :34-37 dX, :235-244 dW accumulate).
 //
-// Tiling: one workgroup owns a BM x BN tile of C and walks K in steps of 64.  Global loads
-// are 16 B per lane into registers, then written to a double-buffered LDS tile, so the loads
-// of step k+1 are in flight while the MFMAs of step k run.  "R" operands are stored [row][k]
-// with 8 elements of padding and read with ds_read_b128; "T" operands are stored [k][row] as
-// they sit in memory and read with ds_read_b64_tr_b16, the LDS transpose read of gfx950, so
-// no operand is ever transposed through HBM.  Each wave owns a (BM/WR) x (BN/WC) sub-tile
-// built from v_mfma_f32_32x32x16_bf16.
+// The kernels are in gemm_dma.hip (256x256 and 128x256 tiles) and gemm_ring.hip (128x128 .. 64x64 tiles); all of them
+// add the products of an output in the same order, so the choice of a tile never changes its bits (a split of K does).
 #include <atomic>
 
 #include "common.h"
@@ -22,12 +17,6 @@
 namespace elf {
 
 constexpr int BK = 64;
-// turn counters of split tiles (see gemm_kernel)
-constexpr int TURN_RS_SLOTS = 4096;
-static __device__ uint32_t turn_rs[TURN_RS_SLOTS];
-// polls of ~1 us: about a millisecond, several times a predecessor's epilogue; a workgroup that uses them up is counted
-constexpr int TURN_RS_SPIN_LIMIT = 1 << 10;
-static __device__ unsigned int turn_rs_giveups;
 
 // One sequence of tags for every launch of every GEMM kernel that splits tiles: a counter value left behind by any
 // earlier launch then never equals a value a later launch waits for.
@@ -35,344 +24,86 @@ uint32_t next_turn_tag() {
 	static std::atomic<uint32_t> launch_tag{0};
 	return (launch_tag.fetch_add(1) % 0xFFFFFFu) + 1;
 }
-int dma_turn_giveups(uint64_t* out);  // gemm_dma.hip
+int dma_turn_giveups(uint64_t* out);   // gemm_dma.hip
+int ring_turn_giveups(uint64_t* out);  // gemm_ring.hip
 // Split-K workgroups / waves (both GEMM kernel families, this device) that stopped waiting for their turn and added out
 // of turn since the library was loaded: the sums are right, only bit-reproducibility lapsed for those launches.
 int gemm_turn_giveups(uint64_t* out) {
-	unsigned int n = 0;
-	uint64_t d = 0;
-	ELF_CHECK_HIP(hipMemcpyFromSymbol(&n, HIP_SYMBOL(turn_rs_giveups), sizeof(n)));
+	uint64_t d = 0, r = 0;
 	if (int rc = dma_turn_giveups(&d)) return rc;
-	*out = d + n;
-	return 0;
-}
-constexpr int PAD_R = 8;    // elements of padding per row of an "R" tile ([row][BK+8])
-constexpr int PAD_T = 16;   // elements of padding per row of a "T" tile ([k][rows+16])
-
-struct GemmArgs {
-	const bf16_t* A;
-	const bf16_t* B;
-	void* C;
-	const bf16_t* R;  // residual (EPI_BF16_RESID)
-	int64_t lda, ldb, ldc, ldr;
-	int M, N, K;
-	int tiles_m, tiles_n;
-	int k_splits;      // >1: split-K with fp32 atomics (EPI_F32_ACC only)
-	uint32_t turn_tag; // split-K: this launch's tag in the turn counters, 0 = the splits add in any order
-};
-
-template <int ROWS, bool T>
-struct TileShape {
-	static constexpr int LD = T ? (ROWS + PAD_T) : (BK + PAD_R);
-	static constexpr int ELEMS = T ? BK * LD : ROWS * LD;
-};
-
-// Global -> register staging of one operand tile. NT threads cooperatively fetch ROWS x BK
-// (or BK x ROWS) elements as 16-byte chunks.
-template <int ROWS, bool T, int NT>
-struct TileLoader {
-	static constexpr int CHUNKS = ROWS * BK / 8 / NT;  // 16-byte chunks per thread
-	static constexpr int CPR = T ? ROWS / 8 : BK / 8;  // chunks per stored row
-	static constexpr int RPP = NT / CPR;               // stored rows per pass
-	static_assert(CHUNKS >= 1 && (NT % CPR) == 0, "tile/threads mismatch");
-
-	u32x4 regs[CHUNKS];
-
-	// p points at the tile origin: for R, &A[row0][k0]; for T, &A[k0][row0].
-	__device__ __forceinline__ void load(const bf16_t* __restrict__ p, int64_t ld, int tid) {
-		const int c = tid % CPR, r = tid / CPR;
-#pragma unroll
-		for (int i = 0; i < CHUNKS; i++) {
-			const bf16_t* q = p + (int64_t)(r + i * RPP) * ld + c * 8;
-			regs[i] = *reinterpret_cast<const u32x4*>(q);
-		}
-	}
-	__device__ __forceinline__ void store(bf16_t* lds, int tid) const {
-		constexpr int LD = TileShape<ROWS, T>::LD;
-		const int c = tid % CPR, r = tid / CPR;
-#pragma unroll
-		for (int i = 0; i < CHUNKS; i++) {
-			*reinterpret_cast<u32x4*>(lds + (r + i * RPP) * LD + c * 8) = regs[i];
-		}
-	}
-};
-
-// One MFMA operand fragment (8 consecutive k for row lane%32, k-group lane/32) for the
-// 32-row slab starting at `row`, k-step `ks` (16 wide).
-template <int ROWS, bool T>
-__device__ __forceinline__ bf16x8 read_frag(const bf16_t* lds, int row, int ks, int lane) {
-	constexpr int LD = TileShape<ROWS, T>::LD;
-	if constexpr (!T) {
-		const bf16_t* p = lds + (row + (lane & 31)) * LD + ks * 16 + 8 * (lane >> 5);
-		return *reinterpret_cast<const bf16x8*>(p);
-	} else {
-		// Transposing read: inside each group of 16 lanes, lane j supplies the address of the
-		// 8-byte chunk (k = k0 + j/4, rows 4*(j%4)..+3) and receives rows (j) of k0..k0+3.
-		const int j = lane & 15;
-		const int rbase = row + 16 * ((lane & 31) >> 4) + 4 * (j & 3);
-		const int k0 = ks * 16 + 8 * (lane >> 5) + (j >> 2);
-		const bf16_t* p0 = lds + k0 * LD + rbase;
-		const bf16_t* p1 = p0 + 4 * LD;
-		s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 ELF_LDS*)(p0));
-		s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 ELF_LDS*)(p1));
-		s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-		return __builtin_bit_cast(bf16x8, v);
-	}
-}
-
-template <int BM, int BN, int WR, int WC, bool AT, bool BT, int EPI>
-__global__ __launch_bounds__(WR* WC * 64) void gemm_kernel(GemmArgs g) {
-	constexpr int NT = WR * WC * 64;
-	constexpr int WM = BM / WR, WN = BN / WC;
-	constexpr int TM = WM / 32, TN = WN / 32;
-	constexpr int A_ELEMS = TileShape<BM, AT>::ELEMS;
-	constexpr int B_ELEMS = TileShape<BN, BT>::ELEMS;
-
-	extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-	// Buffers are addressed as smem + integer offset (never through an array of pointers) so that
-	// every access stays a DS instruction; a generic pointer would turn them into FLAT accesses
-	// that also wait on the global-load counter.
-	bf16_t* const smem = reinterpret_cast<bf16_t*>(smem_raw);
-	constexpr int STAGE = A_ELEMS + B_ELEMS;
-
-	const int tid = threadIdx.x;
-	const int lane = tid & 63;
-	const int wave = tid >> 6;
-	const int wr = wave / WC, wc = wave % WC;
-
-	// Tile assignment. Workgroups are dealt round-robin to the 8 XCDs, each with a private
-	// L2: give every XCD a contiguous run of tile ids, then walk tiles in column-major
-	// groups of GROUP_M tile rows so that a group shares its B panel and A rows in L2.
-	int pid = blockIdx.x;
-	const int ntiles = g.tiles_m * g.tiles_n;
-	int ksplit = 0;
-	if (g.k_splits > 1) {
-		ksplit = pid / ntiles;
-		pid = pid % ntiles;
-	}
-	if ((ntiles & 7) == 0) pid = (pid & 7) * (ntiles >> 3) + (pid >> 3);
-	constexpr int GROUP_M = 8;
-	const int per_group = GROUP_M * g.tiles_n;
-	const int group = pid / per_group;
-	const int first_m = group * GROUP_M;
-	const int gsz = min(g.tiles_m - first_m, GROUP_M);
-	const int tm_idx = first_m + (pid % per_group) % gsz;
-	const int tn_idx = (pid % per_group) / gsz;
-	const int m0 = tm_idx * BM, n0 = tn_idx * BN;
-
-	const int nk_total = g.K / BK;
-	const int nk_per = (nk_total + g.k_splits - 1) / g.k_splits;
-	const int kt_begin = ksplit * nk_per;
-	const int kt_end = min(nk_total, kt_begin + nk_per);
-	// Split tiles add in turn (bit-reproducible sums): split s starts its atomics when turn_rs[tile] holds this
-	// launch's tag with count s and publishes s + 1 when they have been performed.  Splits of lower index are
-	// dispatched first, so the one waited for is running or done; the wait is bounded, and a workgroup that gives
-	// up adds out of turn (the right sum, only its rounding may differ).
-	uint32_t* const my_turn = turn_rs + (((uint32_t)pid + g.turn_tag * 977u) % (uint32_t)TURN_RS_SLOTS);
-	const uint32_t turn_want = (g.turn_tag << 8) | (uint32_t)ksplit;
-	// The poll and the publication are relaxed: the adds are atomics performed at the memory side, so what has to
-	// be known is only that they have been performed - every lane awaits the acknowledgement of its own
-	// (vmcnt(0)) before the workgroup barrier that precedes the publication.
-	auto take_turn = [&]() {
-		if (g.k_splits > 1 && g.turn_tag) {
-			if (tid == 0 && ksplit > 0) {
-				int spin = 0;
-				for (; spin < TURN_RS_SPIN_LIMIT && __hip_atomic_load(my_turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != turn_want; spin++)
-					__builtin_amdgcn_s_sleep(8);
-				if (spin >= TURN_RS_SPIN_LIMIT) atomicAdd(&turn_rs_giveups, 1u);
-			}
-			__syncthreads();
-		}
-	};
-	auto pass_turn = [&]() {
-		if (g.k_splits > 1 && g.turn_tag) {
-			wait_vmcnt<0>();
-			__syncthreads();
-			if (tid == 0) __hip_atomic_store(my_turn, turn_want + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-		}
-	};
-	if (kt_begin >= kt_end) {
-		take_turn();
-		pass_turn();
-		return;
-	}
-
-	const bf16_t* Ap = AT ? g.A + (int64_t)kt_begin * BK * g.lda + m0 : g.A + (int64_t)m0 * g.lda + (int64_t)kt_begin * BK;
-	const bf16_t* Bp = BT ? g.B + (int64_t)kt_begin * BK * g.ldb + n0 : g.B + (int64_t)n0 * g.ldb + (int64_t)kt_begin * BK;
-	const int64_t a_step = AT ? (int64_t)BK * g.lda : BK;
-	const int64_t b_step = BT ? (int64_t)BK * g.ldb : BK;
-
-	TileLoader<BM, AT, NT> la;
-	TileLoader<BN, BT, NT> lb;
-
-	f32x16 acc[TM][TN];
-#pragma unroll
-	for (int i = 0; i < TM; i++)
-#pragma unroll
-		for (int j = 0; j < TN; j++)
-#pragma unroll
-			for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
-
-	la.load(Ap, g.lda, tid);
-	lb.load(Bp, g.ldb, tid);
-	la.store(smem, tid);
-	lb.store(smem + A_ELEMS, tid);
-	__syncthreads();
-
-	for (int kt = kt_begin; kt < kt_end; kt++) {
-		const int cur = (kt - kt_begin) & 1;
-		const bool more = (kt + 1) < kt_end;
-		if (more) {
-			Ap += a_step;
-			Bp += b_step;
-			la.load(Ap, g.lda, tid);
-			lb.load(Bp, g.ldb, tid);
-		}
-		const bf16_t* a_s = smem + cur * STAGE;
-		const bf16_t* b_s = a_s + A_ELEMS;
-#pragma unroll
-		for (int ks = 0; ks < BK / 16; ks++) {
-			bf16x8 af[TM], bfr[TN];
-#pragma unroll
-			for (int i = 0; i < TM; i++) af[i] = read_frag<BM, AT>(a_s, wr * WM + i * 32, ks, lane);
-#pragma unroll
-			for (int j = 0; j < TN; j++) bfr[j] = read_frag<BN, BT>(b_s, wc * WN + j * 32, ks, lane);
-#pragma unroll
-			for (int i = 0; i < TM; i++)
-#pragma unroll
-				for (int j = 0; j < TN; j++)
-					acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i], bfr[j], acc[i][j], 0, 0, 0);
-		}
-		if (more) {
-			la.store(smem + (cur ^ 1) * STAGE, tid);
-			lb.store(smem + (cur ^ 1) * STAGE + A_ELEMS, tid);
-		}
-		__syncthreads();
-	}
-
-	// Epilogue. Accumulator register r of a 32x32 tile holds row (r/4)*8 + (lane/32)*4 + r%4,
-	// column lane%32: lanes 0..31 cover 32 consecutive columns of one row.
-	if constexpr (EPI == EPI_F32_ACC) take_turn();
-	const int col_l = lane & 31;
-	const int row_l = (lane >> 5) * 4;
-#pragma unroll
-	for (int i = 0; i < TM; i++) {
-#pragma unroll
-		for (int j = 0; j < TN; j++) {
-			const int col = n0 + wc * WN + j * 32 + col_l;
-#pragma unroll
-			for (int r = 0; r < 16; r++) {
-				const int row = m0 + wr * WM + i * 32 + (r >> 2) * 8 + row_l + (r & 3);
-				const float v = acc[i][j][r];
-				if constexpr (EPI == EPI_BF16) {
-					reinterpret_cast<bf16_t*>(g.C)[(int64_t)row * g.ldc + col] = f2bf(v);
-				} else if constexpr (EPI == EPI_BF16_RESID) {
-					const float res = bf2f(g.R[(int64_t)row * g.ldr + col]);
-					reinterpret_cast<bf16_t*>(g.C)[(int64_t)row * g.ldc + col] = f2bf(v + res);
-				} else if constexpr (EPI == EPI_F32_ACC) {
-					float* c = reinterpret_cast<float*>(g.C) + (int64_t)row * g.ldc + col;
-					if (g.k_splits > 1) {
-						unsafeAtomicAdd(c, v);
-					} else {
-						*c += v;
-					}
-				} else {
-					reinterpret_cast<float*>(g.C)[(int64_t)row * g.ldc + col] = v;
-				}
-			}
-		}
-	}
-	if constexpr (EPI == EPI_F32_ACC) pass_turn();
-}
-
-template <int BM, int BN, int WR, int WC, bool AT, bool BT, int EPI>
-static int launch_cfg(const GemmArgs& g, hipStream_t stream) {
-	constexpr int smem = 2 * (TileShape<BM, AT>::ELEMS + TileShape<BN, BT>::ELEMS) * (int)sizeof(bf16_t);
-	auto kern = gemm_kernel<BM, BN, WR, WC, AT, BT, EPI>;
-	static bool attr_set = false;
-	if (!attr_set) {
-		ELF_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-		                                  hipFuncAttributeMaxDynamicSharedMemorySize, smem));
-		attr_set = true;
-	}
-	GemmArgs a = g;
-	a.tiles_m = g.M / BM;
-	a.tiles_n = g.N / BN;
-	a.turn_tag = EPI == EPI_F32_ACC && a.k_splits > 1 && a.tiles_m * a.tiles_n <= TURN_RS_SLOTS ? next_turn_tag() : 0;
-	const int grid = a.tiles_m * a.tiles_n * a.k_splits;
-	ELF_LAUNCH(kern, dim3(grid), dim3(WR * WC * 64), smem, stream, a);
-	ELF_CHECK_HIP(hipGetLastError());
+	if (int rc = ring_turn_giveups(&r)) return rc;
+	*out = d + r;
 	return 0;
 }
 
-template <bool AT, bool BT, int EPI>
-static int launch_layout(GemmArgs& g, int tile_cfg, hipStream_t stream) {
-	const int M = g.M, N = g.N;
-	// Tile choice: the 256x256 tile (8 waves, 128x64 each) has the best MFMA : HBM ratio;
-	// smaller tiles keep all 256 CUs busy when the output is small.
-	int cfg = tile_cfg;
-	if (cfg <= 0) {
-		const int64_t t256 = (M % 256 == 0 && N % 256 == 0) ? (int64_t)(M / 256) * (N / 256) : 0;
-		const int64_t t128 = (M % 128 == 0 && N % 128 == 0) ? (int64_t)(M / 128) * (N / 128) : 0;
-		if (t256 >= 256) cfg = 1;
-		else if (t128 >= 128) cfg = 2;
-		else cfg = 3;
-	}
-	if (EPI == EPI_F32_ACC && g.k_splits <= 0) {
-		// Split K when the weight-gradient tile count cannot fill the chip.
-		int bm = cfg == 1 ? 256 : cfg == 2 ? 128 : 64;
-		int64_t tiles = (int64_t)(M / bm) * (N / bm);
-		int ks = 1;
-		while (tiles * ks < 256 && (g.K / BK) / (ks * 2) >= 8 && ks < 16) ks *= 2;
-		g.k_splits = ks;
-	}
-	if (g.k_splits <= 0 || EPI != EPI_F32_ACC) g.k_splits = 1;
-	switch (cfg) {
-		case 1:
-			ELF_REQUIRE(M % 256 == 0 && N % 256 == 0, "gemm: tile 256 needs M,N multiples of 256 (M=%d N=%d)", M, N);
-			return launch_cfg<256, 256, 2, 4, AT, BT, EPI>(g, stream);
-		case 2:
-			ELF_REQUIRE(M % 128 == 0 && N % 128 == 0, "gemm: tile 128 needs M,N multiples of 128 (M=%d N=%d)", M, N);
-			return launch_cfg<128, 128, 2, 2, AT, BT, EPI>(g, stream);
-		case 3:
-			ELF_REQUIRE(M % 64 == 0 && N % 64 == 0, "gemm: M and N must be multiples of 64 (M=%d N=%d)", M, N);
-			return launch_cfg<64, 64, 2, 2, AT, BT, EPI>(g, stream);
-		case 5:
-			ELF_REQUIRE(M % 256 == 0 && N % 128 == 0, "gemm: tile 256x128 needs M%%256==0, N%%128==0 (M=%d N=%d)", M, N);
-			return launch_cfg<256, 128, 2, 2, AT, BT, EPI>(g, stream);
-		default:
-			set_error("gemm: unknown tile config %d", cfg);
-			return -1;
-	}
+// ------------------------------------------------------------------------------------------
+// Tile choice.  Estimated time of a product on tiles of bm x bn: rounds of 256 workgroups (one per compute unit) times the
+// time of a K slice of 64 times the slices, plus what a round costs besides (filling the ring, the epilogue).  The constants
+// are microseconds fitted to cold-operand timings of 33 shapes from 512 x 512 x 512 to 4096 x 50304 x 768 (operands rotated
+// through more than the 256 MB cache); the estimate is within 15 % of nearly all of them.  A large tile has the cheaper products (per slice
+// and output: 22 ps on 256x256, 26 on 128x256, 35 on 128x128, 66 on 64x64: the smaller the tile, the more operand bytes go
+// through the 64 B/clk path into LDS for each product) and loses where its tiles leave compute units idle:
+//   1920 x 1600 x 1600: 44 us on 56 tiles of 256x256, 27 on 105 of 128x256, 19.9 on 195 of 128x128, 25 on 750 of 64x64;
+//   1920 x 4800 x 1600: 46 us on 152 tiles of 256x256, 52 on 285 of 128x256, 49 on 570 of 128x128.
+struct TileTime {
+	int bm, bn;
+	float slice, round;
+};
+static constexpr TileTime TILES_BF16[] = {{256, 256, 1.45f, 6.f}, {128, 256, 0.854f, 5.5f}, {128, 128, 0.58f, 4.f}, {64, 128, 0.38f, 2.f}, {128, 64, 0.40f, 2.f}, {64, 64, 0.27f, 1.3f}};
+// weight gradients: both operands reduction-major, fp32 read-modify-write of the output
+static constexpr TileTime TILES_F32[] = {{256, 256, 1.33f, 20.f}, {128, 256, 0.79f, 11.f}, {128, 128, 0.55f, 5.f}, {64, 128, 0.44f, 2.f}, {128, 64, 0.44f, 2.f}, {64, 64, 0.30f, 1.5f}};
+
+struct Plan {
+	int bm = 0, bn = 0, k_splits = 1;
+	float us = 1e30f;
+	bool dma() const { return bn == 256; }
+};
+
+static float tile_us(const TileTime& t, int M, int N, int slices, int k_splits = 1) {
+	const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * k_splits;
+	const float rounds = (float)((tiles + 255) / 256);
+	// workgroups that walk several 256x256 tiles fill their ring once
+	return rounds * (slices + k_splits - 1) / k_splits * t.slice + (t.bm == 256 && t.round < 10.f ? t.round : rounds * t.round);
 }
 
-template <bool AT, bool BT>
-static int launch_epi(GemmArgs& g, int epi, int tile_cfg, hipStream_t stream) {
-	switch (epi) {
-		case EPI_BF16: return launch_layout<AT, BT, EPI_BF16>(g, tile_cfg, stream);
-		case EPI_BF16_RESID: return launch_layout<AT, BT, EPI_BF16_RESID>(g, tile_cfg, stream);
-		case EPI_F32_ACC: return launch_layout<AT, BT, EPI_F32_ACC>(g, tile_cfg, stream);
-		case EPI_F32_STORE: return launch_layout<AT, BT, EPI_F32_STORE>(g, tile_cfg, stream);
-		default: set_error("gemm: unknown epilogue %d", epi); return -1;
+// The tile with the smallest estimate.  ring_extra: what the caller pays on top if it is one of the small ring tiles (a
+// pass of its own for an epilogue that only the 256-column tiles have).
+static Plan plan_tiles(bool f32, int M, int N, int K, float ring_extra = 0.f) {
+	Plan best;
+	for (const TileTime& t : f32 ? TILES_F32 : TILES_BF16) {
+		if (M < t.bm || N < t.bn) continue;
+		const float us = tile_us(t, M, N, K / BK) + (t.bn == 256 ? 0.f : ring_extra);
+		if (us < best.us) best = Plan{t.bm, t.bn, 1, us};
 	}
+	return best;
 }
 
-// Which direct-to-LDS tile a forward / input-gradient product runs on: 256 rows when 192 or more such tiles fill
-// the chip, else 128 rows (k-contiguous A) when 128 or more of those do, else neither (0).  A choice by estimated
-// rounds of workgroups x time per workgroup - 128-row tiles where the 256-row ones leave a mostly empty last round,
-// e.g. 8192 x 2304 x 768 - wins 4-11 % back to back on operands that stay cached and loses 3.6 % inside the
-// GPT-2-small stream, where they are cold and the narrower tile fetches B twice as often: not used.
-static int dma_tile_rows(bool a_t, int M, int N, int K) {
-	if (N % 256 != 0 || K % 64 != 0) return 0;
-	if (M % 256 == 0 && (int64_t)(M / 256) * (N / 256) >= 192) return 256;
-	if (M % 128 == 0 && !a_t && (int64_t)(M / 128) * (N / 256) >= 128) return 128;
-	return 0;
+// Weight gradients on 128x256 tiles with K split k_splits ways (at least 16 slices each): the splits of a tile add with
+// atomics, 2.3 us per million output elements and split (2048 x 2048 x 8192: 107 us whole, 82 us in two; 768 x 768 x 8192:
+// 107 and 43 in four, but 41 whole on 64x64 tiles).
+static Plan plan_weight_gradient(int M, int N, int K) {
+	Plan best = plan_tiles(true, M, N, K);
+	const TileTime& t = TILES_F32[1];
+	if (M >= t.bm && N >= t.bn)
+		for (int ks = 2; ks <= 16 && K / BK / ks >= 16; ks++) {
+			const float us = tile_us(t, M, N, K / BK, ks) + 2.3e-6f * ks * (float)M * N;
+			if (us < best.us) best = Plan{t.bm, t.bn, ks, us};
+		}
+	return best;
 }
+
+// 256 or 128: the direct-to-LDS tile of 256 columns a forward / input-gradient product runs on, 0: one of the ring tiles.
+static int dma_tile_rows(int M, int N, int K, float ring_extra) {
+	const Plan p = plan_tiles(false, M, N, K, ring_extra);
+	return p.dma() ? p.bm : 0;
+}
+// what a pass of its own over `bytes` costs (5 TB/s and a launch)
+static float pass_us(double bytes) { return 3.f + (float)(bytes / 5e6); }
 
 // K split of a weight gradient on 256x256 direct-to-LDS tiles when the caller leaves it open: *k_splits ways for the last
 // *tail_tiles tiles (-1: all of them).
 static void dw_split_plan(int M, int N, int K, int* k_splits, int* tail_tiles) {
-	const int64_t tiles = (int64_t)(M / 256) * (N / 256);
+	const int64_t tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
 	const int nk = K / 64;
 	*k_splits = 1;
 	*tail_tiles = -1;
@@ -403,54 +134,37 @@ int gemm_bf16(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda,
 	// the turn counters of split tiles hold the split index in 8 bits next to the launch tag
 	ELF_REQUIRE(k_splits <= 255, "gemm: k_splits must be at most 255 (got %d)", k_splits);
 	ProfScope prof(PROF_GEMM, 2.0 * M * N * K, stream);
-	GemmArgs g;
-	g.A = (const bf16_t*)A;
-	g.B = (const bf16_t*)B;
-	g.C = C;
-	g.R = (const bf16_t*)R;
-	g.lda = lda;
-	g.ldb = ldb;
-	g.ldc = ldc;
-	g.ldr = ldr;
-	g.M = M;
-	g.N = N;
-	g.K = K;
-	g.tiles_m = g.tiles_n = 0;
-	g.k_splits = k_splits;
-	// small weight gradients (12..128 tiles of 128x256, e.g. 2304x768 or 2048x2048 at K = 8192): 128x256 tiles with K
-	// split so that the workgroups just fill the chip once - 7-28 % faster than 256x256 tiles split further.  A split
-	// keeps at least 32 K slices, 16 where the tiles are so few (768x768: 18) that half of the chip would idle otherwise
-	if (tile_cfg <= 0 && epi == EPI_F32_ACC && a_t && b_t && k_splits <= 0 && M % 128 == 0 && N % 256 == 0 && K >= 4096) {
-		const int64_t tiles = (int64_t)(M / 128) * (N / 256);
-		if (tiles >= 12 && tiles <= 128) {
-			int ks = (int)(256 / tiles);
-			const int min_slices = tiles < 24 ? 16 : 32;
-			if (ks > K / 64 / min_slices) ks = K / 64 / min_slices;
-			return gemm_bf16_dma(a_t, b_t, M, N, K, A, lda, B, ldb, C, ldc, epi, R, ldr, ks < 1 ? 1 : ks, -1, 128, stream);
+	ELF_REQUIRE(M % 64 == 0 && N % 64 == 0, "gemm: M and N must be multiples of 64 (M=%d N=%d)", M, N);
+	ELF_REQUIRE(tile_cfg >= 0 && tile_cfg <= 12 && tile_cfg != 4 && tile_cfg != 6, "gemm: unknown tile config %d", tile_cfg);
+	int bm = 0, bn = 0, tail_tiles = -1;  // an explicit k_splits splits every tile
+	switch (tile_cfg) {
+		case 0: break;
+		case 1: case 7: bm = 256, bn = 256; break;
+		case 8: bm = 128, bn = 256; break;
+		case 2: case 5: case 9: bm = 128, bn = 128; break;
+		case 10: bm = 64, bn = 128; break;
+		case 11: bm = 128, bn = 64; break;
+		default: bm = bn = 64; break;
+	}
+	ELF_REQUIRE(M >= bm && N >= bn, "gemm: tile config %d needs M of at least %d and N of at least %d (M=%d N=%d)", tile_cfg, bm, bn, M, N);
+	if (bm == 0) {
+		Plan p;
+		if (epi != EPI_F32_ACC) {
+			p = plan_tiles(false, M, N, K);
+		} else if (k_splits > 0) {
+			p = plan_tiles(true, M, N, K);
+		} else if (M >= 256 && N >= 256 && (int64_t)((M + 255) / 256) * ((N + 255) / 256) >= 192 && K >= 4096) {
+			p = Plan{256, 256, 0};  // the split of the tail included, see below
+		} else {
+			p = plan_weight_gradient(M, N, K);
 		}
+		bm = p.bm, bn = p.bn;
+		if (epi == EPI_F32_ACC && k_splits <= 0) k_splits = p.k_splits;
 	}
-	// Tile choice when the caller leaves it open: the direct-to-LDS 256x256 kernel whenever its
-	// tiles can fill the chip, the register-staged kernels (smaller tiles) otherwise.
-	if (tile_cfg <= 0 && epi == EPI_F32_ACC && M % 256 == 0 && N % 256 == 0 && K % 64 == 0) {
-		// weight gradients (long K, fp32 accumulate) also when the tiles are few: K is split instead
-		const int64_t tiles = (int64_t)(M / 256) * (N / 256);
-		if (tiles >= 192 || (tiles >= 24 && K >= 4096)) tile_cfg = 7;
-	}
-	if (tile_cfg <= 0 && epi != EPI_F32_ACC) {
-		const int rows = dma_tile_rows(a_t, M, N, K);
-		tile_cfg = rows == 256 ? 7 : rows == 128 ? 8 : tile_cfg;
-	}
-	if (tile_cfg == 7) {
-		int tail_tiles = -1;  // an explicit k_splits splits every tile
-		if (epi == EPI_F32_ACC && k_splits <= 0) dw_split_plan(M, N, K, &k_splits, &tail_tiles);
-		return gemm_bf16_dma(a_t, b_t, M, N, K, A, lda, B, ldb, C, ldc, epi, R, ldr, k_splits, tail_tiles, 256, stream);
-	}
-	if (tile_cfg == 8) return gemm_bf16_dma(a_t, b_t, M, N, K, A, lda, B, ldb, C, ldc, epi, R, ldr, epi == EPI_F32_ACC && k_splits > 1 ? k_splits : 1, -1, 128, stream);
-	if (!a_t && !b_t) return launch_epi<false, false>(g, epi, tile_cfg, stream);
-	if (!a_t && b_t) return launch_epi<false, true>(g, epi, tile_cfg, stream);
-	if (a_t && b_t) return launch_epi<true, true>(g, epi, tile_cfg, stream);
-	set_error("gemm: layout A=T,B=R is not used by any stage contraction");
-	return -1;
+	if (epi != EPI_F32_ACC) k_splits = 1;
+	if (bm == 256 && k_splits <= 0) dw_split_plan(M, N, K, &k_splits, &tail_tiles);
+	if (bn == 256) return gemm_bf16_dma(a_t, b_t, M, N, K, A, lda, B, ldb, C, ldc, epi, R, ldr, k_splits < 1 ? 1 : k_splits, tail_tiles, bm, stream);
+	return gemm_bf16_ring(a_t, b_t, M, N, K, A, lda, B, ldb, C, ldc, epi, R, ldr, k_splits, bm, bn, stream);
 }
 
 int gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, const void* W, int64_t ldw, void* pre,
@@ -458,12 +172,11 @@ int gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, cons
 	ELF_REQUIRE(act == ACT_GELU || act == ACT_SWIGLU, "gemm_act: unknown activation %d", act);
 	ELF_REQUIRE(M > 0 && F > 0 && K > 0 && A && W && pre && out, "gemm_act: empty problem or null operand");
 	const int N = act == ACT_SWIGLU ? 2 * F : F;
-	// the same tile choice as gemm_bf16 makes for this shape; the SwiGLU epilogue pairs 64 gate with 64 up
-	// columns per wave, so a 256-column tile covers 128 outputs
+	// the SwiGLU epilogue pairs 64 gate with 64 up columns per wave, so a 256-column tile covers 128 outputs
 	int bm = 0;
-	if (act == ACT_SWIGLU && K % 64 == 0 && N % 256 == 0 && lda % 8 == 0 && ldw % 8 == 0 && ldpre >= N && ldout >= F && ldpre % 8 == 0 && ldout % 8 == 0 &&
+	if (act == ACT_SWIGLU && M % 64 == 0 && F % 64 == 0 && K % 64 == 0 && lda % 8 == 0 && ldw % 8 == 0 && ldpre >= N && ldout >= F && ldpre % 8 == 0 && ldout % 8 == 0 &&
 	    ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)pre % 16) == 0 && ((uintptr_t)out % 16) == 0 && lda >= K && ldw >= K) {
-		bm = dma_tile_rows(false, M, N, K);
+		bm = dma_tile_rows(M, N, K, pass_us(6.0 * M * F));
 	}
 	if (bm) {
 		ProfScope prof(PROF_GEMM, 2.0 * M * N * K, stream);
@@ -478,7 +191,7 @@ int gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, cons
 int gemm_dw_final(int M, int N, int K, const void* dY, int64_t lddy, const void* X, int64_t ldx, float* acc, void* grad_bf16, float scale,
                   hipStream_t stream) {
 	ELF_REQUIRE(M > 0 && N > 0 && K > 0 && dY && X && acc && grad_bf16, "gemm_dw_final: bad argument");
-	const bool fused = M % 256 == 0 && N % 256 == 0 && K % 64 == 0 && (int64_t)(M / 256) * (N / 256) >= 192 && lddy % 8 == 0 && ldx % 8 == 0 && lddy >= M &&
+	const bool fused = M % 64 == 0 && N % 64 == 0 && K % 64 == 0 && M >= 256 && N >= 256 && (int64_t)((M + 255) / 256) * ((N + 255) / 256) >= 192 && K >= 4096 && lddy % 8 == 0 && ldx % 8 == 0 && lddy >= M &&
 	                   ldx >= N && ((uintptr_t)dY % 16) == 0 && ((uintptr_t)X % 16) == 0 && ((uintptr_t)acc % 16) == 0 && ((uintptr_t)grad_bf16 % 8) == 0;
 	if (fused) {
 		// the same K split as the plain weight gradient (same rounding); tiles shared by several workgroups along K have no
@@ -492,10 +205,12 @@ int gemm_dw_final(int M, int N, int K, const void* dY, int64_t lddy, const void*
 	return scale_grads(acc, grad_bf16, (int64_t)M * N, scale, stream);
 }
 
+static int rope_tile_rows(int M, int N, int K, int D) {
+	if (!(M >= 64 && N >= 64 && M % 64 == 0 && N % 64 == 0 && K % 64 == 0 && (D == 64 || D == 128) && N % D == 0)) return 0;
+	return dma_tile_rows(M, N, K, pass_us(4.0 * M * N));
+}
 bool gemm_rope_fused(int M, int N, int K, int D) {
-	if (!(M > 0 && N > 0 && K > 0 && K % 64 == 0 && N % 256 == 0 && (D == 64 || D == 128))) return false;
-	// the tile choice gemm_bf16 makes for this shape
-	return dma_tile_rows(false, M, N, K) != 0;
+	return rope_tile_rows(M, N, K, D) != 0;
 }
 
 int gemm_rope_bf16(int M, int N, int K, const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, const void* cs,
@@ -506,7 +221,7 @@ int gemm_rope_bf16(int M, int N, int K, const void* A, int64_t lda, const void* 
 	    ((uintptr_t)W % 16) == 0 && ((uintptr_t)C % 16) == 0 && ((uintptr_t)cs % 16) == 0) {
 		// the rotation's arithmetic is not counted: the figure stays the GEMM's
 		ProfScope prof(PROF_GEMM, 2.0 * M * N * K, stream);
-		const int bm = dma_tile_rows(false, M, N, K);
+		const int bm = rope_tile_rows(M, N, K, D);
 		return gemm_bf16_dma(0, 0, M, N, K, A, lda, W, ldw, C, ldc, EPI_BF16_ROPE, nullptr, 0, 1, 0, bm, stream, nullptr, 0, cs, S, n_rot_heads * D, D);
 	}
 	if (int rc = gemm_bf16(0, 0, M, N, K, A, lda, W, ldw, C, ldc, EPI_BF16, nullptr, 0, 0, 0, stream)) return rc;
@@ -514,7 +229,11 @@ int gemm_rope_bf16(int M, int N, int K, const void* A, int64_t lda, const void* 
 }
 
 bool gemm_swiglu_bwd_fused(int M, int F, int K) {
-	return M > 0 && F > 0 && K > 0 && M % 256 == 0 && F % 256 == 0 && K % 64 == 0 && (int64_t)(M / 256) * (F / 256) >= 192;
+	if (!(M >= 256 && F >= 256 && M % 64 == 0 && F % 64 == 0 && K % 64 == 0)) return false;
+	// 256x256 tiles only: against the best tile of the plain product and the pass over d, g, u and their gradients (the
+	// epilogue itself reads and writes four of those five at 256 tiles a time)
+	const float rounds = (float)(((int64_t)((M + 255) / 256) * ((F + 255) / 256) + 255) / 256);
+	return rounds * K / BK * TILES_BF16[0].slice + rounds * 12.f < plan_tiles(false, M, F, K).us + pass_us(10.0 * M * F);
 }
 
 int gemm_swiglu_bwd_bf16(int M, int F, int K, const void* dY, int64_t lddy, const void* W, int64_t ldw, const void* gu,

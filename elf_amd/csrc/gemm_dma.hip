@@ -1,6 +1,6 @@
 // 256x256 (and 128x256) bf16 MFMA GEMM tile kernel with direct global->LDS loads, for gfx950.
 //
-// Same contraction and layouts as gemm_bf16.hip (C (+)= sum_k A(m,k) B(n,k); "R" operands are
+// The contraction of gemm_bf16.hip (C (+)= sum_k A(m,k) B(n,k); "R" operands are
 // k-contiguous, "T" operands reduction-major), different data movement:
 //   * global_load_lds_dwordx4 moves 16 B per lane straight into LDS (no VGPR staging, no
 //     ds_write); two 64-wide K slices (2 x 64 KiB) alternate, the next slice being fetched while
@@ -17,14 +17,13 @@
 // workgroup barrier for the other waves' slices and for the reuse of the oldest stage.
 #include "common.h"
 #include "kernels.h"
-#include "lds_dma.h"
-#include <type_traits>
+#include "gemm_tile.h"
 
 namespace elf {
 
 namespace dma {
 
-constexpr int BN = 256, BKS = 64;
+constexpr int BN = 256;
 constexpr int PERS_WORKGROUPS = 256;  // one per compute unit: the persistent kernel's grid
 constexpr int B_BYTES = BN * BKS * 2;  // 32 KiB per stage
 
@@ -44,15 +43,6 @@ struct Shape {
 	static constexpr int LOADS_PER_STAGE = LOADS_A + LOADS_B;
 	static_assert(LOADS_PER_STAGE % 2 == 0, "the loads of a slice are issued in two halves");
 };
-
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N-1>), unrolled at compile time.
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-	if constexpr (N > 0) {
-		static_for<N - 1>(f);
-		f(std::integral_constant<int, N - 1>{});
-	}
-}
 
 struct Args {
 	const bf16_t* A;
@@ -92,85 +82,6 @@ static __device__ uint32_t turn[TURN_TILES * TURN_PER_TILE];
 constexpr int TURN_SPIN_LIMIT = 1 << 10;
 static __device__ unsigned int turn_giveups;
 __device__ __forceinline__ void note_turn_giveup() { atomicAdd(&turn_giveups, 1u); }
-
-// Byte offsets (relative to the tile origin of the current K slice) of the 16-byte chunks this
-// lane fetches for one operand (< 2^31: 256 rows of at most 64 K elements).  "R" tiles are
-// [256 rows][128 B], "T" tiles [64 k][512 B] ([64 k][256 B] for the 128 rows of A in a 128x256 tile); LDS chunk slot s of a row holds global chunk
-// s ^ f(row) with f chosen so that the lanes of a fragment read spread over all banks: an "R"
-// read takes one chunk from each of 32 rows (f = (row / 2) % 8), a "T" transpose read takes 64
-// contiguous bytes from each of four k rows per half-wave (f = 4 * (k % 8): the four rows land in
-// four different 64-byte bank groups; with 2 * (k % 8) pairs of rows shared one and the bank-conflict
-// counter read half of the LDS-active cycles).
-// chunk swizzle of reduction-major ("T") tiles as a function of the k row
-// ROWS = 128 (a k row is 256 bytes, exactly one row of banks): the four k rows of a half-wave's transpose read
-// are moved into four different 64-byte groups by (k % 4) * 4 chunks, rows k and k + 8 apart by two chunks
-template <int ROWS = 256>
-__device__ __forceinline__ int t_swz(int k) {
-	return ((k & (ROWS == 256 ? 7 : 3)) << 2) ^ (((k >> 3) & 1) << 1);
-}
-
-// PAIRED (k-contiguous operands only): the 256 tile rows are not 256 consecutive operand rows but, for
-// each 128-row half, 64 consecutive rows followed by the 64 rows `pair_rows` further down — the gate and
-// up rows of the same 64 SwiGLU columns, which thereby land in one wave's accumulators.
-template <bool T, int LPO, bool PAIRED = false, int ROWS = 256>
-__device__ __forceinline__ void lane_offsets(int wave, int lane, int64_t ld, uint32_t (&off)[LPO], int64_t pair_rows = 0) {
-#pragma unroll
-	for (int i = 0; i < LPO; i++) {
-		const int q = wave * LPO + i;  // which 1 KiB piece of the operand tile
-		if constexpr (!T) {
-			const int row = q * 8 + (lane >> 3), slot = lane & 7;
-			const int64_t grow = PAIRED ? (row >> 7) * 64 + (row & 63) + ((row >> 6) & 1) * pair_rows : row;
-			off[i] = (uint32_t)((grow * ld + ((slot ^ ((row >> 1) & 7)) << 3)) * 2);
-		} else {
-			constexpr int CPR = ROWS / 8;  // 16-byte chunks per k row; a 1 KiB piece holds 64 / CPR k rows
-			const int krow = q * (64 / CPR) + lane / CPR, slot = lane % CPR;
-			off[i] = (uint32_t)((krow * ld + ((slot ^ t_swz<ROWS>(krow)) << 3)) * 2);
-		}
-	}
-}
-
-// Operand fragment of v_mfma_f32_16x16x32_bf16 for the 16-row slab at `row0` and the k32 half `kq`
-// of the current slice: lane l holds row (or column) row0 + l % 16 at k = 32 kq + 8 (l / 16) .. + 7.
-// "R" tiles give it with one 16-byte read; "T" tiles with two transpose reads, each of which hands
-// the 16 lanes of a group the 4 (k) x 16 (rows) block they address row-wise.
-template <bool T, int ROWS = 256>
-__device__ __forceinline__ bf16x8 frag(const unsigned char* base, int row0, int kq, int lane) {
-	if constexpr (!T) {
-		const int r = row0 + (lane & 15);
-		const int c = (4 * kq + (lane >> 4)) ^ ((r >> 1) & 7);
-		return *reinterpret_cast<const bf16x8*>(base + r * 128 + c * 16);
-	} else {
-		const int j = lane & 15;
-		const int m = row0 + 4 * (j & 3);
-		const int kk = kq * 32 + 8 * (lane >> 4) + (j >> 2);
-		const int c0 = (m >> 3) ^ t_swz<ROWS>(kk);
-		const int c1 = (m >> 3) ^ t_swz<ROWS>(kk + 4);
-		const unsigned char* p0 = base + kk * (ROWS * 2) + c0 * 16 + (j & 1) * 8;
-		const unsigned char* p1 = base + (kk + 4) * (ROWS * 2) + c1 * 16 + (j & 1) * 8;
-		s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 ELF_LDS*)(p0));
-		s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 ELF_LDS*)(p1));
-		return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-	}
-}
-
-// The two byte offsets (within the operand tile of stage 0, k32 half 0) that frag<true> reads for the
-// 16-row slab at row0, and the fragment read from them for k32 half kq of the tile at `base`.
-template <int ROWS = 256>
-__device__ __forceinline__ void frag_t_offsets(int row0, int lane, uint32_t (&o)[2]) {
-	const int j = lane & 15;
-	const int m = row0 + 4 * (j & 3);
-	const int kk = 8 * (lane >> 4) + (j >> 2);
-	o[0] = (uint32_t)(kk * (ROWS * 2) + (((m >> 3) ^ t_swz<ROWS>(kk)) << 4) + (j & 1) * 8);
-	o[1] = (uint32_t)((kk + 4) * (ROWS * 2) + (((m >> 3) ^ t_swz<ROWS>(kk + 4)) << 4) + (j & 1) * 8);
-}
-// o: LDS byte addresses; imm: a compile-time byte offset (stage and k32 half) that ends up in the
-// instructions' offset fields.  t_swz only looks at k % 16, so the second k32 half of a tile lies 32 rows
-// (of 2 * ROWS bytes) further on.
-__device__ __forceinline__ bf16x8 frag_t_at(const uint32_t (&o)[2], uint32_t imm) {
-	s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 ELF_LDS*)(uintptr_t)(o[0] + imm));
-	s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 ELF_LDS*)(uintptr_t)(o[1] + imm));
-	return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-}
 
 // NW = 4, RT = 4: 256x256 workgroup tile, one wave per SIMD with a 128x128 wave tile: 16 fragment reads per
 // k32 for 64 MFMAs, a third less LDS traffic per FLOP than the eight-wave shape, which on this power-limited
@@ -251,6 +162,16 @@ __device__ __forceinline__ void tile_origin(const Args& g, int pid, int& m0, int
 	}
 }
 
+// Ragged sizes: the last tile of a row or column of tiles moves back so that it ends with the matrix, and stores only what
+// its neighbour does not (it needs M >= BM, N >= 256).  Every operand load stays inside the matrix without a bounds check
+// in the K loop, and the partly empty tile multiplies rows its neighbour multiplies as well instead of padding.  (M, N
+// multiples of 64: what is skipped are whole 32-row strips and whole 64-column halves.)
+template <int BM>
+__device__ __forceinline__ void clip_tile(const Args& g, int& m0, int& n0) {
+	m0 = min(m0, g.M - BM);
+	n0 = min(n0, g.N - BN);
+}
+
 // Tile, K range and turn counter of workgroup `bid` of the problem `g` (the block index of a launch with one problem).
 // The first ntiles - tail_tiles tiles are computed whole, one workgroup each; each of the last tail_tiles is shared by
 // k_splits workgroups that take a K range each and add their part with atomics.  Splitting only the tail turns the
@@ -277,7 +198,8 @@ __device__ __forceinline__ void locate_tile(const Args& g, const int bid, int& p
 
 // One workgroup: tile `pid` of the problem `g`, K range `ksplit` of `splits`; a split tile's turn counters are those of
 // `turn_slot`.
-template <int NW, int RT, bool AT, bool BT, int EPI>
+// EDGE: M or N is no multiple of the tile (see clip_tile).
+template <int NW, int RT, bool AT, bool BT, int EPI, bool EDGE>
 __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, const int ksplit, const int splits, const int turn_slot) {
 	using Sh = Shape<NW, RT>;
 	constexpr int BM = Sh::BM, A_BYTES = Sh::A_BYTES, STAGE_BYTES = Sh::STAGE_BYTES;
@@ -304,6 +226,8 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 	tile_origin<BM>(g, pid, m0, n0);
 	m0 = __builtin_amdgcn_readfirstlane(m0);
 	n0 = __builtin_amdgcn_readfirstlane(n0);
+	const int m_lo = m0, n_lo = n0;  // first row and column this tile stores
+	if constexpr (EDGE) clip_tile<BM>(g, m0, n0);
 
 	const int nk_total = g.K / BKS;
 	const int nk_per = (nk_total + splits - 1) / splits;
@@ -315,6 +239,7 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 			const uint32_t want = (g.turn_tag << 8) | (uint32_t)ksplit;
 			int patience = TURN_SPIN_LIMIT;
 			for (int i = 0; i < RT; i++) {
+				if (EDGE && m0 + wr * (RT * 32) + i * 32 < m_lo) continue;
 				uint32_t* t = turn + turn_slot * TURN_PER_TILE + wave * RT + i;
 				int spin = 0;
 				for (; ksplit > 0 && spin < patience && __hip_atomic_load(t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != want; spin++)
@@ -515,11 +440,14 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 				for (int r = 0; r < 4; r++) ws[(ii * 16 + row_l + r) * PITCH + j * 16 + col_l] = acc[i * 2 + ii][j][r];
 		const int grow0 = m0 + wr * (RT * 32) + i * 32;
 		const int gcol0 = n0 + wc * 128;
+		if (EDGE && grow0 < m_lo) continue;  // the neighbouring tile's rows (the same strips for every K split of a tile)
+		const int c_lo = EDGE ? n_lo - gcol0 : 0;  // columns of the wave's 128 below c_lo are the neighbouring tile's
 		if constexpr (EPI == EPI_BF16_SWIGLU) {
 			// the strip's columns are 64 gate columns then the 64 up columns of the same outputs: both go to
 			// their places in C = [gate | up] (kept for the backward) and silu(gate) * up, computed from the
 			// rounded values exactly as a separate pass over C would, to C2
 			const int F = g.N / 2, cg0 = n0 / 2 + wc * 64;
+			if (EDGE && cg0 < n_lo / 2) continue;
 #pragma unroll
 			for (int it = 0; it < 4; it++) {
 				const int row = it * 8 + (lane >> 3), c8 = (lane & 7) * 8;
@@ -543,6 +471,7 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 			// their gradients likewise in C.  All loads of the strip first (see the residual epilogue below); d is
 			// rounded to bf16 before it is used, as a separate pass over a stored d would read it
 			const int F = g.N;
+			if (EDGE && (lane & 15) * 8 < c_lo) continue;
 			bf16x8 gs[8], us[8];
 #pragma unroll
 			for (int it = 0; it < 8; it++) {
@@ -583,8 +512,9 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 			// entries of the whole strip are fetched before the first store (see the residual epilogue below).
 			const int half = g.rope_D >> 1, cph = half >> 3;  // chunks of 8 columns per half head
 			const int j = lane & 7;
-			const int c_lo = (j / cph) * g.rope_D + (j % cph) * 8, c_hi = c_lo + half;
-			const bool rot = gcol0 + c_lo < g.rope_cols;
+			const int h_lo = (j / cph) * g.rope_D + (j % cph) * 8, h_hi = h_lo + half;
+			if (EDGE && h_lo < c_lo) continue;  // (a launch's tiles only overlap by whole heads: see gemm_bf16_dma)
+			const bool rot = gcol0 + h_lo < g.rope_cols;
 			f32x4 tab[4][4];
 			if (rot) {
 #pragma unroll
@@ -599,8 +529,8 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 			for (int it = 0; it < 4; it++) {
 				const int row = it * 8 + (lane >> 3);
 				const float* w = ws + row * PITCH;
-				const f32x4 a0 = *reinterpret_cast<const f32x4*>(w + c_lo), a1 = *reinterpret_cast<const f32x4*>(w + c_lo + 4);
-				const f32x4 b0 = *reinterpret_cast<const f32x4*>(w + c_hi), b1 = *reinterpret_cast<const f32x4*>(w + c_hi + 4);
+				const f32x4 a0 = *reinterpret_cast<const f32x4*>(w + h_lo), a1 = *reinterpret_cast<const f32x4*>(w + h_lo + 4);
+				const f32x4 b0 = *reinterpret_cast<const f32x4*>(w + h_hi), b1 = *reinterpret_cast<const f32x4*>(w + h_hi + 4);
 				bf16x8 olo, ohi;
 #pragma unroll
 				for (int t = 0; t < 8; t++) {
@@ -611,12 +541,13 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 					ohi[t] = (bf16_t)rb;
 				}
 				bf16_t* c = reinterpret_cast<bf16_t*>(g.C) + (int64_t)(grow0 + row) * g.ldc + gcol0;
-				*reinterpret_cast<bf16x8*>(c + c_lo) = olo;
-				*reinterpret_cast<bf16x8*>(c + c_hi) = ohi;
+				*reinterpret_cast<bf16x8*>(c + h_lo) = olo;
+				*reinterpret_cast<bf16x8*>(c + h_hi) = ohi;
 			}
 		} else if constexpr (EPI == EPI_BF16 || EPI == EPI_BF16_RESID) {
 			// the strip's residual values first, all loads in flight together: read inside the loop below each
 			// one would be awaited (a full trip to HBM) before the store that follows it in program order
+			if (EDGE && (lane & 15) * 8 < c_lo) continue;
 			bf16x8 rs[EPI == EPI_BF16_RESID ? 8 : 1];
 			if constexpr (EPI == EPI_BF16_RESID) {
 #pragma unroll
@@ -664,7 +595,8 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 					const int row = it * 2 + (lane >> 5);
 					float* c = reinterpret_cast<float*>(g.C) + (int64_t)(grow0 + row) * g.ldc + gcol0 + (lane & 31);
 #pragma unroll
-					for (int cg = 0; cg < 4; cg++) unsafeAtomicAdd(c + cg * 32, ws[row * PITCH + cg * 32 + (lane & 31)]);
+					for (int cg = 0; cg < 4; cg++)
+						if (!EDGE || cg * 32 >= c_lo) unsafeAtomicAdd(c + cg * 32, ws[row * PITCH + cg * 32 + (lane & 31)]);
 				}
 				if (g.turn_tag) {
 					// wait until this wave's adds have been performed (they complete in vmcnt; no cache write-back is
@@ -678,6 +610,7 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 			// loop each load is awaited on its own, 16 trips to HBM in a row per strip: 43 k cycles of a
 			// 360 k-cycle dW tile)
 			constexpr bool ACCUM = EPI == EPI_F32_ACC || EPI == EPI_F32_ACC_SCALE;
+			if (EDGE && (lane & 31) * 4 < c_lo) continue;
 			f32x4 cv[ACCUM ? 16 : 1];
 			if constexpr (ACCUM) {
 #pragma unroll
@@ -706,11 +639,11 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 	}
 }
 
-template <int NW, int RT, bool AT, bool BT, int EPI>
+template <int NW, int RT, bool AT, bool BT, int EPI, bool EDGE>
 __global__ __launch_bounds__(NW * 64) void gemm_dma_kernel(Args g) {
 	int pid, ksplit, splits, turn_slot;
 	locate_tile(g, (int)blockIdx.x, pid, ksplit, splits, turn_slot);
-	gemm_dma_tile<NW, RT, AT, BT, EPI>(g, pid, ksplit, splits, turn_slot);
+	gemm_dma_tile<NW, RT, AT, BT, EPI, EDGE>(g, pid, ksplit, splits, turn_slot);
 }
 
 // Several weight gradients in one launch (the W pass of a stage: every linear layer's dW += dY^T X over the same
@@ -732,7 +665,7 @@ struct GroupArgs {
 	int first[GROUP_MAX], count[GROUP_MAX];
 	Args a[GROUP_MAX];
 };
-template <int EPI>
+template <int EPI, bool EDGE>
 __global__ __launch_bounds__(512) void gemm_dw_group_kernel(GroupArgs ga) {
 	int p = 0, pid, ksplit = 0, splits = 1, turn_slot = 0;
 	if (ga.compact) {
@@ -762,7 +695,7 @@ __global__ __launch_bounds__(512) void gemm_dw_group_kernel(GroupArgs ga) {
 		if (bid >= ga.count[p]) return;
 		locate_tile(ga.a[p], bid, pid, ksplit, splits, turn_slot);
 	}
-	gemm_dma_tile<8, 2, true, true, EPI>(ga.a[p], pid, ksplit, splits, turn_slot);
+	gemm_dma_tile<8, 2, true, true, EPI, EDGE>(ga.a[p], pid, ksplit, splits, turn_slot);
 }
 
 // ------------------------------------------------------------------------------------------------------------
@@ -800,7 +733,7 @@ __device__ __forceinline__ void mfma_init(f32x4& acc, const bf16x8& a, const bf1
 	asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(acc) : "v"(a), "v"(b));
 }
 
-template <int EPI>
+template <int EPI, bool EDGE>
 __global__ __launch_bounds__(256) void gemm_pers_kernel(Args g) {
 	using Sh = Shape<4, 4>;
 	constexpr int BM = 256, RT = 4, RF = 8, NST = 2, A_BYTES = Sh::A_BYTES, STAGE_BYTES = Sh::STAGE_BYTES;
@@ -826,6 +759,7 @@ __global__ __launch_bounds__(256) void gemm_pers_kernel(Args g) {
 		tile_origin<BM>(g, tile, m0, n0);
 		m0 = __builtin_amdgcn_readfirstlane(m0);
 		n0 = __builtin_amdgcn_readfirstlane(n0);
+		if constexpr (EDGE) clip_tile<BM>(g, m0, n0);
 		Ap = g.A + (int64_t)m0 * g.lda;
 		Bp = g.B + (int64_t)(PAIRED ? n0 / 2 : n0) * g.ldb;
 	};
@@ -950,6 +884,9 @@ __global__ __launch_bounds__(256) void gemm_pers_kernel(Args g) {
 		asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 		const int grow0 = m0 + wr * 128 + rr;
 		const int gcol0 = n0 + wc * 128;
+		// a tile that was moved back (clip_tile): 16-row groups below i_lo and 64-column halves below h_lo are its neighbour's
+		const int i_lo = EDGE ? ((m0 + BM - 1) / BM * BM - m0 - wr * 128) >> 4 : 0;
+		const int h_lo = EDGE ? (PAIRED ? ((n0 + BN - 1) / BN * BN - n0) / 2 - wc * 64 : (n0 + BN - 1) / BN * BN - n0 - wc * 128) >> 6 : 0;
 		// the lane's run t (0..3) of 8 consecutive columns: columns (t / 2) * 64 + (t % 2) * 32 + 8 g4 .. + 7 of the wave's 128
 		auto run = [&](int i, int t, float (&v)[8]) {
 #pragma unroll
@@ -962,6 +899,7 @@ __global__ __launch_bounds__(256) void gemm_pers_kernel(Args g) {
 #pragma unroll
 			for (int i = 0; i < RF; i++) {
 				__builtin_amdgcn_sched_barrier(0);  // one row group at a time (see the residual epilogue below)
+				if (EDGE && (i < i_lo || h_lo > 0)) continue;
 				const int64_t row = grow0 + i * 16;
 #pragma unroll
 				for (int t = 0; t < 2; t++) {
@@ -999,9 +937,11 @@ __global__ __launch_bounds__(256) void gemm_pers_kernel(Args g) {
 #pragma unroll
 			for (int i = 0; i < RF; i++) {
 				__builtin_amdgcn_sched_barrier(0);
+				if (EDGE && i < i_lo) continue;
 				bf16_t* cp = reinterpret_cast<bf16_t*>(g.C) + (int64_t)(grow0 + i * 16) * g.ldc + gcol0;
 #pragma unroll
 				for (int t = 0; t < 4; t++) {
+					if (EDGE && (t >> 1) < h_lo) continue;
 					float v[8];
 					run(i, t, v);
 					bf16x8 o;
@@ -1021,11 +961,11 @@ __global__ __launch_bounds__(256) void gemm_pers_kernel(Args g) {
 	wait_vmcnt<0>();  // the loads past the last tile land in LDS too
 }
 
-template <int EPI>
-static int launch_pers(const Args& a, hipStream_t stream) {
+template <int EPI, bool EDGE>
+static int launch_pers_sized(const Args& a, hipStream_t stream) {
 	using Sh = Shape<4, 4>;
 	constexpr int smem = Sh::NST * Sh::STAGE_BYTES + Sh::LOADS_A * 1024;
-	auto kern = gemm_pers_kernel<EPI>;
+	auto kern = gemm_pers_kernel<EPI, EDGE>;
 	static bool attr_set = false;
 	if (!attr_set) {
 		ELF_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
@@ -1035,6 +975,10 @@ static int launch_pers(const Args& a, hipStream_t stream) {
 	ELF_LAUNCH(kern, dim3(ntiles < PERS_WORKGROUPS ? ntiles : PERS_WORKGROUPS), dim3(256), smem, stream, a);
 	ELF_CHECK_HIP(hipGetLastError());
 	return 0;
+}
+template <int EPI>
+static int launch_pers(const Args& a, hipStream_t stream) {
+	return a.M % 256 || a.N % BN ? launch_pers_sized<EPI, true>(a, stream) : launch_pers_sized<EPI, false>(a, stream);
 }
 
 
@@ -1050,6 +994,7 @@ __global__ __launch_bounds__(256) void scale_tail_kernel(Args g) {
 	float* C = reinterpret_cast<float*>(g.C);
 	for (int i = threadIdx.x; i < 32 * 64; i += 256) {
 		const int row = i >> 6, c4 = (i & 63) * 4;
+		if (m0 + row >= g.M || n0 + c4 >= g.N) continue;  // ragged sizes
 		float* c = C + (int64_t)(m0 + row) * g.ldc + n0 + c4;
 		f32x4 v = *reinterpret_cast<const f32x4*>(c);
 		v *= g.scale;
@@ -1061,14 +1006,14 @@ __global__ __launch_bounds__(256) void scale_tail_kernel(Args g) {
 	}
 }
 
-template <int NW, int RT, bool AT, bool BT, int EPI>
-static int launch(const Args& a, hipStream_t stream) {
+template <int NW, int RT, bool AT, bool BT, int EPI, bool EDGE>
+static int launch_sized(const Args& a, hipStream_t stream) {
 	// the ring + the target of the loads past the end of K (as many KiB as a wave issues loads per
 	// operand); the epilogue needs a 32 x 136 fp32 strip per wave
 	using Sh = Shape<NW, RT>;
 	constexpr int ring = Sh::NST * Sh::STAGE_BYTES + (Sh::LOADS_A > Sh::LOADS_B ? Sh::LOADS_A : Sh::LOADS_B) * 1024, epi = NW * 32 * 136 * 4;
 	constexpr int smem = ring > epi ? ring : epi;
-	auto kern = gemm_dma_kernel<NW, RT, AT, BT, EPI>;
+	auto kern = gemm_dma_kernel<NW, RT, AT, BT, EPI, EDGE>;
 	static bool attr_set = false;
 	if (!attr_set) {
 		ELF_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
@@ -1077,6 +1022,11 @@ static int launch(const Args& a, hipStream_t stream) {
 	ELF_LAUNCH(kern, dim3(a.tiles_m * a.tiles_n + a.tail_tiles * (a.k_splits - 1)), dim3(NW * 64), smem, stream, a);
 	ELF_CHECK_HIP(hipGetLastError());
 	return 0;
+}
+
+template <int NW, int RT, bool AT, bool BT, int EPI>
+static int launch(const Args& a, hipStream_t stream) {
+	return a.M % Shape<NW, RT>::BM || a.N % BN ? launch_sized<NW, RT, AT, BT, EPI, true>(a, stream) : launch_sized<NW, RT, AT, BT, EPI, false>(a, stream);
 }
 
 template <int NW, int RT, bool AT, bool BT>
@@ -1116,15 +1066,17 @@ int gemm_bf16_dma(int a_t, int b_t, int M, int N, int K, const void* A, int64_t 
                   int64_t ldc, int epi, const void* R, int64_t ldr, int k_splits, int tail_tiles, int bm, hipStream_t stream,
                   void* C2, int64_t ldc2, const void* rope_cs, int rope_S, int rope_cols, int rope_D, float scale) {
 	ELF_REQUIRE(bm == 256 || bm == 128, "gemm (dma tile): 256- or 128-row tiles");
-	ELF_REQUIRE(M % bm == 0 && N % dma::BN == 0 && K % dma::BKS == 0, "gemm (dma tile): M multiple of %d, N of 256 and K of 64 required", bm);
-	const int ntiles = (M / bm) * (N / dma::BN);
+	ELF_REQUIRE(M >= bm && N >= dma::BN && M % 64 == 0 && N % 64 == 0 && K % dma::BKS == 0, "gemm (dma tile): M at least %d, N at least 256, all sizes multiples of 64", bm);
+	const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + dma::BN - 1) / dma::BN, ntiles = tiles_m * tiles_n;
+	// a tile's columns are taken in heads: the last one may only move back by whole heads
+	ELF_REQUIRE(epi != EPI_BF16_ROPE || N % rope_D == 0, "gemm (dma tile): the RoPE epilogue needs N to be a multiple of the head width");
 	ELF_REQUIRE(epi != EPI_BF16_SWIGLU || (C2 && !a_t && !b_t), "gemm (dma tile): the SwiGLU epilogue needs k-contiguous operands and a second output");
 	// the paired rows of the SwiGLU epilogue are addressed with 32-bit byte offsets from the tile's first row
 	ELF_REQUIRE(epi != EPI_BF16_SWIGLU || (int64_t)(N / 2 + 256) * ldb * 2 < (int64_t(1) << 31), "gemm (dma tile): weight too large for the paired-row epilogue");
 	ELF_REQUIRE(epi != EPI_F32_ACC_SCALE || (C2 && a_t && b_t && bm == 256), "gemm (dma tile): the scaling accumulate epilogue needs reduction-major operands, 256-row tiles and a bf16 output");
 	ELF_REQUIRE(epi != EPI_BF16_ROPE || (rope_cs && rope_S > 0 && !a_t && !b_t && (rope_D == 64 || rope_D == 128) && rope_cols % rope_D == 0 && rope_cols <= N),
 	            "gemm (dma tile): the RoPE epilogue needs k-contiguous operands, a table and heads of 64 or 128 columns");
-	dma::Args a{(const bf16_t*)A, (const bf16_t*)B, C, (const bf16_t*)R, (bf16_t*)C2, lda, ldb, ldc, ldr, ldc2, M, N, K, M / bm, N / dma::BN, k_splits < 1 ? 1 : k_splits,
+	dma::Args a{(const bf16_t*)A, (const bf16_t*)B, C, (const bf16_t*)R, (bf16_t*)C2, lda, ldb, ldc, ldr, ldc2, M, N, K, tiles_m, tiles_n, k_splits < 1 ? 1 : k_splits,
 	            tail_tiles < 0 || tail_tiles > ntiles ? ntiles : tail_tiles, 0, (const float2*)rope_cs, rope_S, rope_cols, rope_D, 0, scale};
 	// The band walk fetches every row slab of A from HBM in one round only and B once per band; the default
 	// walk wants A in the 256 MB memory-side cache for the whole launch and streams B once.  Inside the stage's
@@ -1171,7 +1123,7 @@ int gemm_bf16_dma(int a_t, int b_t, int M, int N, int K, const void* A, int64_t 
 }
 
 bool gemm_dw_groupable(int M, int N, int K, const void* dY, int64_t lddy, const void* X, int64_t ldx, const void* acc) {
-	return M > 0 && N > 0 && K > 0 && M % 256 == 0 && N % dma::BN == 0 && K % dma::BKS == 0 && lddy % 8 == 0 && ldx % 8 == 0 && lddy >= M && ldx >= N &&
+	return M >= 256 && N >= dma::BN && K > 0 && M % 64 == 0 && N % 64 == 0 && K % dma::BKS == 0 && lddy % 8 == 0 && ldx % 8 == 0 && lddy >= M && ldx >= N &&
 	       ((uintptr_t)dY % 16) == 0 && ((uintptr_t)X % 16) == 0 && ((uintptr_t)acc % 16) == 0;
 }
 
@@ -1179,11 +1131,14 @@ int gemm_dw_group(int n, const DwProblem* pr, int K, float scale, hipStream_t st
 	ELF_REQUIRE(n > 0 && n <= dma::GROUP_MAX && pr, "gemm_dw_group: 1..%d problems", dma::GROUP_MAX);
 	int64_t tiles = 0;
 	double flops = 0;
+	bool edge = false;
+	auto tiles_of = [](const DwProblem& q) { return ((q.M + 255) / 256) * ((q.N + dma::BN - 1) / dma::BN); };
 	for (int i = 0; i < n; i++) {
 		ELF_REQUIRE(pr[i].dY && pr[i].X && pr[i].acc && gemm_dw_groupable(pr[i].M, pr[i].N, K, pr[i].dY, pr[i].lddy, pr[i].X, pr[i].ldx, pr[i].acc),
-		            "gemm_dw_group: problem %d (M=%d N=%d K=%d) needs M, N multiples of 256, K of 64 and 16-byte aligned operands", i, pr[i].M, pr[i].N, K);
+		            "gemm_dw_group: problem %d (M=%d N=%d K=%d) needs M, N of at least 256, all sizes multiples of 64 and 16-byte aligned operands", i, pr[i].M, pr[i].N, K);
 		ELF_REQUIRE(scale == 0.f || (pr[i].grad_bf16 && ((uintptr_t)pr[i].grad_bf16 % 8) == 0), "gemm_dw_group: a scaling pass needs the bf16 gradient buffers");
-		tiles += (int64_t)(pr[i].M / 256) * (pr[i].N / dma::BN);
+		tiles += tiles_of(pr[i]);
+		edge = edge || pr[i].M % 256 || pr[i].N % dma::BN;
 		flops += 2.0 * pr[i].M * pr[i].N * K;
 	}
 	// Whole tiles, one workgroup each, except in the launch's last round: when that round would fill at most half of the
@@ -1201,7 +1156,7 @@ int gemm_dw_group(int n, const DwProblem* pr, int K, float scale, hipStream_t st
 	ga.n = n;
 	ga.compact = 1;
 	for (int i = 0; i < n; i++)
-		if ((pr[i].M / 256) * (pr[i].N / dma::BN) >= 256) ga.compact = 0;
+		if (tiles_of(pr[i]) >= 256) ga.compact = 0;
 	ga.tiles = (int)tiles, ga.tail = tail, ga.splits = splits;
 	const uint32_t tag = tail ? next_turn_tag() : 0;
 	uint32_t turn_base = tag * 977u;
@@ -1211,12 +1166,12 @@ int gemm_dw_group(int n, const DwProblem* pr, int K, float scale, hipStream_t st
 	int next = 0;
 	for (int i = 0; i < n; i++) {
 		const DwProblem& q = pr[i];
-		const int ntiles = (q.M / 256) * (q.N / dma::BN);
+		const int ntiles = tiles_of(q);
 		// this problem's share of the launch's last `tail` tiles
 		const int64_t tail_from = tiles - tail;
 		const int tail_i = before + ntiles <= tail_from ? 0 : (int)(before + ntiles - (tail_from > before ? tail_from : before));
 		dma::Args& a = ga.a[i];
-		a = dma::Args{(const bf16_t*)q.dY, (const bf16_t*)q.X, q.acc, nullptr, (bf16_t*)q.grad_bf16, q.lddy, q.ldx, q.N, 0, q.N, q.M, q.N, K, q.M / 256, q.N / dma::BN,
+		a = dma::Args{(const bf16_t*)q.dY, (const bf16_t*)q.X, q.acc, nullptr, (bf16_t*)q.grad_bf16, q.lddy, q.ldx, q.N, 0, q.N, q.M, q.N, K, (q.M + 255) / 256, (q.N + dma::BN - 1) / dma::BN,
 		              tail_i ? splits : 1, tail_i, 0, nullptr, 0, 0, 0, tail_i ? tag : 0, scale, turn_base};
 		a.walk = ga.compact ? 2 : !((int64_t)q.M * K * 2 < big && (int64_t)q.N * K * 2 >= big);
 		turn_base += (uint32_t)tail_i;
@@ -1231,14 +1186,14 @@ int gemm_dw_group(int n, const DwProblem* pr, int K, float scale, hipStream_t st
 		using Sh = dma::Shape<8, 2>;
 		constexpr int ring = Sh::NST * Sh::STAGE_BYTES + (Sh::LOADS_A > Sh::LOADS_B ? Sh::LOADS_A : Sh::LOADS_B) * 1024, epi = 8 * 32 * 136 * 4;
 		constexpr int smem = ring > epi ? ring : epi;
-		static bool attr_set = false;
-		if (!attr_set) {
-			ELF_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(dma::gemm_dw_group_kernel<EPI_F32_ACC>), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
-			ELF_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(dma::gemm_dw_group_kernel<EPI_F32_ACC_SCALE>), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
-			attr_set = true;
+		auto kern = scale != 0.f ? (edge ? dma::gemm_dw_group_kernel<EPI_F32_ACC_SCALE, true> : dma::gemm_dw_group_kernel<EPI_F32_ACC_SCALE, false>)
+		                         : (edge ? dma::gemm_dw_group_kernel<EPI_F32_ACC, true> : dma::gemm_dw_group_kernel<EPI_F32_ACC, false>);
+		static bool attr_set[2][2] = {};
+		if (bool& set = attr_set[scale != 0.f][edge]; !set) {
+			ELF_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
+			set = true;
 		}
-		if (scale != 0.f) ELF_LAUNCH(dma::gemm_dw_group_kernel<EPI_F32_ACC_SCALE>, dim3(next), dim3(512), smem, stream, ga);
-		else ELF_LAUNCH(dma::gemm_dw_group_kernel<EPI_F32_ACC>, dim3(next), dim3(512), smem, stream, ga);
+		ELF_LAUNCH(kern, dim3(next), dim3(512), smem, stream, ga);
 		ELF_CHECK_HIP(hipGetLastError());
 	}
 	// split tiles have no single epilogue that could scale them: a small kernel behind the launch does those

@@ -36,6 +36,9 @@ int gemm_bf16_dma(int a_t, int b_t, int M, int N, int K, const void* A, int64_t 
                   int64_t ldc, int epi, const void* R, int64_t ldr, int k_splits, int tail_tiles, int bm, hipStream_t stream,
                   void* C2 = nullptr, int64_t ldc2 = 0, const void* rope_cs = nullptr, int rope_S = 0, int rope_cols = 0, int rope_D = 0,
                   float scale = 1.f);
+// the same on small tiles (bm, bn: 128 or 64) with a deep ring of K slices (gemm_ring.hip)
+int gemm_bf16_ring(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb, void* C, int64_t ldc, int epi, const void* R,
+                   int64_t ldr, int k_splits, int bm, int bn, hipStream_t stream);
 
 // The weight gradient of the step's last micro-batch with the step's gradient scale folded in: acc [M, N] (fp32, dense)
 // = (acc + dY^T X) * scale and grad_bf16 [M, N] = bf16(acc), with dY [K, M] and X [K, N] (both reduction-major).  One
@@ -73,7 +76,7 @@ int gemm_rope_bf16(int M, int N, int K, const void* A, int64_t lda, const void* 
                    int S, int n_rot_heads, int D, hipStream_t stream);
 
 // Tag of one GEMM launch whose tiles are split along K (24 bits, never 0, different from launch to launch); see the
-// turn counters in gemm_dma.hip and gemm_bf16.hip.
+// turn counters in gemm_dma.hip and gemm_ring.hip.
 uint32_t next_turn_tag();
 // Waves / workgroups of split-K launches on the current device that used up their bounded wait for their turn and added
 // out of turn (right sums, rounding order not fixed) since the library was loaded.  Synchronous (one 4-byte copy each

@@ -33,9 +33,9 @@ int elf_abi_version(void);
  *   epilogue: 0 C(bf16) = acc; 1 C(bf16) = acc + R(bf16, leading dim ldr; ldr = 0: R is one row of N values
  *             added to every row of C, the bias of nn.Linear);
  *             2 C(fp32) += acc; 3 C(fp32) = acc.
- *   tile_cfg = 0 picks a tile shape from M,N (1: 256x256, 2: 128x128, 3: 64x64, 5: 256x128 register-staged;
- *   7: 256x256 with direct-to-LDS loads; 8: 128x256 with direct-to-LDS loads: a_t = 1 is accepted only together with
- *   b_t = 1, and k_splits is honoured for epilogue 2);
+ *   tile_cfg = 0 picks the tile by estimated time (7: 256x256, 8: 128x256, 9: 128x128, 10: 64x128, 11: 128x64, 12: 64x64;
+ *   1 is another name of 7, 2 and 5 of 9, 3 of 12; M and N must be at least the tile's): a_t = 1 is accepted only together
+ *   with b_t = 1; k_splits is honoured for epilogue 2;
  *   k_splits = 0 picks a K split (epilogue 2 only; at most 255).
  * Replaces: F.linear in LinearDX.forward (elf/zb_utils.py:20)            -> a_t=0,b_t=0
  *           torch.mm(grad_output, weight) in LinearDX.backward (:34-37)  -> a_t=0,b_t=1
@@ -79,9 +79,8 @@ int elf_gemm_dw_group(int n, const elf_dw_problem* problems, int K, float scale,
 /* The MLP's up-projection with its activation: pre = A W^T with A [M, K] and W [N, K], both k contiguous;
  * act 0 (GELU): N = F, out[M, F] = gelu(pre); act 1 (SwiGLU): N = 2F, W = [gate rows; up rows],
  * pre[M, 2F] = [g | u], out[M, F] = silu(g) * u.  pre is kept because the backward needs it.  SwiGLU is
- * computed in the GEMM epilogue (one kernel, the pre-activation never re-read); GELU, and shapes the
- * fused tiles do not cover (M not a multiple of 128, N not of 256, or too few tiles to fill the chip),
- * run elf_gemm_bf16 (epilogue 0) followed by elf_gelu_fwd / elf_swiglu_fwd.  Same bits either way.
+ * computed in the GEMM epilogue (one kernel, the pre-activation never re-read); GELU, and shapes that
+ * run faster on tiles too small for that epilogue, run elf_gemm_bf16 (epilogue 0) followed by elf_gelu_fwd / elf_swiglu_fwd.  Same bits either way.
  * Replaces: fc1 + nn.GELU() of the GPT block's MLP (benchmarks/models/simple.py:44-52) run through
  *           LinearDX.forward (elf/zb_utils.py:20); no reference module for SwiGLU. */
 int elf_gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, const void* W, int64_t ldw,
@@ -89,7 +88,7 @@ int elf_gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, 
 /* Backward of the down-projection into the SwiGLU: d = dY W with dY [M, K] and W [K, F] (the down
  * projection's weight [d_model, F] as it lies in memory), then dgu[M, 2F] = [d silu'(g) u | d silu(g)]
  * from the saved gu[M, 2F] = [g | u].  One kernel (activation backward in the GEMM epilogue, d never
- * reaches memory) when M and F are multiples of 256, K of 64 and the tiles fill the chip; otherwise
+ * reaches memory) where 256x256 tiles are the faster choice (sizes multiples of 64, M and F at least 256); otherwise
  * elf_gemm_bf16(0, 1, ...) into scratch [M, F] followed by elf_swiglu_bwd (scratch may be null only for
  * the fused shapes).  Same bits either way.
  * Replaces: LinearDX.backward of fc2 (elf/zb_utils.py:29-41) followed by autograd's backward of
@@ -101,7 +100,7 @@ int elf_gemm_swiglu_bwd_bf16(int M, int F, int K, const void* dY, int64_t lddy, 
  * C[M, N] = A W^T (A [M, K], W [N, K], both k contiguous) rounded to bf16, then the rotation of elf_rope_apply
  * on the first n_rot_heads heads of width D (64 or 128); cs is the table of elf_rope_table for sequence length
  * S, row r of A is the token at position r mod S.  One kernel (rotation in the GEMM epilogue, the projection
- * is never read back) when M is a multiple of 128, N of 256, K of 64 and the tiles fill the chip; otherwise
+ * is never read back) where tiles of 256 columns are the faster choice (N a multiple of D); otherwise
  * elf_gemm_bf16 followed by elf_rope_apply.  Same bits either way.
  * Replaces: the q / k / v projections of the attention block run through LinearDX.forward
  *           (elf/zb_utils.py:20); no reference module for the rotary embedding. */

@@ -156,6 +156,63 @@ def test_persistent_forward_gemm_equals_the_tile_kernel_bit_for_bit(K, monkeypat
 	_close(new[4], torch.nn.functional.silu(new[3][:, :F].float()) * new[3][:, F:].float(), what="persistent swiglu")
 
 
+@pytest.mark.parametrize("layout", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("tile_cfg,shape", [
+	(7, (256, 320, 64)), (7, (320, 256, 192)), (7, (1984, 576, 128)), (8, (128, 256, 64)), (8, (192, 448, 320)),
+	(9, (128, 128, 64)), (9, (192, 320, 192)), (9, (832, 1600, 320)), (10, (64, 192, 448)), (11, (192, 64, 448)), (12, (64, 64, 64)), (12, (192, 128, 1088)),
+	(0, (64, 64, 64)), (0, (576, 832, 192)), (0, (1088, 3136, 128)),
+])
+def test_gemm_ragged_sizes_on_every_tile(K, tile_cfg, shape, layout):
+	"""Sizes that are multiples of 64 but not of the tile (the last tile moves back over its neighbour's rows or columns), down
+	to the smallest a tile takes, with fewer and more K slices than the ring holds: every epilogue, and a K split with more
+	splits than slices.  Bounds: one bf16 rounding of the fp32 sum for bf16 outputs, fp32 summation for the others."""
+	M, N, Kd = shape
+	A, B, R, bias = _randn(M, Kd, seed=31), _randn(N, Kd, seed=32, scale=0.05), _randn(M, N, seed=33), _randn(1, N, seed=34)
+	ref = A.float() @ B.float().t()
+	a, b, kw = {"nt": (A, B, {}), "nn": (A, B.t().contiguous(), dict(b_t=True)), "tn": (A.t().contiguous(), B.t().contiguous(), dict(a_t=True, b_t=True))}[layout]
+	kw["tile_cfg"] = tile_cfg
+	big = torch.full((M + 64, N + 64), 7.0, dtype=torch.bfloat16, device="cuda")  # what lies around the output stays untouched
+	K.gemm(a, b, out=big[:M, :N], **kw)
+	_close(big[:M, :N], ref, what="bf16")
+	assert (big[M:] == 7).all() and (big[:, N:] == 7).all()
+	assert torch.equal(K.gemm(a, b, **kw), big[:M, :N])
+	_close(K.gemm(a, b, epilogue=K.EPI_BF16_RESID, residual=R, **kw), ref + R.float(), what="resid")
+	_close(K.gemm(a, b, epilogue=K.EPI_BF16_RESID, residual=bias, residual_ld=0, **kw), ref + bias.float(), what="bias")
+	_close(K.gemm(a, b, epilogue=K.EPI_F32_STORE, **kw), ref, rel_fro=1e-5, rel_max=1e-5, what="f32 store")
+	before = K.gemm_turn_giveups()
+	for ks in (0, 1, 3, 20):
+		acc = torch.full((M, N), 0.25, dtype=torch.float32, device="cuda")
+		for _ in range(2):
+			K.gemm(a, b, out=acc, epilogue=K.EPI_F32_ACC, k_splits=ks, **kw)
+		_close(acc, 2 * ref + 0.25, rel_fro=1e-5, rel_max=1e-5, what=f"f32 acc ks={ks}")
+	assert K.gemm_turn_giveups() == before, "every split finds its predecessor's turn"
+
+
+def test_gemm_bits_do_not_depend_on_the_tile(K):
+	"""Every tile adds an output's products in the same order: equal bits from all of them, ragged tiles included."""
+	A, B = _randn(320, 704, seed=41), _randn(448, 704, seed=42, scale=0.05)
+	for kw, a, b in (({}, A, B), (dict(b_t=True), A, B.t().contiguous())):
+		want = K.gemm(a, b, tile_cfg=7, **kw)
+		for cfg in (8, 9, 10, 11, 12):
+			assert torch.equal(K.gemm(a, b, tile_cfg=cfg, **kw), want), f"tile config {cfg} {kw}"
+
+
+@pytest.mark.parametrize("dims", [(4160, 5504, 128), (2880, 2880, 64), (320, 320, 128)])
+def test_fused_epilogues_at_ragged_sizes_equal_the_separate_passes(K, dims):
+	"""SwiGLU forward and backward and the rotary embedding in the GEMM epilogue on tiles that move back at the matrix's
+	edges (and at sizes where the separate passes are taken): the bits of the GEMM followed by the pass."""
+	T, F, Kd = dims
+	S, D = 64, 64
+	a, w, w2 = _randn(T, Kd, seed=51), _randn(2 * F, Kd, seed=52, scale=0.05), _randn(Kd, F, seed=53, scale=0.05)
+	gu, act = K.gemm_act(a, w, K.ACT_SWIGLU)
+	assert torch.equal(gu, K.gemm(a, w)) and torch.equal(act, K.swiglu_fwd(gu))
+	dy = _randn(T, Kd, seed=54)
+	assert torch.equal(K.gemm_swiglu_bwd(dy, w2, gu), K.gemm_swiglu_bwd(dy, w2, gu, fused=False))
+	cs = K.rope_table(S, D, 1e4)
+	n_rot = F // D - 1
+	assert torch.equal(K.gemm_rope(a, w[:F], cs, S, n_rot, D), K.gemm_rope(a, w[:F], cs, S, n_rot, D, fused=False))
+
+
 def test_gemm_strided_views(K):
 	# operands that are column slices of wider buffers (leading dimension > row length)
 	big = _randn(512, 1024, seed=6)

@@ -87,6 +87,38 @@ def test_fbw_matches_oracle(kind):
 
 
 @pytest.mark.parametrize("kind", ["gpt", "llama"])
+def test_widths_that_no_tile_divides_match_oracle(kind):
+	"""Widths and FFN sizes that are multiples of 64 only: the grouped weight gradients (with the gradient scale folded into
+	the last one) and every other product run on tiles that move back at the edges."""
+	from elf_amd import models
+
+	mb = 2
+	stage = models.gpt_stage(1, 320, 5, 832, 128, seed=6) if kind == "gpt" else models.llama_stage(1, 576, 3, 1, 1088, 128, head_dim=128, seed=6)
+	perturb_norms(stage)
+	R, cfg, ref = _oracle(stage, mb)
+	blk = _block(stage, mb)
+	xs, dys = R.make_boundary(cfg, 2, seed=12)
+	blk.set_boundary(inputs=[x.cuda() for x in xs], grads=[d.cuda() for d in dys], keep_sent=True)
+	for m in range(2):
+		blk.recv_forward(m, mb, src=0)
+		blk.forward(m)
+		blk.send_forward(m, dst=2)
+		assert_close(blk.sent_forward[m], ref.forward(m, xs[m]), f"{kind} y[{m}]")
+		blk.recv_backward(m, mb, src=2)
+		blk.backward_inputs(m)
+		blk.send_backward(m, dst=0)
+		assert_close(blk.sent_backward[m], ref.backward_inputs(m, dys[m]), f"{kind} dx[{m}]")
+		blk.backward_params(m, **({"final_scale": 0.25} if m else {}))
+		ref.backward_params(m)
+	blk.scale_grads(4)
+	ref.scale_grads(4)
+	got, got16, want = product_grads(stage), product_grads(stage, "grad"), ref.grads()
+	for name in sorted(want):
+		assert_close(got[name], want[name], f"{kind} grad {name}")
+		assert torch.equal(got16[name], got[name].to(torch.bfloat16)), name
+
+
+@pytest.mark.parametrize("kind", ["gpt", "llama"])
 def test_short_micro_batches_share_a_stage(kind):
 	"""Micro-batches of 3, 1 and 2 sequences on a stage sized for 3 (an uneven split of the batch,
 	elf/pipeline.py:497-503): each against the oracle, with a recompute of the 1-sequence one, an offload
