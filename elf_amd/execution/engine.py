@@ -35,6 +35,15 @@ def _fake_p2p(data):
 	return [None, data.detach()]
 
 
+def _timed(block, name):
+	"""A timer of ``block`` (kept in its ``compute_time``), or nothing while a step runs that no timer is read of."""
+	if not getattr(block, "times_ops", True):
+		return contextlib.nullcontext()
+	timer = Timer(name=name)
+	block.compute_time.append(timer)
+	return timer
+
+
 def _capturing():
 	return _GPU() and torch.cuda.is_current_stream_capturing()
 
@@ -45,7 +54,12 @@ def _sync():
 
 
 def _mem():
-	return (torch.cuda.memory_allocated(), torch.cuda.max_memory_allocated()) if _GPU() else (0, 0)
+	"""(allocated, peak) bytes of the current device, from one query of the allocator: ``memory_allocated`` and
+	``max_memory_allocated`` flatten and sort its whole statistics tree per call, 190 us an operation for the two."""
+	if not _GPU():
+		return 0, 0
+	st = torch.cuda.memory_stats_as_nested_dict().get("allocated_bytes", {}).get("all", {})
+	return st.get("current", 0), st.get("peak", 0)
 
 
 def preallocate_pool(blocks):
@@ -102,6 +116,16 @@ class Engine:
 		with ELF_TIMINGS), ``detailed_stats`` = {"all_events": {timer name: s}, "memories":
 		{str(op): bytes allocated after it}, "peak_memory": {str(op): peak bytes}}; with a
 		HipStageBlock the byte counts include the library's own stash."""
+		# the blocks' timers are read below with ELF_TIMINGS only: without it their events (two per op) are not recorded
+		for b in self.blocks:
+			b.times_ops = bool(precise_timings)
+		try:
+			return self._train_step(batch, target, loss_fn, schedule, mb_sizes, profile)
+		finally:
+			for b in self.blocks:
+				b.times_ops = True
+
+	def _train_step(self, batch, target, loss_fn, schedule, mb_sizes, profile):
 		if batch is not None:
 			microbatches = iter(zip(*[t.split(mb_sizes, dim=0) for t in batch]))
 		if target is not None:
@@ -141,14 +165,15 @@ class Engine:
 		warmup_time = None
 		memories, peak_memories = OrderedDict(), OrderedDict()
 		T = OperationType
+		on_gpu = _GPU()
 
 		for op_index, op in enumerate(schedule):
 			block = self.id_to_block.get(op.block_id)
 			if block is None:
 				continue
-			if profile and _GPU():
+			if profile and on_gpu:
 				torch.cuda.nvtx.range_push(f"{block}:{op}")
-			if precise_memory and _GPU():
+			if precise_memory and on_gpu:
 				torch.cuda.reset_peak_memory_stats()
 				if hasattr(block, "reset_peak"):
 					block.reset_peak()
@@ -205,9 +230,8 @@ class Engine:
 					logger.warning(f"Tried to compute loss backward on a non-last block {block}")
 					continue
 				assert op.mb_id < len(losses), f"Loss backward for mb {op.mb_id} but only {len(losses)} losses computed"
-				with Timer(name=f"backward({block.id}:{op.mb_id})") as timer:
+				with _timed(block, f"backward({block.id}:{op.mb_id})"):
 					grads = grad_fns.popleft()()
-				block.compute_time.append(timer)
 				if self.offload_stream is not None and not _capturing():  # a captured step keeps its outputs on the GPU
 					self.offload_stream.wait_stream(torch.cuda.current_stream())
 					with torch.cuda.stream(self.offload_stream), torch.no_grad():
@@ -229,13 +253,14 @@ class Engine:
 
 			if precise_memory:
 				_sync()
-			alloc, peak = _mem()
+			alloc, peak = _mem() if on_gpu else (0, 0)
 			if hasattr(block, "mem_stats"):
 				st = block.mem_stats()
 				alloc, peak = alloc + st["live_bytes"], peak + st["peak_bytes"]
-			memories[str(op)] = alloc
-			peak_memories[str(op)] = peak
-			if profile and _GPU():
+			op_name = str(op)
+			memories[op_name] = alloc
+			peak_memories[op_name] = peak
+			if profile and on_gpu:
 				torch.cuda.nvtx.range_pop()
 
 		if precise_timings:
@@ -341,17 +366,15 @@ def compute_loss(block, output, target, loss_fn):
 	fused = getattr(loss_fn, "loss_and_grad", None)
 	if fused is not None:
 		# loss and gradient from one kernel (elf_amd.losses): nothing for autograd to record
-		with Timer(name="loss_forward") as timer:
+		with _timed(block, "loss_forward"):
 			loss, grad = fused(output.detach(), target, reduction="sum", scale=1.0 / elems)
-		block.compute_time.append(timer)
 		return (loss / elems).detach(), lambda: (grad,)
 	output = output.detach().requires_grad_()
-	with Timer(name="loss_forward") as timer:
+	with _timed(block, "loss_forward"):
 		try:
 			loss = loss_fn(output, target, reduction="sum")
 		except TypeError:
 			loss = loss_fn(output, target)
-	block.compute_time.append(timer)
 	loss = loss / elems
 
 	def grad_fn():

@@ -15,8 +15,7 @@ EPI_BF16, EPI_BF16_RESID, EPI_F32_ACC, EPI_F32_STORE = 0, 1, 2, 3
 NORM_RMS, NORM_LAYER = 0, 1
 
 
-def _stream():
-	return torch.cuda.current_stream().cuda_stream
+_stream = _lib.raw_stream
 
 
 def _ptr(t):

@@ -14,8 +14,7 @@ from . import _lib
 _PAD = 64  # gradient rows are padded to this many columns, the layout the stage's head GEMM reads
 
 
-def _stream():
-	return torch.cuda.current_stream().cuda_stream
+_stream = _lib.raw_stream
 
 
 def _rows_view(pred, V):
