@@ -49,7 +49,40 @@ struct AttnBwdArgs {
 	// non-null: the q and k heads carry a rotary embedding whose backward (the inverse rotation) is applied to
 	// dQ and dK before they are stored; (cos, sin) table [S, D / 2] of rope_table()
 	const float2* rope_cs;
+	// A pass's walk (query heads of the group x query tiles) shared by h_splits x q_splits workgroups, each of which leaves its
+	// dK and dV as fp32 partial sums in dkv_part ([split][dK, dV][token][Hkv * D]) for the reduction kernel; 1 x 1: they are
+	// stored as they are.  See split_walk().
+	int h_splits, q_splits;
+	float* dkv_part;
 };
+
+// The walk of one workgroup: query heads [h0, h0 + nh) and, per head, query tiles [q_lo, q_hi) of a pass.
+struct Walk {
+	int pair, b, hk, split, h0, nh;
+	__device__ __forceinline__ void tiles(const AttnBwdArgs& a, int qt_first, int nqt, int& q_lo, int& q_hi) const {
+		const int qs = split % a.q_splits, len = nqt - qt_first;
+		q_lo = qt_first + len * qs / a.q_splits;
+		q_hi = qt_first + len * (qs + 1) / a.q_splits;
+	}
+};
+__device__ __forceinline__ Walk locate_walk(const AttnBwdArgs& a, int npair) {
+	const int ns = a.h_splits * a.q_splits, per_group = npair * ns;
+	int rest = blockIdx.x % per_group, bh = blockIdx.x / per_group;
+	// all workgroups of a (batch, kv head) group on one XCD (workgroup w runs on XCD w % 8)
+	const int ngroups = (int)(gridDim.x / per_group);
+	if (ngroups % 8 == 0) {
+		const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+		bh = xcd + 8 * (slot / per_group);
+		rest = slot % per_group;
+	}
+	Walk w;
+	w.split = rest % ns;
+	w.pair = rest / ns;
+	w.hk = bh % a.Hkv, w.b = bh / a.Hkv;
+	w.nh = a.Hq / a.Hkv / a.h_splits;
+	w.h0 = w.hk * (a.Hq / a.Hkv) + (w.split / a.q_splits) * w.nh;
+	return w;
+}
 
 // dQ partials.  Every 128-key tile contributes a [queries, Hq*D] partial dQ; the partials are written
 // with plain stores, each by exactly one workgroup, rounded to bf16 (like the P and dS operands of the
@@ -174,6 +207,22 @@ __device__ __forceinline__ void store_dk_dv(const f32x16 (&acc_dk)[D / 32], cons
 	}
 }
 
+// The same accumulators as fp32 partial sums: dK at p, dV `stride` floats further on.
+template <int D>
+__device__ __forceinline__ void store_dkv_part(const f32x16 (&acc_dk)[D / 32], const f32x16 (&acc_dv)[D / 32], float* p, int64_t stride, int g) {
+#pragma unroll
+	for (int dt = 0; dt < D / 32; dt++) {
+#pragma unroll
+		for (int r4 = 0; r4 < 4; r4++) {
+			f32x4 k4, v4;
+#pragma unroll
+			for (int u = 0; u < 4; u++) k4[u] = acc_dk[dt][r4 * 4 + u], v4[u] = acc_dv[dt][r4 * 4 + u];
+			*reinterpret_cast<f32x4*>(p + dt * 32 + r4 * 8 + 4 * g) = k4;
+			*reinterpret_cast<f32x4*>(p + stride + dt * 32 + r4 * 8 + 4 * g) = v4;
+		}
+	}
+}
+
 // One workgroup pass = 128 keys of one (batch, kv head); wave w owns keys [32w, 32w+32) and
 // keeps their K / V rows (MFMA B operands) and dK^T / dV^T accumulators in registers while the
 // workgroup walks over the 32-query tiles of every query head of the group.  Q and dO tiles
@@ -208,19 +257,8 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kernel(AttnBwdA
 	const int g = lane >> 5, kl = lane & 31;
 	const int nkt = a.S / BKV;
 	const int npair = CAUSAL ? (nkt + 1) / 2 : nkt;
-	int pair = blockIdx.x % npair;
-	int bh = blockIdx.x / npair;
-	{
-		// all key-tile workgroups of a (batch, kv head) group on one XCD (workgroup w runs on XCD w % 8)
-		const int ngroups = (int)(gridDim.x / npair);
-		if (ngroups % 8 == 0) {
-			const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-			bh = xcd + 8 * (slot / npair);
-			pair = slot % npair;
-		}
-	}
-	const int hk = bh % a.Hkv, b = bh / a.Hkv;
-	const int G = a.Hq / a.Hkv;
+	const Walk wk = locate_walk(a, npair);
+	const int pair = wk.pair, hk = wk.hk, b = wk.b;
 	const int64_t tok0 = (int64_t)b * a.S;
 	const int64_t HqD = (int64_t)a.Hq * D;
 	const float sc = a.scale * LOG2E;
@@ -298,10 +336,12 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kernel(AttnBwdA
 
 		// Walk over (query head in group, query tile); causal: only tiles that reach key0.
 		const int qt_first = CAUSAL ? key0 / BQ : 0;
-		const int n_iter = G * (nqt_all - qt_first);
+		int q_lo, q_hi;
+		wk.tiles(a, qt_first, nqt_all, q_lo, q_hi);
+		const int n_iter = wk.nh * (q_hi - q_lo);  // at least one: a pass has four query tiles or more, q_splits is at most four
 
 		// tile whose loads are issued next: running pointers, recomputed when the walk moves to the next head
-		int ld_h = hk * G, ld_qt = qt_first;
+		int ld_h = wk.h0, ld_qt = q_lo;
 		const bf16_t* ld_q;
 		const bf16_t* ld_do;
 		const float* ld_stat;  // lanes 0..31: nlse2 of the tile's queries, lanes 32..63: delta
@@ -321,8 +361,8 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kernel(AttnBwdA
 				dma16(ld_do, dooff[i], __builtin_amdgcn_readfirstlane(st + Q_BYTES + i * TL::RPI * TL::ROW_BYTES));
 			}
 			if (wave == 0) dma4(ld_stat, __builtin_amdgcn_readfirstlane(st + 2 * Q_BYTES));
-			if (++ld_qt == nqt_all) {
-				ld_qt = qt_first;
+			if (++ld_qt == q_hi) {
+				ld_qt = q_lo;
 				ld_h++;
 				seek();
 			} else {
@@ -342,10 +382,10 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kernel(AttnBwdA
 		for (int i = 0; i < NQ; i++) ktf[i] = TL::template cols<false>(sKt, i * 16, dq_dt * 32, lane);
 
 		// position of the current tile; dq_prev_tile = where the dQ tile of iteration it-1 goes
-		int cur_h = hk * G, cur_qt = qt_first;
+		int cur_h = wk.h0, cur_qt = q_lo;
 		// rows of this key tile's slice: first query of the slice = key0 (causal) or 0
 		bf16_t* const part = a.dq_part + ((int64_t)b * part_rows(a.S, CAUSAL) + part_row0(kt_idx, a.S, CAUSAL) - qt_first * BQ) * HqD;
-		bf16_t* dq_prev_tile = part + (int64_t)(qt_first * BQ) * HqD + cur_h * D;
+		bf16_t* dq_prev_tile = part + (int64_t)(q_lo * BQ) * HqD + cur_h * D;
 
 		for (int it = 0; it < n_iter; it++) {
 			if (it + 1 < n_iter) issue((it + 1) & 1);
@@ -448,8 +488,8 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kernel(AttnBwdA
 				acc_dk[i % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bC[i], dsf[i / DT], acc_dk[i % DT], 0, 0, 0);
 			dq_out(dq_prev_tile, dq, 12, 16);
 			dq_prev_tile = part + (int64_t)q0 * HqD + cur_h * D;
-			if (++cur_qt == nqt_all) {
-				cur_qt = qt_first;
+			if (++cur_qt == q_hi) {
+				cur_qt = q_lo;
 				cur_h++;
 			}
 			// the next tile's loads were issued before this step's 4 partial stores and vector memory
@@ -471,6 +511,10 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kernel(AttnBwdA
 		}
 
 		// dK^T / dV^T accumulators: register r <-> d = dt*32 + (r/4)*8 + 4g + r%4, lane <-> key
+		if (a.dkv_part) {
+			store_dkv_part<D>(acc_dk, acc_dv, a.dkv_part + (((int64_t)wk.split * 2 * a.B * a.S + tok0 + wkey0 + kl) * a.Hkv + hk) * D, (int64_t)a.B * a.S * a.Hkv * D, g);
+			continue;
+		}
 		bf16_t* dkp = a.dk + (tok0 + wkey0 + kl) * a.lddk + hk * D;
 		bf16_t* dvp = a.dv + (tok0 + wkey0 + kl) * a.lddv + hk * D;
 		store_dk_dv<D>(acc_dk, acc_dv, dkp, dvp, a.scale, g, a.rope_cs ? a.rope_cs + (int64_t)(wkey0 + kl) * (D / 2) : nullptr);
@@ -505,19 +549,8 @@ __global__ __launch_bounds__(256) void attn_bwd_kernel_lone(AttnBwdArgs a) {
 	const int g = lane >> 5, kl = lane & 31;
 	const int nkt = a.S / BKV;
 	const int npair = CAUSAL ? (nkt + 1) / 2 : nkt;
-	int pair = blockIdx.x % npair;
-	int bh = blockIdx.x / npair;
-	{
-		// all key-tile workgroups of a (batch, kv head) group on one XCD (workgroup w runs on XCD w % 8)
-		const int ngroups = (int)(gridDim.x / npair);
-		if (ngroups % 8 == 0) {
-			const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-			bh = xcd + 8 * (slot / npair);
-			pair = slot % npair;
-		}
-	}
-	const int hk = bh % a.Hkv, b = bh / a.Hkv;
-	const int G = a.Hq / a.Hkv;
+	const Walk wk = locate_walk(a, npair);
+	const int pair = wk.pair, hk = wk.hk, b = wk.b;
 	const int64_t tok0 = (int64_t)b * a.S;
 	const int64_t HqD = (int64_t)a.Hq * D;
 	const float sc = a.scale * LOG2E;
@@ -591,10 +624,12 @@ __global__ __launch_bounds__(256) void attn_bwd_kernel_lone(AttnBwdArgs a) {
 
 		// Walk over (query head in group, query tile); causal: only tiles that reach key0.
 		const int qt_first = CAUSAL ? key0 / BQ : 0;
-		const int n_iter = G * (nqt_all - qt_first);
+		int q_lo, q_hi;
+		wk.tiles(a, qt_first, nqt_all, q_lo, q_hi);
+		const int n_iter = wk.nh * (q_hi - q_lo);  // at least one: a pass has four query tiles or more, q_splits is at most four
 
 		// tile whose loads are issued next: running pointers, recomputed when the walk moves to the next head
-		int ld_h = hk * G, ld_qt = qt_first;
+		int ld_h = wk.h0, ld_qt = q_lo;
 		const bf16_t* ld_q;
 		const bf16_t* ld_do;
 		const float* ld_stat;  // lanes 0..31: nlse2 of the tile's queries, lanes 32..63: delta
@@ -614,8 +649,8 @@ __global__ __launch_bounds__(256) void attn_bwd_kernel_lone(AttnBwdArgs a) {
 				dma16(ld_do, dooff[i], __builtin_amdgcn_readfirstlane(st + Q_BYTES + i * TL::RPI * TL::ROW_BYTES));
 			}
 			if (wave == 0) dma4(ld_stat, __builtin_amdgcn_readfirstlane(st + 2 * Q_BYTES));
-			if (++ld_qt == nqt_all) {
-				ld_qt = qt_first;
+			if (++ld_qt == q_hi) {
+				ld_qt = q_lo;
 				ld_h++;
 				seek();
 			} else {
@@ -636,10 +671,10 @@ __global__ __launch_bounds__(256) void attn_bwd_kernel_lone(AttnBwdArgs a) {
 		for (int i = 0; i < NQ; i++) ktf[i] = TL::template cols<false>(sKt, i * 16, dq_dt * 32, lane);
 
 		// position of the current tile; dq_prev_tile = where the dQ tile of iteration it-1 goes
-		int cur_h = hk * G, cur_qt = qt_first;
+		int cur_h = wk.h0, cur_qt = q_lo;
 		// rows of this key tile's slice: first query of the slice = key0 (causal) or 0
 		bf16_t* const part = a.dq_part + ((int64_t)b * part_rows(a.S, CAUSAL) + part_row0(kt_idx, a.S, CAUSAL) - qt_first * BQ) * HqD;
-		bf16_t* dq_prev_tile = part + (int64_t)(qt_first * BQ) * HqD + cur_h * D;
+		bf16_t* dq_prev_tile = part + (int64_t)(q_lo * BQ) * HqD + cur_h * D;
 
 		// One step = one (head, 32-query tile).  Two fragment buffers alternate roles so that every LDS
 		// read is issued one product ahead of the MFMAs that consume it (one wave per SIMD: nothing else
@@ -753,8 +788,8 @@ __global__ __launch_bounds__(256) void attn_bwd_kernel_lone(AttnBwdArgs a) {
 				__builtin_amdgcn_sched_barrier(0);
 			}
 			dq_prev_tile = part + (int64_t)q0 * HqD + cur_h * D;
-			if (++cur_qt == nqt_all) {
-				cur_qt = qt_first;
+			if (++cur_qt == q_hi) {
+				cur_qt = q_lo;
 				cur_h++;
 			}
 			// the loads of the tile after next were issued before this step's 4 partial stores and vector
@@ -784,6 +819,10 @@ __global__ __launch_bounds__(256) void attn_bwd_kernel_lone(AttnBwdArgs a) {
 		}
 
 		// dK^T / dV^T accumulators: register r <-> d = dt*32 + (r/4)*8 + 4g + r%4, lane <-> key
+		if (a.dkv_part) {
+			store_dkv_part<D>(acc_dk, acc_dv, a.dkv_part + (((int64_t)wk.split * 2 * a.B * a.S + tok0 + wkey0 + kl) * a.Hkv + hk) * D, (int64_t)a.B * a.S * a.Hkv * D, g);
+			continue;
+		}
 		bf16_t* dkp = a.dk + (tok0 + wkey0 + kl) * a.lddk + hk * D;
 		bf16_t* dvp = a.dv + (tok0 + wkey0 + kl) * a.lddv + hk * D;
 		store_dk_dv<D>(acc_dk, acc_dv, dkp, dvp, a.scale, g, a.rope_cs ? a.rope_cs + (int64_t)(wkey0 + kl) * (D / 2) : nullptr);
@@ -795,14 +834,60 @@ __global__ __launch_bounds__(256) void attn_bwd_kernel_lone(AttnBwdArgs a) {
 // half a head further on; with a rotary embedding on the q heads (cs non-null) these are the pairs of the
 // rotation, which is undone on the scaled, bf16-rounded sums before they are stored (what a separate RoPE
 // pass over the stored gradient would compute).
+//
+// dkv.splits > 1: the launch's last dkv.blocks workgroups add the fp32 partial sums of dK and dV in ascending split order,
+// 8 + 8 columns per thread, scale (dK), round, undo the rotation (dK) and store them.
+struct DkvReduce {
+	const float* part;
+	bf16_t *dk, *dv;
+	int64_t lddk, lddv;
+	int splits, Hkv, blocks;
+};
 __global__ __launch_bounds__(256) void dq_reduce_kernel(const bf16_t* __restrict__ part, bf16_t* __restrict__ dq, int B, int S, int cols,
-                                                        int64_t ld, float scale, int causal, int D, const float2* __restrict__ cs) {
+                                                        int64_t ld, float scale, int causal, int D, const float2* __restrict__ cs, DkvReduce dkv) {
+	const int dq_blocks = (int)gridDim.x - dkv.blocks;
+	if ((int)blockIdx.x >= dq_blocks) {
+		const int half = D / 2, cph = half / 8, ppr = dkv.Hkv * cph;  // chunk pairs per row
+		const int64_t n = (int64_t)B * S * ppr, stride = (int64_t)B * S * dkv.Hkv * D;
+		for (int64_t i = ((int64_t)blockIdx.x - dq_blocks) * 256 + threadIdx.x; i < 2 * n; i += (int64_t)dkv.blocks * 256) {
+			const bool is_v = i >= n;
+			const int64_t k = is_v ? i - n : i, row = k / ppr;
+			const int pr = (int)(k - row * ppr), c = (pr / cph) * D + (pr % cph) * 8;
+			const float* p = dkv.part + (is_v ? stride : 0) + row * dkv.Hkv * D + c;
+			f32x4 s[4] = {};
+			for (int t = 0; t < dkv.splits; t++, p += 2 * stride) {
+#pragma unroll
+				for (int u = 0; u < 4; u++) s[u] += __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p + (u >> 1) * half + (u & 1) * 4));
+			}
+			const float f = is_v ? 1.f : scale;
+			bf16x8 lo, hi;
+#pragma unroll
+			for (int t = 0; t < 8; t++) {
+				lo[t] = (bf16_t)(s[t >> 2][t & 3] * f);
+				hi[t] = (bf16_t)(s[2 + (t >> 2)][t & 3] * f);
+			}
+			if (cs && !is_v) {
+				const float2* tab = cs + (row % S) * half + (pr % cph) * 8;
+#pragma unroll
+				for (int t = 0; t < 8; t++) {
+					float rl, rh;
+					rope_rot((float)lo[t], (float)hi[t], tab[t].x, -tab[t].y, rl, rh);
+					lo[t] = (bf16_t)rl;
+					hi[t] = (bf16_t)rh;
+				}
+			}
+			bf16_t* out = (is_v ? dkv.dv + row * dkv.lddv : dkv.dk + row * dkv.lddk) + c;
+			*reinterpret_cast<bf16x8*>(out) = lo;
+			*reinterpret_cast<bf16x8*>(out + half) = hi;
+		}
+		return;
+	}
 	const int half = D / 2, cph = half / 8;  // 8-column chunks per half head
 	const int ppr = cols / 16;               // chunk pairs per row
 	const int64_t n = (int64_t)B * S * ppr;
 	const int nkt = S / 128;
 	const int64_t rows_b = part_rows(S, causal);
-	for (int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; j < n; j += (int64_t)gridDim.x * blockDim.x) {
+	for (int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; j < n; j += (int64_t)dq_blocks * blockDim.x) {
 		// last rows first: under a causal mask they sum the most partials, and the launch then ends on the short ones
 		const int64_t i = n - 1 - j;
 		const int64_t row = i / ppr;
@@ -865,9 +950,49 @@ int launch_bwd(const AttnBwdArgs& a, dim3 grid, hipStream_t stream) {
 
 using namespace attn;
 
+// How the walks of a launch are shared out.  A workgroup's walk over the query heads of its group and their query tiles is
+// serial (one 32-query tile per step), and B * Hkv * (key tile pairs) walks leave the chip idle where there are few of them:
+// then the heads of a group and, after those, the query tiles are split, as long as the estimate gets smaller.  Steps and the
+// fixed part of a walk (K / V rows in, first tiles in, dK / dV out) are in microseconds as measured; a split adds
+// 16 bytes per element of dK to write and to read again.  The whole call, before -> after (us): 2 x 2048 tokens, 16 / 4 heads
+// of 128 346 -> 160 (64 walks, heads split 4 ways); 3 x 896, 32 / 8 heads of 128 189 -> 134 (2 ways); 4096 tokens, 6 / 1 heads
+// of 128 886 -> 125 (6 x 2); 2 x 1024, 16 / 4 heads of 64 196 -> 59 (4 x 2).  Full launches stay whole: 2 x 4096, 32 / 8 heads
+// of 128 takes 1000 us whole and 1030 in two.
+struct Splits {
+	int h = 1, q = 1;
+};
+static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal) {
+	const int nkt = S / 128, G = Hq / Hkv;
+	const int64_t walks = (int64_t)B * Hkv * (causal ? (nkt + 1) / 2 : nkt);
+	const int tiles = causal ? (nkt + 1) * 4 : nkt * 4;  // query tiles of a walk and head (a pair of key tiles has nkt + 1 of four)
+	const float slots = D == 128 ? 256.f : 512.f, step = D == 128 ? 1.2f : 1.1f, fixed = 8.f;
+	Splits best;
+	float best_us = 1e30f;
+	for (int h = 1; h <= G; h++) {
+		if (G % h) continue;
+		for (int q = 1; q <= 4; q *= 2) {
+			if (q > 1 && h < G) continue;
+			const int ns = h * q;
+			const float rounds = ceilf((float)(walks * ns) / slots);
+			const float us = rounds * (fixed + (float)(G / h) * ((tiles + q - 1) / q) * step) + (ns > 1 ? 2.f + (float)ns * B * S * Hkv * D * 16 / 5e6f : 0.f);
+			if (us < best_us * (ns > 1 ? 0.95f : 1.f)) best_us = us, best = Splits{h, q};
+		}
+	}
+	return best;
+}
+static int64_t dkv_part_bytes(const Splits& sp, int B, int S, int Hkv, int D) { return sp.h * sp.q > 1 ? (int64_t)sp.h * sp.q * 2 * B * S * Hkv * D * 4 : 0; }
+
 int64_t attn_bwd_workspace_bytes(int B, int S, int Hq, int D, int causal) {
-	// bf16 dQ partials of every key tile + delta + scaled log-sum-exp
-	return (int64_t)B * part_rows(S, causal != 0) * Hq * D * 2 + 2 * (int64_t)B * S * Hq * 4;
+	// bf16 dQ partials of every key tile + delta + scaled log-sum-exp + the largest set of dK / dV partials that any number of
+	// kv heads and any smaller batch asks for (few walks are split the more: it is 150 MB at most)
+	int64_t dkv = 0;
+	for (int b = 1; b <= B; b++)
+		for (int hkv = 1; hkv <= Hq; hkv++)
+			if (Hq % hkv == 0) {
+				const int64_t n = dkv_part_bytes(split_walk(b, S, Hq, hkv, D, causal != 0), b, S, hkv, D);
+				if (n > dkv) dkv = n;
+			}
+	return (int64_t)B * part_rows(S, causal != 0) * Hq * D * 2 + 2 * (int64_t)B * S * Hq * 4 + dkv;
 }
 
 int attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* dO, const void* lse, void* dq,
@@ -895,18 +1020,25 @@ int attn_bwd(const void* q, const void* k, const void* v, const void* o, const v
 		ELF_LAUNCH(attn_delta_kernel, dim3((unsigned)(want < 8192 ? want : 8192)), dim3(256), 0, stream, (const bf16_t*)dO,
 	                   (const bf16_t*)o, (const float*)lse, delta, nlse2, lddo, ldo, B, S, Hq, D);
 	}
+	const Splits sp = split_walk(B, S, Hq, Hkv, D, causal != 0);
+	float* dkv_part = sp.h * sp.q > 1 ? nlse2 + T * Hq : nullptr;
 	AttnBwdArgs a{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)dO, nlse2, delta, dq_part,
-	              (bf16_t*)dk, (bf16_t*)dv, ldq, ldk, ldv, lddo, lddk, lddv, B, S, Hq, Hkv, scale, (const float2*)rope_cs};
+	              (bf16_t*)dk, (bf16_t*)dv, ldq, ldk, ldv, lddo, lddk, lddv, B, S, Hq, Hkv, scale, (const float2*)rope_cs, sp.h, sp.q, dkv_part};
 	const int nkt = S / 128;
-	const dim3 grid((unsigned)((int64_t)B * Hkv * (causal ? (nkt + 1) / 2 : nkt))), block(256);
+	const dim3 grid((unsigned)((int64_t)B * Hkv * (causal ? (nkt + 1) / 2 : nkt) * sp.h * sp.q)), block(256);
 	int rc;
 	if (D == 128) rc = causal ? launch_bwd<128, true>(a, grid, stream) : launch_bwd<128, false>(a, grid, stream);
 	else rc = causal ? launch_bwd<64, true>(a, grid, stream) : launch_bwd<64, false>(a, grid, stream);
 	if (rc) return rc;
 	const int64_t n16 = T * (Hq * D / 16);
 	const int64_t blocks = (n16 + 255) / 256;
-	ELF_LAUNCH(dq_reduce_kernel, dim3((unsigned)(blocks < 16384 ? blocks : 16384)), dim3(256), 0, stream, dq_part, (bf16_t*)dq, B, S,
-	                   Hq * D, lddq, scale, causal, D, (const float2*)rope_cs);
+	DkvReduce dkv{dkv_part, (bf16_t*)dk, (bf16_t*)dv, lddk, lddv, sp.h * sp.q, Hkv, 0};
+	if (dkv_part) {
+		const int64_t want = (2 * T * Hkv * (D / 16) + 255) / 256;
+		dkv.blocks = (int)(want < 4096 ? want : 4096);
+	}
+	ELF_LAUNCH(dq_reduce_kernel, dim3((unsigned)(blocks < 16384 ? blocks : 16384) + dkv.blocks), dim3(256), 0, stream, dq_part, (bf16_t*)dq, B, S,
+	                   Hq * D, lddq, scale, causal, D, (const float2*)rope_cs, dkv);
 	ELF_CHECK_HIP(hipGetLastError());
 	return 0;
 }

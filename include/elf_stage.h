@@ -199,7 +199,9 @@ int elf_cross_entropy_reduce(const void* row_loss, const void* target, int64_t r
  * elf_attn_bwd_workspace_bytes() of 16-byte aligned scratch (the bf16 partial dQ of every 128-key tile,
  * which a second kernel sums in fp32 in a fixed order — no atomics, run-to-run identical gradients —
  * plus two fp32 values per query and head): B * S * (S/128 + 1) / 2 * Hq * D * 2 bytes with a causal
- * mask, B * S * (S/128) * Hq * D * 2 without, + 8 * B * S * Hq. */
+ * mask, B * S * (S/128) * Hq * D * 2 without, + 8 * B * S * Hq, and where a batch or a group of kv heads is too small to
+ * fill the chip, fp32 partial sums of dK and dV (about 150 MB at most; they too are added in a fixed order).  The size
+ * covers every Hkv that divides Hq and every smaller batch. */
 int elf_attn_fwd(const void* q, const void* k, const void* v, void* o, void* lse, int64_t ldq,
                  int64_t ldk, int64_t ldv, int64_t ldo, int B, int S, int Hq, int Hkv, int D,
                  int causal, float scale, void* stream);

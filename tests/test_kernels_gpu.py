@@ -460,6 +460,30 @@ def test_attention_fwd_bwd(K, cfg):
 	assert torch.equal(fused, K.rope_apply_(dqkv.clone(), cs, S, Hq + Hkv, D, backward=True))
 
 
+@pytest.mark.parametrize("cfg", [(1, 2176, 6, 1, 128, True), (1, 896, 6, 2, 128, False), (1, 1664, 12, 4, 64, True), (3, 640, 5, 5, 64, False), (2, 384, 16, 16, 128, True)])
+def test_attention_backward_with_walks_shared_by_workgroups(K, cfg):
+	"""Few key tiles and kv heads: the query heads of a group and the query tiles of a pass (in two and four parts that the
+	tile count does not divide evenly) go to different workgroups, whose dK and dV meet as fp32 partial sums.  Against fp32
+	autograd, equal bits from run to run, the rotation undone as by a pass of its own, and a workspace sized for a batch that
+	also holds every smaller one."""
+	from elf_amd import _lib
+
+	B, S, Hq, Hkv, D, causal = cfg
+	T = B * S
+	qkv, do = _randn(T, (Hq + 2 * Hkv) * D, seed=55), _randn(T, Hq * D, seed=56)
+	o_ref, _, dqkv_ref = _attn_ref(qkv, B, S, Hq, Hkv, D, causal, do)
+	o, lse = K.attn_fwd(qkv, B, S, Hq, Hkv, D, causal)
+	dqkv = K.attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal)
+	for name, sl in (("dq", slice(0, Hq * D)), ("dk", slice(Hq * D, (Hq + Hkv) * D)), ("dv", slice((Hq + Hkv) * D, None))):
+		_close(dqkv[:, sl], dqkv_ref[:, sl], rel_fro=1.5e-2, what=f"attn {name} {cfg}")
+	assert torch.equal(dqkv, K.attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal))
+	cs = K.rope_table(S, D, 5e5)
+	fused = K.attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal, rope_cs=cs)
+	assert torch.equal(fused, K.rope_apply_(dqkv.clone(), cs, S, Hq + Hkv, D, backward=True))
+	sizes = [_lib.load().elf_attn_bwd_workspace_bytes(b, S, Hq, D, int(causal)) for b in range(1, 9)]
+	assert sizes == sorted(sizes)
+
+
 @pytest.mark.parametrize("D,causal,ramp,gain", [(128, True, 6.0, 1.0), (128, False, 6.0, 1.0), (64, True, 6.0, 1.0), (128, True, 0.0, 6.0),
                                                (128, False, -6.0, 3.0), (64, False, 0.0, 6.0)])
 def test_attention_forward_with_scores_that_climb_along_the_keys(K, D, causal, ramp, gain):
