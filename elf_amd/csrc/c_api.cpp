@@ -90,6 +90,11 @@ int elf_cross_entropy(const void* logits, int64_t ld, const void* target, int64_
                       const void* dev_div, void* row_loss, void* dlogits, int64_t ld_out, void* stream) {
 	return elf::cross_entropy(logits, ld, target, rows, V, ignore_index, scale, dev_div, row_loss, dlogits, ld_out, S_(stream));
 }
+int elf_cross_entropy_dense(const void* logits, const void* target, int64_t rows, int64_t V, int64_t ignore_index, float scale, const void* dev_div,
+                            void* row_loss, void* dlogits, void* stream) {
+	return elf::cross_entropy_dense(logits, target, rows, V, ignore_index, scale, dev_div, row_loss, dlogits, S_(stream));
+}
+int elf_scale_by_bf16(const void* x, const void* g_f32, void* y, int64_t n, void* stream) { return elf::scale_by_bf16(x, g_f32, y, n, S_(stream)); }
 int elf_cross_entropy_reduce(const void* row_loss, const void* target, int64_t rows, int64_t ignore_index, void* out2, void* stream) {
 	return elf::cross_entropy_reduce(row_loss, target, rows, ignore_index, out2, S_(stream));
 }

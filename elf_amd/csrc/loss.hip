@@ -5,9 +5,9 @@
 //     dlogits[r,c] = (softmax(x[r, :])[c] - (c == target[r])) * scale (0 for ignored rows and for
 //                    the padding columns V <= c < ld_out)
 // Forward and backward are one kernel — 4 bytes per logit of HBM traffic instead of the 10+ of a
-// log-softmax / gather / scatter chain.  Short rows (up to 16384 columns) are read once into
+// log-softmax / gather / scatter chain.  Rows of up to 131072 columns are read once into
 // registers, reduced, and their gradient written from the same registers; longer rows are read
-// twice by their workgroup, the second time out of cache.
+// twice by their workgroup.
 #include "common.h"
 #include "kernels.h"
 
@@ -62,28 +62,47 @@ __device__ __forceinline__ float row_loss_of(const LossArgs& a, int64_t row, int
 	return m + logf(s) - (float)a.x[row * a.ld + tgt];
 }
 
-// G threads per row, C 16-byte chunks (8 logits) per thread: rows of up to G * C * 8 columns.
-template <int G, int C>
-__global__ __launch_bounds__(G < 256 ? 256 : G) void cross_entropy_kernel(LossArgs a) {
+// G threads per row, C 16-byte chunks (8 logits) per thread: rows of up to G * C * 8 columns, read once into registers,
+// reduced there, and their gradient written from the same registers.  Bound: HBM (4 bytes per logit) and, close behind, the two
+// exponentials per logit.  Rows beyond 16384 columns used to be read twice by 256 threads, the second time from a cache that
+// the rows in flight on the chip (2048 of 100 KB) do not fit; loss and gradient, before -> after: 4096 x 50304 235 -> 167 us
+// (3.5 -> 4.9 TB/s), 8192 x 20000 168 -> 130, 2048 x 128256 262 -> 241.
+//
+// DENSE: rows of V columns one after the other, so that they start at any 2-byte address; x and dx lie alike modulo 16 bytes.
+// A row is walked in the aligned 16-byte chunks that cover it.  The first and the last of them, where they are shared with the
+// neighbouring rows (or with what lies behind the last column), are read and written element by element by lanes 0 and 1.
+template <int G, int C, bool DENSE>
+__global__ __launch_bounds__(G < 256 ? 256 : G, G >= 256 ? 64 / C : 1) void cross_entropy_kernel(LossArgs a) {
 	constexpr int BLOCK = G < 256 ? 256 : G;
 	constexpr int ROWS = BLOCK / G;
+	constexpr bool WIDE = G * C * 8 > 16384;
 	__shared__ float red[BLOCK / 64];
-	const int lane = threadIdx.x % G;
-	const int64_t row = (int64_t)blockIdx.x * ROWS + threadIdx.x / G;
+	const int lane = ROWS == 1 ? (int)threadIdx.x : (int)threadIdx.x % G;
+	const int64_t row = ROWS == 1 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * ROWS + threadIdx.x / G;
 	if (ROWS > 1 && row >= a.rows) return;  // whole waves leave together (G = 64 when ROWS > 1)
-	const bf16_t* xr = a.x + row * a.ld;
-	const int vchunks = (a.V + 7) / 8;
+	const int rot = DENSE ? (int)(((uintptr_t)(a.x + row * a.ld) >> 1) & 7) : 0;  // columns of chunk 0 that belong to the row before
+	const bf16_t* const xr = a.x + (row * a.ld - rot);  // chunk c holds columns c * 8 - rot .. + 7, at xr + c * 8
+	const int cbeg = rot != 0, cend = (a.V + rot) / 8;  // the chunks that lie inside the row
+	// the edge chunk of this lane, if any, and its elements inside the row
+	const int ec = lane == 0 && rot ? 0 : lane == 1 && (a.V + rot) % 8 && (cend > 0 || !rot) ? cend : -1;
+	const int elo = ec == 0 ? rot : 0, ehi = min(8, a.V + rot - ec * 8);
 
 	bf16x8 reg[C];
 	float m = -INFINITY;
 #pragma unroll
 	for (int j = 0; j < C; j++) {
 		const int c = j * G + lane;
-		if (c < vchunks) {
-			reg[j] = *reinterpret_cast<const bf16x8*>(xr + (int64_t)c * 8);
+		if (c >= cbeg && c < cend) reg[j] = *reinterpret_cast<const bf16x8*>(xr + (int64_t)c * 8);
+	}
+	if (ec >= 0) {
+		for (int i = elo; i < ehi; i++) m = fmaxf(m, (float)xr[(int64_t)ec * 8 + i]);
+	}
 #pragma unroll
-			for (int i = 0; i < 8; i++)
-				if (c * 8 + i < a.V) m = fmaxf(m, (float)reg[j][i]);
+	for (int j = 0; j < C; j++) {
+		const int c = j * G + lane;
+		if (c >= cbeg && c < cend) {
+#pragma unroll
+			for (int i = 0; i < 8; i++) m = fmaxf(m, (float)reg[j][i]);
 		}
 	}
 	m = group_reduce<G, true>(m, red);
@@ -92,47 +111,61 @@ __global__ __launch_bounds__(G < 256 ? 256 : G) void cross_entropy_kernel(LossAr
 #pragma unroll
 	for (int j = 0; j < C; j++) {
 		const int c = j * G + lane;
-		if (c < vchunks) {
+		if (c >= cbeg && c < cend) {
 #pragma unroll
-			for (int i = 0; i < 8; i++)
-				if (c * 8 + i < a.V) s += fast_exp2((float)reg[j][i] * LOG2E_F - m2);
+			for (int i = 0; i < 8; i++) s += fast_exp2(fmaf((float)reg[j][i], LOG2E_F, -m2));
 		}
+	}
+	if (ec >= 0) {
+		for (int i = elo; i < ehi; i++) s += fast_exp2(fmaf((float)xr[(int64_t)ec * 8 + i], LOG2E_F, -m2));
 	}
 	s = group_reduce<G, false>(s, red);
 
 	const int64_t tgt = a.target[row];
 	if (a.row_loss && lane == 0) a.row_loss[row] = row_loss_of(a, row, tgt, m, s);
 	if (!a.dx) return;
-	const bool live = tgt != a.ignore_index;
-	const float g = live ? grad_scale(a) : 0.f;
-	const float gs = g / s;
-	bf16_t* dr = a.dx + row * a.ld_out;
-	const int ochunks = (int)(a.ld_out / 8);
+	const float g = tgt != a.ignore_index ? grad_scale(a) : 0.f;
+	bf16_t* const dr = a.dx + (row * a.ld_out - rot);
+	const int tchunk = tgt >= 0 && tgt < a.V ? (int)((tgt + rot) >> 3) : -1, tcol = (int)((tgt + rot) & 7);
+	// softmax * |g| of the wide rows = exp2(x*log2e - (m + log2(s) - log2|g|)), its sign by an exclusive or: no product per
+	// logit; a zero factor (an ignored row) gives zeros whatever the logits are
+	const bool zero = WIDE && g == 0.f;
+	const float gs = g / s, shift = WIDE ? m2 + log2f(s) - log2f(fabsf(g)) : m2;
+	const uint32_t sign = WIDE && g < 0.f ? 0x80000000u : 0u;
+	auto softmax = [&](bf16_t x) {
+		float v = fast_exp2(fmaf((float)x, LOG2E_F, -shift));
+		if constexpr (WIDE) return zero ? 0.f : __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) ^ sign);
+		return v * gs;
+	};
 #pragma unroll
 	for (int j = 0; j < C; j++) {
 		const int c = j * G + lane;
-		if (c >= ochunks) continue;
+		if (c < cbeg || c >= cend) continue;
+		float v[8];
+#pragma unroll
+		for (int i = 0; i < 8; i++) v[i] = softmax(reg[j][i]);
+		if (c == tchunk) {
+#pragma unroll
+			for (int i = 0; i < 8; i++)
+				if (i == tcol) v[i] -= g;
+		}
 		bf16x8 o;
 #pragma unroll
-		for (int i = 0; i < 8; i++) {
-			const int col = c * 8 + i;
-			float v = 0.f;
-			if (c < vchunks && col < a.V) {
-				v = fast_exp2((float)reg[j][i] * LOG2E_F - m2) * gs;
-				if (col == tgt) v -= g;
-			}
-			o[i] = (bf16_t)v;
-		}
+		for (int i = 0; i < 8; i++) o[i] = (bf16_t)v[i];
 		*reinterpret_cast<bf16x8*>(dr + (int64_t)c * 8) = o;
 	}
+	if (ec >= 0) {
+		for (int i = elo; i < ehi; i++) dr[(int64_t)ec * 8 + i] = (bf16_t)(softmax(xr[(int64_t)ec * 8 + i]) - (ec == tchunk && i == tcol ? g : 0.f));
+	}
+	if constexpr (!DENSE)
+		for (int64_t i = a.V + lane; i < a.ld_out; i += G) dr[i] = (bf16_t)0.f;  // padding columns
 }
 
-// Longer rows: G threads per row (one workgroup), an online max / sum over one read of the row, then
-// a second read (served by the cache hierarchy: the rows in flight on the chip are a few MiB) for the
-// gradient.  The arithmetic is trimmed to what the two exponentials per logit leave room for: the
-// running maximum only rescales the partial sum when it grows, column masks are confined to the last
-// chunk of a row, the 1/sum * scale factor rides in the exponent, and the target column is fixed up
-// by the one thread that holds it.
+// Rows beyond those registers, and wide rows whose gradient nobody asked for (nothing is read twice then, and more and smaller
+// workgroups hide the loads better: 4096 x 50304 82 us against 100, 2048 x 128256 99 against 129): G threads per row (one
+// workgroup), an online max / sum over one read of the row, then a second read for the gradient.  The running maximum only
+// rescales the partial sum when it grows, column masks are confined to the last chunk of a row, the 1/sum * scale factor rides
+// in the exponent, and the target column is fixed up by the one thread that holds it.
 template <bool MASKED>
 __device__ __forceinline__ void online_chunk(const bf16x8& r, int c, int V, float& m, float& s) {
 	float x[8];
@@ -234,11 +267,37 @@ __global__ __launch_bounds__(1024) void cross_entropy_reduce_kernel(const float*
 	}
 }
 
-template <int G, int C>
+template <int G, int C, bool DENSE>
 void launch_rows(const LossArgs& a, hipStream_t s) {
 	constexpr int BLOCK = G < 256 ? 256 : G;
 	constexpr int ROWS = BLOCK / G;
-	ELF_LAUNCH((cross_entropy_kernel<G, C>), dim3((unsigned)((a.rows + ROWS - 1) / ROWS)), dim3(BLOCK), 0, s, a);
+	ELF_LAUNCH((cross_entropy_kernel<G, C, DENSE>), dim3((unsigned)((a.rows + ROWS - 1) / ROWS)), dim3(BLOCK), 0, s, a);
+}
+
+// The narrowest group of threads whose registers hold a row of `width` columns; false: none does.
+template <bool DENSE>
+bool launch_resident(const LossArgs& a, int64_t width, hipStream_t s) {
+	if (width <= 64 * 2 * 8) launch_rows<64, 2, DENSE>(a, s);
+	else if (width <= 64 * 8 * 8) launch_rows<64, 8, DENSE>(a, s);
+	else if (width <= 256 * 8 * 8) launch_rows<256, 8, DENSE>(a, s);
+	else if (width <= 512 * 8 * 8) launch_rows<512, 8, DENSE>(a, s);
+	else if (width <= 1024 * 8 * 8) launch_rows<1024, 8, DENSE>(a, s);
+	else if (width <= 1024 * 16 * 8) launch_rows<1024, 16, DENSE>(a, s);
+	else return false;
+	return true;
+}
+
+// y = x * g, both factors and the product rounded to bf16 once (g is an fp32 scalar on the device).
+__global__ __launch_bounds__(256) void scale_by_kernel(const bf16_t* __restrict__ x, const float* __restrict__ g, bf16_t* __restrict__ y, int64_t n) {
+	const float f = (float)(bf16_t)*g;
+	const int64_t nchunks = n >> 3;
+	for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nchunks; i += (int64_t)gridDim.x * blockDim.x) {
+		bf16x8 v = *reinterpret_cast<const bf16x8*>(x + i * 8);
+#pragma unroll
+		for (int j = 0; j < 8; j++) v[j] = (bf16_t)((float)v[j] * f);
+		*reinterpret_cast<bf16x8*>(y + i * 8) = v;
+	}
+	if (blockIdx.x == 0 && threadIdx.x < (n & 7)) y[nchunks * 8 + threadIdx.x] = (bf16_t)((float)x[nchunks * 8 + threadIdx.x] * f);
 }
 
 }  // namespace
@@ -257,11 +316,31 @@ int cross_entropy(const void* logits, int64_t ld, const void* target, int64_t ro
 	           (float*)row_loss, (bf16_t*)dlogits, dlogits ? ld_out : 0};
 	const int64_t width = dlogits && ld_out > V ? ld_out : V;
 	ProfScope prof(PROF_LOSS, (dlogits ? 4.0 : 2.0) * rows * V, s);
-	if (width <= 64 * 2 * 8) launch_rows<64, 2>(a, s);
-	else if (width <= 64 * 8 * 8) launch_rows<64, 8>(a, s);
-	else if (width <= 256 * 8 * 8) launch_rows<256, 8>(a, s);
-	else if (width <= 65536) ELF_LAUNCH(cross_entropy_stream_kernel<256>, dim3((unsigned)rows), dim3(256), 0, s, a);
-	else ELF_LAUNCH(cross_entropy_stream_kernel<1024>, dim3((unsigned)rows), dim3(1024), 0, s, a);
+	if (!dlogits && width > 16384 && width <= 65536) ELF_LAUNCH(cross_entropy_stream_kernel<256>, dim3((unsigned)rows), dim3(256), 0, s, a);
+	else if ((!dlogits && width > 16384) || !launch_resident<false>(a, width, s)) ELF_LAUNCH(cross_entropy_stream_kernel<1024>, dim3((unsigned)rows), dim3(1024), 0, s, a);
+	ELF_CHECK_HIP(hipGetLastError());
+	return 0;
+}
+
+int cross_entropy_dense(const void* logits, const void* target, int64_t rows, int64_t V, int64_t ignore_index, float scale, const void* dev_div,
+                        void* row_loss, void* dlogits, hipStream_t s) {
+	ELF_REQUIRE(logits && target && rows > 0 && rows < (1ll << 31) && V > 0, "cross_entropy_dense: bad argument");
+	ELF_REQUIRE(V <= 1024 * 16 * 8 - 7, "cross_entropy_dense: rows of at most %d columns (V=%lld)", 1024 * 16 * 8 - 7, (long long)V);
+	ELF_REQUIRE(row_loss || dlogits, "cross_entropy_dense: nothing to compute (no row_loss and no dlogits)");
+	ELF_REQUIRE(((uintptr_t)logits & 1) == 0 && (!dlogits || ((uintptr_t)logits & 15) == ((uintptr_t)dlogits & 15)),
+	            "cross_entropy_dense: logits and their gradient must lie alike modulo 16 bytes");
+	LossArgs a{(const bf16_t*)logits, V, (const int64_t*)target, rows, (int)V, ignore_index, scale, (const float*)dev_div, (float*)row_loss, (bf16_t*)dlogits, V};
+	ProfScope prof(PROF_LOSS, (dlogits ? 4.0 : 2.0) * rows * V, s);
+	launch_resident<true>(a, V + 7, s);  // a row may cover one chunk more than V / 8
+	ELF_CHECK_HIP(hipGetLastError());
+	return 0;
+}
+
+int scale_by_bf16(const void* x, const void* g_f32, void* y, int64_t n, hipStream_t s) {
+	ELF_REQUIRE(x && g_f32 && y && n > 0, "scale_by: bad argument");
+	ELF_REQUIRE(((uintptr_t)x & 15) == 0 && ((uintptr_t)y & 15) == 0 && ((uintptr_t)g_f32 & 3) == 0, "scale_by: pointers must be 16-byte aligned");
+	const int64_t blocks = (n / 8 + 255) / 256;
+	ELF_LAUNCH(scale_by_kernel, dim3((unsigned)(blocks < 1 ? 1 : blocks < 8192 ? blocks : 8192)), dim3(256), 0, s, (const bf16_t*)x, (const float*)g_f32, (bf16_t*)y, n);
 	ELF_CHECK_HIP(hipGetLastError());
 	return 0;
 }

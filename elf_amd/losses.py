@@ -45,10 +45,16 @@ def _check_target(target, rows):
 	return target.contiguous().view(-1)
 
 
-def _run(pred, target, *, ignore_index, scale, mean, want_grad):
-	"""(row_loss fp32 [rows], out2 = [sum, count] fp32, grad [rows, ld_out] bf16 or None)."""
+_DENSE_MAX = 1024 * 16 * 8 - 7  # widest row elf_cross_entropy_dense holds in registers
+
+
+def _run(pred, target, *, ignore_index, scale, mean, want_grad, padded=True):
+	"""(row_loss fp32 [rows], out2 = [sum, count] fp32, grad or None).  The gradient is [rows, ld_out] bf16 with ``ld_out`` a
+	multiple of 64, or, unless ``padded``, [rows, V] where the logits are one dense block: rows that start at any address are
+	then read in place (50257 columns: the padded copy of the logits took half of a loss's time)."""
 	V = pred.shape[-1]
-	src, ld = _rows_view(pred, V)
+	dense = (not padded if want_grad else V % 8 != 0) and pred.dtype == torch.bfloat16 and pred.is_cuda and pred.is_contiguous() and pred.data_ptr() % 16 == 0 and 0 < V <= _DENSE_MAX
+	src, ld = (pred, V) if dense else _rows_view(pred, V)
 	rows = pred.numel() // V
 	target = _check_target(target, rows)
 	lib = _lib.load()
@@ -60,13 +66,20 @@ def _run(pred, target, *, ignore_index, scale, mean, want_grad):
 		_lib.check(lib.elf_cross_entropy_reduce(None, target.data_ptr(), rows, ignore_index, out2.data_ptr(), _stream()), "elf_cross_entropy_reduce")
 		div = out2[1:]
 	if want_grad:
-		ld_out = -(-V // _PAD) * _PAD
+		ld_out = V if dense else -(-V // _PAD) * _PAD
 		grad = torch.empty(rows, ld_out, dtype=torch.bfloat16, device=dev)
-	_lib.check(
-		lib.elf_cross_entropy(src.data_ptr(), ld, target.data_ptr(), rows, V, ignore_index, scale, div.data_ptr() if div is not None else None,
-			row_loss.data_ptr(), grad.data_ptr() if grad is not None else None, ld_out, _stream()),
-		"elf_cross_entropy",
-	)
+	if dense:
+		_lib.check(
+			lib.elf_cross_entropy_dense(src.data_ptr(), target.data_ptr(), rows, V, ignore_index, scale, div.data_ptr() if div is not None else None,
+				row_loss.data_ptr(), grad.data_ptr() if grad is not None else None, _stream()),
+			"elf_cross_entropy_dense",
+		)
+	else:
+		_lib.check(
+			lib.elf_cross_entropy(src.data_ptr(), ld, target.data_ptr(), rows, V, ignore_index, scale, div.data_ptr() if div is not None else None,
+				row_loss.data_ptr(), grad.data_ptr() if grad is not None else None, ld_out, _stream()),
+			"elf_cross_entropy",
+		)
 	_lib.check(lib.elf_cross_entropy_reduce(row_loss.data_ptr(), target.data_ptr(), rows, ignore_index, out2.data_ptr(), _stream()), "elf_cross_entropy_reduce")
 	return row_loss, out2, grad
 
@@ -84,14 +97,20 @@ def _reduced(row_loss, out2, reduction, shape):
 class _CrossEntropy(torch.autograd.Function):
 	@staticmethod
 	def forward(ctx, pred, target, reduction, ignore_index):
-		row_loss, out2, grad = _run(pred, target, ignore_index=ignore_index, scale=1.0, mean=reduction == "mean", want_grad=ctx.needs_input_grad[0])
+		row_loss, out2, grad = _run(pred, target, ignore_index=ignore_index, scale=1.0, mean=reduction == "mean", want_grad=ctx.needs_input_grad[0], padded=False)
 		ctx.grad, ctx.shape, ctx.per_row = grad, pred.shape, reduction == "none"
 		return _reduced(row_loss, out2, reduction, pred.shape[:-1])
 
 	@staticmethod
 	def backward(ctx, g):
 		V = ctx.shape[-1]
-		grad = ctx.grad[:, :V]
+		grad = ctx.grad
+		if grad.shape[1] == V and g.dim() == 0 and g.dtype == torch.float32 and not (torch.is_grad_enabled() and g.requires_grad):
+			# one pass of 16-byte accesses with the same roundings (2048 x 50257: 71 us, 82 as a torch product of the strided view)
+			out = torch.empty(ctx.shape, dtype=grad.dtype, device=grad.device)
+			_lib.check(_lib.load().elf_scale_by_bf16(grad.data_ptr(), g.data_ptr(), out.data_ptr(), out.numel(), _stream()), "elf_scale_by_bf16")
+			return out, None, None, None
+		grad = grad[:, :V]
 		grad = grad * (g.reshape(-1, 1) if ctx.per_row else g).to(grad.dtype)
 		return grad.view(ctx.shape), None, None, None
 

@@ -188,6 +188,13 @@ int elf_embedding_bwd(const void* ids, const void* dx, void* dtable_f32, int64_t
  * number of rows whose target is not ignore_index; fixed summation order (bit-reproducible). */
 int elf_cross_entropy(const void* logits, int64_t ld, const void* target, int64_t rows, int64_t V, int64_t ignore_index, float scale,
                       const void* dev_div, void* row_loss, void* dlogits, int64_t ld_out, void* stream);
+/* The same over dense rows (row stride V, base on any 2-byte boundary; V at most 131065), dlogits dense as well and lying like
+ * logits modulo 16 bytes. */
+int elf_cross_entropy_dense(const void* logits, const void* target, int64_t rows, int64_t V, int64_t ignore_index, float scale,
+                            const void* dev_div, void* row_loss, void* dlogits, void* stream);
+/* y[i] = bf16(x[i] * bf16(*g_f32)), x and y bf16 [n] on 16-byte boundaries, g_f32 an fp32 scalar on the device: the gradient of a
+ * loss multiplied by the gradient that arrives at it. */
+int elf_scale_by_bf16(const void* x, const void* g_f32, void* y, int64_t n, void* stream);
 int elf_cross_entropy_reduce(const void* row_loss, const void* target, int64_t rows, int64_t ignore_index, void* out2, void* stream);
 
 /* ---------------------------------------------------------------------------------------------

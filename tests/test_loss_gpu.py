@@ -63,6 +63,33 @@ def test_cross_entropy_loss_and_gradient(rows, V, ld):
 	_check_grad(xa.grad, xf.grad * (3.0 / live), 3.0 / live)
 
 
+# dense rows that start at every 2-byte phase (odd widths), at the widest of each register depth and one beyond it, and a base
+# that is not 16-byte aligned (the padded copy)
+@pytest.mark.parametrize("V", [1, 7, 9, 1017, 1018, 4089, 4091, 16377, 16379, 32761, 32763, 65529, 65531, 131065, 131067])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_cross_entropy_dense_rows_of_any_width(V, offset):
+	from elf_amd import losses
+
+	rows = 11
+	x, t, _ = _case(rows, V, seed=V)
+	t[3] = V - 1  # the last column
+	t[4] = 0
+	buf = torch.zeros(rows * V + offset, dtype=torch.bfloat16).cuda()
+	buf[offset:] = x.reshape(-1).cuda()
+	xg = buf[offset:].view(rows, V).requires_grad_()
+	xf = x.float().requires_grad_()
+	want = L.cross_entropy_ref(xf, t, "mean")
+	want.backward()
+	got = losses.cross_entropy(xg, t.cuda())
+	assert torch.allclose(got.detach().cpu(), want.detach(), rtol=1e-5, atol=2e-5)
+	(grad,) = torch.autograd.grad(got, xg, retain_graph=True)
+	live = int((t != -100).sum())
+	_check_grad(grad, xf.grad, 1.0 / live)
+	assert V == 1 or grad[t == -100].abs().max().item() == 0
+	(twice,) = torch.autograd.grad(got, xg, grad_outputs=torch.tensor(-2.0).cuda())  # the kept gradient is not consumed
+	assert torch.equal(twice, grad * -2)
+
+
 def test_cross_entropy_rejects_what_it_cannot_run_and_flags_bad_targets():
 	from elf_amd import _lib, losses
 
