@@ -260,6 +260,117 @@ __global__ __launch_bounds__(256) void norm_bwd_kernel(const bf16_t* __restrict_
 	}
 }
 
+constexpr int NORM_TRIP_ROWS = 2;
+// Norm backward of rows of 1025 .. 2048 columns: a workgroup takes two rows at a time, one 16-byte chunk of each per thread, with
+// the next two in flight and one barrier per trip.  A thread owns its columns of dgamma / dbeta outright.  Bound: HBM (8 bytes
+// per element with a residual gradient) and, below some 2000 rows, the latency of a trip.  It takes the place of a wave per row,
+// whose four chunks per lane filled the register file (two waves per SIMD), idled a fifth of the lanes at 1600 columns and
+// folded four waves through LDS in sixteen barriers.  With the fold kernel, before -> after, cold operands: LayerNorm 1920 x 1600
+// 24.4 -> 15.9 us, 8192 x 1600 56.5 -> 30.8, 640 x 1600 12.6 -> 11.1; RMSNorm 4096 x 2048 25.0 -> 18.4, 16384 x 2048
+// 54.1 -> 48.6 (5.5 TB/s).  Rows of up to 1024 columns leave half of the threads without a chunk and stay with a wave per row
+// (8192 x 1024 24.2 us, 28.9 here on 128 threads).
+template <bool LN, bool YOUT>
+__global__ __launch_bounds__(256) void norm_bwd_rows_kernel(const bf16_t* __restrict__ dy, const bf16_t* __restrict__ x, const bf16_t* __restrict__ gamma,
+                                                            const float2* __restrict__ stats, const bf16_t* __restrict__ dres, bf16_t* __restrict__ dx,
+                                                            float* __restrict__ part, int T, int d, const bf16_t* __restrict__ beta,
+                                                            bf16_t* __restrict__ yout) {
+	constexpr int R = NORM_TRIP_ROWS, W = 4;
+	__shared__ float red[2][2 * R][W];  // two buffers: one barrier per trip
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	const bool on = (int)threadIdx.x < (d >> 3);
+	const int col = threadIdx.x * 8;
+	Chunk g, b;
+	float dg[8], db[8];
+#pragma unroll
+	for (int j = 0; j < 8; j++) dg[j] = db[j] = 0.f, g.v[j] = b.v[j] = 0.f;
+	if (on) {
+		g = load8(gamma + col);
+		if (YOUT && LN) b = load8(beta + col);
+	}
+	bf16x8 nx[R], ndy[R], nres[R];  // the rows in flight
+	float2 nst[R];
+	auto fetch = [&](int r0) {
+#pragma unroll
+		for (int k = 0; k < R; k++)
+			if (r0 + k < T) {
+				nst[k] = stats[r0 + k];
+				if (on) {
+					const int64_t at = (int64_t)(r0 + k) * d + col;
+					nx[k] = *reinterpret_cast<const bf16x8*>(x + at);
+					ndy[k] = *reinterpret_cast<const bf16x8*>(dy + at);
+					if (dres) nres[k] = *reinterpret_cast<const bf16x8*>(dres + at);
+				}
+			}
+	};
+	const int step = gridDim.x * R;
+	int row = blockIdx.x * R, buf = 0;
+	fetch(row);
+	for (; row < T; row += step, buf ^= 1) {
+		bf16x8 rx[R], rdy[R], rres[R];
+		float2 st[R];
+#pragma unroll
+		for (int k = 0; k < R; k++) rx[k] = nx[k], rdy[k] = ndy[k], rres[k] = nres[k], st[k] = nst[k];
+		fetch(row + step);  // the next rows' loads travel while these are reduced and stored
+#pragma unroll
+		for (int k = 0; k < R; k++) {
+			float s1 = 0.f, s2 = 0.f;
+			if (on && row + k < T) {
+#pragma unroll
+				for (int j = 0; j < 8; j++) {
+					const float xhat = ((float)rx[k][j] - st[k].x) * st[k].y;
+					const float dyv = (float)rdy[k][j];
+					dg[j] += dyv * xhat;
+					if (LN) db[j] += dyv;
+					const float gv = dyv * g.v[j];
+					s1 += gv;
+					s2 += gv * xhat;
+				}
+			}
+			s2 = wave_sum(s2);
+			if (LN) s1 = wave_sum(s1);
+			if (lane == 0) {
+				red[buf][2 * k][wave] = s2;
+				if (LN) red[buf][2 * k + 1][wave] = s1;
+			}
+		}
+		__syncthreads();
+#pragma unroll
+		for (int k = 0; k < R; k++) {
+			if (row + k >= T || !on) continue;
+			float m2 = 0.f, m1 = 0.f;
+#pragma unroll
+			for (int w = 0; w < W; w++) {
+				m2 += red[buf][2 * k][w];
+				if (LN) m1 += red[buf][2 * k + 1][w];
+			}
+			m2 /= d, m1 /= d;
+			const int64_t at = (int64_t)(row + k) * d + col;
+			Chunk o;
+#pragma unroll
+			for (int j = 0; j < 8; j++) {
+				const float xhat = ((float)rx[k][j] - st[k].x) * st[k].y;
+				const float gv = (float)rdy[k][j] * g.v[j];
+				o.v[j] = st[k].y * (gv - m1 - xhat * m2);
+				if (dres) o.v[j] += (float)rres[k][j];
+			}
+			store8(dx + at, o);
+			if constexpr (YOUT) {
+				Chunk y;
+#pragma unroll
+				for (int j = 0; j < 8; j++) y.v[j] = norm_out<LN>((float)rx[k][j], st[k].x, st[k].y, g.v[j], LN ? b.v[j] : 0.f);
+				store8(yout + at, y);
+			}
+		}
+	}
+	if (!on) return;
+	float* const pg = part + (int64_t)blockIdx.x * 2 * d + col;
+#pragma unroll
+	for (int j = 0; j < 8; j += 4) {
+		*reinterpret_cast<f32x4*>(pg + j) = f32x4{dg[j], dg[j + 1], dg[j + 2], dg[j + 3]};
+		if (LN) *reinterpret_cast<f32x4*>(pg + d + j) = f32x4{db[j], db[j + 1], db[j + 2], db[j + 3]};
+	}
+}
+
 // main_grad[c] += sum_b part[b][which][c].  A workgroup owns 32 columns; its 32 row groups stride over the partial
 // rows and are folded through LDS in a fixed order, and each column has one writer: the sums do not depend on
 // the order in which workgroups run (bit-reproducible gamma / beta gradients).
@@ -456,14 +567,24 @@ static inline bool norm_half_rows(int d) { return d % 256 == 0 && d <= 768; }
 // the full-wave backward kernel can write the norm's output again (see norm_bwd_kernel); the narrow-row one does not
 bool norm_bwd_forms_output(int d) { return !norm_half_rows(d); }
 
+// one chunk of 8 columns per thread of a workgroup of 256 (norm_bwd_rows_kernel)
+static inline bool norm_trip_rows(int d) { return d > 1024 && d <= 2048; }
+
 static inline int norm_bwd_blocks(int T, int d) {
+	if (norm_trip_rows(d)) {
+		// two workgroups per compute unit, one where the rows are few (1024 x 2048 LayerNorm: 13.6 us on 256, 17.3 on 512;
+		// 4096 x 2048 RMSNorm: 21.6 and 18.4), all with the same number of trips but the last
+		const int cap = T <= 2048 ? 256 : 512;
+		const int want = (T + NORM_TRIP_ROWS - 1) / NORM_TRIP_ROWS, trips = (want + cap - 1) / cap;
+		return (want + trips - 1) / trips;
+	}
 	if (norm_half_rows(d)) {
 		// eight rows per workgroup at a time, one workgroup per compute unit: 256 partial rows for the fold kernel (with 512
 		// the pair took 21 us at 8192 x 768, with 256 18 us, with 128 20 us)
 		const int want = (T + 7) / 8;
 		return want < 256 ? want : 256;
 	}
-	const int rows_per_block = d <= 2048 ? ROWS_PER_BLOCK : 1;
+	const int rows_per_block = d <= 1024 ? ROWS_PER_BLOCK : 1;
 	const int want = (T + rows_per_block - 1) / rows_per_block;
 	// fewer, longer workgroups for narrow rows and for the wide ones: the partial rows are overhead traffic that the fold
 	// kernel reads back (d = 8192: 3.8 -> 4.1 TB/s with 512 instead of 1024; d = 4096 inside a stage's stream: 5.28 TB/s
@@ -514,7 +635,12 @@ int norm_fwd(int kind, const void* x, const void* gamma, const void* beta, void*
 	return norm_fwd_dispatch<false>(x, gamma, beta, y, stats, T, d, eps, s);
 }
 
-int64_t norm_bwd_workspace_floats(int T, int d) { return (int64_t)norm_bwd_blocks(T, d) * 2 * d; }
+// never smaller for more rows: a workspace sized for a full micro-batch serves a shorter one (the balanced trips of
+// norm_bwd_blocks are not monotonic, 384 workgroups for 3074 rows and 512 for 3072)
+int64_t norm_bwd_workspace_floats(int T, int d) {
+	const int64_t trip_blocks = ((int64_t)T + NORM_TRIP_ROWS - 1) / NORM_TRIP_ROWS;
+	return (norm_trip_rows(d) ? (trip_blocks < 512 ? trip_blocks : 512) : (int64_t)norm_bwd_blocks(T, d)) * 2 * d;
+}
 
 template <bool LN>
 static int norm_bwd_dispatch(const void* dy, const void* x, const void* gamma, const void* stats, const void* dres,
@@ -539,13 +665,18 @@ static int norm_bwd_dispatch(const void* dy, const void* x, const void* gamma, c
 		if (yout) ELF_NORM_BWD_Y(N, W, true); \
 		else ELF_NORM_BWD_Y(N, W, false);     \
 	} while (0)
+#define ELF_NORM_BWD_ROWS(Y)                                                                                      \
+	ELF_LAUNCH((norm_bwd_rows_kernel<LN, Y>), grid, block, 0, s, (const bf16_t*)dy, (const bf16_t*)x,      \
+	                   (const bf16_t*)gamma, (const float2*)stats, (const bf16_t*)dres, (bf16_t*)dx, part, T, d, (const bf16_t*)beta, (bf16_t*)yout)
 	if (d <= 512) ELF_NORM_BWD(1, 1);
 	else if (d <= 1024) ELF_NORM_BWD(2, 1);
-	else if (d <= 2048) ELF_NORM_BWD(4, 1);
+	else if (norm_trip_rows(d) && yout) ELF_NORM_BWD_ROWS(true);
+	else if (norm_trip_rows(d)) ELF_NORM_BWD_ROWS(false);
 	else if (d <= 4096) ELF_NORM_BWD(2, 4);
 	else ELF_NORM_BWD(4, 4);
 #undef ELF_NORM_BWD
 #undef ELF_NORM_BWD_Y
+#undef ELF_NORM_BWD_ROWS
 	ELF_CHECK_HIP(hipGetLastError());
 	return 0;
 }

@@ -270,6 +270,36 @@ def test_norm_fwd_bwd(K, d, kind):
 	_close(dx2, xr.grad, what="norm dx no residual")
 
 
+@pytest.mark.parametrize("d", [1032, 1600, 2040, 2048])
+@pytest.mark.parametrize("T", [1, 3, 513, 2047, 2050, 3075])
+@pytest.mark.parametrize("kind", ["rms", "ln"])
+def test_norm_bwd_two_rows_a_trip(K, d, T, kind):
+	"""Rows of 1025 to 2048 columns, two a trip: one row alone, odd counts, a last trip that some workgroups miss, the step from
+	one workgroup per compute unit to two, widths with idle threads.  The workspace of more rows is never smaller."""
+	from elf_amd import _lib
+
+	lib = _lib.load()
+	assert all(lib.elf_norm_bwd_workspace_floats(t, d) <= lib.elf_norm_bwd_workspace_floats(t + 1, d) for t in range(max(1, T - 3), T + 3))
+	x, dy, dres = _randn(T, d, seed=41) + 0.25, _randn(T, d, seed=42), _randn(T, d, seed=43)
+	x = x.to(torch.bfloat16)
+	gamma, beta = (1 + 0.1 * _randn(1, d, seed=44).float()).to(torch.bfloat16)[0], _randn(1, d, seed=45)[0]
+	xr, gr, br = (t.double().requires_grad_(True) for t in (x, gamma, beta))
+	yr = torch.nn.functional.layer_norm(xr, (d,), gr, br, 1e-5) if kind == "ln" else xr * torch.rsqrt(xr.pow(2).mean(-1, keepdim=True) + 1e-5) * gr
+	yr.backward(dy.double())
+	k = K.NORM_LAYER if kind == "ln" else K.NORM_RMS
+	_, stats = K.norm_fwd(k, x, gamma, beta if kind == "ln" else None, 1e-5)
+	dgamma, dbeta = torch.zeros(d, device="cuda"), torch.zeros(d, device="cuda") if kind == "ln" else None
+	dx = K.norm_bwd(k, dy, x, gamma, stats, dgamma, dbeta, dres)
+	_close(dx, (xr.grad + dres.double()).float(), what="dx")
+	# fp32 sums of T products, each with the row statistics' few units of 2^-24
+	_close(dgamma, gr.grad.float(), rel_fro=1e-5, rel_max=1e-4, what="dgamma")
+	if kind == "ln":
+		_close(dbeta, br.grad.float(), rel_fro=1e-5, rel_max=1e-4, what="dbeta")
+	again = torch.zeros_like(dgamma)
+	assert torch.equal(K.norm_bwd(k, dy, x, gamma, stats, again, torch.zeros_like(dgamma) if kind == "ln" else None, dres), dx)
+	assert torch.equal(again, dgamma)
+
+
 def test_gelu_swiglu(K):
 	x = _randn(300, 1024, seed=20) * 2
 	x = x.to(torch.bfloat16)
