@@ -115,6 +115,18 @@ bool norm_bwd_forms_output(int d);
 int norm_bwd(int kind, const void* dy, const void* x, const void* gamma, const void* stats, const void* dres,
              void* dx, float* dgamma, float* dbeta, float* workspace, int T, int d, hipStream_t s, const void* beta = nullptr,
              void* y_out = nullptr);
+// The two halves of it: dx and the partial sums of one norm, and the fold of the partial sums of n norms of the same T and d,
+// whose workspaces lie one behind the other, into their (different) accumulators; dbeta null for RMSNorm.  The bits do not
+// depend on how norms are grouped.
+int norm_bwd_partial(int kind, const void* dy, const void* x, const void* gamma, const void* stats, const void* dres, void* dx, float* workspace, int T, int d,
+                     hipStream_t s, const void* beta = nullptr, void* y_out = nullptr);
+constexpr int NORM_FOLD_MAX = 8;
+struct NormFold {
+	int n;
+	float* dgamma[NORM_FOLD_MAX];
+	float* dbeta[NORM_FOLD_MAX];
+};
+int norm_bwd_fold(const NormFold& f, const float* workspace, int T, int d, hipStream_t s);
 // The same with the partial sums in an array of the library's device image instead of a workspace argument
 // (no allocation anywhere on the path); norm_bwd_scratch_prepare looks the array's address up for the
 // current device (done by the first call on a device otherwise).

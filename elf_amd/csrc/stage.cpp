@@ -121,10 +121,10 @@ struct Stage {
 	std::unique_ptr<PinnedPool> pinned;
 	hipStream_t offload_stream = nullptr, prefetch_stream = nullptr;
 	void* rope_cs = nullptr;
-	float* norm_ws = nullptr;
+	float* norm_ws = nullptr;  // partial sums of norm_slots norm backwards
+	int norm_slots = 1;
 	void* attn_ws = nullptr;
 	int64_t ws_bytes = 0;  // fixed device workspaces of the stage (norm / attention backward scratch, rope table, gradient sink)
-	float* dummy_grad = nullptr;  // sink for norm weight gradients during gradient recompute
 	// pinned blocks of released micro-batches whose last copy may still be in flight: they go back to the arena
 	// when their event has fired (polled, never waited for inside a step unless the arena would have to grow)
 	struct HostPending {
@@ -340,6 +340,39 @@ static int run_forward(Stage* s, MbState& m, const void* x, void* y, FwdMode mod
 	return 0;
 }
 
+// The norm backwards of one pass: their partial sums are folded into the accumulators together, when norm_slots of them
+// wait and at the end of the pass.  grads_only: nothing is accumulated.
+struct NormBackwards {
+	Stage* s;
+	bool grads_only;
+	hipStream_t st;
+	NormFold pending{};
+	int run(const void* dy, const void* x, const void* gamma, const void* stats, const void* dres, void* dx, float* dgamma, float* dbeta,
+	        const void* beta = nullptr, void* y_out = nullptr) {
+		const int kind = s->llama ? NORM_RMS : NORM_LAYER;
+		if (!grads_only && s->norm_slots == 1)
+			return norm_bwd(kind, dy, x, gamma, stats, dres, dx, dgamma, dbeta, s->norm_ws, s->T, s->d, st, beta, y_out);
+		ELF_REQUIRE(grads_only || (dgamma && (kind != NORM_LAYER || dbeta)), "norm backward: no gradient buffer is bound");
+		for (int i = 0; i < pending.n; i++)
+			if (pending.dgamma[i] == dgamma || (dbeta && pending.dbeta[i] == dbeta)) {  // a norm shared by blocks
+				ELF_TRY(fold());
+				break;
+			}
+		float* const ws = s->norm_ws + pending.n * norm_bwd_workspace_floats(s->T, s->d);
+		ELF_TRY(norm_bwd_partial(kind, dy, x, gamma, stats, dres, dx, ws, s->T, s->d, st, beta, y_out));
+		if (grads_only) return 0;
+		pending.dgamma[pending.n] = dgamma;
+		pending.dbeta[pending.n++] = kind == NORM_LAYER ? dbeta : nullptr;
+		return pending.n == s->norm_slots ? fold() : 0;
+	}
+	int fold() {
+		if (!pending.n) return 0;
+		ELF_TRY(norm_bwd_fold(pending, s->norm_ws, s->T, s->d, st));
+		pending.n = 0;
+		return 0;
+	}
+};
+
 // grads_only: recompute of the W stash gradients (RECOMPUTE_BACKWARD_INPUTS): no norm weight
 // gradients, and the chain stops once the first block's QKV output gradient is known
 // (elf/zb_utils.py:584-604, elf/execution/block.py:340-374).
@@ -348,6 +381,7 @@ static int run_backward(Stage* s, MbState& m, const void* dy, void* dx, bool gra
 	const int T = s->T, d = s->d, F = s->F;
 	const int norm_kind = s->llama ? NORM_RMS : NORM_LAYER;
 	const float scale = 1.0f / sqrtf((float)s->D);
+	NormBackwards norms{s, grads_only, st};
 	if (s->vocab_out) {
 		// last stage: dy is the gradient of the logits; it is the dY of the head linear's W stash
 		BlockState& hd = m.head;
@@ -364,8 +398,7 @@ static int run_backward(Stage* s, MbState& m, const void* dy, void* dx, bool gra
 			PoolTmp d_hn(s->pool, (size_t)T * d * 2);
 			if (!d_hn.p) return -3;
 			ELF_TRY(gemm_bf16(0, 1, T, d, s->vld, dy, s->vld, s->xw[XP_HEAD], d, d_hn.p, d, EPI_BF16, nullptr, 0, 0, 0, st));
-			ELF_TRY(norm_bwd(norm_kind, d_hn.p, hd.b[B_X].p, s->xw[XP_FNORM_G], hd.b[B_ST1].p, nullptr, last.b[B_DY].p,
-			                 grads_only ? s->dummy_grad : s->xg[XP_FNORM_G], grads_only ? s->dummy_grad + d : s->xg[XP_FNORM_B], s->norm_ws, T, d, st));
+			ELF_TRY(norms.run(d_hn.p, hd.b[B_X].p, s->xw[XP_FNORM_G], hd.b[B_ST1].p, nullptr, last.b[B_DY].p, s->xg[XP_FNORM_G], s->xg[XP_FNORM_B]));
 		} else {
 			ELF_TRY(gemm_bf16(0, 1, T, d, s->vld, dy, s->vld, s->xw[XP_HEAD], d, last.b[B_DY].p, d, EPI_BF16, nullptr, 0, 0, 0, st));
 		}
@@ -468,9 +501,7 @@ static int run_backward(Stage* s, MbState& m, const void* dy, void* dx, bool gra
 			ELF_TRY(buf_alloc(s, bs, B_ST2));
 			ELF_TRY(norm_fwd(norm_kind, bs.b[B_X2].p, p.w[P_NORM2_G], p.w[P_NORM2_B], bs.b[B_H2].p, bs.b[B_ST2].p, T, d, s->cfg.eps, st));
 		}
-		ELF_TRY(norm_bwd(norm_kind, d_h.p, bs.b[B_X2].p, p.w[P_NORM2_G], bs.b[B_ST2].p, dyin, bs.b[B_DX2].p,
-		                 grads_only ? s->dummy_grad : p.g[P_NORM2_G], grads_only ? s->dummy_grad + d : p.g[P_NORM2_B], s->norm_ws, T, d, st,
-		                 p.w[P_NORM2_B], h2_out));
+		ELF_TRY(norms.run(d_h.p, bs.b[B_X2].p, p.w[P_NORM2_G], bs.b[B_ST2].p, dyin, bs.b[B_DX2].p, p.g[P_NORM2_G], p.g[P_NORM2_B], p.w[P_NORM2_B], h2_out));
 		// attention
 		PoolTmp d_o(s->pool, (size_t)T * s->Hq * s->D * 2);
 		if (!d_o.p) return -3;
@@ -502,9 +533,8 @@ static int run_backward(Stage* s, MbState& m, const void* dy, void* dx, bool gra
 				dxout = pv.b[B_DY].p;
 			}
 			if (h1_from_bwd) ELF_TRY(buf_alloc(s, bs, B_H1));
-			ELF_TRY(norm_bwd(norm_kind, d_h.p, bs.b[B_X].p, p.w[P_NORM1_G], bs.b[B_ST1].p, bs.b[B_DX2].p, dxout,
-			                 grads_only ? s->dummy_grad : p.g[P_NORM1_G], grads_only ? s->dummy_grad + d : p.g[P_NORM1_B], s->norm_ws, T, d, st,
-			                 p.w[P_NORM1_B], h1_from_bwd ? bs.b[B_H1].p : nullptr));
+			ELF_TRY(norms.run(d_h.p, bs.b[B_X].p, p.w[P_NORM1_G], bs.b[B_ST1].p, bs.b[B_DX2].p, dxout, p.g[P_NORM1_G], p.g[P_NORM1_B], p.w[P_NORM1_B],
+			                  h1_from_bwd ? bs.b[B_H1].p : nullptr));
 			if (i == 0 && s->vocab_in) {
 				// first stage: the embedding is not a split layer, its gradient accumulates inside B
 				if (!grads_only) ELF_TRY(embedding_bwd(m.ids, d_emb.p, s->xg[XP_EMBED], T, d, s->vocab_in, st));
@@ -514,6 +544,7 @@ static int run_backward(Stage* s, MbState& m, const void* dy, void* dx, bool gra
 		for (int id = 0; id < B_COUNT; id++)
 			if ((ACT_MASK & (1u << id)) && !(WIN_MASK & (1u << id))) buf_free(s, bs, id);
 	}
+	ELF_TRY(norms.fold());
 	m.has_acts = false;
 	m.has_win = true;
 	m.has_wgrad = true;
@@ -750,14 +781,15 @@ int elf_stage_create(const elf_stage_cfg* cfg, elf_stage_t** out) {
 	};
 	if (hipStreamCreateWithFlags(&s->offload_stream, hipStreamNonBlocking) != hipSuccess) return fail("offload stream");
 	if (hipStreamCreateWithFlags(&s->prefetch_stream, hipStreamNonBlocking) != hipSuccess) return fail("prefetch stream");
-	const size_t norm_ws_bytes = (size_t)norm_bwd_workspace_floats(s->T, s->d) * 4;
+	// Norms folded together: up to 8 of rows of at most 2048 columns (67 MB of partial sums, which stay in the memory-side
+	// cache).  The fold of wider rows moves more than its launch costs, and each takes the one workspace in turn.
+	s->norm_slots = s->d > 2048 ? 1 : std::min(NORM_FOLD_MAX, 2 * cfg->n_blocks + 1);
+	const size_t norm_ws_bytes = (size_t)norm_bwd_workspace_floats(s->T, s->d) * 4 * s->norm_slots;
 	const size_t attn_ws_bytes = (size_t)attn_bwd_workspace_bytes(s->B, s->S, s->Hq, s->D, s->cfg.causal);
 	const size_t rope_bytes = s->llama ? (size_t)s->S * (s->D / 2) * 8 : 0;
-	s->ws_bytes = (int64_t)(norm_ws_bytes + attn_ws_bytes + rope_bytes + (size_t)2 * s->d * 4);
+	s->ws_bytes = (int64_t)(norm_ws_bytes + attn_ws_bytes + rope_bytes);
 	if (hipMalloc((void**)&s->norm_ws, norm_ws_bytes) != hipSuccess) return fail("norm workspace");
 	if (hipMalloc(&s->attn_ws, attn_ws_bytes) != hipSuccess) return fail("attention workspace");
-	if (hipMalloc((void**)&s->dummy_grad, (size_t)2 * s->d * 4) != hipSuccess) return fail("gradient sink");
-	if (hipMemset(s->dummy_grad, 0, (size_t)2 * s->d * 4) != hipSuccess) return fail("gradient sink clear");
 	if (s->llama) {
 		if (hipMalloc(&s->rope_cs, rope_bytes) != hipSuccess) return fail("rope table");
 		if (rope_table(s->rope_cs, s->S, s->D, cfg->rope_theta, nullptr) != 0) return fail("rope table fill");
@@ -783,7 +815,6 @@ void elf_stage_destroy(elf_stage_t* h) {
 	if (s->prefetch_stream) (void)hipStreamDestroy(s->prefetch_stream);
 	if (s->norm_ws) (void)hipFree(s->norm_ws);
 	if (s->attn_ws) (void)hipFree(s->attn_ws);
-	if (s->dummy_grad) (void)hipFree(s->dummy_grad);
 	if (s->rope_cs) (void)hipFree(s->rope_cs);
 	delete s;
 }
