@@ -270,6 +270,22 @@ def test_norm_fwd_bwd(K, d, kind):
 	_close(dx2, xr.grad, what="norm dx no residual")
 
 
+@pytest.mark.parametrize("shape", [(64, 64, 64), (192, 320, 192), (512, 832, 128)])
+def test_gemm_output_at_any_element(K, shape):
+	"""Outputs and residuals that start at any element, with an odd leading dimension."""
+	M, N, Kd = shape
+	A, B = _randn(M, Kd, seed=51), _randn(N, Kd, seed=52, scale=0.05)
+	R = _randn(M + 1, N + 3, seed=53)[1:, 1 : N + 1]
+	want, want_r = K.gemm(A, B), K.gemm(A, B, epilogue=K.EPI_BF16_RESID, residual=R.contiguous())
+	for epi, res, ref in ((K.EPI_BF16, None, want), (K.EPI_BF16_RESID, R, want_r)):
+		big = torch.full((M + 2, N + 5), 7.0, dtype=torch.bfloat16, device="cuda")
+		view = big[1 : M + 1, 3 : N + 3]
+		K.gemm(A, B, out=view, epilogue=epi, residual=res)
+		assert torch.equal(view, ref)
+		big[1 : M + 1, 3 : N + 3] = 7
+		assert (big == 7).all()
+
+
 @pytest.mark.parametrize("d", [1032, 1600, 2040, 2048])
 @pytest.mark.parametrize("T", [1, 3, 513, 2047, 2050, 3075])
 @pytest.mark.parametrize("kind", ["rms", "ln"])

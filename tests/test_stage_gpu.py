@@ -543,6 +543,58 @@ def test_preallocate_pool_reserves_the_pinned_arena_before_the_first_step(monkey
 		Engine([blk])
 
 
+def test_norms_folded_together_equal_norms_folded_alone():
+	"""Ten norms (a full group, folded in the middle of the pass, and two more at its end): the gradients of five blocks in one
+	stage against the same blocks in five stages of their own, bit for bit, with a short second micro-batch."""
+	import copy
+
+	from elf_amd import models
+
+	whole = models.gpt_stage(5, 256, 4, 512, 128, causal=True, seed=8)
+	perturb_norms(whole)
+	alone = [models.StageModule([copy.deepcopy(b)], 128) for b in whole]
+	gen = torch.Generator(device="cuda").manual_seed(9)
+	xs, dys = ([torch.randn(n, 128, 256, device="cuda", generator=gen).to(torch.bfloat16) for n in (3, 1)] for _ in range(2))
+
+	def block(stage, inputs, grads):
+		blk = _block(stage, 3)
+		blk.set_boundary(inputs=inputs, grads=grads, keep_sent=True)
+		return blk
+
+	def forward(blk):
+		for m, n in enumerate((3, 1)):
+			blk.recv_forward(m, n, src=0)
+			blk.forward(m)
+			blk.send_forward(m, dst=2)
+
+	def backward(blk):
+		for m, n in enumerate((3, 1)):
+			blk.recv_backward(m, n, src=2)
+			blk.backward_inputs(m)
+			blk.send_backward(m, dst=0)
+			blk.backward_params(m)
+
+	one = block(whole, xs, dys)
+	forward(one)
+	backward(one)
+	ys, blks = xs, []
+	for st in alone:
+		blks.append(block(st, ys, None))
+		forward(blks[-1])
+		ys = [blks[-1].sent_forward[m] for m in range(2)]
+	gs = dys
+	for blk, inputs in reversed(list(zip(blks, [xs] + [[b.sent_forward[m] for m in range(2)] for b in blks]))):
+		blk.set_boundary(inputs=inputs, grads=gs, keep_sent=True)
+		backward(blk)
+		gs = [blk.sent_backward[m] for m in range(2)]
+	torch.cuda.synchronize()
+	assert all(torch.equal(gs[m], one.sent_backward[m]) for m in range(2))
+	for i, (b, st) in enumerate(zip(whole, alone)):
+		for (name, p), (_, q) in zip(b.named_parameters(), st[0].named_parameters()):
+			if "norm" in name:
+				assert torch.equal(p.main_grad, q.main_grad), f"block {i} {name}"
+
+
 @pytest.mark.parametrize("kind", ["gpt", "llama"])
 def test_lean_stash_of_a_middle_width_equals_plain(kind):
 	"""Width 1280, where the norm backward that takes two rows a trip writes the dropped norm outputs again: the same bits, also
