@@ -967,6 +967,9 @@ static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal) {
 	const int tiles = causal ? (nkt + 1) * 4 : nkt * 4;  // query tiles of a walk and head (a pair of key tiles has nkt + 1 of four)
 	const float slots = D == 128 ? 256.f : 512.f, step = D == 128 ? 1.2f : 1.1f, fixed = 8.f;
 	Splits best;
+	// From 2^18 query rows (2 x 4096 tokens of 32 heads) up the workspace holds what it always did, the dQ partials and the row
+	// statistics: such launches fill the chip with eight kv heads, and fewer are rare at these sizes.
+	if ((int64_t)B * S * Hq >= 1 << 18) return best;
 	float best_us = 1e30f;
 	for (int h = 1; h <= G; h++) {
 		if (G % h) continue;
@@ -983,16 +986,17 @@ static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal) {
 static int64_t dkv_part_bytes(const Splits& sp, int B, int S, int Hkv, int D) { return sp.h * sp.q > 1 ? (int64_t)sp.h * sp.q * 2 * B * S * Hkv * D * 4 : 0; }
 
 int64_t attn_bwd_workspace_bytes(int B, int S, int Hq, int D, int causal) {
-	// bf16 dQ partials of every key tile + delta + scaled log-sum-exp + the largest set of dK / dV partials that any number of
-	// kv heads and any smaller batch asks for (few walks are split the more: it is 150 MB at most)
-	int64_t dkv = 0;
-	for (int b = 1; b <= B; b++)
+	// bf16 dQ partials of every key tile + delta + scaled log-sum-exp + the dK / dV partials of shared walks (150 MB at most):
+	// the most that any number of kv heads and any smaller batch asks for
+	const int64_t per_batch = part_rows(S, causal != 0) * Hq * D * 2 + 2 * (int64_t)S * Hq * 4;
+	int64_t most = B * per_batch;
+	for (int b = 1; b <= B && (int64_t)b * S * Hq < 1 << 18; b++)
 		for (int hkv = 1; hkv <= Hq; hkv++)
 			if (Hq % hkv == 0) {
-				const int64_t n = dkv_part_bytes(split_walk(b, S, Hq, hkv, D, causal != 0), b, S, hkv, D);
-				if (n > dkv) dkv = n;
+				const int64_t n = b * per_batch + dkv_part_bytes(split_walk(b, S, Hq, hkv, D, causal != 0), b, S, hkv, D);
+				if (n > most) most = n;
 			}
-	return (int64_t)B * part_rows(S, causal != 0) * Hq * D * 2 + 2 * (int64_t)B * S * Hq * 4 + dkv;
+	return most;
 }
 
 int attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* dO, const void* lse, void* dq,
