@@ -290,7 +290,6 @@ class HipStageBlock(StageBlockBase):
 		self._fused_w, self._fused_g, self._fused_bf16_grad = [], [], []  # the fused buffers (kept alive here)
 		self._w_scaled = []  # indices of the fused buffers of linear layers: what a W with the folded gradient scale covers
 		self._folded_scale = None  # 1 / batch size that the step's last W applied, until scale_grads has run
-		self._grad_views = None  # (parameter, its bf16 gradient: a view of the fused buffer), once every fused buffer has one
 		self._param_loc = {}  # parameter -> (fused buffer index, first row, rows)
 		self.main_grads = {}  # parameter -> fp32 accumulator view
 		handle = ctypes.c_void_p()
@@ -595,10 +594,9 @@ class HipStageBlock(StageBlockBase):
 			if self._fused_bf16_grad[i] is None:
 				self._fused_bf16_grad[i] = torch.empty_like(w)
 			_lib.check(self.lib.elf_scale_grads(g.data_ptr(), self._fused_bf16_grad[i].data_ptr(), g.numel(), inv, _stream()), "elf_scale_grads")
-		if self._grad_views is None:
-			self._grad_views = [(p, self._fused_bf16_grad[i][r : r + n]) for p, (i, r, n) in self._param_loc.items()]
-		for p, view in self._grad_views:
-			p.grad = view
+		# a new view every step: the tensor of the last one is the caller's, who may have given it another storage (p.grad.data = ...)
+		for p, (i, r, n) in self._param_loc.items():
+			p.grad = self._fused_bf16_grad[i][r : r + n]
 
 	def zero_grad(self):
 		self._folded_scale = None

@@ -86,6 +86,30 @@ def test_fbw_matches_oracle(kind):
 	assert attn_ws <= st["workspace_bytes"] <= attn_ws + (64 << 20)
 
 
+@pytest.mark.parametrize("folded", [False, True])
+def test_gradients_whose_storage_the_caller_replaced_come_fresh_next_step(folded):
+	"""``p.grad.data = p.grad.data * c`` (clipping, unscaling, a module moved with ``.to``) gives a gradient tensor another
+	storage.  The next step's gradients must be those of that step all the same, with and without ``zero_grad`` in between."""
+	mb = 1
+	stage = _stage("llama")
+	blk = _block(stage, mb)
+	gen = torch.Generator(device="cuda").manual_seed(3)
+	xs, dys = ([torch.randn(mb, 256, 512, device="cuda", generator=gen).to(torch.bfloat16) for _ in range(3)] for _ in range(2))
+	blk.set_boundary(inputs=xs, grads=dys)
+	for step in range(3):
+		if step != 1:
+			blk.zero_grad()
+		blk.recv_forward(step, mb, src=0)
+		blk.forward(step)
+		blk.recv_backward(step, mb, src=2)
+		blk.backward_inputs(step)
+		blk.backward_params(step, **({"final_scale": 0.5} if folded else {}))
+		blk.scale_grads(2)
+		for name, p in stage.named_parameters():
+			assert torch.equal(p.grad, p.main_grad.to(torch.bfloat16)), f"step {step} {name}"
+			p.grad.data = p.grad.data * 0.25
+
+
 @pytest.mark.parametrize("kind", ["gpt", "llama"])
 def test_widths_that_no_tile_divides_match_oracle(kind):
 	"""Widths and FFN sizes that are multiples of 64 only: the grouped weight gradients (with the gradient scale folded into
