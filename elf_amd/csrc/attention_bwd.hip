@@ -961,14 +961,18 @@ using namespace attn;
 struct Splits {
 	int h = 1, q = 1;
 };
-static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal) {
+static int64_t dkv_part_bytes(const Splits& sp, int B, int S, int Hkv, int D) { return sp.h * sp.q > 1 ? (int64_t)sp.h * sp.q * 2 * B * S * Hkv * D * 4 : 0; }
+// room: bytes there are for the partial sums.  Splits are tried in ascending order of what they need, so the room for the one
+// that an unlimited search takes gives that one.
+static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal, int64_t room) {
 	const int nkt = S / 128, G = Hq / Hkv;
 	const int64_t walks = (int64_t)B * Hkv * (causal ? (nkt + 1) / 2 : nkt);
 	const int tiles = causal ? (nkt + 1) * 4 : nkt * 4;  // query tiles of a walk and head (a pair of key tiles has nkt + 1 of four)
 	const float slots = D == 128 ? 256.f : 512.f, step = D == 128 ? 1.2f : 1.1f, fixed = 8.f;
 	Splits best;
-	// From 2^18 query rows (2 x 4096 tokens of 32 heads) up the workspace holds what it always did, the dQ partials and the row
-	// statistics: such launches fill the chip with eight kv heads, and fewer are rare at these sizes.
+	// From 2^18 query rows (2 x 4096 tokens of 32 heads) up walks stay whole.  With eight kv heads or more and several sequences such
+	// launches fill the chip; one sequence of 4096 tokens with 64 / 8 heads (128 walks for 256 compute units) does not, and sharing
+	// has not been measured there.
 	if ((int64_t)B * S * Hq >= 1 << 18) return best;
 	float best_us = 1e30f;
 	for (int h = 1; h <= G; h++) {
@@ -976,6 +980,7 @@ static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal) {
 		for (int q = 1; q <= 4; q *= 2) {
 			if (q > 1 && h < G) continue;
 			const int ns = h * q;
+			if (dkv_part_bytes(Splits{h, q}, B, S, Hkv, D) > room) continue;
 			const float rounds = ceilf((float)(walks * ns) / slots);
 			const float us = rounds * (fixed + (float)(G / h) * ((tiles + q - 1) / q) * step) + (ns > 1 ? 2.f + (float)ns * B * S * Hkv * D * 16 / 5e6f : 0.f);
 			if (us < best_us * (ns > 1 ? 0.95f : 1.f)) best_us = us, best = Splits{h, q};
@@ -983,26 +988,25 @@ static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal) {
 	}
 	return best;
 }
-static int64_t dkv_part_bytes(const Splits& sp, int B, int S, int Hkv, int D) { return sp.h * sp.q > 1 ? (int64_t)sp.h * sp.q * 2 * B * S * Hkv * D * 4 : 0; }
 
+// bf16 dQ partials of every key tile + delta + scaled log-sum-exp: what a backward whose walks stay whole needs.  It grows with
+// each of its arguments, so a buffer for the largest of a caller's shapes serves the smaller ones.
 int64_t attn_bwd_workspace_bytes(int B, int S, int Hq, int D, int causal) {
-	// bf16 dQ partials of every key tile + delta + scaled log-sum-exp + the dK / dV partials of shared walks (150 MB at most):
-	// the most that any number of kv heads and any smaller batch asks for
-	const int64_t per_batch = part_rows(S, causal != 0) * Hq * D * 2 + 2 * (int64_t)S * Hq * 4;
-	int64_t most = B * per_batch;
-	for (int b = 1; b <= B && (int64_t)b * S * Hq < 1 << 18; b++)
-		for (int hkv = 1; hkv <= Hq; hkv++)
-			if (Hq % hkv == 0) {
-				const int64_t n = b * per_batch + dkv_part_bytes(split_walk(b, S, Hq, hkv, D, causal != 0), b, S, hkv, D);
-				if (n > most) most = n;
-			}
-	return most;
+	return (int64_t)B * part_rows(S, causal != 0) * Hq * D * 2 + 2 * (int64_t)B * S * Hq * 4;
+}
+
+// With the partial sums of the walks this shape shares: 2 x 2048 tokens, 16 / 4 heads of 128 143 + 67 MB; 2 x 4096, 32 / 8 heads
+// 1109 MB, whole.  Not monotonic (a shape that shares needs more than the next larger one that does not).
+int64_t attn_bwd_shared_workspace_bytes(int B, int S, int Hq, int Hkv, int D, int causal) {
+	const int64_t whole = attn_bwd_workspace_bytes(B, S, Hq, D, causal);
+	if (Hkv <= 0 || Hq % Hkv != 0) return whole;
+	return whole + dkv_part_bytes(split_walk(B, S, Hq, Hkv, D, causal != 0, INT64_MAX), B, S, Hkv, D);
 }
 
 int attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* dO, const void* lse, void* dq,
              void* dk, void* dv, void* workspace, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo, int64_t lddo,
              int64_t lddq, int64_t lddk, int64_t lddv, int B, int S, int Hq, int Hkv, int D, int causal, float scale,
-             hipStream_t stream, const void* rope_cs) {
+             hipStream_t stream, const void* rope_cs, int64_t workspace_bytes) {
 	ELF_REQUIRE(q && k && v && o && dO && lse && dq && dk && dv && workspace, "attn_bwd: null pointer");
 	ELF_REQUIRE(((uintptr_t)rope_cs % 16) == 0, "attn_bwd: misaligned rotary table");
 	ELF_REQUIRE(B > 0 && S > 0 && S % 128 == 0, "attn_bwd: sequence length must be a multiple of 128 (S=%d)", S);
@@ -1012,6 +1016,8 @@ int attn_bwd(const void* q, const void* k, const void* v, const void* o, const v
 	                lddk % 8 == 0 && lddv % 8 == 0,
 	            "attn_bwd: strides must be multiples of 8");
 	ELF_REQUIRE(((uintptr_t)workspace % 16) == 0, "attn_bwd: misaligned workspace");
+	const int64_t whole = attn_bwd_workspace_bytes(B, S, Hq, D, causal);
+	ELF_REQUIRE(workspace_bytes >= whole, "attn_bwd: a workspace of %lld bytes, %lld are needed", (long long)workspace_bytes, (long long)whole);
 	ELF_REQUIRE(((uintptr_t)o % 16) == 0 && ((uintptr_t)dO % 16) == 0, "attn_bwd: o and dO must be 16-byte aligned");
 	ProfScope prof(PROF_ATTN_BWD, (causal ? 4.0 : 8.0) * B * Hq * (double)S * S * D, stream);
 	const int64_t T = (int64_t)B * S;
@@ -1024,7 +1030,7 @@ int attn_bwd(const void* q, const void* k, const void* v, const void* o, const v
 		ELF_LAUNCH(attn_delta_kernel, dim3((unsigned)(want < 8192 ? want : 8192)), dim3(256), 0, stream, (const bf16_t*)dO,
 	                   (const bf16_t*)o, (const float*)lse, delta, nlse2, lddo, ldo, B, S, Hq, D);
 	}
-	const Splits sp = split_walk(B, S, Hq, Hkv, D, causal != 0);
+	const Splits sp = split_walk(B, S, Hq, Hkv, D, causal != 0, workspace_bytes - whole);
 	float* dkv_part = sp.h * sp.q > 1 ? nlse2 + T * Hq : nullptr;
 	AttnBwdArgs a{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)dO, nlse2, delta, dq_part,
 	              (bf16_t*)dk, (bf16_t*)dv, ldq, ldk, ldv, lddo, lddk, lddv, B, S, Hq, Hkv, scale, (const float2*)rope_cs, sp.h, sp.q, dkv_part};

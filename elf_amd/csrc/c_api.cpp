@@ -108,7 +108,7 @@ int elf_attn_bwd(const void* q, const void* k, const void* v, const void* o, con
                  int64_t lddq, int64_t lddk, int64_t lddv, int B, int S, int Hq, int Hkv, int D, int causal, float scale,
                  void* stream) {
 	return elf::attn_bwd(q, k, v, o, dO, lse, dq, dk, dv, workspace, ldq, ldk, ldv, ldo, lddo, lddq, lddk, lddv, B, S, Hq,
-	                     Hkv, D, causal, scale, S_(stream));
+	                     Hkv, D, causal, scale, S_(stream), nullptr, elf::attn_bwd_workspace_bytes(B, S, Hq, D, causal));
 }
 
 int elf_attn_bwd_rope(const void* q, const void* k, const void* v, const void* o, const void* dO, const void* lse, void* dq,
@@ -116,7 +116,16 @@ int elf_attn_bwd_rope(const void* q, const void* k, const void* v, const void* o
                       int64_t lddq, int64_t lddk, int64_t lddv, int B, int S, int Hq, int Hkv, int D, int causal, float scale,
                       const void* cs, void* stream) {
 	return elf::attn_bwd(q, k, v, o, dO, lse, dq, dk, dv, workspace, ldq, ldk, ldv, ldo, lddo, lddq, lddk, lddv, B, S, Hq,
-	                     Hkv, D, causal, scale, S_(stream), cs);
+	                     Hkv, D, causal, scale, S_(stream), cs, elf::attn_bwd_workspace_bytes(B, S, Hq, D, causal));
+}
+
+int64_t elf_attn_bwd_shared_workspace_bytes(int B, int S, int Hq, int Hkv, int D, int causal) { return elf::attn_bwd_shared_workspace_bytes(B, S, Hq, Hkv, D, causal); }
+int elf_attn_bwd_shared(const void* q, const void* k, const void* v, const void* o, const void* dO, const void* lse, void* dq,
+                        void* dk, void* dv, void* workspace, int64_t workspace_bytes, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo,
+                        int64_t lddo, int64_t lddq, int64_t lddk, int64_t lddv, int B, int S, int Hq, int Hkv, int D, int causal,
+                        float scale, const void* cs, void* stream) {
+	return elf::attn_bwd(q, k, v, o, dO, lse, dq, dk, dv, workspace, ldq, ldk, ldv, ldo, lddo, lddq, lddk, lddv, B, S, Hq,
+	                     Hkv, D, causal, scale, S_(stream), cs, workspace_bytes);
 }
 
 int elf_hbm_probe(int mode, const void* src, void* dst, int64_t bytes, void* stream) { return elf::hbm_probe(mode, src, dst, bytes, S_(stream)); }

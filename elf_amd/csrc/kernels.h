@@ -160,10 +160,13 @@ int cross_entropy_reduce(const void* row_loss, const void* target, int64_t rows,
 int attn_fwd(const void* q, const void* k, const void* v, void* o, void* lse, int64_t ldq, int64_t ldk, int64_t ldv,
              int64_t ldo, int B, int S, int Hq, int Hkv, int D, int causal, float scale, hipStream_t stream);
 int64_t attn_bwd_workspace_bytes(int B, int S, int Hq, int D, int causal);
+int64_t attn_bwd_shared_workspace_bytes(int B, int S, int Hq, int Hkv, int D, int causal);
+// workspace_bytes: what lies at `workspace`, at least attn_bwd_workspace_bytes(); what it holds beyond that is used for the
+// partial sums of shared walks, and a launch shares its walks only as far as they fit.
 int attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* dO, const void* lse, void* dq,
              void* dk, void* dv, void* workspace, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo, int64_t lddo,
              int64_t lddq, int64_t lddk, int64_t lddv, int B, int S, int Hq, int Hkv, int D, int causal, float scale,
-             hipStream_t stream, const void* rope_cs = nullptr);
+             hipStream_t stream, const void* rope_cs, int64_t workspace_bytes);
 // rope_cs non-null: q and k are the rotated heads (rope_apply with this table); dq and dk come out as the gradients
 // of the heads before the rotation (rope_apply's backward applied to them), bit-identical to the separate pass.
 

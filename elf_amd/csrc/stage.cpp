@@ -124,6 +124,7 @@ struct Stage {
 	float* norm_ws = nullptr;  // partial sums of norm_slots norm backwards
 	int norm_slots = 1;
 	void* attn_ws = nullptr;
+	int64_t attn_ws_bytes = 0;
 	int64_t ws_bytes = 0;  // fixed device workspaces of the stage (norm / attention backward scratch, rope table, gradient sink)
 	// pinned blocks of released micro-batches whose last copy may still be in flight: they go back to the arena
 	// when their event has fired (polled, never waited for inside a step unless the arena would have to grow)
@@ -515,7 +516,7 @@ static int run_backward(Stage* s, MbState& m, const void* dy, void* dx, bool gra
 			// the llama block's q and k carry the rotary embedding: its backward is applied to dQ and dK where they are stored
 			ELF_TRY(attn_bwd(q, q + ko, q + vo, bs.b[B_O].p, d_o.p, bs.b[B_LSE].p, dq, dq + ko, dq + vo, s->attn_ws, s->nqkv, s->nqkv, s->nqkv,
 			                 s->Hq * s->D, s->Hq * s->D, s->nqkv, s->nqkv, s->nqkv, s->B, s->S, s->Hq, s->Hkv, s->D, s->cfg.causal, scale, st,
-			                 s->llama ? s->rope_cs : nullptr));
+			                 s->llama ? s->rope_cs : nullptr, s->attn_ws_bytes));
 		}
 		d_o.release();
 		if (!(grads_only && i == 0)) {
@@ -785,11 +786,12 @@ int elf_stage_create(const elf_stage_cfg* cfg, elf_stage_t** out) {
 	// cache).  The fold of wider rows moves more than its launch costs, and each takes the one workspace in turn.
 	s->norm_slots = s->d > 2048 ? 1 : std::min(NORM_FOLD_MAX, 2 * cfg->n_blocks + 1);
 	const size_t norm_ws_bytes = (size_t)norm_bwd_workspace_floats(s->T, s->d) * 4 * s->norm_slots;
-	const size_t attn_ws_bytes = (size_t)attn_bwd_workspace_bytes(s->B, s->S, s->Hq, s->D, s->cfg.causal);
+	// for every size of micro-batch the most its shared walks use: a shorter one may share more than a full one
+	for (int b = 1; b <= s->B; b++) s->attn_ws_bytes = std::max(s->attn_ws_bytes, attn_bwd_shared_workspace_bytes(b, s->S, s->Hq, s->Hkv, s->D, s->cfg.causal));
 	const size_t rope_bytes = s->llama ? (size_t)s->S * (s->D / 2) * 8 : 0;
-	s->ws_bytes = (int64_t)(norm_ws_bytes + attn_ws_bytes + rope_bytes);
+	s->ws_bytes = (int64_t)(norm_ws_bytes + s->attn_ws_bytes + rope_bytes);
 	if (hipMalloc((void**)&s->norm_ws, norm_ws_bytes) != hipSuccess) return fail("norm workspace");
-	if (hipMalloc(&s->attn_ws, attn_ws_bytes) != hipSuccess) return fail("attention workspace");
+	if (hipMalloc(&s->attn_ws, s->attn_ws_bytes) != hipSuccess) return fail("attention workspace");
 	if (s->llama) {
 		if (hipMalloc(&s->rope_cs, rope_bytes) != hipSuccess) return fail("rope table");
 		if (rope_table(s->rope_cs, s->S, s->D, cfg->rope_theta, nullptr) != 0) return fail("rope table fill");

@@ -266,14 +266,11 @@ def attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal, scale=None, rope_cs=None
 	T, ld = qkv.shape[0], qkv.stride(0)
 	scale = scale if scale is not None else 1.0 / math.sqrt(D)
 	lib = _lib.load()
-	ws = torch.empty(lib.elf_attn_bwd_workspace_bytes(B, S, Hq, D, int(causal)), dtype=torch.uint8, device=qkv.device)
+	ws = torch.empty(lib.elf_attn_bwd_shared_workspace_bytes(B, S, Hq, Hkv, D, int(causal)), dtype=torch.uint8, device=qkv.device)
 	dqkv = torch.empty_like(qkv)
 	q, k, v = qkv[:, : Hq * D], qkv[:, Hq * D : (Hq + Hkv) * D], qkv[:, (Hq + Hkv) * D :]
 	dq, dk, dv = dqkv[:, : Hq * D], dqkv[:, Hq * D : (Hq + Hkv) * D], dqkv[:, (Hq + Hkv) * D :]
-	args = (_ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(do), _ptr(lse), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(ws),
-	        ld, ld, ld, o.stride(0), do.stride(0), dqkv.stride(0), dqkv.stride(0), dqkv.stride(0), B, S, Hq, Hkv, D, int(causal), scale)
-	if rope_cs is None:
-		_lib.check(lib.elf_attn_bwd(*args, _stream()), "elf_attn_bwd")
-	else:
-		_lib.check(lib.elf_attn_bwd_rope(*args, _ptr(rope_cs), _stream()), "elf_attn_bwd_rope")
+	rc = lib.elf_attn_bwd_shared(_ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(do), _ptr(lse), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(ws), ws.numel(),
+	                             ld, ld, ld, o.stride(0), do.stride(0), dqkv.stride(0), dqkv.stride(0), dqkv.stride(0), B, S, Hq, Hkv, D, int(causal), scale, _ptr(rope_cs), _stream())
+	_lib.check(rc, "elf_attn_bwd_shared")
 	return dqkv

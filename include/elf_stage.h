@@ -206,9 +206,8 @@ int elf_cross_entropy_reduce(const void* row_loss, const void* target, int64_t r
  * elf_attn_bwd_workspace_bytes() of 16-byte aligned scratch (the bf16 partial dQ of every 128-key tile,
  * which a second kernel sums in fp32 in a fixed order — no atomics, run-to-run identical gradients —
  * plus two fp32 values per query and head): B * S * (S/128 + 1) / 2 * Hq * D * 2 bytes with a causal
- * mask, B * S * (S/128) * Hq * D * 2 without, + 8 * B * S * Hq, and where a batch or a group of kv heads is too small to
- * fill the chip, fp32 partial sums of dK and dV (about 150 MB at most; they too are added in a fixed order).  The size
- * covers every Hkv that divides Hq and every smaller batch. */
+ * mask, B * S * (S/128) * Hq * D * 2 without, + 8 * B * S * Hq.  Every term grows with every argument: a buffer for the
+ * largest shape serves the smaller ones. */
 int elf_attn_fwd(const void* q, const void* k, const void* v, void* o, void* lse, int64_t ldq,
                  int64_t ldk, int64_t ldv, int64_t ldo, int B, int S, int Hq, int Hkv, int D,
                  int causal, float scale, void* stream);
@@ -229,6 +228,18 @@ int elf_attn_bwd_rope(const void* q, const void* k, const void* v, const void* o
                       int64_t ldk, int64_t ldv, int64_t ldo, int64_t lddo, int64_t lddq, int64_t lddk,
                       int64_t lddv, int B, int S, int Hq, int Hkv, int D, int causal, float scale,
                       const void* cs, void* stream);
+
+/* elf_attn_bwd_rope that is told how large its workspace is (at least elf_attn_bwd_workspace_bytes(), else it is refused).
+ * Where a batch or a group of kv heads is too small to fill the chip, the walk over a group's query heads and their queries
+ * is shared by several workgroups, which leave dK and dV as fp32 partial sums (added in a fixed order) in what the workspace
+ * holds beyond that: 2 x 2048 tokens, 16 / 4 heads of 128 160 us instead of 346.  elf_attn_bwd_shared_workspace_bytes(): the
+ * size with which a shape shares as much as pays (h * q * 8 * B * S * Hkv * D bytes more for a walk shared h * q ways);
+ * with less it shares less.  The size decides in which order partial sums are added, and with it the rounding of dK and dV. */
+int64_t elf_attn_bwd_shared_workspace_bytes(int B, int S, int Hq, int Hkv, int D, int causal);
+int elf_attn_bwd_shared(const void* q, const void* k, const void* v, const void* o, const void* dO, const void* lse,
+                        void* dq, void* dk, void* dv, void* workspace, int64_t workspace_bytes, int64_t ldq, int64_t ldk,
+                        int64_t ldv, int64_t ldo, int64_t lddo, int64_t lddq, int64_t lddk, int64_t lddv, int B, int S,
+                        int Hq, int Hkv, int D, int causal, float scale, const void* cs, void* stream);
 
 /* ---------------------------------------------------------------------------------------------
  * Stage executor: one pipeline stage = n_blocks transformer blocks on T = mb * seq tokens.

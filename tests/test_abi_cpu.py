@@ -62,6 +62,40 @@ def test_argument_errors_without_device(lib):
 	assert lib.elf_attn_bwd_workspace_bytes(2, 4096, 32, 128, 1) == 2 * sum(4096 - 128 * kt for kt in range(32)) * 32 * 128 * 2 + stats
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal", [0, 1])
+def test_attention_workspace_of_a_larger_shape_serves_the_smaller_ones(lib, D, causal):
+	"""The size is the header's formula at every shape, whether its walks would be shared or not, and grows with every argument:
+	elf_attn_bwd is not told how large its buffer is, and a caller keeps one for its longest sequence."""
+	heads, batches, tiles = (1, 2, 4, 6, 8, 16, 32), (1, 2, 3, 4, 8), (1, 2, 3, 7, 15, 16, 17, 31, 32, 33, 64)
+	size = {}
+	for B in batches:
+		for nkt in tiles:
+			for Hq in heads:
+				S = 128 * nkt
+				rows = S * (nkt + 1) // 2 if causal else S * nkt
+				size[B, nkt, Hq] = lib.elf_attn_bwd_workspace_bytes(B, S, Hq, D, causal)
+				assert size[B, nkt, Hq] == B * rows * Hq * D * 2 + 8 * B * S * Hq, (B, S, Hq)
+				for Hkv in (h for h in heads if Hq % h == 0):
+					more = lib.elf_attn_bwd_shared_workspace_bytes(B, S, Hq, Hkv, D, causal) - size[B, nkt, Hq]
+					# room for a whole number of splits, four per query head at most
+					assert more >= 0 and more % (8 * B * S * Hkv * D) == 0 and more // (8 * B * S * Hkv * D) <= 4 * Hq // Hkv
+	for (B, nkt, Hq), n in size.items():
+		for axis, values in enumerate((batches, tiles, heads)):
+			key = [B, nkt, Hq]
+			i = values.index(key[axis])
+			if i:
+				key[axis] = values[i - 1]
+				assert size[tuple(key)] < n
+	assert lib.elf_attn_bwd_workspace_bytes(2, 4096, 8, D, 0) > lib.elf_attn_bwd_workspace_bytes(2, 4096, 8, D, 1)
+
+
+def test_attention_backward_refuses_a_workspace_that_is_too_small(lib):
+	n = lib.elf_attn_bwd_workspace_bytes(1, 128, 4, 64, 1)
+	rc = lib.elf_attn_bwd_shared(*[16] * 10, n - 1, *[64 * 12] * 8, 1, 128, 4, 4, 64, 1, 0.125, None, None)
+	assert rc == -1 and str(n).encode() in lib.elf_last_error()
+
+
 def test_stage_create_rejects_bad_configs(lib):
 	from elf_amd.execution.block import StageConfig
 

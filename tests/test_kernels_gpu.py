@@ -530,6 +530,38 @@ def test_attention_backward_with_walks_shared_by_workgroups(K, cfg):
 	assert sizes == sorted(sizes)
 
 
+@pytest.mark.parametrize("cfg", [(1, 4096, 4, 4, 64, False), (2, 2048, 8, 4, 64, False), (1, 896, 8, 1, 128, True)])
+@pytest.mark.parametrize("ways", [None, 1, 2, 3, 64])
+def test_attention_backward_stays_inside_its_workspace(K, cfg, ways):
+	"""Shapes whose walks are shared where there is room: the entry point that is not told its workspace's size (ways None) keeps
+	to the size the formula gives, elf_attn_bwd_shared to the partial sums of at most `ways` parts that it is given room for.
+	What lies behind the workspace keeps its value; the gradients are those of autograd in fp32."""
+	from elf_amd import _lib
+
+	B, S, Hq, Hkv, D, causal = cfg
+	lib, T = _lib.load(), B * S
+	whole = lib.elf_attn_bwd_workspace_bytes(B, S, Hq, D, int(causal))
+	assert lib.elf_attn_bwd_shared_workspace_bytes(B, S, Hq, Hkv, D, int(causal)) > whole, "a shape whose walks are shared"
+	part = 8 * B * S * Hkv * D
+	n = whole if ways in (None, 1) else whole + ways * part
+	ws = torch.full((n + 8 * part,), 0x5A, dtype=torch.uint8, device="cuda")  # as much again as eight parts behind it
+	qkv, do = _randn(T, (Hq + 2 * Hkv) * D, seed=57), _randn(T, Hq * D, seed=58)
+	o_ref, _, dqkv_ref = _attn_ref(qkv, B, S, Hq, Hkv, D, causal, do)
+	o, lse = K.attn_fwd(qkv, B, S, Hq, Hkv, D, causal)
+	dqkv = torch.empty_like(qkv)
+	ld, at = qkv.stride(0), [0, 2 * Hq * D, 2 * (Hq + Hkv) * D]  # q, k, v: byte offsets in a row
+	stream = torch.cuda.current_stream().cuda_stream
+	ptrs = [qkv.data_ptr() + a for a in at] + [o.data_ptr(), do.data_ptr(), lse.data_ptr()] + [dqkv.data_ptr() + a for a in at] + [ws.data_ptr()]
+	rest = [ld, ld, ld, Hq * D, Hq * D, ld, ld, ld, B, S, Hq, Hkv, D, int(causal), 1 / math.sqrt(D)]
+	if ways is None:
+		_lib.check(lib.elf_attn_bwd(*ptrs, *rest, stream), "elf_attn_bwd")
+	else:
+		_lib.check(lib.elf_attn_bwd_shared(*ptrs, n, *rest, None, stream), "elf_attn_bwd_shared")
+	assert bool((ws[n:] == 0x5A).all()), "wrote behind its workspace"
+	for name, sl in (("dq", slice(0, Hq * D)), ("dk", slice(Hq * D, (Hq + Hkv) * D)), ("dv", slice((Hq + Hkv) * D, None))):
+		_close(dqkv[:, sl], dqkv_ref[:, sl], rel_fro=1.5e-2, what=f"attn {name} {cfg} {ways}")
+
+
 @pytest.mark.parametrize("D,causal,ramp,gain", [(128, True, 6.0, 1.0), (128, False, 6.0, 1.0), (64, True, 6.0, 1.0), (128, True, 0.0, 6.0),
                                                (128, False, -6.0, 3.0), (64, False, 0.0, 6.0)])
 def test_attention_forward_with_scores_that_climb_along_the_keys(K, D, causal, ramp, gain):
