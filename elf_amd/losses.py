@@ -53,7 +53,7 @@ def _run(pred, target, *, ignore_index, scale, mean, want_grad, padded=True):
 	multiple of 64, or, unless ``padded``, [rows, V] where the logits are one dense block: rows that start at any address are
 	then read in place (50257 columns: the padded copy of the logits took half of a loss's time)."""
 	V = pred.shape[-1]
-	dense = (not padded if want_grad else V % 8 != 0) and pred.dtype == torch.bfloat16 and pred.is_cuda and pred.is_contiguous() and pred.data_ptr() % 16 == 0 and 0 < V <= _DENSE_MAX
+	dense = (not padded if want_grad else V % 8 != 0) and pred.dtype == torch.bfloat16 and pred.is_cuda and pred.is_contiguous() and not pred.is_neg() and pred.data_ptr() % 16 == 0 and 0 < V <= _DENSE_MAX
 	src, ld = (pred, V) if dense else _rows_view(pred, V)
 	rows = pred.numel() // V
 	target = _check_target(target, rows)
@@ -94,6 +94,13 @@ def _reduced(row_loss, out2, reduction, shape):
 	raise ValueError(f"{reduction} is not a valid value for reduction")
 
 
+def _plain(t):
+	"""Whether a kernel may read ``t`` through its pointer: under vmap it is a batch without storage of its own, and a view
+	such as ``z.conj().imag`` holds its values negated."""
+	return (type(t) is torch.Tensor and torch._C._has_storage(t) and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+	        and not t.is_neg() and not t._is_zerotensor())
+
+
 class _CrossEntropy(torch.autograd.Function):
 	@staticmethod
 	def forward(ctx, pred, target, reduction, ignore_index):
@@ -105,7 +112,7 @@ class _CrossEntropy(torch.autograd.Function):
 	def backward(ctx, g):
 		V = ctx.shape[-1]
 		grad = ctx.grad
-		if grad.shape[1] == V and g.dim() == 0 and g.dtype == torch.float32 and not (torch.is_grad_enabled() and g.requires_grad):
+		if _plain(g) and grad.shape[1] == V and g.dim() == 0 and g.dtype == torch.float32 and not (torch.is_grad_enabled() and g.requires_grad):
 			# one pass of 16-byte accesses with the same roundings (2048 x 50257: 71 us, 82 as a torch product of the strided view)
 			out = torch.empty(ctx.shape, dtype=grad.dtype, device=grad.device)
 			_lib.check(_lib.load().elf_scale_by_bf16(grad.data_ptr(), g.data_ptr(), out.data_ptr(), out.numel(), _stream()), "elf_scale_by_bf16")

@@ -90,6 +90,27 @@ def test_cross_entropy_dense_rows_of_any_width(V, offset):
 	assert torch.equal(twice, grad * -2)
 
 
+@pytest.mark.parametrize("V", [1000, 1003])
+def test_cross_entropy_gradients_for_a_batch_of_incoming_gradients(V):
+	"""``is_grads_batched``: the backward is run once under vmap, with an incoming gradient that has no storage of its own; and an
+	incoming gradient whose storage holds something else than its value."""
+	from elf_amd import losses
+
+	x, t, xg = _case(11, V, seed=V)
+	xg = xg.detach().clone().requires_grad_()
+	loss = losses.cross_entropy(xg, t.cuda())
+	(one,) = torch.autograd.grad(loss, xg, retain_graph=True)
+	g = torch.tensor([1.0, -2.0, 0.5]).cuda()
+	(many,) = torch.autograd.grad(loss, xg, grad_outputs=g, is_grads_batched=True)
+	assert tuple(many.shape) == (3, 11, V)
+	for i in range(3):
+		assert torch.equal(many[i], one * g[i].to(torch.bfloat16))
+	lazy = torch.tensor(3 - 2j).cuda().conj().imag  # 2, kept as the negation of -2
+	assert lazy.is_neg() and lazy.item() == 2
+	(twice,) = torch.autograd.grad(loss, xg, grad_outputs=lazy)
+	assert torch.equal(twice, one * 2)
+
+
 def test_cross_entropy_rejects_what_it_cannot_run_and_flags_bad_targets():
 	from elf_amd import _lib, losses
 
