@@ -228,8 +228,11 @@ int gemm_rope_bf16(int M, int N, int K, const void* A, int64_t lda, const void* 
 	return n_rot_heads ? rope_apply(C, cs, M, S, (int)ldc, n_rot_heads, D, 0, stream) : 0;
 }
 
+// What the fused kernel can run at all (a caller without scratch or with strided buffers relies on it) ...
+static bool swiglu_bwd_fits(int M, int F, int K) { return M >= 256 && F >= 256 && M % 64 == 0 && F % 64 == 0 && K % 64 == 0; }
+// ... and where it is also the faster way.
 bool gemm_swiglu_bwd_fused(int M, int F, int K) {
-	if (!(M >= 256 && F >= 256 && M % 64 == 0 && F % 64 == 0 && K % 64 == 0)) return false;
+	if (!swiglu_bwd_fits(M, F, K)) return false;
 	// 256x256 tiles only: against the best tile of the plain product and the pass over d, g, u and their gradients (the
 	// epilogue itself reads and writes four of those five at 256 tiles a time)
 	const float rounds = (float)(((int64_t)((M + 255) / 256) * ((F + 255) / 256) + 255) / 256);
@@ -239,7 +242,8 @@ bool gemm_swiglu_bwd_fused(int M, int F, int K) {
 int gemm_swiglu_bwd_bf16(int M, int F, int K, const void* dY, int64_t lddy, const void* W, int64_t ldw, const void* gu,
                          int64_t ldgu, void* dgu, int64_t lddgu, void* scratch, hipStream_t stream, void* act, int64_t ldact) {
 	ELF_REQUIRE(M > 0 && F > 0 && K > 0 && dY && W && gu && dgu, "gemm_swiglu_bwd: empty problem or null operand");
-	if (gemm_swiglu_bwd_fused(M, F, K) && lddy >= K && ldw >= F && ldgu >= 2 * F && lddgu >= 2 * F && lddy % 8 == 0 && ldw % 8 == 0 && ldgu % 8 == 0 &&
+	const bool apart = scratch && ldgu == 2 * F && lddgu == 2 * F && (!act || ldact == F);  // what the separate passes need
+	if ((apart ? gemm_swiglu_bwd_fused(M, F, K) : swiglu_bwd_fits(M, F, K)) && lddy >= K && ldw >= F && ldgu >= 2 * F && lddgu >= 2 * F && lddy % 8 == 0 && ldw % 8 == 0 && ldgu % 8 == 0 &&
 	    lddgu % 8 == 0 && ((uintptr_t)dY % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)gu % 16) == 0 && ((uintptr_t)dgu % 16) == 0) {
 		// the activation backward's arithmetic is not counted: the figure stays the GEMM's
 		ProfScope prof(PROF_GEMM, 2.0 * M * F * K, stream);

@@ -88,9 +88,9 @@ int elf_gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, 
 /* Backward of the down-projection into the SwiGLU: d = dY W with dY [M, K] and W [K, F] (the down
  * projection's weight [d_model, F] as it lies in memory), then dgu[M, 2F] = [d silu'(g) u | d silu(g)]
  * from the saved gu[M, 2F] = [g | u].  One kernel (activation backward in the GEMM epilogue, d never
- * reaches memory) where 256x256 tiles are the faster choice (sizes multiples of 64, M and F at least 256); otherwise
- * elf_gemm_bf16(0, 1, ...) into scratch [M, F] followed by elf_swiglu_bwd (scratch may be null only for
- * the fused shapes).  Same bits either way.
+ * reaches memory) or elf_gemm_bf16(0, 1, ...) into scratch [M, F] followed by elf_swiglu_bwd, whichever is faster.  The one
+ * kernel runs every M and F of at least 256 (sizes multiples of 64, leading dimensions of 8, 16-byte aligned operands): there
+ * scratch may be null and gu / dgu may have rows further apart than 2 F, and it is then taken.  Same bits either way.
  * Replaces: LinearDX.backward of fc2 (elf/zb_utils.py:29-41) followed by autograd's backward of
  *           silu(gate) * up; no reference module for SwiGLU. */
 int elf_gemm_swiglu_bwd_bf16(int M, int F, int K, const void* dY, int64_t lddy, const void* W, int64_t ldw,

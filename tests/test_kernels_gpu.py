@@ -419,6 +419,24 @@ def test_gemm_with_activation_strided_outputs(K):
 	assert pre[:, 2 * F :].abs().max().item() == 0 and out[:, F:].abs().max().item() == 0
 
 
+@pytest.mark.parametrize("dims", [(1024, 16640, 8192), (8192, 2304, 8192), (256, 256, 64), (320, 448, 128)])
+@pytest.mark.parametrize("strided", [False, True])
+def test_swiglu_backward_without_scratch_at_any_size_a_tile_fits(K, dims, strided):
+	"""M and F of at least 256: neither scratch nor dense buffers are needed, also where the product and the activation backward
+	one after the other are faster (1024 x 16640 x 8192: 260 tiles on 256 compute units).  The same bits as those two."""
+	from elf_amd import _lib
+
+	M, F, Kd = dims
+	dy, w2, gu = _randn(M, Kd, seed=47), _randn(Kd, F, seed=48, scale=0.05), _randn(M, 2 * F, seed=49)
+	pad = 8 if strided else 0
+	gin, dgu = torch.zeros(M, 2 * F + pad, dtype=torch.bfloat16, device="cuda"), torch.zeros(M, 2 * F + pad, dtype=torch.bfloat16, device="cuda")
+	gin[:, : 2 * F] = gu
+	_lib.check(_lib.load().elf_gemm_swiglu_bwd_bf16(M, F, Kd, dy.data_ptr(), Kd, w2.data_ptr(), F, gin.data_ptr(), gin.stride(0), dgu.data_ptr(), dgu.stride(0), None,
+	                                                torch.cuda.current_stream().cuda_stream), "elf_gemm_swiglu_bwd_bf16")
+	assert torch.equal(dgu[:, : 2 * F], K.gemm_swiglu_bwd(dy, w2, gu, fused=False))
+	assert dgu[:, 2 * F :].float().abs().sum().item() == 0
+
+
 def _rope_ref(x, S, D, theta):
 	# x: [T, H, D] fp32; half-split rotation, angles in fp64
 	T = x.shape[0]
