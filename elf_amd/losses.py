@@ -8,6 +8,7 @@ the reference transformer's loss (benchmarks/models/simple.py:520-524): logits f
 """
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -96,9 +97,10 @@ def _reduced(row_loss, out2, reduction, shape):
 
 def _plain(t):
 	"""Whether a kernel may read ``t`` through its pointer: under vmap it is a batch without storage of its own, and a view
-	such as ``z.conj().imag`` holds its values negated."""
+	such as ``z.conj().imag`` holds its values negated.  Nor may it where somebody follows the operations on ``t``: in a
+	forward-mode level (a tangent) or under a dispatch mode (a trace)."""
 	return (type(t) is torch.Tensor and torch._C._has_storage(t) and not torch._C._functorch.is_functorch_wrapped_tensor(t)
-	        and not t.is_neg() and not t._is_zerotensor())
+	        and not t.is_neg() and not t._is_zerotensor() and forward_ad._current_level < 0 and not torch._C._len_torch_dispatch_stack())
 
 
 class _CrossEntropy(torch.autograd.Function):
