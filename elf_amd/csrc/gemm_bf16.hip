@@ -92,7 +92,9 @@ static Plan plan_weight_gradient(int M, int N, int K) {
 	return best;
 }
 
-// 256 or 128: the direct-to-LDS tile of 256 columns a forward / input-gradient product runs on, 0: one of the ring tiles.
+// 256 or 128: the direct-to-LDS tile of 256 columns a forward / input-gradient product runs on, 0: one of the ring tiles
+// (never with ring_extra = NO_RING, unless no tile of 256 columns fits).
+constexpr float NO_RING = 1e20f;
 static int dma_tile_rows(int M, int N, int K, float ring_extra) {
 	const Plan p = plan_tiles(false, M, N, K, ring_extra);
 	return p.dma() ? p.bm : 0;
@@ -176,7 +178,8 @@ int gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, cons
 	int bm = 0;
 	if (act == ACT_SWIGLU && M % 64 == 0 && F % 64 == 0 && K % 64 == 0 && lda % 8 == 0 && ldw % 8 == 0 && ldpre >= N && ldout >= F && ldpre % 8 == 0 && ldout % 8 == 0 &&
 	    ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)pre % 16) == 0 && ((uintptr_t)out % 16) == 0 && lda >= K && ldw >= K) {
-		bm = dma_tile_rows(M, N, K, pass_us(6.0 * M * F));
+		// rows that lie further apart only the fused kernel writes
+		bm = dma_tile_rows(M, N, K, ldpre == N && ldout == F ? pass_us(6.0 * M * F) : NO_RING);
 	}
 	if (bm) {
 		ProfScope prof(PROF_GEMM, 2.0 * M * N * K, stream);

@@ -402,11 +402,13 @@ def test_gemm_with_rope_epilogue(K, shape):
 	_close(got[:, :nrot], ref, what="rotated projection")
 
 
-def test_gemm_with_activation_strided_outputs(K):
-	# outputs that are column slices of wider buffers, as a caller that packs activations would pass
+@pytest.mark.parametrize("dims", [(1024, 2048, 128), (512, 4096, 1664), (256, 8192, 1024), (128, 128, 64), (192, 320, 128), (576, 192, 192)])
+def test_gemm_with_activation_strided_outputs(K, dims):
+	"""Outputs that are column slices of wider buffers, as a caller that packs activations would pass: at every M and F of at least
+	128, also where the product and the activation one after the other are faster.  The same bits as those two."""
 	from elf_amd import _lib
 
-	M, F, Kd = 1024, 2048, 128
+	M, F, Kd = dims
 	A = _randn(M, Kd, seed=43)
 	W = _randn(2 * F, Kd, seed=44, scale=0.12)
 	pre = torch.zeros(M, 2 * F + 64, dtype=torch.bfloat16, device="cuda")
@@ -416,6 +418,7 @@ def test_gemm_with_activation_strided_outputs(K):
 	_lib.check(rc, "elf_gemm_act_bf16")
 	p2, o2 = K.gemm_act(A, W, K.ACT_SWIGLU)
 	assert torch.equal(pre[:, : 2 * F], p2) and torch.equal(out[:, :F], o2)
+	assert torch.equal(p2, K.gemm(A, W)) and torch.equal(o2, K.swiglu_fwd(p2))
 	assert pre[:, 2 * F :].abs().max().item() == 0 and out[:, F:].abs().max().item() == 0
 
 
