@@ -63,6 +63,25 @@ def test_cross_entropy_loss_and_gradient(rows, V, ld):
 	_check_grad(xa.grad, xf.grad * (3.0 / live), 3.0 / live)
 
 
+@pytest.mark.parametrize("rows,V,ld", [(9, 3, 8), (300, 1003, 1024), (37, 1230, 1232), (5, 4095, 4160), (7, 16381, 16384), (6, 20003, 20032), (3, 65533, 65536), (3, 100001, 100008)])
+def test_last_columns_of_rows_no_chunk_divides(rows, V, ld):
+	"""V that is no multiple of 8, in rows that lie ld apart with NaN between them: every register depth, the target and infinities
+	in the last columns, and zeros from column V to the end of the gradient's rows."""
+	from elf_amd import losses
+
+	x, t, xg = _case(rows, V, seed=V, ld=ld)
+	x[0, V - 1] = xg[0, V - 1] = float("-inf")
+	t[0] = 1  # (not ignored)
+	t[rows - 1] = V - 1
+	xf = x.float().requires_grad_()
+	L.cross_entropy_ref(xf, t, "sum").backward()
+	loss, grad = losses.cross_entropy.loss_and_grad(xg, t.cuda(), reduction="sum")
+	assert float(loss) == pytest.approx(float(L.cross_entropy_ref(x, t, "sum")), rel=1e-5)
+	_check_grad(grad, xf.grad, 1.0)
+	base = torch.as_strided(grad, (rows, grad.stride(0)), (grad.stride(0), 1))
+	assert base[:, V:].float().abs().sum().item() == 0
+
+
 # dense rows that start at every 2-byte phase (odd widths), at the widest of each register depth and one beyond it, and a base
 # that is not 16-byte aligned (the padded copy)
 @pytest.mark.parametrize("V", [1, 7, 9, 1017, 1018, 4089, 4091, 16377, 16379, 32761, 32763, 65529, 65531, 131065, 131067])
