@@ -38,20 +38,24 @@ int gemm_turn_giveups(uint64_t* out) {
 
 // ------------------------------------------------------------------------------------------
 // Tile choice.  Estimated time of a product on tiles of bm x bn: rounds of 256 workgroups (one per compute unit) times the
-// time of a K slice of 64 times the slices, plus what a round costs besides (filling the ring, the epilogue).  The constants
-// are microseconds fitted to cold-operand timings of 33 shapes from 512 x 512 x 512 to 4096 x 50304 x 768 (operands rotated
-// through more than the 256 MB cache); the estimate is within 15 % of nearly all of them.  A large tile has the cheaper products (per slice
+// time of a K slice of 64 times the slices and what a round costs besides (filling the ring, the epilogue), plus what a launch
+// costs once.  The constants are microseconds, the bf16 ones fitted to cold-operand timings of 33 shapes from 512 x 512 x 512 to
+// 4096 x 50304 x 768, those of the weight gradients to every tile and split on 2100 shapes from 64 x 64 x 64 to 8192 x 8192 x
+// 16384 (the tile and split that are picked take 0.4 % longer than the best on average).  A large tile has the cheaper products (per slice
 // and output: 22 ps on 256x256, 26 on 128x256, 35 on 128x128, 66 on 64x64: the smaller the tile, the more operand bytes go
 // through the 64 B/clk path into LDS for each product) and loses where its tiles leave compute units idle:
 //   1920 x 1600 x 1600: 44 us on 56 tiles of 256x256, 27 on 105 of 128x256, 19.9 on 195 of 128x128, 25 on 750 of 64x64;
 //   1920 x 4800 x 1600: 46 us on 152 tiles of 256x256, 52 on 285 of 128x256, 49 on 570 of 128x128.
 struct TileTime {
 	int bm, bn;
-	float slice, round;
+	float slice, round, launch;
 };
-static constexpr TileTime TILES_BF16[] = {{256, 256, 1.45f, 6.f}, {128, 256, 0.854f, 5.5f}, {128, 128, 0.58f, 4.f}, {64, 128, 0.38f, 2.f}, {128, 64, 0.40f, 2.f}, {64, 64, 0.27f, 1.3f}};
+static constexpr int N_TILES = 6;
+static constexpr TileTime TILES_BF16[N_TILES] = {{256, 256, 1.45f, 0.f, 6.f}, {128, 256, 0.854f, 5.5f, 0.f}, {128, 128, 0.58f, 4.f, 0.f},
+                                                 {64, 128, 0.38f, 2.f, 0.f}, {128, 64, 0.40f, 2.f, 0.f}, {64, 64, 0.27f, 1.3f, 0.f}};
 // weight gradients: both operands reduction-major, fp32 read-modify-write of the output
-static constexpr TileTime TILES_F32[] = {{256, 256, 1.33f, 20.f}, {128, 256, 0.79f, 11.f}, {128, 128, 0.55f, 5.f}, {64, 128, 0.44f, 2.f}, {128, 64, 0.44f, 2.f}, {64, 64, 0.30f, 1.5f}};
+static constexpr TileTime TILES_F32[N_TILES] = {{256, 256, 1.3f, 22.f, 0.f}, {128, 256, 0.757f, 12.9f, 0.f}, {128, 128, 0.537f, 9.9f, 0.f},
+                                                {64, 128, 0.442f, 5.9f, 0.f}, {128, 64, 0.416f, 7.5f, 0.f}, {64, 64, 0.26f, 4.f, 0.f}};
 
 struct Plan {
 	int bm = 0, bn = 0, k_splits = 1;
@@ -62,15 +66,14 @@ struct Plan {
 static float tile_us(const TileTime& t, int M, int N, int slices, int k_splits = 1) {
 	const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) * k_splits;
 	const float rounds = (float)((tiles + 255) / 256);
-	// workgroups that walk several 256x256 tiles fill their ring once
-	return rounds * (slices + k_splits - 1) / k_splits * t.slice + (t.bm == 256 && t.round < 10.f ? t.round : rounds * t.round);
+	return rounds * ((slices + k_splits - 1) / k_splits * t.slice + t.round) + t.launch;
 }
 
-// The tile with the smallest estimate.  ring_extra: what the caller pays on top if it is one of the small ring tiles (a
-// pass of its own for an epilogue that only the 256-column tiles have).
-static Plan plan_tiles(bool f32, int M, int N, int K, float ring_extra = 0.f) {
+// The tile of a bf16 output with the smallest estimate.  ring_extra: what the caller pays on top if it is one of the small ring
+// tiles (a pass of its own for an epilogue that only the 256-column tiles have).
+static Plan plan_tiles(int M, int N, int K, float ring_extra = 0.f) {
 	Plan best;
-	for (const TileTime& t : f32 ? TILES_F32 : TILES_BF16) {
+	for (const TileTime& t : TILES_BF16) {
 		if (M < t.bm || N < t.bn) continue;
 		const float us = tile_us(t, M, N, K / BK) + (t.bn == 256 ? 0.f : ring_extra);
 		if (us < best.us) best = Plan{t.bm, t.bn, 1, us};
@@ -78,17 +81,20 @@ static Plan plan_tiles(bool f32, int M, int N, int K, float ring_extra = 0.f) {
 	return best;
 }
 
-// Weight gradients on 128x256 tiles with K split k_splits ways (at least 16 slices each): the splits of a tile add with
-// atomics, 2.3 us per million output elements and split (2048 x 2048 x 8192: 107 us whole, 82 us in two; 768 x 768 x 8192:
-// 107 and 43 in four, but 41 whole on 64x64 tiles).
-static Plan plan_weight_gradient(int M, int N, int K) {
-	Plan best = plan_tiles(true, M, N, K);
-	const TileTime& t = TILES_F32[1];
-	if (M >= t.bm && N >= t.bn)
-		for (int ks = 2; ks <= 16 && K / BK / ks >= 16; ks++) {
-			const float us = tile_us(t, M, N, K / BK, ks) + 2.3e-6f * ks * (float)M * N;
+// Weight gradients, with K split up to max_splits ways where that fills the chip.  The splits of a tile add with atomics, one
+// after the other: 2 us per split, and more on the ring's tiles, which take a whole tile's turn at a time, and for a large output.
+// Only 128x256 tiles used to be split since the register-staged kernel went; before -> after splitting them all (us):
+// 256 x 704 x 14080 68 -> 31, 512 x 384 x 10112 54 -> 26, 64 x 5632 x 13696 83 -> 53, 1536 x 192 x 12608 68 -> 39.
+static Plan plan_weight_gradient(int M, int N, int K, int max_splits = 16) {
+	Plan best;
+	for (const TileTime& t : TILES_F32) {
+		if (M < t.bm || N < t.bn) continue;
+		for (int ks = 1; ks <= max_splits && (ks == 1 || K / BK / ks >= 3); ks++) {
+			const float add = ks == 1 ? 0.f : t.bn == 256 ? ks * (1.6f + 1.3e-6f * (float)M * N) : ks * (2.2f + 1.2e-4f * t.bm * t.bn + 7.4e-6f * (float)M * N);
+			const float us = tile_us(t, M, N, K / BK, ks) + add;
 			if (us < best.us) best = Plan{t.bm, t.bn, ks, us};
 		}
+	}
 	return best;
 }
 
@@ -96,7 +102,7 @@ static Plan plan_weight_gradient(int M, int N, int K) {
 // (never with ring_extra = NO_RING, unless no tile of 256 columns fits).
 constexpr float NO_RING = 1e20f;
 static int dma_tile_rows(int M, int N, int K, float ring_extra) {
-	const Plan p = plan_tiles(false, M, N, K, ring_extra);
+	const Plan p = plan_tiles(M, N, K, ring_extra);
 	return p.dma() ? p.bm : 0;
 }
 // what a pass of its own over `bytes` costs (5 TB/s and a launch)
@@ -152,9 +158,9 @@ int gemm_bf16(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda,
 	if (bm == 0) {
 		Plan p;
 		if (epi != EPI_F32_ACC) {
-			p = plan_tiles(false, M, N, K);
+			p = plan_tiles(M, N, K);
 		} else if (k_splits > 0) {
-			p = plan_tiles(true, M, N, K);
+			p = plan_weight_gradient(M, N, K, 1);
 		} else if (M >= 256 && N >= 256 && (int64_t)((M + 255) / 256) * ((N + 255) / 256) >= 192 && K >= 4096) {
 			p = Plan{256, 256, 0};  // the split of the tail included, see below
 		} else {
@@ -239,7 +245,7 @@ bool gemm_swiglu_bwd_fused(int M, int F, int K) {
 	// 256x256 tiles only: against the best tile of the plain product and the pass over d, g, u and their gradients (the
 	// epilogue itself reads and writes four of those five at 256 tiles a time)
 	const float rounds = (float)(((int64_t)((M + 255) / 256) * ((F + 255) / 256) + 255) / 256);
-	return rounds * K / BK * TILES_BF16[0].slice + rounds * 12.f < plan_tiles(false, M, F, K).us + pass_us(10.0 * M * F);
+	return rounds * K / BK * TILES_BF16[0].slice + rounds * 12.f < plan_tiles(M, F, K).us + pass_us(10.0 * M * F);
 }
 
 int gemm_swiglu_bwd_bf16(int M, int F, int K, const void* dY, int64_t lddy, const void* W, int64_t ldw, const void* gu,

@@ -197,6 +197,35 @@ def test_gemm_bits_do_not_depend_on_the_tile(K):
 			assert torch.equal(K.gemm(a, b, tile_cfg=cfg, **kw), want), f"tile config {cfg} {kw}"
 
 
+@pytest.mark.parametrize("shape", [(64, 64, 15424), (256, 704, 14080), (512, 384, 10112), (1536, 192, 12608), (64, 5632, 13696), (128, 256, 192)])
+def test_small_weight_gradients_are_split_along_the_tokens(K, shape):
+	"""Outputs too small for the chip with long reductions: the choice left open runs about as fast as the best of a few explicit
+	splits of the small tiles (2.5 times as long without a split), with fp32 sums and equal bits from run to run."""
+	M, N, Kd = shape
+	A, B = _randn(Kd, M, seed=61), _randn(Kd, N, seed=62, scale=0.05)
+	before = K.gemm_turn_giveups()
+	acc = [K.gemm(A, B, a_t=True, b_t=True, epilogue=K.EPI_F32_ACC) for _ in range(2)]
+	assert torch.equal(acc[0], acc[1]) and K.gemm_turn_giveups() == before
+	_close(acc[0], A.float().t() @ B.float(), rel_fro=1e-5, rel_max=1e-5, what=f"weight gradient {shape}")
+	if Kd < 4096:
+		return
+
+	def ms(**kw):
+		times = []
+		for _ in range(5):
+			e0, e1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+			e0.record()
+			for _ in range(20):
+				K.gemm(A, B, a_t=True, b_t=True, out=acc[0], epilogue=K.EPI_F32_ACC, **kw)
+			e1.record()
+			e1.synchronize()
+			times.append(e0.elapsed_time(e1))
+		return sorted(times)[2]
+
+	best = min(ms(tile_cfg=12, k_splits=ks) for ks in (1, 2, 3, 4))
+	assert ms() < 1.6 * best
+
+
 @pytest.mark.parametrize("dims", [(4160, 5504, 128), (2880, 2880, 64), (320, 320, 128)])
 def test_fused_epilogues_at_ragged_sizes_equal_the_separate_passes(K, dims):
 	"""SwiGLU forward and backward and the rotary embedding in the GEMM epilogue on tiles that move back at the matrix's
