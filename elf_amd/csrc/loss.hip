@@ -5,9 +5,9 @@
 //     dlogits[r,c] = (softmax(x[r, :])[c] - (c == target[r])) * scale (0 for ignored rows and for
 //                    the padding columns V <= c < ld_out)
 // Forward and backward are one kernel — 4 bytes per logit of HBM traffic instead of the 10+ of a
-// log-softmax / gather / scatter chain.  Rows of up to 131072 columns are read once into
-// registers, reduced, and their gradient written from the same registers; longer rows are read
-// twice by their workgroup.
+// log-softmax / gather / scatter chain.  Rows of up to 65536 columns, and most of up to 131072, are
+// read once into registers, reduced, and their gradient written from the same registers; longer rows
+// are read twice by their workgroup.
 #include "common.h"
 #include "kernels.h"
 
@@ -175,9 +175,10 @@ __global__ __launch_bounds__(G < 256 ? 256 : G, G >= 256 ? 64 / C : 1) void cros
 		for (int64_t c = cend + lane; c < a.ld_out / 8; c += G) *reinterpret_cast<bf16x8*>(dr + c * 8) = bf16x8{};  // padding columns
 }
 
-// Rows beyond those registers, and wide rows whose gradient nobody asked for (nothing is read twice then, and more and smaller
-// workgroups hide the loads better: 4096 x 50304 82 us against 100, 2048 x 128256 99 against 129): G threads per row (one
-// workgroup), an online max / sum over one read of the row, then a second read for the gradient.  The running maximum only
+// Rows beyond those registers; of rows that start on 16-byte boundaries also those that do not fill them well (see
+// cross_entropy()) and wide ones whose gradient nobody asked for (nothing is read twice then, and more and smaller workgroups
+// hide the loads better: 4096 x 50304 82 us against 100, 2048 x 128256 99 against 129).  Dense rows have the kernel above only.
+// G threads per row (one workgroup), an online max / sum over one read of the row, then a second read for the gradient.  The running maximum only
 // rescales the partial sum when it grows, column masks are confined to the last chunk of a row, the 1/sum * scale factor rides
 // in the exponent, and the target column is fixed up by the one thread that holds it.
 template <bool MASKED>
@@ -330,8 +331,12 @@ int cross_entropy(const void* logits, int64_t ld, const void* target, int64_t ro
 	           (float*)row_loss, (bf16_t*)dlogits, dlogits ? ld_out : 0};
 	const int64_t width = dlogits && ld_out > V ? ld_out : V;
 	ProfScope prof(PROF_LOSS, (dlogits ? 4.0 : 2.0) * rows * V, s);
+	// 1024 threads with 16 chunks each leave room for one row per compute unit, the two-read kernel for two: it is the faster one
+	// where the registers are little more than half filled (4096 x 70656 as fast, 136 x 67936 12.9 us against 14.5) and where rows
+	// make a little more than one round (279 x 130568 44 against 54); 4096 x 100000 371 us against 356, 4096 x 128256 483 and 450
+	const bool twice = width > 65536 && (width < 98304 || rows < 512);
 	if (!dlogits && width > 16384 && width <= 65536) ELF_LAUNCH(cross_entropy_stream_kernel<256>, dim3((unsigned)rows), dim3(256), 0, s, a);
-	else if ((!dlogits && width > 16384) || !launch_resident<false>(a, width, s)) ELF_LAUNCH(cross_entropy_stream_kernel<1024>, dim3((unsigned)rows), dim3(1024), 0, s, a);
+	else if ((!dlogits && width > 16384) || twice || !launch_resident<false>(a, width, s)) ELF_LAUNCH(cross_entropy_stream_kernel<1024>, dim3((unsigned)rows), dim3(1024), 0, s, a);
 	ELF_CHECK_HIP(hipGetLastError());
 	return 0;
 }
