@@ -39,10 +39,10 @@ int gemm_turn_giveups(uint64_t* out) {
 // ------------------------------------------------------------------------------------------
 // Tile choice.  Estimated time of a product on tiles of bm x bn: rounds of 256 workgroups (one per compute unit) times the
 // time of a K slice of 64 times the slices and what a round costs besides (filling the ring, the epilogue), plus what a launch
-// costs once.  The constants are microseconds, the bf16 ones fitted to cold-operand timings of 33 shapes from 512 x 512 x 512 to
-// 4096 x 50304 x 768, those of the weight gradients to every tile and split on 2100 shapes from 64 x 64 x 64 to 8192 x 8192 x
-// 16384 (the tile and split that are picked take 0.4 % longer than the best on average).  A large tile has the cheaper products (per slice
-// and output: 22 ps on 256x256, 26 on 128x256, 35 on 128x128, 66 on 64x64: the smaller the tile, the more operand bytes go
+// costs once.  The constants are microseconds fitted to timings of every tile on some 10000 shapes (sizes spread over the
+// logarithm from 64 to 16384, operands rotated through 1 GB): over these the tile that is picked takes 0.3 to 0.4 % longer than
+// the best one on average, and more than 7 % longer for one shape in fifty.  A large tile has the cheaper products (per slice
+// and output: 21 ps on 256x256, 25 on 128x256, 35 on 128x128, 64 on 64x64: the smaller the tile, the more operand bytes go
 // through the 64 B/clk path into LDS for each product) and loses where its tiles leave compute units idle:
 //   1920 x 1600 x 1600: 44 us on 56 tiles of 256x256, 27 on 105 of 128x256, 19.9 on 195 of 128x128, 25 on 750 of 64x64;
 //   1920 x 4800 x 1600: 46 us on 152 tiles of 256x256, 52 on 285 of 128x256, 49 on 570 of 128x128.
@@ -51,8 +51,8 @@ struct TileTime {
 	float slice, round, launch;
 };
 static constexpr int N_TILES = 6;
-static constexpr TileTime TILES_BF16[N_TILES] = {{256, 256, 1.45f, 0.f, 6.f}, {128, 256, 0.854f, 5.5f, 0.f}, {128, 128, 0.58f, 4.f, 0.f},
-                                                 {64, 128, 0.38f, 2.f, 0.f}, {128, 64, 0.40f, 2.f, 0.f}, {64, 64, 0.27f, 1.3f, 0.f}};
+static constexpr TileTime TILES_BF16[N_TILES] = {{256, 256, 1.362f, 5.8f, 4.1f}, {128, 256, 0.811f, 5.5f, 1.4f}, {128, 128, 0.55f, 2.96f, 0.7f},
+                                                 {64, 128, 0.38f, 2.27f, 0.7f}, {128, 64, 0.395f, 2.06f, 0.6f}, {64, 64, 0.272f, 1.93f, 0.f}};
 // weight gradients: both operands reduction-major, fp32 read-modify-write of the output
 static constexpr TileTime TILES_F32[N_TILES] = {{256, 256, 1.3f, 22.f, 0.f}, {128, 256, 0.757f, 12.9f, 0.f}, {128, 128, 0.537f, 9.9f, 0.f},
                                                 {64, 128, 0.442f, 5.9f, 0.f}, {128, 64, 0.416f, 7.5f, 0.f}, {64, 64, 0.26f, 4.f, 0.f}};
@@ -69,12 +69,13 @@ static float tile_us(const TileTime& t, int M, int N, int slices, int k_splits =
 	return rounds * ((slices + k_splits - 1) / k_splits * t.slice + t.round) + t.launch;
 }
 
-// The tile of a bf16 output with the smallest estimate.  ring_extra: what the caller pays on top if it is one of the small ring
-// tiles (a pass of its own for an epilogue that only the 256-column tiles have).
-static Plan plan_tiles(int M, int N, int K, float ring_extra = 0.f) {
+// The tile of a bf16 output with the smallest estimate.  For an epilogue that only the 256-column tiles have: epi_extra, its time
+// per round of 256x256 tiles, and ring_extra, the time of the pass of its own that the small ring tiles need instead.
+static Plan plan_tiles(int M, int N, int K, float ring_extra = 0.f, float epi_extra = 0.f) {
 	Plan best;
-	for (const TileTime& t : TILES_BF16) {
+	for (TileTime t : TILES_BF16) {
 		if (M < t.bm || N < t.bn) continue;
+		if (t.bn == 256) t.round += epi_extra * t.bm / 256;
 		const float us = tile_us(t, M, N, K / BK) + (t.bn == 256 ? 0.f : ring_extra);
 		if (us < best.us) best = Plan{t.bm, t.bn, 1, us};
 	}
@@ -101,12 +102,14 @@ static Plan plan_weight_gradient(int M, int N, int K, int max_splits = 16) {
 // 256 or 128: the direct-to-LDS tile of 256 columns a forward / input-gradient product runs on, 0: one of the ring tiles
 // (never with ring_extra = NO_RING, unless no tile of 256 columns fits).
 constexpr float NO_RING = 1e20f;
-static int dma_tile_rows(int M, int N, int K, float ring_extra) {
-	const Plan p = plan_tiles(M, N, K, ring_extra);
+static int dma_tile_rows(int M, int N, int K, float ring_extra, float epi_extra) {
+	const Plan p = plan_tiles(M, N, K, ring_extra, epi_extra);
 	return p.dma() ? p.bm : 0;
 }
 // what a pass of its own over `bytes` costs (5 TB/s and a launch)
-static float pass_us(double bytes) { return 3.f + (float)(bytes / 5e6); }
+static float pass_us(double bytes) { return 2.f + (float)(bytes / 5e6); }
+// what an epilogue adds to a round of 256x256 tiles (half of it to one of 128x256)
+constexpr float SWIGLU_FWD_US = 4.f, ROPE_US = 5.f;
 
 // K split of a weight gradient on 256x256 direct-to-LDS tiles when the caller leaves it open: *k_splits ways for the last
 // *tail_tiles tiles (-1: all of them).
@@ -185,7 +188,7 @@ int gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, cons
 	if (act == ACT_SWIGLU && M % 64 == 0 && F % 64 == 0 && K % 64 == 0 && lda % 8 == 0 && ldw % 8 == 0 && ldpre >= N && ldout >= F && ldpre % 8 == 0 && ldout % 8 == 0 &&
 	    ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)pre % 16) == 0 && ((uintptr_t)out % 16) == 0 && lda >= K && ldw >= K) {
 		// rows that lie further apart only the fused kernel writes
-		bm = dma_tile_rows(M, N, K, ldpre == N && ldout == F ? pass_us(6.0 * M * F) : NO_RING);
+		bm = dma_tile_rows(M, N, K, ldpre == N && ldout == F ? pass_us(6.0 * M * F) : NO_RING, SWIGLU_FWD_US);
 	}
 	if (bm) {
 		ProfScope prof(PROF_GEMM, 2.0 * M * N * K, stream);
@@ -216,7 +219,7 @@ int gemm_dw_final(int M, int N, int K, const void* dY, int64_t lddy, const void*
 
 static int rope_tile_rows(int M, int N, int K, int D) {
 	if (!(M >= 64 && N >= 64 && M % 64 == 0 && N % 64 == 0 && K % 64 == 0 && (D == 64 || D == 128) && N % D == 0)) return 0;
-	return dma_tile_rows(M, N, K, pass_us(4.0 * M * N));
+	return dma_tile_rows(M, N, K, pass_us(4.0 * M * N), ROPE_US);
 }
 bool gemm_rope_fused(int M, int N, int K, int D) {
 	return rope_tile_rows(M, N, K, D) != 0;
@@ -242,10 +245,11 @@ static bool swiglu_bwd_fits(int M, int F, int K) { return M >= 256 && F >= 256 &
 // ... and where it is also the faster way.
 bool gemm_swiglu_bwd_fused(int M, int F, int K) {
 	if (!swiglu_bwd_fits(M, F, K)) return false;
-	// 256x256 tiles only: against the best tile of the plain product and the pass over d, g, u and their gradients (the
-	// epilogue itself reads and writes four of those five at 256 tiles a time)
-	const float rounds = (float)(((int64_t)((M + 255) / 256) * ((F + 255) / 256) + 255) / 256);
-	return rounds * K / BK * TILES_BF16[0].slice + rounds * 12.f < plan_tiles(M, F, K).us + pass_us(10.0 * M * F);
+	// 256x256 tiles only: against the best tile of the plain product and the pass over d, g, u and their gradients.  The epilogue
+	// reads and writes four of those five at 256 tiles a time, 20 us more per round than the plain one (fitted to 700 shapes;
+	// with 12 us for the whole round 1024 x 3072 x 64 took 25 us fused, 13 apart, and 8448 x 512 x 512 32 and 20)
+	const TileTime fused{256, 256, 1.24f, 27.f, 0.f};
+	return tile_us(fused, M, F, K / BK) < plan_tiles(M, F, K).us + pass_us(10.0 * M * F);
 }
 
 int gemm_swiglu_bwd_bf16(int M, int F, int K, const void* dY, int64_t lddy, const void* W, int64_t ldw, const void* gu,

@@ -226,6 +226,32 @@ def test_small_weight_gradients_are_split_along_the_tokens(K, shape):
 	assert ms() < 1.6 * best
 
 
+PROF_ACT_FWD, PROF_ACT_BWD, PROF_ROPE = 5, 6, 7
+
+
+def _launches(kind, call):
+	"""``call()`` and how many kernels of a family (``elf_prof_launches``) it ran: none where a fused epilogue did the work."""
+	from elf_amd import _lib
+
+	lib = _lib.load()
+	lib.elf_prof_enable(1)
+	try:
+		return call(), lib.elf_prof_launches(kind, None)
+	finally:
+		lib.elf_prof_enable(0)
+
+
+@pytest.mark.parametrize("dims,fused", [((1024, 3072, 64), False), ((8448, 512, 512), False), ((3072, 2304, 768), False), ((8192, 7168, 512), True), ((4096, 4096, 4096), True)])
+def test_swiglu_backward_is_fused_where_that_is_faster(K, dims, fused):
+	"""The epilogue of a 256x256 tile takes 27 us a round: one partly filled round of few K slices is faster apart (1024 x 3072 x 64:
+	13 us against 25), full rounds are faster fused (8192 x 14336 x 4096: 842 us against 932)."""
+	M, F, Kd = dims
+	dy, w2, gu = _randn(M, Kd, seed=71), _randn(Kd, F, seed=72, scale=0.05), _randn(M, 2 * F, seed=73)
+	got, passes = _launches(PROF_ACT_BWD, lambda: K.gemm_swiglu_bwd(dy, w2, gu))
+	assert (passes == 0) == fused
+	assert torch.equal(got, K.gemm_swiglu_bwd(dy, w2, gu, fused=False))
+
+
 @pytest.mark.parametrize("dims", [(4160, 5504, 128), (2880, 2880, 64), (320, 320, 128)])
 def test_fused_epilogues_at_ragged_sizes_equal_the_separate_passes(K, dims):
 	"""SwiGLU forward and backward and the rotary embedding in the GEMM epilogue on tiles that move back at the matrix's
