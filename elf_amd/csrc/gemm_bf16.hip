@@ -53,6 +53,9 @@ struct TileTime {
 static constexpr int N_TILES = 6;
 static constexpr TileTime TILES_BF16[N_TILES] = {{256, 256, 1.362f, 5.8f, 4.1f}, {128, 256, 0.811f, 5.5f, 1.4f}, {128, 128, 0.55f, 2.96f, 0.7f},
                                                  {64, 128, 0.38f, 2.27f, 0.7f}, {128, 64, 0.395f, 2.06f, 0.6f}, {64, 64, 0.272f, 1.93f, 0.f}};
+// K of at most RING_SHORT_K: the small tiles on the ring of two slices
+static constexpr TileTime TILES_SHORT[N_TILES] = {{256, 256, 1.293f, 7.15f, 2.5f}, {128, 256, 0.996f, 4.9f, 0.44f}, {128, 128, 0.388f, 1.94f, 3.5f},
+                                                  {64, 128, 0.285f, 0.93f, 3.7f}, {128, 64, 0.325f, 1.0f, 2.4f}, {64, 64, 0.184f, 0.55f, 2.9f}};
 // weight gradients: both operands reduction-major, fp32 read-modify-write of the output
 static constexpr TileTime TILES_F32[N_TILES] = {{256, 256, 1.3f, 22.f, 0.f}, {128, 256, 0.757f, 12.9f, 0.f}, {128, 128, 0.537f, 9.9f, 0.f},
                                                 {64, 128, 0.442f, 5.9f, 0.f}, {128, 64, 0.416f, 7.5f, 0.f}, {64, 64, 0.26f, 4.f, 0.f}};
@@ -73,7 +76,7 @@ static float tile_us(const TileTime& t, int M, int N, int slices, int k_splits =
 // per round of 256x256 tiles, and ring_extra, the time of the pass of its own that the small ring tiles need instead.
 static Plan plan_tiles(int M, int N, int K, float ring_extra = 0.f, float epi_extra = 0.f) {
 	Plan best;
-	for (TileTime t : TILES_BF16) {
+	for (TileTime t : K <= RING_SHORT_K ? TILES_SHORT : TILES_BF16) {
 		if (M < t.bm || N < t.bn) continue;
 		if (t.bn == 256) t.round += epi_extra * t.bm / 256;
 		const float us = tile_us(t, M, N, K / BK) + (t.bn == 256 ? 0.f : ring_extra);

@@ -40,10 +40,14 @@ static __device__ uint32_t turn[TURN_TILES * 4];
 constexpr int TURN_SPIN_LIMIT = 1 << 10;
 static __device__ unsigned int turn_giveups;
 
-template <int BM, int BN>
+// SHORT: two slices, for a K of at most RING_SHORT_K and bf16 outputs.  A deep ring fetches all of its slices up front whether K
+// has them or not, and holds the compute unit's LDS alone; of these, two to four workgroups share one, and the epilogue of one
+// hides behind the loads of the next.  11392 x 640 x 64 10.0 -> 8.1 us, 7232 x 576 x 128 7.6 -> 6.3, 9344 x 896 x 256 13.0 -> 10.2;
+// with five to eight slices of K the deep ring is 5 % ahead, with sixteen 30 %.
+template <int BM, int BN, bool SHORT>
 struct Shape {
 	static constexpr int A_BYTES = BM * BKS * 2, B_BYTES = BN * BKS * 2, STAGE_BYTES = A_BYTES + B_BYTES;
-	static constexpr int NST = BM == 64 && BN == 64 ? 8 : BM == 128 && BN == 128 ? 4 : 6;  // 128 .. 144 KiB of slices
+	static constexpr int NST = SHORT ? 2 : BM == 64 && BN == 64 ? 8 : BM == 128 && BN == 128 ? 4 : 6;  // 128 .. 144 KiB of slices
 	static constexpr int LOADS_A = A_BYTES / 4096, LOADS_B = B_BYTES / 4096, LOADS = LOADS_A + LOADS_B;  // 1 KiB pieces per wave and slice
 	static constexpr int SMEM = NST * STAGE_BYTES + (LOADS_A > LOADS_B ? LOADS_A : LOADS_B) * 1024;
 };
@@ -64,9 +68,9 @@ __device__ __forceinline__ void pair_slabs(f32x4& lo, f32x4& hi) {
 	}
 }
 
-template <int BM, int BN, bool AT, bool BT, int EPI>
+template <int BM, int BN, bool AT, bool BT, int EPI, bool SHORT>
 __global__ __launch_bounds__(256) void gemm_ring_kernel(Args g) {
-	using Sh = Shape<BM, BN>;
+	using Sh = Shape<BM, BN, SHORT>;
 	constexpr int NST = Sh::NST, A_BYTES = Sh::A_BYTES, B_BYTES = Sh::B_BYTES, LOADS_A = Sh::LOADS_A, LOADS_B = Sh::LOADS_B, P = Sh::LOADS;
 	constexpr int WM = BM / 2, WN = BN / 2, RF = WM / 16, CF = WN / 16, NM = RF * CF, NR = RF + CF;
 	extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
@@ -319,27 +323,32 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(Args g) {
 	wait_vmcnt<0>();  // the loads past the end of K land in LDS too
 }
 
-template <int BM, int BN, bool AT, bool BT, int EPI>
+template <int BM, int BN, bool AT, bool BT, int EPI, bool SHORT>
 static int launch(const Args& g, hipStream_t stream) {
-	auto kern = gemm_ring_kernel<BM, BN, AT, BT, EPI>;
+	using Sh = Shape<BM, BN, SHORT>;
+	auto kern = gemm_ring_kernel<BM, BN, AT, BT, EPI, SHORT>;
 	static bool attr_set = false;
 	if (!attr_set) {
-		ELF_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Shape<BM, BN>::SMEM));
+		ELF_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Sh::SMEM));
 		attr_set = true;
 	}
 	const int ntiles = g.tiles_m * g.tiles_n;
-	ELF_LAUNCH(kern, dim3(8 * ((ntiles + 7) / 8) * g.k_splits), dim3(256), (Shape<BM, BN>::SMEM), stream, g);
+	ELF_LAUNCH(kern, dim3(8 * ((ntiles + 7) / 8) * g.k_splits), dim3(256), (Sh::SMEM), stream, g);
 	ELF_CHECK_HIP(hipGetLastError());
 	return 0;
 }
 
 template <int BM, int BN, bool AT, bool BT>
 static int launch_epi(const Args& g, int epi, hipStream_t stream) {
+	if constexpr (!AT) {
+		if (g.K <= RING_SHORT_K && epi == EPI_BF16) return launch<BM, BN, AT, BT, EPI_BF16, true>(g, stream);
+		if (g.K <= RING_SHORT_K && epi == EPI_BF16_RESID) return launch<BM, BN, AT, BT, EPI_BF16_RESID, true>(g, stream);
+	}
 	switch (epi) {
-		case EPI_BF16: return launch<BM, BN, AT, BT, EPI_BF16>(g, stream);
-		case EPI_BF16_RESID: return launch<BM, BN, AT, BT, EPI_BF16_RESID>(g, stream);
-		case EPI_F32_ACC: return launch<BM, BN, AT, BT, EPI_F32_ACC>(g, stream);
-		case EPI_F32_STORE: return launch<BM, BN, AT, BT, EPI_F32_STORE>(g, stream);
+		case EPI_BF16: return launch<BM, BN, AT, BT, EPI_BF16, false>(g, stream);
+		case EPI_BF16_RESID: return launch<BM, BN, AT, BT, EPI_BF16_RESID, false>(g, stream);
+		case EPI_F32_ACC: return launch<BM, BN, AT, BT, EPI_F32_ACC, false>(g, stream);
+		case EPI_F32_STORE: return launch<BM, BN, AT, BT, EPI_F32_STORE, false>(g, stream);
 	}
 	set_error("gemm: unknown epilogue %d", epi);
 	return -1;

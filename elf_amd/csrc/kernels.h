@@ -36,7 +36,9 @@ int gemm_bf16_dma(int a_t, int b_t, int M, int N, int K, const void* A, int64_t 
                   int64_t ldc, int epi, const void* R, int64_t ldr, int k_splits, int tail_tiles, int bm, hipStream_t stream,
                   void* C2 = nullptr, int64_t ldc2 = 0, const void* rope_cs = nullptr, int rope_S = 0, int rope_cols = 0, int rope_D = 0,
                   float scale = 1.f);
-// the same on small tiles (bm, bn: 128 or 64) with a deep ring of K slices (gemm_ring.hip)
+// the same on small tiles (bm, bn: 128 or 64) with a deep ring of K slices (gemm_ring.hip); products of at most RING_SHORT_K
+// with a bf16 output and k-contiguous A on a ring of two slices
+constexpr int RING_SHORT_K = 256;
 int gemm_bf16_ring(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb, void* C, int64_t ldc, int epi, const void* R,
                    int64_t ldr, int k_splits, int bm, int bn, hipStream_t stream);
 

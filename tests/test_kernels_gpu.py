@@ -226,6 +226,22 @@ def test_small_weight_gradients_are_split_along_the_tokens(K, shape):
 	assert ms() < 1.6 * best
 
 
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+@pytest.mark.parametrize("Kd", [64, 128, 192, 256, 320])
+@pytest.mark.parametrize("tile_cfg,mn", [(9, (448, 320)), (10, (192, 320)), (11, (320, 192)), (12, (192, 64))])
+def test_short_reductions_on_the_small_tiles(K, tile_cfg, mn, Kd, layout):
+	"""K of 64 to 256 runs on a ring of two slices, K of 320 on the deep one: the bits of the 64x64 tile's fp32 sums, rounded once."""
+	M, N = mn
+	A, B, R = _randn(M, Kd, seed=81), _randn(N, Kd, seed=82, scale=0.05), _randn(M, N, seed=83)
+	b, kw = (B, {}) if layout == "nt" else (B.t().contiguous(), dict(b_t=True))
+	want = K.gemm(A, b, epilogue=K.EPI_F32_STORE, tile_cfg=12, **kw)
+	_close(want, A.float() @ B.float().t(), rel_fro=1e-5, rel_max=1e-5, what="f32 store")
+	big = torch.full((M + 64, N + 64), 7.0, dtype=torch.bfloat16, device="cuda")
+	K.gemm(A, b, out=big[:M, :N], tile_cfg=tile_cfg, **kw)
+	assert torch.equal(big[:M, :N], want.to(torch.bfloat16)) and (big[M:] == 7).all() and (big[:, N:] == 7).all()
+	assert torch.equal(K.gemm(A, b, epilogue=K.EPI_BF16_RESID, residual=R, tile_cfg=tile_cfg, **kw), (want + R.float()).to(torch.bfloat16))
+
+
 PROF_ACT_FWD, PROF_ACT_BWD, PROF_ROPE = 5, 6, 7
 
 
