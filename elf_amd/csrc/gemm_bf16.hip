@@ -149,7 +149,8 @@ int gemm_bf16(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda,
 	ELF_REQUIRE(k_splits <= 255, "gemm: k_splits must be at most 255 (got %d)", k_splits);
 	ProfScope prof(PROF_GEMM, 2.0 * M * N * K, stream);
 	ELF_REQUIRE(M % 64 == 0 && N % 64 == 0, "gemm: M and N must be multiples of 64 (M=%d N=%d)", M, N);
-	ELF_REQUIRE(tile_cfg >= 0 && tile_cfg <= 12 && tile_cfg != 4 && tile_cfg != 6, "gemm: unknown tile config %d", tile_cfg);
+	if (tile_cfg < 0) tile_cfg = 0;
+	ELF_REQUIRE(tile_cfg <= 12 && tile_cfg != 4 && tile_cfg != 6, "gemm: unknown tile config %d", tile_cfg);
 	int bm = 0, bn = 0, tail_tiles = -1;  // an explicit k_splits splits every tile
 	switch (tile_cfg) {
 		case 0: break;

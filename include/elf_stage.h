@@ -33,10 +33,10 @@ int elf_abi_version(void);
  *   epilogue: 0 C(bf16) = acc; 1 C(bf16) = acc + R(bf16, leading dim ldr; ldr = 0: R is one row of N values
  *             added to every row of C, the bias of nn.Linear);
  *             2 C(fp32) += acc; 3 C(fp32) = acc.
- *   tile_cfg = 0 picks the tile by estimated time (7: 256x256, 8: 128x256, 9: 128x128, 10: 64x128, 11: 128x64, 12: 64x64;
+ *   tile_cfg <= 0 picks the tile by estimated time (7: 256x256, 8: 128x256, 9: 128x128, 10: 64x128, 11: 128x64, 12: 64x64;
  *   1 is another name of 7, 2 and 5 of 9, 3 of 12; M and N must be at least the tile's): a_t = 1 is accepted only together
  *   with b_t = 1; k_splits is honoured for epilogue 2;
- *   k_splits = 0 picks a K split (epilogue 2 only; at most 255).
+ *   k_splits <= 0 picks a K split (epilogue 2 only; at most 255).
  * Replaces: F.linear in LinearDX.forward (elf/zb_utils.py:20)            -> a_t=0,b_t=0
  *           torch.mm(grad_output, weight) in LinearDX.backward (:34-37)  -> a_t=0,b_t=1
  *           torch.mm(go.t(), inp) + weight.grad.add_ in LinearDW.backward (:238-244) -> a_t=1,b_t=1, epilogue 2

@@ -226,6 +226,13 @@ def test_small_weight_gradients_are_split_along_the_tokens(K, shape):
 	assert ms() < 1.6 * best
 
 
+def test_gemm_takes_any_tile_choice_below_one_as_open(K):
+	A, B = _randn(192, 128, seed=85), _randn(320, 128, seed=86, scale=0.05)
+	assert torch.equal(K.gemm(A, B, tile_cfg=-1), K.gemm(A, B))
+	acc = K.gemm(A, B, tile_cfg=-1, k_splits=-1, epilogue=K.EPI_F32_ACC)
+	_close(acc, A.float() @ B.float().t(), rel_fro=1e-5, rel_max=1e-5, what="f32 acc")
+
+
 @pytest.mark.parametrize("layout", ["nt", "nn"])
 @pytest.mark.parametrize("Kd", [64, 128, 192, 256, 320])
 @pytest.mark.parametrize("tile_cfg,mn", [(9, (448, 320)), (10, (192, 320)), (11, (320, 192)), (12, (192, 64))])
