@@ -187,9 +187,10 @@ int gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, cons
 	ELF_REQUIRE(act == ACT_GELU || act == ACT_SWIGLU, "gemm_act: unknown activation %d", act);
 	ELF_REQUIRE(M > 0 && F > 0 && K > 0 && A && W && pre && out, "gemm_act: empty problem or null operand");
 	const int N = act == ACT_SWIGLU ? 2 * F : F;
-	// the SwiGLU epilogue pairs 64 gate with 64 up columns per wave, so a 256-column tile covers 128 outputs
+	// the SwiGLU epilogue pairs 64 gate with 64 up columns per wave, so a 256-column tile covers 128 outputs; it reaches the up rows
+	// with 32-bit byte offsets from the gate rows
 	int bm = 0;
-	if (act == ACT_SWIGLU && M % 64 == 0 && F % 64 == 0 && K % 64 == 0 && lda % 8 == 0 && ldw % 8 == 0 && ldpre >= N && ldout >= F && ldpre % 8 == 0 && ldout % 8 == 0 &&
+	if (act == ACT_SWIGLU && (int64_t)(F + 256) * ldw * 2 < (int64_t(1) << 31) && M % 64 == 0 && F % 64 == 0 && K % 64 == 0 && lda % 8 == 0 && ldw % 8 == 0 && ldpre >= N && ldout >= F && ldpre % 8 == 0 && ldout % 8 == 0 &&
 	    ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)pre % 16) == 0 && ((uintptr_t)out % 16) == 0 && lda >= K && ldw >= K) {
 		// rows that lie further apart only the fused kernel writes
 		bm = dma_tile_rows(M, N, K, ldpre == N && ldout == F ? pass_us(6.0 * M * F) : NO_RING, SWIGLU_FWD_US);

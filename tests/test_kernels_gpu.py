@@ -226,6 +226,16 @@ def test_small_weight_gradients_are_split_along_the_tokens(K, shape):
 	assert ms() < 1.6 * best
 
 
+def test_gemm_with_activation_whose_up_rows_lie_far_off(K):
+	"""A weight whose up rows start 1.3 GB behind the gate rows, too far for the fused epilogue: the separate passes."""
+	M, F, Kd, ldw = 192, 320, 64, 1 << 21
+	a = _randn(M, Kd, seed=87)
+	w = torch.empty(2 * F, ldw, dtype=torch.bfloat16, device="cuda")[:, :Kd]
+	w.copy_(_randn(2 * F, Kd, seed=88, scale=0.05))
+	gu, act = K.gemm_act(a, w, K.ACT_SWIGLU)
+	assert torch.equal(gu, K.gemm(a, w.contiguous())) and torch.equal(act, K.swiglu_fwd(gu))
+
+
 def test_gemm_takes_any_tile_choice_below_one_as_open(K):
 	A, B = _randn(192, 128, seed=85), _randn(320, 128, seed=86, scale=0.05)
 	assert torch.equal(K.gemm(A, B, tile_cfg=-1), K.gemm(A, B))
