@@ -175,6 +175,7 @@ int gemm_bf16(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda,
 		}
 		bm = p.bm, bn = p.bn;
 		if (epi == EPI_F32_ACC && k_splits <= 0) k_splits = p.k_splits;
+		if (!gemm_reaches(a_t ? BK : bm, lda) || !gemm_reaches(b_t ? BK : bn, ldb)) bm = bn = 64;  // rows 16 MB apart and more
 	}
 	if (epi != EPI_F32_ACC) k_splits = 1;
 	if (bm == 256 && k_splits <= 0) dw_split_plan(M, N, K, &k_splits, &tail_tiles);
@@ -191,7 +192,7 @@ int gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, cons
 	// with 32-bit byte offsets from the gate rows
 	int bm = 0;
 	if (act == ACT_SWIGLU && (int64_t)(F + 256) * ldw * 2 < (int64_t(1) << 31) && M % 64 == 0 && F % 64 == 0 && K % 64 == 0 && lda % 8 == 0 && ldw % 8 == 0 && ldpre >= N && ldout >= F && ldpre % 8 == 0 && ldout % 8 == 0 &&
-	    ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)pre % 16) == 0 && ((uintptr_t)out % 16) == 0 && lda >= K && ldw >= K) {
+	    ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)pre % 16) == 0 && ((uintptr_t)out % 16) == 0 && lda >= K && ldw >= K && gemm_reaches(256, lda)) {
 		// rows that lie further apart only the fused kernel writes
 		bm = dma_tile_rows(M, N, K, ldpre == N && ldout == F ? pass_us(6.0 * M * F) : NO_RING, SWIGLU_FWD_US);
 	}
@@ -208,7 +209,7 @@ int gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, cons
 int gemm_dw_final(int M, int N, int K, const void* dY, int64_t lddy, const void* X, int64_t ldx, float* acc, void* grad_bf16, float scale,
                   hipStream_t stream) {
 	ELF_REQUIRE(M > 0 && N > 0 && K > 0 && dY && X && acc && grad_bf16, "gemm_dw_final: bad argument");
-	const bool fused = M % 64 == 0 && N % 64 == 0 && K % 64 == 0 && M >= 256 && N >= 256 && (int64_t)((M + 255) / 256) * ((N + 255) / 256) >= 192 && K >= 4096 && lddy % 8 == 0 && ldx % 8 == 0 && lddy >= M &&
+	const bool fused = gemm_reaches(BK, lddy) && gemm_reaches(BK, ldx) && M % 64 == 0 && N % 64 == 0 && K % 64 == 0 && M >= 256 && N >= 256 && (int64_t)((M + 255) / 256) * ((N + 255) / 256) >= 192 && K >= 4096 && lddy % 8 == 0 && ldx % 8 == 0 && lddy >= M &&
 	                   ldx >= N && ((uintptr_t)dY % 16) == 0 && ((uintptr_t)X % 16) == 0 && ((uintptr_t)acc % 16) == 0 && ((uintptr_t)grad_bf16 % 8) == 0;
 	if (fused) {
 		// the same K split as the plain weight gradient (same rounding); tiles shared by several workgroups along K have no
@@ -235,7 +236,7 @@ int gemm_rope_bf16(int M, int N, int K, const void* A, int64_t lda, const void* 
 	ELF_REQUIRE(M > 0 && N > 0 && K > 0 && A && W && C && cs, "gemm_rope: empty problem or null operand");
 	ELF_REQUIRE(S > 0 && M % S == 0 && n_rot_heads >= 0 && (int64_t)n_rot_heads * D <= N, "gemm_rope: bad head layout (S=%d, heads=%d, D=%d, N=%d)", S, n_rot_heads, D, N);
 	if (gemm_rope_fused(M, N, K, D) && lda % 8 == 0 && ldw % 8 == 0 && ldc % 8 == 0 && lda >= K && ldw >= K && ldc >= N && ((uintptr_t)A % 16) == 0 &&
-	    ((uintptr_t)W % 16) == 0 && ((uintptr_t)C % 16) == 0 && ((uintptr_t)cs % 16) == 0) {
+	    ((uintptr_t)W % 16) == 0 && ((uintptr_t)C % 16) == 0 && ((uintptr_t)cs % 16) == 0 && gemm_reaches(256, lda) && gemm_reaches(256, ldw)) {
 		// the rotation's arithmetic is not counted: the figure stays the GEMM's
 		ProfScope prof(PROF_GEMM, 2.0 * M * N * K, stream);
 		const int bm = rope_tile_rows(M, N, K, D);
@@ -262,7 +263,7 @@ int gemm_swiglu_bwd_bf16(int M, int F, int K, const void* dY, int64_t lddy, cons
 	ELF_REQUIRE(M > 0 && F > 0 && K > 0 && dY && W && gu && dgu, "gemm_swiglu_bwd: empty problem or null operand");
 	const bool apart = scratch && ldgu == 2 * F && lddgu == 2 * F && (!act || ldact == F);  // what the separate passes need
 	if ((apart ? gemm_swiglu_bwd_fused(M, F, K) : swiglu_bwd_fits(M, F, K)) && lddy >= K && ldw >= F && ldgu >= 2 * F && lddgu >= 2 * F && lddy % 8 == 0 && ldw % 8 == 0 && ldgu % 8 == 0 &&
-	    lddgu % 8 == 0 && ((uintptr_t)dY % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)gu % 16) == 0 && ((uintptr_t)dgu % 16) == 0) {
+	    lddgu % 8 == 0 && ((uintptr_t)dY % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)gu % 16) == 0 && ((uintptr_t)dgu % 16) == 0 && gemm_reaches(256, lddy) && gemm_reaches(BK, ldw)) {
 		// the activation backward's arithmetic is not counted: the figure stays the GEMM's
 		ProfScope prof(PROF_GEMM, 2.0 * M * F * K, stream);
 		ELF_REQUIRE(!act || (ldact >= F && ldact % 8 == 0 && ((uintptr_t)act % 16) == 0), "gemm_swiglu_bwd: bad activation output");

@@ -1068,6 +1068,7 @@ int gemm_bf16_dma(int a_t, int b_t, int M, int N, int K, const void* A, int64_t 
 	ELF_REQUIRE(bm == 256 || bm == 128, "gemm (dma tile): 256- or 128-row tiles");
 	ELF_REQUIRE(M >= bm && N >= dma::BN && M % 64 == 0 && N % 64 == 0 && K % dma::BKS == 0, "gemm (dma tile): M at least %d, N at least 256, all sizes multiples of 64", bm);
 	const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + dma::BN - 1) / dma::BN, ntiles = tiles_m * tiles_n;
+	ELF_REQUIRE(gemm_reaches(a_t ? dma::BKS : bm, lda) && gemm_reaches(b_t ? dma::BKS : dma::BN, ldb), "gemm (dma tile): leading dimension too large (%lld, %lld)", (long long)lda, (long long)ldb);
 	// a tile's columns are taken in heads: the last one may only move back by whole heads
 	ELF_REQUIRE(epi != EPI_BF16_ROPE || N % rope_D == 0, "gemm (dma tile): the RoPE epilogue needs N to be a multiple of the head width");
 	ELF_REQUIRE(epi != EPI_BF16_SWIGLU || (C2 && !a_t && !b_t), "gemm (dma tile): the SwiGLU epilogue needs k-contiguous operands and a second output");
@@ -1123,7 +1124,7 @@ int gemm_bf16_dma(int a_t, int b_t, int M, int N, int K, const void* A, int64_t 
 }
 
 bool gemm_dw_groupable(int M, int N, int K, const void* dY, int64_t lddy, const void* X, int64_t ldx, const void* acc) {
-	return M >= 256 && N >= dma::BN && K > 0 && M % 64 == 0 && N % 64 == 0 && K % dma::BKS == 0 && lddy % 8 == 0 && ldx % 8 == 0 && lddy >= M && ldx >= N &&
+	return M >= 256 && N >= dma::BN && K > 0 && gemm_reaches(dma::BKS, lddy) && gemm_reaches(dma::BKS, ldx) && M % 64 == 0 && N % 64 == 0 && K % dma::BKS == 0 && lddy % 8 == 0 && ldx % 8 == 0 && lddy >= M && ldx >= N &&
 	       ((uintptr_t)dY % 16) == 0 && ((uintptr_t)X % 16) == 0 && ((uintptr_t)acc % 16) == 0;
 }
 

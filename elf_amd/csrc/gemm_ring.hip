@@ -380,6 +380,7 @@ int ring_turn_giveups(uint64_t* out) {
 int gemm_bf16_ring(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb, void* C, int64_t ldc, int epi, const void* R,
                    int64_t ldr, int k_splits, int bm, int bn, hipStream_t stream) {
 	ELF_REQUIRE(M % 64 == 0 && N % 64 == 0 && K % dma::BKS == 0, "gemm (ring tile): sizes must be multiples of 64");
+	ELF_REQUIRE(gemm_reaches(a_t ? dma::BKS : bm, lda) && gemm_reaches(b_t ? dma::BKS : bn, ldb), "gemm (ring tile): leading dimension too large (%lld, %lld)", (long long)lda, (long long)ldb);
 	ring::Args g{(const bf16_t*)A, (const bf16_t*)B, C, (const bf16_t*)R, lda, ldb, ldc, ldr, M, N, K, 0, 0, k_splits, 0};
 	if (bm == 128 && bn == 128) return ring::launch_layout<128, 128>(g, a_t, b_t, epi, stream);
 	if (bm == 64 && bn == 128) return ring::launch_layout<64, 128>(g, a_t, b_t, epi, stream);

@@ -96,6 +96,16 @@ def test_attention_backward_refuses_a_workspace_that_is_too_small(lib):
 	assert rc == -1 and str(n).encode() in lib.elf_last_error()
 
 
+def test_gemm_refuses_rows_too_far_apart_for_its_offsets(lib):
+	"""The kernels reach a tile's rows with 32-bit byte offsets: 256 rows of 2^24 elements reach too far, 128 of 2^25,
+	64 of 2^26."""
+	for cfg, lda, ldb in ((7, 24, 6), (7, 6, 24), (8, 25, 6), (8, 6, 24), (9, 25, 6), (9, 6, 25), (10, 6, 25), (11, 25, 6), (12, 26, 6), (12, 6, 26), (0, 26, 6), (0, 6, 26)):
+		rc = lib.elf_gemm_bf16(0, 0, 256, 256, 64, 16, 1 << lda, 16, 1 << ldb, 16, 256, 0, None, 0, cfg, 0, None)
+		assert rc == -1 and b"leading dimension too large" in lib.elf_last_error(), (cfg, lda, ldb)
+	rc = lib.elf_gemm_bf16(1, 1, 256, 256, 64, 16, 1 << 26, 16, 256, 16, 256, 2, None, 0, 0, 0, None)
+	assert rc == -1 and b"leading dimension too large" in lib.elf_last_error()
+
+
 def test_stage_create_rejects_bad_configs(lib):
 	from elf_amd.execution.block import StageConfig
 
