@@ -127,6 +127,35 @@ def test_compute_loss_matches_mean_reduction_after_batch_scaling():
 	assert blk.compute_time[0].name == "loss_forward"
 
 
+@pytest.mark.parametrize("timings", [False, True])
+def test_timers_run_in_steps_whose_timings_are_read(monkeypatch, timings):
+	"""Inside a step ``times_ops`` of every block says whether anybody reads its timers (ELF_TIMINGS); outside, and after a step
+	that failed, blocks time their ops as ever."""
+	from elf_amd.execution import engine as E
+
+	monkeypatch.setattr(E, "precise_timings", timings)
+	seen = []
+
+	class Watching(FakeBlock):
+		def forward(self, mb, **opts):
+			seen.append(self.times_ops)
+			if fail:
+				raise ValueError("stop")
+			return super().forward(mb, **opts)
+
+	fail = False
+	blocks = [Watching(i, [0, 0]) for i in range(2)]
+	schedule = COMM_SCHEDULERS["pipelined"](add_comms(SCHEDULERS["afab"]([0, 0], 2), sequential_signatures([0, 0])))
+	args = ((torch.arange(8.0).reshape(4, 2),), torch.zeros(4, 2), torch.nn.functional.mse_loss, schedule, [2, 2])
+	_, _, _, detailed = Engine(blocks).train_step(*args)
+	assert seen == [timings] * 4 and all(b.times_ops and not b.compute_time for b in blocks)
+	assert ("loss_forward" in detailed["all_events"]) == timings and ("backward(1:1)" in detailed["all_events"]) == timings
+	fail = True
+	with pytest.raises(ValueError):
+		Engine(blocks).train_step(*args)
+	assert seen[-1] is timings and all(b.times_ops for b in blocks)
+
+
 @pytest.mark.parametrize("scheduler,placement,nmb", [("1f1b", [0, 1], 4), ("zbh1", [0, 1, 2, 3], 8), ("1f1b", [0, 1, 0, 1], 4), ("afab", [0, 1, 2], 3), ("zbh2", [0, 1, 2, 3], 4)])
 @pytest.mark.parametrize("comm", ["pipelined", "topo", "simulation"])
 def test_sequential_order_lets_one_process_play_every_rank(scheduler, placement, nmb, comm):

@@ -301,6 +301,21 @@ def test_fused_epilogues_at_ragged_sizes_equal_the_separate_passes(K, dims):
 	assert torch.equal(K.gemm_rope(a, w[:F], cs, S, n_rot, D), K.gemm_rope(a, w[:F], cs, S, n_rot, D, fused=False))
 
 
+# (tokens, F, K), the head width, and whether the epilogue runs in the GEMM.  1984 x 3200 x 512: 208 tiles of 128x256, the last ones
+# moved back by 64 rows and 128 columns (two heads of 64 or one of 128); 4160 x 11136 x 128: 256x256, moved back by 192 rows and 128 columns
+@pytest.mark.parametrize("dims,D,fused", [((1984, 1600, 512), 64, True), ((1984, 1600, 512), 128, True), ((4160, 5568, 128), 128, True), ((320, 320, 128), 64, False)])
+def test_fused_epilogues_on_moved_tiles(K, dims, D, fused):
+	T, F, Kd = dims
+	a, w = _randn(T, Kd, seed=55), _randn(2 * F, Kd, seed=56, scale=0.05)
+	(gu, act), passes = _launches(PROF_ACT_FWD, lambda: K.gemm_act(a, w, K.ACT_SWIGLU))
+	assert (passes == 0) == fused
+	assert torch.equal(gu, K.gemm(a, w)) and torch.equal(act, K.swiglu_fwd(gu))
+	cs, n_rot = K.rope_table(64, D, 1e4), 2 * F // D - 1
+	got, passes = _launches(PROF_ROPE, lambda: K.gemm_rope(a, w, cs, 64, n_rot, D))
+	assert (passes == 0) == fused
+	assert torch.equal(got, K.gemm_rope(a, w, cs, 64, n_rot, D, fused=False))
+
+
 def test_gemm_strided_views(K):
 	# operands that are column slices of wider buffers (leading dimension > row length)
 	big = _randn(512, 1024, seed=6)
@@ -372,6 +387,25 @@ def test_gemm_output_at_any_element(K, shape):
 		assert torch.equal(view, ref)
 		big[1 : M + 1, 3 : N + 3] = 7
 		assert (big == 7).all()
+
+
+@pytest.mark.parametrize("tile_cfg,shape", [(7, (320, 576, 128)), (8, (192, 448, 192)), (9, (192, 320, 192)), (12, (64, 128, 320)), (0, (192, 320, 128))])
+def test_gemm_output_at_any_element_on_every_kind_of_tile(K, tile_cfg, shape):
+	"""The same on ragged tiles of both kernels, and for fp32 outputs (added to and stored, whole and in K ranges)."""
+	M, N, Kd = shape
+	A, B = _randn(M, Kd, seed=51), _randn(N, Kd, seed=52, scale=0.05)
+	R = _randn(M + 1, N + 3, seed=53)[1:, 1 : N + 1]
+	for epi, res, ks in ((K.EPI_BF16, None, 0), (K.EPI_BF16_RESID, R, 0), (K.EPI_F32_STORE, None, 0), (K.EPI_F32_ACC, None, 1), (K.EPI_F32_ACC, None, 2)):
+		kw = dict(epilogue=epi, tile_cfg=tile_cfg, k_splits=ks)
+		dt = torch.bfloat16 if res is not None or epi == K.EPI_BF16 else torch.float32
+		want = torch.full((M, N), 7.0, dtype=dt, device="cuda")
+		K.gemm(A, B, out=want, residual=res.contiguous() if res is not None else None, **kw)
+		big = torch.full((M + 2, N + 5), 7.0, dtype=dt, device="cuda")
+		view = big[1 : M + 1, 3 : N + 3]
+		K.gemm(A, B, out=view, residual=res, **kw)
+		assert torch.equal(view, want), (epi, ks)
+		view.fill_(7)
+		assert (big == 7).all(), (epi, ks)
 
 
 @pytest.mark.parametrize("d", [1032, 1600, 2040, 2048])

@@ -118,3 +118,38 @@ def test_pipeline_rejects_what_this_build_does_not_run():
 	pipe = Pipeline(st, None, scheduler="afab", partitioner=False, placement=[0], mb_size=2)
 	with pytest.raises(ValueError):
 		pipe(torch.zeros(6, 128, 256, dtype=torch.bfloat16, device="cuda"), None, None, split_size=3)  # larger than the stage was sized for
+
+
+def test_memory_figures_of_one_allocator_query():
+	from elf_amd.execution import engine as E
+
+	keep = torch.empty(3 << 20, dtype=torch.uint8, device="cuda")
+	del keep
+	held = torch.empty(1 << 20, dtype=torch.uint8, device="cuda")
+	assert E._mem() == (torch.cuda.memory_allocated(), torch.cuda.max_memory_allocated())
+	torch.cuda.reset_peak_memory_stats()
+	assert E._mem() == (torch.cuda.memory_allocated(), torch.cuda.max_memory_allocated())
+	del held
+
+
+def test_steps_in_a_row_hand_over_their_own_outputs():
+	"""Six steps on six batches without a wait in between: the host is never more than two steps' output copies ahead, and every
+	step's outputs and loss are those the same step gives alone."""
+	from elf_amd.pipeline import Pipeline, PipelineConfig
+
+	g = torch.Generator().manual_seed(11)
+	batches = [torch.randn(4, 128, 256, generator=g).to(torch.bfloat16).cuda() for _ in range(6)]
+	target = torch.zeros_like(batches[0])
+	pipe = Pipeline(_stages(2), batches[0][:2], config=PipelineConfig(scheduler="afab", partitioner=False, placement=[0, 0]))
+	alone = []
+	for b in batches:
+		out, loss = pipe(b, target, F.mse_loss, split_size=2)
+		torch.cuda.synchronize()
+		alone.append(([o.clone() for o in out], float(loss)))
+	got = []
+	for b in batches:
+		got.append(pipe(b, target, F.mse_loss, split_size=2))
+		assert len(pipe.engine._output_copies) <= 2
+	torch.cuda.synchronize()
+	for (out, loss), (want, want_loss) in zip(got, alone):
+		assert all(o.device.type == "cpu" and torch.equal(o, w) for o, w in zip(out, want)) and float(loss) == want_loss
