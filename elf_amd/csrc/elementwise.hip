@@ -640,7 +640,7 @@ int norm_fwd(int kind, const void* x, const void* gamma, const void* beta, void*
 }
 
 // never smaller for more rows: a workspace sized for a full micro-batch serves a shorter one (the balanced trips of
-// norm_bwd_blocks are not monotonic, 384 workgroups for 3074 rows and 512 for 3072)
+// norm_bwd_blocks are not monotonic, 385 workgroups for 3074 rows and 512 for 3072)
 int64_t norm_bwd_workspace_floats(int T, int d) {
 	const int64_t trip_blocks = ((int64_t)T + NORM_TRIP_ROWS - 1) / NORM_TRIP_ROWS;
 	return (norm_trip_rows(d) ? (trip_blocks < 512 ? trip_blocks : 512) : (int64_t)norm_bwd_blocks(T, d)) * 2 * d;

@@ -12,7 +12,6 @@
 
 #include "common.h"
 #include "kernels.h"
-#include "lds_dma.h"
 
 namespace elf {
 

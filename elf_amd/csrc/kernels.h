@@ -58,7 +58,7 @@ int gemm_dw_final(int M, int N, int K, const void* dY, int64_t lddy, const void*
 // filled round per launch instead of one per layer; when that round would leave half of the chip idle its tiles are
 // split along K and add in a fixed order).  scale != 0: every accumulator leaves multiplied by it, with its bf16 copy in
 // grad_bf16 (from the epilogue for whole tiles, by a small kernel behind the launch for split ones: same bits).  gemm_dw_groupable: a problem's
-// shape and operands fit (M, N multiples of 256, K of 64, 16-byte aligned, dense enough).
+// shape and operands fit (M, N of at least 256, all sizes multiples of 64, 16-byte aligned, dense enough).
 struct DwProblem {
 	const void* dY;
 	int64_t lddy;

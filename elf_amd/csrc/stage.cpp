@@ -125,7 +125,7 @@ struct Stage {
 	int norm_slots = 1;
 	void* attn_ws = nullptr;
 	int64_t attn_ws_bytes = 0;
-	int64_t ws_bytes = 0;  // fixed device workspaces of the stage (norm / attention backward scratch, rope table, gradient sink)
+	int64_t ws_bytes = 0;  // fixed device workspaces of the stage (norm / attention backward scratch, rope table)
 	// pinned blocks of released micro-batches whose last copy may still be in flight: they go back to the arena
 	// when their event has fired (polled, never waited for inside a step unless the arena would have to grow)
 	struct HostPending {
@@ -558,7 +558,7 @@ static int run_backward_params(Stage* s, MbState& m, hipStream_t st, float scale
 	const int T = s->T, d = s->d, F = s->F;
 	// dW[N_out, K_in] += dY[T, N_out]^T X[T, K_in] for every linear layer of the stage: the layers whose shapes fit go
 	// into launches of up to 16 (their workgroups fill the chip together), in the stage's layer order; the others
-	// (a head whose vocabulary is not a multiple of 256) run one by one.  Which way a layer goes depends on its shape
+	// (narrower than 256, or with an unaligned accumulator) run one by one.  Which way a layer goes depends on its shape
 	// alone, so every stream that reaches this W pass accumulates its gradients in the same order of roundings.
 	DwProblem group[16];
 	int ng = 0;
