@@ -39,9 +39,13 @@ int gemm_turn_giveups(uint64_t* out) {
 // Tile choice.  Estimated time of a product on tiles of bm x bn: rounds of 256 workgroups (one per compute unit) times the
 // time of a K slice of 64 times the slices and what a round costs besides (filling the ring, the epilogue), plus what a launch
 // costs once.  The constants are microseconds fitted to timings of every tile on some 10000 shapes (sizes spread over the
-// logarithm from 64 to 16384, operands rotated through 1 GB): over these the tile that is picked takes 0.3 to 0.4 % longer than
-// the best one on average, and more than 7 % longer for one shape in fifty.  A large tile has the cheaper products (per slice
-// and output: 21 ps on 256x256, 25 on 128x256, 35 on 128x128, 64 on 64x64: the smaller the tile, the more operand bytes go
+// logarithm from 64 to 16384, operands rotated through 1 GB): over these the tile that is picked takes 0.4 % longer than the best
+// one on average, and more than 7 % longer for one shape in fifty.  For K beyond RING_SHORT_K the bf16 constants are those of 33
+// shapes with cold operands instead, as good on average (0.35 %) and fonder of 256x256 tiles where several rounds of them are
+// close to more of 128x256: alone 8192 x 2304 x 768 and 8192 x 3072 x 768 are as fast on either, inside a stage's stream, where the
+// narrower tile's second fetch of B goes to memory, a GPT-2-small stage takes 7.86 ms with the first and 8.26 with the second.
+// A large tile has the cheaper products (per slice
+// and output: 22 ps on 256x256, 26 on 128x256, 35 on 128x128, 66 on 64x64: the smaller the tile, the more operand bytes go
 // through the 64 B/clk path into LDS for each product) and loses where its tiles leave compute units idle:
 //   1920 x 1600 x 1600: 44 us on 56 tiles of 256x256, 27 on 105 of 128x256, 19.9 on 195 of 128x128, 25 on 750 of 64x64;
 //   1920 x 4800 x 1600: 46 us on 152 tiles of 256x256, 52 on 285 of 128x256, 49 on 570 of 128x128.
@@ -50,8 +54,8 @@ struct TileTime {
 	float slice, round, launch;
 };
 static constexpr int N_TILES = 6;
-static constexpr TileTime TILES_BF16[N_TILES] = {{256, 256, 1.362f, 5.8f, 4.1f}, {128, 256, 0.811f, 5.5f, 1.4f}, {128, 128, 0.55f, 2.96f, 0.7f},
-                                                 {64, 128, 0.38f, 2.27f, 0.7f}, {128, 64, 0.395f, 2.06f, 0.6f}, {64, 64, 0.272f, 1.93f, 0.f}};
+static constexpr TileTime TILES_BF16[N_TILES] = {{256, 256, 1.45f, 0.f, 6.f}, {128, 256, 0.854f, 5.5f, 0.f}, {128, 128, 0.58f, 4.f, 0.f},
+                                                 {64, 128, 0.38f, 2.f, 0.f}, {128, 64, 0.40f, 2.f, 0.f}, {64, 64, 0.27f, 1.3f, 0.f}};
 // K of at most RING_SHORT_K: the small tiles on the ring of two slices
 static constexpr TileTime TILES_SHORT[N_TILES] = {{256, 256, 1.293f, 7.15f, 2.5f}, {128, 256, 0.996f, 4.9f, 0.44f}, {128, 128, 0.388f, 1.94f, 3.5f},
                                                   {64, 128, 0.285f, 0.93f, 3.7f}, {128, 64, 0.325f, 1.0f, 2.4f}, {64, 64, 0.184f, 0.55f, 2.9f}};
