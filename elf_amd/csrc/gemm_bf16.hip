@@ -96,7 +96,9 @@ static Plan plan_weight_gradient(int M, int N, int K, int max_splits = 16) {
 	Plan best;
 	for (const TileTime& t : TILES_F32) {
 		if (M < t.bm || N < t.bn) continue;
-		for (int ks = 1; ks <= max_splits && (ks == 1 || K / BK / ks >= 3); ks++) {
+		const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+		// (what was measured: three slices or more a split, little more than two rounds of workgroups)
+		for (int ks = 1; ks <= max_splits && (ks == 1 || (K / BK / ks >= 3 && tiles * ks <= 600)); ks++) {
 			const float add = ks == 1 ? 0.f : t.bn == 256 ? ks * (1.6f + 1.3e-6f * (float)M * N) : ks * (2.2f + 1.2e-4f * t.bm * t.bn + 7.4e-6f * (float)M * N);
 			const float us = tile_us(t, M, N, K / BK, ks) + add;
 			if (us < best.us) best = Plan{t.bm, t.bn, ks, us};
