@@ -51,10 +51,10 @@ _DENSE_MAX = 1024 * 16 * 8 - 7  # widest row elf_cross_entropy_dense holds in re
 
 def _run(pred, target, *, ignore_index, scale, mean, want_grad, padded=True):
 	"""(row_loss fp32 [rows], out2 = [sum, count] fp32, grad or None).  The gradient is [rows, ld_out] bf16 with ``ld_out`` a
-	multiple of 64, or, unless ``padded``, [rows, V] where the logits are one dense block: rows that start at any address are
-	then read in place (50257 columns: the padded copy of the logits took half of a loss's time)."""
+	multiple of 64, or, unless ``padded``, [rows, V] where V is a multiple of 8 or the logits are one dense block: rows that start
+	at any address are then read in place (50257 columns: the padded copy of the logits took half of a loss's time)."""
 	V = pred.shape[-1]
-	dense = (not padded if want_grad else V % 8 != 0) and pred.dtype == torch.bfloat16 and pred.is_cuda and pred.is_contiguous() and not pred.is_neg() and pred.data_ptr() % 16 == 0 and 0 < V <= _DENSE_MAX
+	dense = V % 8 != 0 and not (want_grad and padded) and pred.dtype == torch.bfloat16 and pred.is_cuda and pred.is_contiguous() and not pred.is_neg() and pred.data_ptr() % 16 == 0 and 0 < V <= _DENSE_MAX
 	src, ld = (pred, V) if dense else _rows_view(pred, V)
 	rows = pred.numel() // V
 	target = _check_target(target, rows)
@@ -67,7 +67,7 @@ def _run(pred, target, *, ignore_index, scale, mean, want_grad, padded=True):
 		_lib.check(lib.elf_cross_entropy_reduce(None, target.data_ptr(), rows, ignore_index, out2.data_ptr(), _stream()), "elf_cross_entropy_reduce")
 		div = out2[1:]
 	if want_grad:
-		ld_out = V if dense else -(-V // _PAD) * _PAD
+		ld_out = V if dense or (V % 8 == 0 and not padded) else -(-V // _PAD) * _PAD
 		grad = torch.empty(rows, ld_out, dtype=torch.bfloat16, device=dev)
 	if dense:
 		_lib.check(
