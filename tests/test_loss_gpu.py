@@ -109,6 +109,18 @@ def test_cross_entropy_dense_rows_of_any_width(V, offset):
 	assert torch.equal(twice, grad * -2)
 
 
+@pytest.mark.parametrize("n", [1, 7, 8, 2047, 2048, 2049, 4103, (1 << 25) - 9, (1 << 25) - 1, 1 << 25, (1 << 25) + 4095, (1 << 25) + 8191])
+def test_scaling_pass_at_the_edges_of_its_grids(n):
+	"""Whole and partly filled workgroups of one and two chunks a thread, the last elements of no whole chunk, the step to the pass
+	that goes past the caches: the bits of the torch product, nothing behind the end touched."""
+	from elf_amd import _lib
+
+	x = torch.randn(n, device="cuda", generator=torch.Generator(device="cuda").manual_seed(n)).to(torch.bfloat16)
+	g, y = torch.tensor(-1.7, device="cuda"), torch.full((n + 4096,), 7.0, dtype=torch.bfloat16, device="cuda")
+	_lib.check(_lib.load().elf_scale_by_bf16(x.data_ptr(), g.data_ptr(), y.data_ptr(), n, torch.cuda.current_stream().cuda_stream), "elf_scale_by_bf16")
+	assert torch.equal(y[:n], x * g.to(torch.bfloat16)) and bool((y[n:] == 7).all())
+
+
 @pytest.mark.parametrize("V", [1000, 1003])
 def test_cross_entropy_gradients_for_a_batch_of_incoming_gradients(V):
 	"""``is_grads_batched``: the backward is run once under vmap, with an incoming gradient that has no storage of its own; and an
