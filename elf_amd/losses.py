@@ -58,13 +58,13 @@ def _run(pred, target, *, ignore_index, scale, mean, want_grad, padded=True):
 	src, ld = (pred, V) if dense else _rows_view(pred, V)
 	rows = pred.numel() // V
 	target = _check_target(target, rows)
-	lib = _lib.load()
+	lib, stream = _lib.load(), _stream()
 	dev = pred.device
 	row_loss = torch.empty(rows, dtype=torch.float32, device=dev)
 	out2 = torch.empty(2, dtype=torch.float32, device=dev)
 	grad, ld_out, div = None, 0, None
 	if mean:  # the gradient divides by the number of live rows, which only depends on the target
-		_lib.check(lib.elf_cross_entropy_reduce(None, target.data_ptr(), rows, ignore_index, out2.data_ptr(), _stream()), "elf_cross_entropy_reduce")
+		_lib.check(lib.elf_cross_entropy_reduce(None, target.data_ptr(), rows, ignore_index, out2.data_ptr(), stream), "elf_cross_entropy_reduce")
 		div = out2[1:]
 	if want_grad:
 		ld_out = V if dense or (V % 8 == 0 and not padded) else -(-V // _PAD) * _PAD
@@ -72,16 +72,16 @@ def _run(pred, target, *, ignore_index, scale, mean, want_grad, padded=True):
 	if dense:
 		_lib.check(
 			lib.elf_cross_entropy_dense(src.data_ptr(), target.data_ptr(), rows, V, ignore_index, scale, div.data_ptr() if div is not None else None,
-				row_loss.data_ptr(), grad.data_ptr() if grad is not None else None, _stream()),
+				row_loss.data_ptr(), grad.data_ptr() if grad is not None else None, stream),
 			"elf_cross_entropy_dense",
 		)
 	else:
 		_lib.check(
 			lib.elf_cross_entropy(src.data_ptr(), ld, target.data_ptr(), rows, V, ignore_index, scale, div.data_ptr() if div is not None else None,
-				row_loss.data_ptr(), grad.data_ptr() if grad is not None else None, ld_out, _stream()),
+				row_loss.data_ptr(), grad.data_ptr() if grad is not None else None, ld_out, stream),
 			"elf_cross_entropy",
 		)
-	_lib.check(lib.elf_cross_entropy_reduce(row_loss.data_ptr(), target.data_ptr(), rows, ignore_index, out2.data_ptr(), _stream()), "elf_cross_entropy_reduce")
+	_lib.check(lib.elf_cross_entropy_reduce(row_loss.data_ptr(), target.data_ptr(), rows, ignore_index, out2.data_ptr(), stream), "elf_cross_entropy_reduce")
 	return row_loss, out2, grad
 
 
@@ -95,12 +95,15 @@ def _reduced(row_loss, out2, reduction, shape):
 	raise ValueError(f"{reduction} is not a valid value for reduction")
 
 
+_has_storage, _wrapped, _dispatch_modes = torch._C._has_storage, torch._C._functorch.is_functorch_wrapped_tensor, torch._C._len_torch_dispatch_stack
+
+
 def _plain(t):
 	"""Whether a kernel may read ``t`` through its pointer: under vmap it is a batch without storage of its own, and a view
 	such as ``z.conj().imag`` holds its values negated.  Nor may it where somebody follows the operations on ``t``: in a
 	forward-mode level (a tangent) or under a dispatch mode (a trace)."""
-	return (type(t) is torch.Tensor and torch._C._has_storage(t) and not torch._C._functorch.is_functorch_wrapped_tensor(t)
-	        and not t.is_neg() and not t._is_zerotensor() and forward_ad._current_level < 0 and not torch._C._len_torch_dispatch_stack())
+	return (type(t) is torch.Tensor and _has_storage(t) and not _wrapped(t) and not t.is_neg() and not t._is_zerotensor()
+	        and forward_ad._current_level < 0 and not _dispatch_modes())
 
 
 class _CrossEntropy(torch.autograd.Function):
@@ -114,7 +117,7 @@ class _CrossEntropy(torch.autograd.Function):
 	def backward(ctx, g):
 		V = ctx.shape[-1]
 		grad = ctx.grad
-		if _plain(g) and grad.shape[1] == V and g.dim() == 0 and g.dtype == torch.float32 and not (torch.is_grad_enabled() and g.requires_grad):
+		if grad.shape[1] == V and g.dim() == 0 and g.dtype == torch.float32 and not (g.requires_grad and torch.is_grad_enabled()) and _plain(g):
 			# one pass of 16-byte accesses with the same roundings (2048 x 50257: 60 us, 82 as a torch product of the strided view)
 			out = torch.empty(ctx.shape, dtype=grad.dtype, device=grad.device)
 			_lib.check(_lib.load().elf_scale_by_bf16(grad.data_ptr(), g.data_ptr(), out.data_ptr(), out.numel(), _stream()), "elf_scale_by_bf16")
