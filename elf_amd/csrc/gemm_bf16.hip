@@ -39,28 +39,29 @@ int gemm_turn_giveups(uint64_t* out) {
 // Tile choice.  Estimated time of a product on tiles of bm x bn: rounds of 256 workgroups (one per compute unit) times the
 // time of a K slice of 64 times the slices and what a round costs besides (filling the ring, the epilogue), plus what a launch
 // costs once.  The constants are microseconds fitted to timings of every tile on some 10000 shapes (sizes spread over the
-// logarithm from 64 to 16384, operands rotated through 1 GB): over these the tile that is picked takes 0.4 % longer than the best
-// one on average, and more than 7 % longer for one shape in fifty.  For K beyond RING_SHORT_K the bf16 constants are those of 33
-// shapes with cold operands instead, as good on average (0.35 %) and fonder of 256x256 tiles where several rounds of them are
-// close to more of 128x256: alone 8192 x 2304 x 768 and 8192 x 3072 x 768 are as fast on either, inside a stage's stream, where the
-// narrower tile's second fetch of B goes to memory, a GPT-2-small stage takes 7.86 ms with the first and 8.26 with the second.
-// A large tile has the cheaper products (per slice
-// and output: 22 ps on 256x256, 26 on 128x256, 35 on 128x128, 66 on 64x64: the smaller the tile, the more operand bytes go
-// through the 64 B/clk path into LDS for each product) and loses where its tiles leave compute units idle:
-//   1920 x 1600 x 1600: 44 us on 56 tiles of 256x256, 27 on 105 of 128x256, 19.9 on 195 of 128x128, 25 on 750 of 64x64;
-//   1920 x 4800 x 1600: 46 us on 152 tiles of 256x256, 52 on 285 of 128x256, 49 on 570 of 128x128.
+// logarithm from 64 to 16384, operands rotated through 1 GB).  For K beyond RING_SHORT_K the bf16 constants come from 226 of
+// them: the tile that is picked takes 0.4 % longer than the best one on average, and more than 7 % longer for 5 of the 226.
+// A large tile has the cheaper products (per slice and output: 18 ps on 256x256, 23 on 128x256, 30 on 128x128, 52 on 64x64: the
+// smaller the tile, the more operand bytes go through the 64 B/clk path into LDS for each product) and loses where its tiles leave
+// compute units idle.  The tiles of 160, 192 and 224 rows are for sizes of which 256-row tiles leave a round partly empty and
+// 128-row ones make twice the rounds (without them the best tile takes 2.9 % longer on average): before -> after (us)
+//   2688 x 4096 x 28672 (a Llama-3-8B block's input gradient over 3 x 896 tokens) 504 on 176 tiles of 256 rows, 463 on 224 of 192;
+//   2688 x 4096 x 14336 with a residual 266 -> 231, 1920 x 4800 x 1600 32.1 on 152 tiles, 28.0 on 228 of 160,
+//   8192 x 2304 x 768 37.4 on 288 tiles of 256 rows, 31.1 on 468 of 160, 4096 x 5504 x 2048 with the SwiGLU backward 131 on 352
+//   tiles of 256 rows, 117 on 484 of 192; 1920 x 1600 x 1600 stays on 195 tiles of 128x128 (14.6; 24 on 84 of 160 rows).
 struct TileTime {
 	int bm, bn;
 	float slice, round, launch;
 };
-static constexpr int N_TILES = 6;
-static constexpr TileTime TILES_BF16[N_TILES] = {{256, 256, 1.45f, 0.f, 6.f}, {128, 256, 0.854f, 5.5f, 0.f}, {128, 128, 0.58f, 4.f, 0.f},
-                                                 {64, 128, 0.38f, 2.f, 0.f}, {128, 64, 0.40f, 2.f, 0.f}, {64, 64, 0.27f, 1.3f, 0.f}};
+static constexpr TileTime TILES_BF16[] = {{256, 256, 1.18f, 6.f, 0.f}, {128, 256, 0.739f, 5.f, 0.f}, {128, 128, 0.487f, 2.9f, 0.4f}, {64, 128, 0.32f, 2.2f, 0.9f},
+                                          {128, 64, 0.341f, 1.9f, 1.f}, {64, 64, 0.213f, 1.5f, 1.3f}};
+// the tiles between 128 and 256 rows (k-contiguous A and bf16 outputs only)
+static constexpr TileTime TILES_MID[] = {{224, 256, 1.01f, 11.1f, 0.f}, {192, 256, 0.938f, 6.5f, 0.f}, {160, 256, 0.854f, 6.2f, 0.f}};
 // K of at most RING_SHORT_K: the small tiles on the ring of two slices
-static constexpr TileTime TILES_SHORT[N_TILES] = {{256, 256, 1.293f, 7.15f, 2.5f}, {128, 256, 0.996f, 4.9f, 0.44f}, {128, 128, 0.388f, 1.94f, 3.5f},
+static constexpr TileTime TILES_SHORT[] = {{256, 256, 1.293f, 7.15f, 2.5f}, {128, 256, 0.996f, 4.9f, 0.44f}, {128, 128, 0.388f, 1.94f, 3.5f},
                                                   {64, 128, 0.285f, 0.93f, 3.7f}, {128, 64, 0.325f, 1.0f, 2.4f}, {64, 64, 0.184f, 0.55f, 2.9f}};
 // weight gradients: both operands reduction-major, fp32 read-modify-write of the output
-static constexpr TileTime TILES_F32[N_TILES] = {{256, 256, 1.3f, 22.f, 0.f}, {128, 256, 0.757f, 12.9f, 0.f}, {128, 128, 0.537f, 9.9f, 0.f},
+static constexpr TileTime TILES_F32[] = {{256, 256, 1.3f, 22.f, 0.f}, {128, 256, 0.757f, 12.9f, 0.f}, {128, 128, 0.537f, 9.9f, 0.f},
                                                 {64, 128, 0.442f, 5.9f, 0.f}, {128, 64, 0.416f, 7.5f, 0.f}, {64, 64, 0.26f, 4.f, 0.f}};
 
 struct Plan {
@@ -75,16 +76,24 @@ static float tile_us(const TileTime& t, int M, int N, int slices, int k_splits =
 	return rounds * ((slices + k_splits - 1) / k_splits * t.slice + t.round) + t.launch;
 }
 
-// The tile of a bf16 output with the smallest estimate.  For an epilogue that only the 256-column tiles have: epi_extra, its time
-// per round of 256x256 tiles, and ring_extra, the time of the pass of its own that the small ring tiles need instead.
-static Plan plan_tiles(int M, int N, int K, float ring_extra = 0.f, float epi_extra = 0.f) {
+// The tile of a bf16 output with the smallest estimate.  mid: the tiles between 128 and 256 rows are to be had.  For an epilogue
+// that only the 256-column tiles have: epi_extra, its time per round of 256x256 tiles, and ring_extra, the time of the pass of its
+// own that the small ring tiles need instead.
+static Plan plan_tiles(int M, int N, int K, bool mid = true, float ring_extra = 0.f, float epi_extra = 0.f) {
 	Plan best;
-	for (TileTime t : K <= RING_SHORT_K ? TILES_SHORT : TILES_BF16) {
-		if (M < t.bm || N < t.bn) continue;
+	auto weigh = [&](TileTime t) {
+		if (M < t.bm || N < t.bn) return;
 		if (t.bn == 256) t.round += epi_extra * t.bm / 256;
 		const float us = tile_us(t, M, N, K / BK) + (t.bn == 256 ? 0.f : ring_extra);
 		if (us < best.us) best = Plan{t.bm, t.bn, 1, us};
+	};
+	if (K <= RING_SHORT_K) {
+		for (const TileTime& t : TILES_SHORT) weigh(t);
+		return best;
 	}
+	for (const TileTime& t : TILES_BF16) weigh(t);
+	if (mid)
+		for (const TileTime& t : TILES_MID) weigh(t);
 	return best;
 }
 
@@ -107,11 +116,11 @@ static Plan plan_weight_gradient(int M, int N, int K, int max_splits = 16) {
 	return best;
 }
 
-// 256 or 128: the direct-to-LDS tile of 256 columns a forward / input-gradient product runs on, 0: one of the ring tiles
+// The rows of the direct-to-LDS tile of 256 columns a forward / input-gradient product runs on, 0: one of the ring tiles
 // (never with ring_extra = NO_RING, unless no tile of 256 columns fits).
 constexpr float NO_RING = 1e20f;
 static int dma_tile_rows(int M, int N, int K, float ring_extra, float epi_extra) {
-	const Plan p = plan_tiles(M, N, K, ring_extra, epi_extra);
+	const Plan p = plan_tiles(M, N, K, true, ring_extra, epi_extra);
 	return p.dma() ? p.bm : 0;
 }
 // what a pass of its own over `bytes` costs (5 TB/s and a launch)
@@ -170,7 +179,7 @@ int gemm_bf16(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda,
 	if (bm == 0) {
 		Plan p;
 		if (epi != EPI_F32_ACC) {
-			p = plan_tiles(M, N, K);
+			p = plan_tiles(M, N, K, !a_t && (epi == EPI_BF16 || epi == EPI_BF16_RESID));
 		} else if (k_splits > 0) {
 			p = plan_weight_gradient(M, N, K, 1);
 		} else if (M >= 256 && N >= 256 && (int64_t)((M + 255) / 256) * ((N + 255) / 256) >= 192 && K >= 4096) {
@@ -253,14 +262,25 @@ int gemm_rope_bf16(int M, int N, int K, const void* A, int64_t lda, const void* 
 
 // What the fused kernel can run at all (a caller without scratch or with strided buffers relies on it) ...
 static bool swiglu_bwd_fits(int M, int F, int K) { return M >= 256 && F >= 256 && M % 64 == 0 && F % 64 == 0 && K % 64 == 0; }
-// ... and where it is also the faster way.
+// The tile it runs on.  The epilogue reads and writes four of d, g, u and their two gradients at 256 tiles a time: 20 us more per
+// round of 256-row tiles than the plain one (fitted to 700 shapes; with 12 us for the whole round 1024 x 3072 x 64 took 25 us
+// fused, 13 apart, and 8448 x 512 x 512 32 and 20).
+static Plan swiglu_bwd_tile(int M, int F, int K) {
+	Plan best;
+	auto weigh = [&](TileTime t) {
+		if (M < t.bm) return;
+		t.round += 20.f * t.bm / 256;
+		const float us = tile_us(t, M, F, K / BK);
+		if (us < best.us) best = Plan{t.bm, t.bn, 1, us};
+	};
+	weigh(TILES_BF16[0]);
+	if (K > RING_SHORT_K)
+		for (const TileTime& t : TILES_MID) weigh(t);
+	return best;
+}
+// ... and where it is also the faster way: against the best tile of the plain product and the pass over d, g, u and their gradients.
 bool gemm_swiglu_bwd_fused(int M, int F, int K) {
-	if (!swiglu_bwd_fits(M, F, K)) return false;
-	// 256x256 tiles only: against the best tile of the plain product and the pass over d, g, u and their gradients.  The epilogue
-	// reads and writes four of those five at 256 tiles a time, 20 us more per round than the plain one (fitted to 700 shapes;
-	// with 12 us for the whole round 1024 x 3072 x 64 took 25 us fused, 13 apart, and 8448 x 512 x 512 32 and 20)
-	const TileTime fused{256, 256, 1.24f, 27.f, 0.f};
-	return tile_us(fused, M, F, K / BK) < plan_tiles(M, F, K).us + pass_us(10.0 * M * F);
+	return swiglu_bwd_fits(M, F, K) && swiglu_bwd_tile(M, F, K).us < plan_tiles(M, F, K).us + pass_us(10.0 * M * F);
 }
 
 int gemm_swiglu_bwd_bf16(int M, int F, int K, const void* dY, int64_t lddy, const void* W, int64_t ldw, const void* gu,
@@ -272,7 +292,7 @@ int gemm_swiglu_bwd_bf16(int M, int F, int K, const void* dY, int64_t lddy, cons
 		// the activation backward's arithmetic is not counted: the figure stays the GEMM's
 		ProfScope prof(PROF_GEMM, 2.0 * M * F * K, stream);
 		ELF_REQUIRE(!act || (ldact >= F && ldact % 8 == 0 && ((uintptr_t)act % 16) == 0), "gemm_swiglu_bwd: bad activation output");
-		return gemm_bf16_dma(0, 1, M, F, K, dY, lddy, W, ldw, dgu, lddgu, EPI_BF16_SWIGLU_BWD, gu, ldgu, 1, 0, 256, stream, act, ldact);
+		return gemm_bf16_dma(0, 1, M, F, K, dY, lddy, W, ldw, dgu, lddgu, EPI_BF16_SWIGLU_BWD, gu, ldgu, 1, 0, swiglu_bwd_tile(M, F, K).bm, stream, act, ldact);
 	}
 	ELF_REQUIRE(scratch, "gemm_swiglu_bwd: this shape needs a scratch buffer of M x F bf16");
 	ELF_REQUIRE(ldgu == 2 * F && lddgu == 2 * F, "gemm_swiglu_bwd: the unfused path needs dense [M, 2F] buffers");

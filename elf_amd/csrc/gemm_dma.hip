@@ -112,7 +112,7 @@ int dma_turn_giveups(uint64_t* out) {
 int gemm_bf16_dma(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb, void* C,
                   int64_t ldc, int epi, const void* R, int64_t ldr, int k_splits, int tail_tiles, int bm, hipStream_t stream,
                   void* C2, int64_t ldc2, const void* rope_cs, int rope_S, int rope_cols, int rope_D, float scale) {
-	ELF_REQUIRE(bm == 256 || bm == 128, "gemm (dma tile): 256- or 128-row tiles");
+	ELF_REQUIRE(bm == 256 || bm == 128 || (!a_t && gemm_mid_rows(bm)), "gemm (dma tile): 256- or 128-row tiles, 160, 192 or 224 rows with a k-contiguous A");
 	ELF_REQUIRE(M >= bm && N >= dma::BN && M % 64 == 0 && N % 64 == 0 && K % dma::BKS == 0, "gemm (dma tile): M at least %d, N at least 256, all sizes multiples of 64", bm);
 	const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + dma::BN - 1) / dma::BN, ntiles = tiles_m * tiles_n;
 	ELF_REQUIRE(gemm_reaches(a_t ? dma::BKS : bm, lda) && gemm_reaches(b_t ? dma::BKS : dma::BN, ldb), "gemm (dma tile): leading dimension too large (%lld, %lld)", (long long)lda, (long long)ldb);

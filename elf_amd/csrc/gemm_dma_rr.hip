@@ -20,7 +20,28 @@ static int launch_epi(const Args& a, int epi, hipStream_t stream) {
 	return -1;
 }
 
-int launch_rr(int bm, const Args& a, int epi, hipStream_t stream) { return bm == 128 ? launch_epi<4>(a, epi, stream) : launch_epi<8>(a, epi, stream); }
+// the tiles between them: bf16 outputs, always clipped (an aligned size loses nothing by it)
+template <int RF>
+static int launch_mid(const Args& a, int epi, hipStream_t stream) {
+	switch (epi) {
+		case EPI_BF16: return launch_sized<4, RF, false, false, EPI_BF16, true>(a, stream);
+		case EPI_BF16_RESID: return launch_sized<4, RF, false, false, EPI_BF16_RESID, true>(a, stream);
+		case EPI_BF16_SWIGLU: return launch_sized<4, RF, false, false, EPI_BF16_SWIGLU, true>(a, stream);
+		case EPI_BF16_ROPE: return launch_sized<4, RF, false, false, EPI_BF16_ROPE, true>(a, stream);
+	}
+	set_error("gemm: epilogue %d has no %d-row tile", epi, RF * 32);
+	return -1;
+}
+
+int launch_rr(int bm, const Args& a, int epi, hipStream_t stream) {
+	switch (bm) {
+		case 128: return launch_epi<4>(a, epi, stream);
+		case 160: return launch_mid<5>(a, epi, stream);
+		case 192: return launch_mid<6>(a, epi, stream);
+		case 224: return launch_mid<7>(a, epi, stream);
+		default: return launch_epi<8>(a, epi, stream);
+	}
+}
 
 int rr_turn_giveups(uint64_t* sum) { return add_turn_giveups(sum); }
 

@@ -698,4 +698,7 @@ int rt_turn_giveups(uint64_t* sum);
 
 }  // namespace dma
 
+// the tiles between 128 and 256 rows
+inline bool gemm_mid_rows(int bm) { return bm == 160 || bm == 192 || bm == 224; }
+
 }  // namespace elf

@@ -197,6 +197,29 @@ def test_gemm_bits_do_not_depend_on_the_tile(K):
 			assert torch.equal(K.gemm(a, b, tile_cfg=cfg, **kw), want), f"tile config {cfg} {kw}"
 
 
+@pytest.mark.parametrize("M,N,Kd", [(2112, 3968, 320), (2624, 4160, 320), (2624, 4160, 448), (4096, 3072, 2048), (896, 14336, 512)])
+def test_gemm_tiles_between_128_and_256_rows(K, M, N, Kd):
+	"""Sizes for which the tile rule takes 160, 192 and 224 rows (for one of the epilogues at least), with moved last tiles that end
+	inside a wave's 32-row strip, and fewer and more K slices than a turn of the ring: the bits of the 64x64 tile for every
+	epilogue (all tiles add the products in the same order), nothing written outside the output."""
+	a, w, r, bias = _randn(M, Kd, seed=71), _randn(N, Kd, seed=72, scale=0.05), _randn(M, N, seed=73), _randn(1, N, seed=74)
+	for kw, b in ((dict(), w), (dict(b_t=True), w.t().contiguous())):
+		want = K.gemm(a, b, tile_cfg=12, **kw)
+		big = torch.full((M + 64, N + 64), 7.0, dtype=torch.bfloat16, device="cuda")
+		K.gemm(a, b, out=big[:M, :N], **kw)
+		assert torch.equal(big[:M, :N], want) and (big[M:] == 7).all() and (big[:, N:] == 7).all()
+		for res in (dict(residual=r), dict(residual=bias, residual_ld=0)):
+			assert torch.equal(K.gemm(a, b, epilogue=K.EPI_BF16_RESID, **res, **kw), K.gemm(a, b, epilogue=K.EPI_BF16_RESID, tile_cfg=12, **res, **kw))
+	S, D = 64, 128 if N % 128 == 0 else 64
+	cs, n_rot = K.rope_table(S, D, 5e5), N // D // 2
+	assert torch.equal(K.gemm_rope(a, w, cs, S, n_rot, D), K.gemm_rope(a, w, cs, S, n_rot, D, fused=False))
+	if N % 128 == 0:
+		gu, act = K.gemm_act(a, w, K.ACT_SWIGLU)
+		assert torch.equal(gu, K.gemm(a, w, tile_cfg=12)) and torch.equal(act, K.swiglu_fwd(gu))
+	g, wt = _randn(M, 2 * N, seed=75), w.t().contiguous()
+	assert torch.equal(K.gemm_swiglu_bwd(a, wt, g), K.gemm_swiglu_bwd(a, wt, g, fused=False))
+
+
 @pytest.mark.parametrize("shape", [(64, 64, 15424), (256, 704, 14080), (512, 384, 10112), (1536, 192, 12608), (64, 5632, 13696), (128, 256, 192)])
 def test_small_weight_gradients_are_split_along_the_tokens(K, shape):
 	"""Outputs too small for the chip with long reductions: the choice left open runs about as fast as the best of a few explicit
