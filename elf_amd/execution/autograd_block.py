@@ -10,7 +10,7 @@ several inputs and outputs.  There is no CPU path: construction needs the GPU an
 """
 
 import logging
-from contextlib import contextmanager
+from contextlib import contextmanager, nullcontext
 
 import torch
 from torch.utils.checkpoint import checkpoint
@@ -76,8 +76,8 @@ class AutogradStageBlock(StageBlockBase):
 			if x.is_floating_point() or x.is_complex():
 				x.requires_grad_(True)
 			inputs.append(x)
-		strategy = options.get(OpOptions.REMAT_STRATEGY) or (lambda *_: False)
-		with self._selective_remat(strategy, mb_id):
+		strategy = options.get(OpOptions.REMAT_STRATEGY)
+		with self._selective_remat(strategy, mb_id) if strategy else nullcontext():
 			y = self._run(inputs, f"forward({self.id}:{mb_id})")
 			for m in self._layers_dw():
 				m.move_last_computed("input", mb_id)

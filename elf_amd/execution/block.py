@@ -651,5 +651,11 @@ class HipStageBlock(StageBlockBase):
 		_lib.check(self.lib.elf_stage_mem_stats(self._handle, ctypes.byref(st)), "elf_stage_mem_stats")
 		return {n: getattr(st, n) for n, _ in MemStats._fields_}
 
+	def live_and_peak(self):
+		"""The two of ``mem_stats`` that the Engine books after every operation."""
+		st = MemStats()
+		_lib.check(self.lib.elf_stage_mem_stats(self._handle, ctypes.byref(st)), "elf_stage_mem_stats")
+		return st.live_bytes, st.peak_bytes
+
 	def reset_peak(self):
 		_lib.check(self.lib.elf_stage_reset_peak(self._handle), "elf_stage_reset_peak")

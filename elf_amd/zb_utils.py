@@ -40,7 +40,7 @@ class LinearDX(torch.autograd.Function):
 		ctx.save_for_backward(input.detach())  # marks the input as needed by the backward, so that torch.utils.checkpoint recomputes it
 		x = _as_rows(input)
 		if bias is not None:
-			y = kernels.gemm(x, weight, epilogue=kernels.EPI_BF16_RESID, residual=bias.reshape(1, -1).expand(1, weight.shape[0]), residual_ld=0)
+			y = kernels.gemm(x, weight, epilogue=kernels.EPI_BF16_RESID, residual=bias, residual_ld=0)
 		else:
 			y = kernels.gemm(x, weight)
 		return y.view(*input.shape[:-1], weight.shape[0])
@@ -88,17 +88,18 @@ class LayerDW:
 	def _state(self):
 		return f"({sum(x is not None for x in self.ctx['input'])},{sum(x is not None for x in self.ctx['grad_output'])})"
 
+	# (last_input and last_grad_output are plain attributes: nn.Module.__setattr__ first looks for a parameter, a module and a
+	# buffer of that name, 3 us each time)
 	def _store_input(self, input):
-		self.last_input = input.detach()
+		last = input.detach()
 		# an input without a grad_fn is the stage's own input: checkpointing will not recompute it, so the
 		# remat logic must not drop it
-		setattr(self.last_input, "is_model_input", input.grad_fn is None)
+		last.is_model_input = input.grad_fn is None
+		self.__dict__["last_input"] = last
 
 	def _accumulate_grad_output(self, grad_output):
-		if getattr(self, "last_grad_output", None) is None:
-			self.last_grad_output = grad_output
-		else:
-			self.last_grad_output = self.last_grad_output + grad_output
+		last = getattr(self, "last_grad_output", None)
+		self.__dict__["last_grad_output"] = grad_output if last is None else last + grad_output
 
 	def set(self, queue, idx, value):
 		values = self.ctx[queue]
@@ -119,7 +120,7 @@ class LayerDW:
 		if last_value is None:
 			return  # a sub-module the forward did not use
 		self.set(queue, idx, last_value)
-		setattr(self, f"last_{queue}", None)
+		self.__dict__[f"last_{queue}"] = None
 
 	def offload_last(self, idx, to="cpu"):
 		with torch.no_grad():
