@@ -54,6 +54,7 @@ struct AttnBwdArgs {
 	// stored as they are.  See split_walk().
 	int h_splits, q_splits;
 	float* dkv_part;
+	int paired;  // causal: a workgroup takes two key tiles one after the other (see attn_bwd_kernel); 0: one
 };
 
 // The walk of one workgroup: query heads [h0, h0 + nh) and, per head, query tiles [q_lo, q_hi) of a pass.
@@ -235,7 +236,7 @@ __device__ __forceinline__ void store_dkv_part(const f32x16 (&acc_dk)[D / 32], c
 // partial dQ buffer (bf16).  The softmax scale of dK and dQ is applied by the epilogue / the
 // reduction kernel.  With a causal mask key tile kt meets 1 - kt/nkt of the query tiles, so
 // a workgroup takes the tiles kt and nkt-1-kt one after the other: every workgroup then does
-// the same amount of work.
+// the same amount of work.  (Where there are workgroups to spare each takes one tile: split_walk().)
 template <int D, bool CAUSAL>
 __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kernel(AttnBwdArgs a) {
 	using TL = BwdTile<D>;
@@ -256,7 +257,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kernel(AttnBwdA
 	const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 	const int g = lane >> 5, kl = lane & 31;
 	const int nkt = a.S / BKV;
-	const int npair = CAUSAL ? (nkt + 1) / 2 : nkt;
+	const int npair = CAUSAL && a.paired ? (nkt + 1) / 2 : nkt;
 	const Walk wk = locate_walk(a, npair);
 	const int pair = wk.pair, hk = wk.hk, b = wk.b;
 	const int64_t tok0 = (int64_t)b * a.S;
@@ -295,7 +296,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kernel(AttnBwdA
 			}
 	};
 
-	const int n_pass = (CAUSAL && nkt - 1 - pair != pair) ? 2 : 1;
+	const int n_pass = (CAUSAL && a.paired && nkt - 1 - pair != pair) ? 2 : 1;
 #pragma unroll 1
 	for (int pass = 0; pass < n_pass; pass++) {
 		const int kt_idx = pass == 0 ? pair : nkt - 1 - pair;
@@ -548,7 +549,7 @@ __global__ __launch_bounds__(256) void attn_bwd_kernel_lone(AttnBwdArgs a) {
 	const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 	const int g = lane >> 5, kl = lane & 31;
 	const int nkt = a.S / BKV;
-	const int npair = CAUSAL ? (nkt + 1) / 2 : nkt;
+	const int npair = CAUSAL && a.paired ? (nkt + 1) / 2 : nkt;
 	const Walk wk = locate_walk(a, npair);
 	const int pair = wk.pair, hk = wk.hk, b = wk.b;
 	const int64_t tok0 = (int64_t)b * a.S;
@@ -586,7 +587,7 @@ __global__ __launch_bounds__(256) void attn_bwd_kernel_lone(AttnBwdArgs a) {
 			}
 	};
 
-	const int n_pass = (CAUSAL && nkt - 1 - pair != pair) ? 2 : 1;
+	const int n_pass = (CAUSAL && a.paired && nkt - 1 - pair != pair) ? 2 : 1;
 #pragma unroll 1
 	for (int pass = 0; pass < n_pass; pass++) {
 		const int kt_idx = pass == 0 ? pair : nkt - 1 - pair;
@@ -957,17 +958,19 @@ using namespace attn;
 // 16 bytes per element of dK to write and to read again.  The whole call, before -> after (us): 2 x 2048 tokens, 16 / 4 heads
 // of 128 346 -> 160 (64 walks, heads split 4 ways); 3 x 896, 32 / 8 heads of 128 189 -> 134 (2 ways); 4096 tokens, 6 / 1 heads
 // of 128 886 -> 125 (6 x 2); 2 x 1024, 16 / 4 heads of 64 196 -> 59 (4 x 2).  Full launches stay whole: 2 x 4096, 32 / 8 heads
-// of 128 takes 1000 us whole and 1030 in two.
+// of 128 takes 1000 us whole and 1030 in two.  Causal: where even the key tiles by themselves fit the chip at once a pair is
+// taken apart as well, which spares the chain the fixed part of its second tile and needs no partial sums.  The whole call, before
+// -> after (us): 2 x 256 tokens, 4 / 2 heads of 128 32.4 -> 22.5; 3 x 640, 25 heads of 64 63.9 -> 56.4; 4 x 512, 12 heads of 64
+// 48.9 -> 38.5; 896 tokens, 32 / 8 heads of 128 66.5 -> 60.9.
 struct Splits {
 	int h = 1, q = 1;
+	bool paired = true;
 };
 static int64_t dkv_part_bytes(const Splits& sp, int B, int S, int Hkv, int D) { return sp.h * sp.q > 1 ? (int64_t)sp.h * sp.q * 2 * B * S * Hkv * D * 4 : 0; }
-// room: bytes there are for the partial sums.  Splits are tried in ascending order of what they need, so the room for the one
-// that an unlimited search takes gives that one.
+// room: bytes there are for the partial sums.  Splits are tried in ascending order of what they need, first of pairs and then of
+// single key tiles.
 static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal, int64_t room) {
 	const int nkt = S / 128, G = Hq / Hkv;
-	const int64_t walks = (int64_t)B * Hkv * (causal ? (nkt + 1) / 2 : nkt);
-	const int tiles = causal ? (nkt + 1) * 4 : nkt * 4;  // query tiles of a walk and head (a pair of key tiles has nkt + 1 of four)
 	const float slots = D == 128 ? 256.f : 512.f, step = D == 128 ? 1.2f : 1.1f, fixed = 8.f;
 	Splits best;
 	// From 2^18 query rows (2 x 4096 tokens of 32 heads) up walks stay whole.  With eight kv heads or more and several sequences such
@@ -975,15 +978,22 @@ static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal, int6
 	// has not been measured there.
 	if ((int64_t)B * S * Hq >= 1 << 18) return best;
 	float best_us = 1e30f;
-	for (int h = 1; h <= G; h++) {
-		if (G % h) continue;
-		for (int q = 1; q <= 4; q *= 2) {
-			if (q > 1 && h < G) continue;
-			const int ns = h * q;
-			if (dkv_part_bytes(Splits{h, q}, B, S, Hkv, D) > room) continue;
-			const float rounds = ceilf((float)(walks * ns) / slots);
-			const float us = rounds * (fixed + (float)(G / h) * ((tiles + q - 1) / q) * step) + (ns > 1 ? 2.f + (float)ns * B * S * Hkv * D * 16 / 5e6f : 0.f);
-			if (us < best_us * (ns > 1 ? 0.95f : 1.f)) best_us = us, best = Splits{h, q};
+	for (int paired = 1; paired >= (causal && nkt > 1 ? 0 : 1); paired--) {
+		if (!paired) best_us += fixed;  // that of a pair's second tile, which all sharings of pairs have alike
+		const bool two = causal && paired && nkt > 1;  // key tiles one after the other
+		const int64_t walks = (int64_t)B * Hkv * (two ? (nkt + 1) / 2 : nkt);
+		const int tiles = two ? (nkt + 1) * 4 : nkt * 4;  // query tiles of the longest walk and head (a pair of key tiles has nkt + 1 of four)
+		for (int h = 1; h <= G; h++) {
+			if (G % h) continue;
+			for (int q = 1; q <= 4; q *= 2) {
+				if (q > 1 && h < G) continue;
+				const int ns = h * q;
+				if (dkv_part_bytes(Splits{h, q}, B, S, Hkv, D) > room) continue;
+				const float rounds = ceilf((float)(walks * ns) / slots);
+				if (!paired && rounds > 1.f) continue;
+				const float us = rounds * (fixed + (float)(G / h) * ((tiles + q - 1) / q) * step) + (ns > 1 ? 2.f + (float)ns * B * S * Hkv * D * 16 / 5e6f : 0.f);
+				if (us < best_us * (ns > 1 ? 0.95f : 1.f)) best_us = us, best = Splits{h, q, paired != 0};
+			}
 		}
 	}
 	return best;
@@ -1033,9 +1043,9 @@ int attn_bwd(const void* q, const void* k, const void* v, const void* o, const v
 	const Splits sp = split_walk(B, S, Hq, Hkv, D, causal != 0, workspace_bytes - whole);
 	float* dkv_part = sp.h * sp.q > 1 ? nlse2 + T * Hq : nullptr;
 	AttnBwdArgs a{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)dO, nlse2, delta, dq_part,
-	              (bf16_t*)dk, (bf16_t*)dv, ldq, ldk, ldv, lddo, lddk, lddv, B, S, Hq, Hkv, scale, (const float2*)rope_cs, sp.h, sp.q, dkv_part};
+	              (bf16_t*)dk, (bf16_t*)dv, ldq, ldk, ldv, lddo, lddk, lddv, B, S, Hq, Hkv, scale, (const float2*)rope_cs, sp.h, sp.q, dkv_part, sp.paired};
 	const int nkt = S / 128;
-	const dim3 grid((unsigned)((int64_t)B * Hkv * (causal ? (nkt + 1) / 2 : nkt) * sp.h * sp.q)), block(256);
+	const dim3 grid((unsigned)((int64_t)B * Hkv * (causal && sp.paired ? (nkt + 1) / 2 : nkt) * sp.h * sp.q)), block(256);
 	int rc;
 	if (D == 128) rc = causal ? launch_bwd<128, true>(a, grid, stream) : launch_bwd<128, false>(a, grid, stream);
 	else rc = causal ? launch_bwd<64, true>(a, grid, stream) : launch_bwd<64, false>(a, grid, stream);

@@ -696,6 +696,24 @@ def test_attention_backward_with_walks_shared_by_workgroups(K, cfg):
 	assert sizes == sorted(sizes)
 
 
+@pytest.mark.parametrize("cfg", [(1, 128, 8, 2, 128, True), (3, 256, 4, 2, 128, True), (4, 512, 12, 12, 64, True), (1, 1152, 6, 3, 64, True), (1, 640, 12, 2, 128, True)])
+def test_attention_backward_with_a_workgroup_per_key_tile(K, cfg):
+	"""Causal, key tiles (one, two, an odd number) that all fit the chip at once: each goes to a workgroup of its own, with and
+	without shared walks.  Against fp32 autograd, equal bits from run to run, the rotation undone as by a pass of its own."""
+	B, S, Hq, Hkv, D, causal = cfg
+	T = B * S
+	qkv, do = _randn(T, (Hq + 2 * Hkv) * D, seed=57), _randn(T, Hq * D, seed=58)
+	o_ref, _, dqkv_ref = _attn_ref(qkv, B, S, Hq, Hkv, D, causal, do)
+	o, lse = K.attn_fwd(qkv, B, S, Hq, Hkv, D, causal)
+	dqkv = K.attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal)
+	for name, sl in (("dq", slice(0, Hq * D)), ("dk", slice(Hq * D, (Hq + Hkv) * D)), ("dv", slice((Hq + Hkv) * D, None))):
+		_close(dqkv[:, sl], dqkv_ref[:, sl], rel_fro=1.5e-2, what=f"attn {name} {cfg}")
+	assert torch.equal(dqkv, K.attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal))
+	cs = K.rope_table(S, D, 5e5)
+	fused = K.attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal, rope_cs=cs)
+	assert torch.equal(fused, K.rope_apply_(dqkv.clone(), cs, S, Hq + Hkv, D, backward=True))
+
+
 @pytest.mark.parametrize("cfg", [(1, 4096, 4, 4, 64, False), (2, 2048, 8, 4, 64, False), (1, 896, 8, 1, 128, True)])
 @pytest.mark.parametrize("ways", [None, 1, 2, 3, 64])
 def test_attention_backward_stays_inside_its_workspace(K, cfg, ways):
