@@ -263,13 +263,13 @@ int gemm_rope_bf16(int M, int N, int K, const void* A, int64_t lda, const void* 
 // What the fused kernel can run at all (a caller without scratch or with strided buffers relies on it) ...
 static bool swiglu_bwd_fits(int M, int F, int K) { return M >= 256 && F >= 256 && M % 64 == 0 && F % 64 == 0 && K % 64 == 0; }
 // The tile it runs on.  The epilogue reads and writes four of d, g, u and their two gradients at 256 tiles a time: 20 us more per
-// round of 256-row tiles than the plain one (fitted to 700 shapes; with 12 us for the whole round 1024 x 3072 x 64 took 25 us
+// round of 256-row tiles than the plain one, and 4 us a launch (without these 3072 x 2304 x 768 took 33 us fused, 30.6 apart; with 12 us for the whole round 1024 x 3072 x 64 took 25 us
 // fused, 13 apart, and 8448 x 512 x 512 32 and 20).
 static Plan swiglu_bwd_tile(int M, int F, int K) {
 	Plan best;
 	auto weigh = [&](TileTime t) {
 		if (M < t.bm) return;
-		t.round += 20.f * t.bm / 256;
+		t.round += 20.f * t.bm / 256, t.launch += 4.f;
 		const float us = tile_us(t, M, F, K / BK);
 		if (us < best.us) best = Plan{t.bm, t.bn, 1, us};
 	};
