@@ -33,6 +33,8 @@ int elf_gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, 
 
 int elf_gemm_swiglu_bwd_bf16(int M, int F, int K, const void* dY, int64_t lddy, const void* W, int64_t ldw,
                              const void* gu, int64_t ldgu, void* dgu, int64_t lddgu, void* scratch, void* stream) {
+	// (the launcher also does without scratch wherever 64x64 tiles are the faster way; this entry point refuses it, as its header says)
+	ELF_REQUIRE(scratch || (M >= 256 && F >= 256), "gemm_swiglu_bwd: this shape needs a scratch buffer of M x F bf16");
 	return elf::gemm_swiglu_bwd_bf16(M, F, K, dY, lddy, W, ldw, gu, ldgu, dgu, lddgu, scratch, (hipStream_t)stream);
 }
 

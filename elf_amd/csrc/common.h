@@ -51,6 +51,11 @@ __device__ __forceinline__ bf16_t f2bf(float v) { return (bf16_t)v; }
 // MLP activations.  swiglu_f is shared by the activation kernel and the GEMM epilogue that fuses it, so
 // that both give the same bits.  GELU is the exact (erf) form of nn.GELU(): 0.5 x (1 + erf(x / sqrt 2)).
 __device__ __forceinline__ float gelu_f(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
+__device__ __forceinline__ float gelu_grad_f(float x) {
+	const float cdf = 0.5f * (1.f + erff(x * 0.70710678118654752f));
+	const float pdf = 0.3989422804014327f * __expf(-0.5f * x * x);
+	return cdf + x * pdf;
+}
 __device__ __forceinline__ float swiglu_f(float g, float u) {
 	// hardware reciprocal (1 ulp): a correctly rounded division is ten more instructions per element, which
 	// a GEMM epilogue cannot hide, and the result is rounded to bf16 anyway

@@ -773,12 +773,6 @@ int norm_bwd_noalloc(int kind, const void* dy, const void* x, const void* gamma,
 // ------------------------------------------------------------------------------------------
 // Activations.  GELU is the exact (erf) form of nn.GELU():  y = 0.5 x (1 + erf(x / sqrt 2)).
 // SwiGLU: h = silu(g) * u with g = gu[:, :F], u = gu[:, F:].
-__device__ __forceinline__ float gelu_grad_f(float x) {
-	const float cdf = 0.5f * (1.f + erff(x * 0.70710678118654752f));
-	const float pdf = 0.3989422804014327f * __expf(-0.5f * x * x);
-	return cdf + x * pdf;
-}
-
 __global__ __launch_bounds__(256) void gelu_fwd_kernel(const bf16_t* __restrict__ x, bf16_t* __restrict__ y, int64_t nchunks) {
 	for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nchunks; i += (int64_t)gridDim.x * blockDim.x) {
 		Chunk c = load8(x + i * 8);

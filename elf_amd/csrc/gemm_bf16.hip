@@ -116,15 +116,22 @@ static Plan plan_weight_gradient(int M, int N, int K, int max_splits = 16) {
 	return best;
 }
 
-// The rows of the direct-to-LDS tile of 256 columns a forward / input-gradient product runs on, 0: one of the ring tiles
-// (never with ring_extra = NO_RING, unless no tile of 256 columns fits).
+// ring_extra of a product that a ring tile cannot do
 constexpr float NO_RING = 1e20f;
-static int dma_tile_rows(int M, int N, int K, float ring_extra, float epi_extra) {
-	const Plan p = plan_tiles(M, N, K, true, ring_extra, epi_extra);
-	return p.dma() ? p.bm : 0;
-}
 // what a pass of its own over `bytes` costs (5 TB/s and a launch)
 static float pass_us(double bytes) { return 2.f + (float)(bytes / 5e6); }
+// Estimate for 64x64 ring tiles with an epilogue of `extra` us a round.  From K = 256 up, the narrowest a stage was measured at;
+// below, products and passes stay apart.
+static float small_us(int M, int N, int K, float extra) {
+	TileTime t = K <= RING_SHORT_K ? TILES_SHORT[5] : TILES_BF16[5];
+	t.round += extra;
+	return M < 64 || N < 64 || M % 64 || N % 64 || K % BK || K < 256 ? 1e30f : tile_us(t, M, N, K / BK);
+}
+// What an epilogue adds to a round of 64x64 tiles.  Of the smallest products a pass of its own costs more than that whatever its
+// size: a launch, 3 us on the GPU and as much on the host.  Product and pass, before -> after on one kernel (us): SwiGLU 512 x 768
+// x 512 (M x F x K) 7.3 -> 5.3 and its backward 7.6 -> 6.3, GELU 512 x 1024 x 256 6.5 -> 5.6, RoPE 512 x 1024 x 512 7.2 -> 5.2;
+// with more than a round of tiles the larger ones and a pass are as fast: GELU 1024 x 2048 x 512 11.5 and 11.4.
+constexpr float SMALL_SWIGLU_US = 0.5f, SMALL_ROPE_US = 0.5f, SMALL_GELU_US = 1.2f, SMALL_GELU_BWD_US = 1.8f, SMALL_SWIGLU_BWD_US = 1.6f;
 // what an epilogue adds to a round of 256x256 tiles (half of it to one of 128x256)
 constexpr float SWIGLU_FWD_US = 4.f, ROPE_US = 5.f;
 
@@ -205,10 +212,21 @@ int gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, cons
 	// the SwiGLU epilogue pairs 64 gate with 64 up columns per wave, so a 256-column tile covers 128 outputs; it reaches the up rows
 	// with 32-bit byte offsets from the gate rows
 	int bm = 0;
-	if (act == ACT_SWIGLU && (int64_t)(F + 256) * ldw * 2 < (int64_t(1) << 31) && M % 64 == 0 && F % 64 == 0 && K % 64 == 0 && lda % 8 == 0 && ldw % 8 == 0 && ldpre >= N && ldout >= F && ldpre % 8 == 0 && ldout % 8 == 0 &&
-	    ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)pre % 16) == 0 && ((uintptr_t)out % 16) == 0 && lda >= K && ldw >= K && gemm_reaches(256, lda)) {
-		// rows that lie further apart only the fused kernel writes
-		bm = dma_tile_rows(M, N, K, ldpre == N && ldout == F ? pass_us(6.0 * M * F) : NO_RING, SWIGLU_FWD_US);
+	bool small = false;
+	if (M % 64 == 0 && F % 64 == 0 && K % 64 == 0 && lda % 8 == 0 && ldw % 8 == 0 && ldpre >= N && ldout >= F && ldpre % 8 == 0 && ldout % 8 == 0 && ((uintptr_t)A % 16) == 0 &&
+	    ((uintptr_t)W % 16) == 0 && ((uintptr_t)pre % 16) == 0 && ((uintptr_t)out % 16) == 0 && lda >= K && ldw >= K && gemm_reaches(256, lda) && (int64_t)(F + 256) * ldw * 2 < (int64_t(1) << 31)) {
+		const bool dense = ldpre == N && ldout == F;  // rows that lie further apart only the fused kernel of the large tiles writes
+		float us = plan_tiles(M, N, K).us + pass_us((act == ACT_SWIGLU ? 6.0 : 4.0) * M * F);
+		if (act == ACT_SWIGLU) {
+			const Plan p = plan_tiles(M, N, K, true, dense ? pass_us(6.0 * M * F) : NO_RING, SWIGLU_FWD_US);
+			bm = p.dma() ? p.bm : 0;
+			us = p.us;
+		}
+		small = dense && small_us(M, N, K, act == ACT_SWIGLU ? SMALL_SWIGLU_US : SMALL_GELU_US) < us;
+	}
+	if (small) {
+		ProfScope prof(PROF_GEMM, 2.0 * M * N * K, stream);
+		return gemm_ring_act(M, N, K, A, lda, W, ldw, pre, ldpre, act == ACT_SWIGLU ? EPI_BF16_SWIGLU : EPI_BF16_GELU, nullptr, 0, stream, out, ldout);
 	}
 	if (bm) {
 		ProfScope prof(PROF_GEMM, 2.0 * M * N * K, stream);
@@ -237,9 +255,12 @@ int gemm_dw_final(int M, int N, int K, const void* dY, int64_t lddy, const void*
 	return scale_grads(acc, grad_bf16, (int64_t)M * N, scale, stream);
 }
 
+// The way of a projection with its rotary embedding: the rows of a 256-column tile, 64: a 64x64 ring tile, 0: two passes.
 static int rope_tile_rows(int M, int N, int K, int D) {
 	if (!(M >= 64 && N >= 64 && M % 64 == 0 && N % 64 == 0 && K % 64 == 0 && (D == 64 || D == 128) && N % D == 0)) return 0;
-	return dma_tile_rows(M, N, K, pass_us(4.0 * M * N), ROPE_US);
+	const Plan p = plan_tiles(M, N, K, true, pass_us(4.0 * M * N), ROPE_US);
+	if (small_us(M, N, K, SMALL_ROPE_US) < p.us) return 64;
+	return p.dma() ? p.bm : 0;
 }
 bool gemm_rope_fused(int M, int N, int K, int D) {
 	return rope_tile_rows(M, N, K, D) != 0;
@@ -254,6 +275,7 @@ int gemm_rope_bf16(int M, int N, int K, const void* A, int64_t lda, const void* 
 		// the rotation's arithmetic is not counted: the figure stays the GEMM's
 		ProfScope prof(PROF_GEMM, 2.0 * M * N * K, stream);
 		const int bm = rope_tile_rows(M, N, K, D);
+		if (bm == 64) return gemm_ring_act(M, N, K, A, lda, W, ldw, C, ldc, EPI_BF16_ROPE, nullptr, 0, stream, nullptr, 0, cs, S, n_rot_heads * D, D);
 		return gemm_bf16_dma(0, 0, M, N, K, A, lda, W, ldw, C, ldc, EPI_BF16_ROPE, nullptr, 0, 1, 0, bm, stream, nullptr, 0, cs, S, n_rot_heads * D, D);
 	}
 	if (int rc = gemm_bf16(0, 0, M, N, K, A, lda, W, ldw, C, ldc, EPI_BF16, nullptr, 0, 0, 0, stream)) return rc;
@@ -263,7 +285,8 @@ int gemm_rope_bf16(int M, int N, int K, const void* A, int64_t lda, const void* 
 // What the fused kernel can run at all (a caller without scratch or with strided buffers relies on it) ...
 static bool swiglu_bwd_fits(int M, int F, int K) { return M >= 256 && F >= 256 && M % 64 == 0 && F % 64 == 0 && K % 64 == 0; }
 // The tile it runs on.  The epilogue reads and writes four of d, g, u and their two gradients at 256 tiles a time: 20 us more per
-// round of 256-row tiles than the plain one, and 4 us a launch (without these 3072 x 2304 x 768 took 33 us fused, 30.6 apart; with 12 us for the whole round 1024 x 3072 x 64 took 25 us
+// round of 256-row tiles than the plain one, and 4 us a launch (without these 3072 x 2304 x 768 took 33 us fused, 30.6 apart;
+// with 12 us for the whole round 1024 x 3072 x 64 took 25 us
 // fused, 13 apart, and 8448 x 512 x 512 32 and 20).
 static Plan swiglu_bwd_tile(int M, int F, int K) {
 	Plan best;
@@ -278,20 +301,35 @@ static Plan swiglu_bwd_tile(int M, int F, int K) {
 		for (const TileTime& t : TILES_MID) weigh(t);
 	return best;
 }
-// ... and where it is also the faster way: against the best tile of the plain product and the pass over d, g, u and their gradients.
-bool gemm_swiglu_bwd_fused(int M, int F, int K) {
-	return swiglu_bwd_fits(M, F, K) && swiglu_bwd_tile(M, F, K).us < plan_tiles(M, F, K).us + pass_us(10.0 * M * F);
+// The faster way, dense buffers: the fused kernel on large tiles, on 64x64 ones, or the best tile of the plain product and the pass
+// over d, g, u and their gradients.
+enum { WAY_APART, WAY_LARGE, WAY_SMALL };
+static int swiglu_bwd_way(int M, int F, int K) {
+	const float apart = plan_tiles(M, F, K).us + pass_us(10.0 * M * F), large = swiglu_bwd_fits(M, F, K) ? swiglu_bwd_tile(M, F, K).us : 1e30f;
+	// (of more than a round of 64x64 tiles the epilogue's five operands are not hidden: 896 x 1408 x 512 10.8 us apart, 11.1 fused)
+	const bool one_round = (int64_t)(M / 64) * (F / 64) <= 256;
+	if (one_round && small_us(M, F, K, SMALL_SWIGLU_BWD_US) < (large < apart ? large : apart)) return WAY_SMALL;
+	return large < apart ? WAY_LARGE : WAY_APART;
 }
+bool gemm_swiglu_bwd_fused(int M, int F, int K) { return swiglu_bwd_way(M, F, K) != WAY_APART; }
 
 int gemm_swiglu_bwd_bf16(int M, int F, int K, const void* dY, int64_t lddy, const void* W, int64_t ldw, const void* gu,
                          int64_t ldgu, void* dgu, int64_t lddgu, void* scratch, hipStream_t stream, void* act, int64_t ldact) {
 	ELF_REQUIRE(M > 0 && F > 0 && K > 0 && dY && W && gu && dgu, "gemm_swiglu_bwd: empty problem or null operand");
-	const bool apart = scratch && ldgu == 2 * F && lddgu == 2 * F && (!act || ldact == F);  // what the separate passes need
-	if ((apart ? gemm_swiglu_bwd_fused(M, F, K) : swiglu_bwd_fits(M, F, K)) && lddy >= K && ldw >= F && ldgu >= 2 * F && lddgu >= 2 * F && lddy % 8 == 0 && ldw % 8 == 0 && ldgu % 8 == 0 &&
-	    lddgu % 8 == 0 && ((uintptr_t)dY % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)gu % 16) == 0 && ((uintptr_t)dgu % 16) == 0 && gemm_reaches(256, lddy) && gemm_reaches(BK, ldw)) {
+	const bool dense = ldgu == 2 * F && lddgu == 2 * F && (!act || ldact == F);
+	const bool fits = lddy >= K && ldw >= F && ldgu >= 2 * F && lddgu >= 2 * F && lddy % 8 == 0 && ldw % 8 == 0 && ldgu % 8 == 0 && lddgu % 8 == 0 && ((uintptr_t)dY % 16) == 0 &&
+	                  ((uintptr_t)W % 16) == 0 && ((uintptr_t)gu % 16) == 0 && ((uintptr_t)dgu % 16) == 0 && gemm_reaches(256, lddy) && gemm_reaches(BK, ldw);
+	int way = WAY_APART;
+	if (fits) {
+		way = dense ? swiglu_bwd_way(M, F, K) : WAY_APART;
+		// what the separate passes cannot do goes to the large tiles wherever these fit
+		if (way == WAY_APART && !(dense && scratch) && swiglu_bwd_fits(M, F, K)) way = WAY_LARGE;
+	}
+	if (way != WAY_APART) {
 		// the activation backward's arithmetic is not counted: the figure stays the GEMM's
 		ProfScope prof(PROF_GEMM, 2.0 * M * F * K, stream);
 		ELF_REQUIRE(!act || (ldact >= F && ldact % 8 == 0 && ((uintptr_t)act % 16) == 0), "gemm_swiglu_bwd: bad activation output");
+		if (way == WAY_SMALL) return gemm_ring_act(M, F, K, dY, lddy, W, ldw, dgu, lddgu, EPI_BF16_SWIGLU_BWD, gu, ldgu, stream, act, ldact);
 		return gemm_bf16_dma(0, 1, M, F, K, dY, lddy, W, ldw, dgu, lddgu, EPI_BF16_SWIGLU_BWD, gu, ldgu, 1, 0, swiglu_bwd_tile(M, F, K).bm, stream, act, ldact);
 	}
 	ELF_REQUIRE(scratch, "gemm_swiglu_bwd: this shape needs a scratch buffer of M x F bf16");
@@ -299,6 +337,22 @@ int gemm_swiglu_bwd_bf16(int M, int F, int K, const void* dY, int64_t lddy, cons
 	if (int rc = gemm_bf16(0, 1, M, F, K, dY, lddy, W, ldw, scratch, F, EPI_BF16, nullptr, 0, 0, 0, stream)) return rc;
 	ELF_REQUIRE(!act || ldact == F, "gemm_swiglu_bwd: the unfused path needs a dense activation output");
 	return swiglu_bwd(scratch, gu, dgu, M, F, stream, act);
+}
+
+// GELU: fused on 64x64 tiles only (on larger ones the error function costs more than the pass it saves).
+bool gemm_gelu_bwd_fused(int M, int F, int K) {
+	return small_us(M, F, K, SMALL_GELU_BWD_US) < plan_tiles(M, F, K).us + pass_us(6.0 * M * F);
+}
+
+int gemm_gelu_bwd_bf16(int M, int F, int K, const void* dY, const void* W, const void* pre, void* dpre, void* scratch, hipStream_t stream) {
+	ELF_REQUIRE(M > 0 && F > 0 && K > 0 && dY && W && pre && dpre, "gemm_gelu_bwd: empty problem or null operand");
+	if (gemm_gelu_bwd_fused(M, F, K) && ((uintptr_t)dY % 16) == 0 && ((uintptr_t)W % 16) == 0 && ((uintptr_t)pre % 16) == 0 && ((uintptr_t)dpre % 16) == 0) {
+		ProfScope prof(PROF_GEMM, 2.0 * M * F * K, stream);
+		return gemm_ring_act(M, F, K, dY, K, W, F, dpre, F, EPI_BF16_GELU_BWD, pre, F, stream);
+	}
+	ELF_REQUIRE(scratch, "gemm_gelu_bwd: this shape needs a scratch buffer of M x F bf16");
+	if (int rc = gemm_bf16(0, 1, M, F, K, dY, K, W, F, scratch, F, EPI_BF16, nullptr, 0, 0, 0, stream)) return rc;
+	return gelu_bwd(scratch, pre, dpre, (int64_t)M * F, stream);
 }
 
 }  // namespace elf

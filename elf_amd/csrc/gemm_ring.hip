@@ -8,7 +8,8 @@
 //
 // Bound: the 64 B/clk path into LDS (a slice of the 128x128 tile is 512 cycles of it and 512 of MFMA, of the 64x64 tile 256
 // against 128) and LDS reads; results leave from registers, two neighbouring column slabs exchanged between lane groups so
-// that a lane stores 16 bytes.  Against the register-staged tiles (global -> VGPR -> LDS, two stages) that these replace, cold
+// that a lane stores 16 bytes.  The activations and the rotary embedding of the smallest products ride in the epilogue of the
+// 64x64 tile (gemm_ring_act: what bounds these is the number of launches).  Against the register-staged tiles (global -> VGPR -> LDS, two stages) that these replace, cold
 // operands: 1920 x 1600 x 1600 23.1 -> 19.9 us, 2112 x 832 x 4288 50 -> 31, 512 x 512 x 1536 14.2 -> 7.9; weight
 // gradients: 1600 x 1600 x 1920 36.7 -> 25.6, 832 x 4288 x 2112 50 -> 29, 768 x 768 x 4096 31 -> 22.
 #include "common.h"
@@ -31,6 +32,11 @@ struct Args {
 	int tiles_m, tiles_n;
 	int k_splits;       // K is split this many ways (fp32 atomics, EPI_F32_ACC only)
 	uint32_t turn_tag;  // this launch's tag in the turn counters, 0 = the splits add in any order
+	// epilogues of gemm_ring_act
+	bf16_t* C2;
+	int64_t ldc2;
+	const float2* rope_cs;
+	int rope_S, rope_cols, rope_D;
 };
 
 // Turn counters of split tiles, one per tile and wave (the scheme of gemm_dma.hip: split s adds when the counter holds this
@@ -73,6 +79,10 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(Args g) {
 	using Sh = Shape<BM, BN, SHORT>;
 	constexpr int NST = Sh::NST, A_BYTES = Sh::A_BYTES, B_BYTES = Sh::B_BYTES, LOADS_A = Sh::LOADS_A, LOADS_B = Sh::LOADS_B, P = Sh::LOADS;
 	constexpr int WM = BM / 2, WN = BN / 2, RF = WM / 16, CF = WN / 16, NM = RF * CF, NR = RF + CF;
+	// A wave's columns are 16 columns (gate, or a head's first half) and the 16 that belong to them `pair` rows of B further on (up,
+	// or its second half): both halves of a pair are in one lane's accumulators
+	constexpr bool PAIRED = EPI == EPI_BF16_SWIGLU || EPI == EPI_BF16_ROPE;
+	static_assert(!PAIRED || (BM == 64 && BN == 64 && !AT && !BT), "the paired row order is defined for 64x64 tiles of k-contiguous operands");
 	extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 	const int tid = threadIdx.x, lane = tid & 63;
 	const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -130,12 +140,24 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(Args g) {
 	}
 
 	const bf16_t* const Ap = AT ? g.A + (int64_t)kt0 * BKS * g.lda + m0 : g.A + (int64_t)m0 * g.lda + (int64_t)kt0 * BKS;
-	const bf16_t* const Bp = BT ? g.B + (int64_t)kt0 * BKS * g.ldb + n0 : g.B + (int64_t)n0 * g.ldb + (int64_t)kt0 * BKS;
+	// the tile's first column in C: a paired tile covers half as many gate columns, or two runs of 32 columns of one head
+	const int c_lo = EPI == EPI_BF16_SWIGLU ? n0 / 2 : EPI == EPI_BF16_ROPE ? n0 / g.rope_D * g.rope_D + n0 % g.rope_D / 2 : n0;
+	const int pair = EPI == EPI_BF16_SWIGLU ? g.N / 2 : EPI == EPI_BF16_ROPE ? g.rope_D / 2 : 0;
+	const bf16_t* const Bp = BT ? g.B + (int64_t)kt0 * BKS * g.ldb + n0 : g.B + (int64_t)c_lo * g.ldb + (int64_t)kt0 * BKS;
 	const int64_t a_step = AT ? (int64_t)BKS * g.lda : BKS;
 	const int64_t b_step = BT ? (int64_t)BKS * g.ldb : BKS;
 	uint32_t aoff[LOADS_A], boff[LOADS_B];
 	dma::lane_offsets<AT, LOADS_A, false, BM>(wave, lane, g.lda, aoff);
-	dma::lane_offsets<BT, LOADS_B, false, BN>(wave, lane, g.ldb, boff);
+	if constexpr (PAIRED) {
+#pragma unroll
+		for (int i = 0; i < LOADS_B; i++) {
+			const int row = (wave * LOADS_B + i) * 8 + (lane >> 3), slot = lane & 7;
+			const int64_t grow = (row >> 5) * 16 + (row & 15) + ((row >> 4) & 1) * (int64_t)pair;
+			boff[i] = (uint32_t)((grow * g.ldb + ((slot ^ ((row >> 1) & 7)) << 3)) * 2);
+		}
+	} else {
+		dma::lane_offsets<BT, LOADS_B, false, BN>(wave, lane, g.ldb, boff);
+	}
 	const uint32_t lds_a = lds_addr(smem) + wave * (LOADS_A * 1024);
 	const uint32_t lds_b = lds_addr(smem) + NST * A_BYTES + wave * (LOADS_B * 1024);
 	const uint32_t lds_dummy = lds_addr(smem) + NST * Sh::STAGE_BYTES;
@@ -266,7 +288,93 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(Args g) {
 		if (g.k_splits > 1) take_turn();
 	}
 	if (mine) {
-		if constexpr (EPI == EPI_BF16 || EPI == EPI_BF16_RESID) {
+		if constexpr (PAIRED) {
+			// four consecutive columns of the first half (acc[i][0]) and the four that belong to them (acc[i][1]); the arithmetic is
+			// that of the separate passes, on the rounded values they would read
+			const int c = c_lo + wc * 16 + 4 * g4;
+			f32x4 tab[RF][2];
+			[[maybe_unused]] bool rot = false;
+			if constexpr (EPI == EPI_BF16_ROPE) {
+				rot = c < g.rope_cols;
+				if (rot) {
+#pragma unroll
+					for (int i = 0; i < RF; i++) {
+						const f32x4* tp = reinterpret_cast<const f32x4*>(g.rope_cs + (int64_t)((row0 + i * 16) % g.rope_S) * pair + c % g.rope_D);
+						tab[i][0] = tp[0], tab[i][1] = tp[1];
+					}
+				}
+			}
+#pragma unroll
+			for (int i = 0; i < RF; i++) {
+				bf16x4 lo, hi, oa;
+#pragma unroll
+				for (int t = 0; t < 4; t++) {
+					lo[t] = (bf16_t)acc[i][0][t];
+					hi[t] = (bf16_t)acc[i][1][t];
+					if constexpr (EPI == EPI_BF16_SWIGLU) {
+						oa[t] = (bf16_t)swiglu_f((float)lo[t], (float)hi[t]);
+					} else if (rot) {
+						float rl, rh;
+						rope_rot((float)lo[t], (float)hi[t], tab[i][t >> 1][(t & 1) * 2], tab[i][t >> 1][(t & 1) * 2 + 1], rl, rh);
+						lo[t] = (bf16_t)rl;
+						hi[t] = (bf16_t)rh;
+					}
+				}
+				bf16_t* const cp = reinterpret_cast<bf16_t*>(g.C) + (int64_t)(row0 + i * 16) * g.ldc + c;
+				*reinterpret_cast<bf16x4*>(cp) = lo;
+				*reinterpret_cast<bf16x4*>(cp + pair) = hi;
+				if constexpr (EPI == EPI_BF16_SWIGLU) *reinterpret_cast<bf16x4*>(g.C2 + (int64_t)(row0 + i * 16) * g.ldc2 + c) = oa;
+			}
+		} else if constexpr (EPI == EPI_BF16_GELU || EPI == EPI_BF16_GELU_BWD || EPI == EPI_BF16_SWIGLU_BWD) {
+			const int c = col0 + 16 * (g4 & 1) + 8 * (g4 >> 1);
+			constexpr bool SW = EPI == EPI_BF16_SWIGLU_BWD;
+			bf16x8 p[RF][CF / 2], u[SW ? RF : 1][CF / 2];  // what the backwards read, all of it before the first store
+			if constexpr (EPI != EPI_BF16_GELU) {
+#pragma unroll
+				for (int i = 0; i < RF; i++)
+#pragma unroll
+					for (int j = 0; j < CF; j += 2) {
+						const bf16_t* r = g.R + (int64_t)(row0 + i * 16) * g.ldr + c + j * 16;
+						p[i][j / 2] = *reinterpret_cast<const bf16x8*>(r);
+						if constexpr (SW) u[i][j / 2] = *reinterpret_cast<const bf16x8*>(r + g.N);
+					}
+			}
+#pragma unroll
+			for (int i = 0; i < RF; i++)
+#pragma unroll
+				for (int j = 0; j < CF; j += 2) {
+					pair_slabs(acc[i][j], acc[i][j + 1]);
+					bf16x8 o, o2;
+#pragma unroll
+					for (int t = 0; t < 8; t++) {
+						const float d = (float)(bf16_t)(t < 4 ? acc[i][j][t] : acc[i][j + 1][t - 4]);
+						if constexpr (EPI == EPI_BF16_GELU) {
+							o[t] = (bf16_t)d;
+							o2[t] = (bf16_t)gelu_f(d);
+						} else if constexpr (EPI == EPI_BF16_GELU_BWD) {
+							o[t] = (bf16_t)(d * gelu_grad_f((float)p[i][j / 2][t]));
+						} else {
+							float dg, du;
+							swiglu_bwd_f(d, (float)p[i][j / 2][t], (float)u[i][j / 2][t], dg, du);
+							o[t] = (bf16_t)dg;
+							o2[t] = (bf16_t)du;
+						}
+					}
+					const int64_t row = row0 + i * 16;
+					bf16_t* const cp = reinterpret_cast<bf16_t*>(g.C) + row * g.ldc + c + j * 16;
+					*reinterpret_cast<bf16x8*>(cp) = o;
+					if constexpr (SW) *reinterpret_cast<bf16x8*>(cp + g.N) = o2;
+					if constexpr (EPI == EPI_BF16_GELU) *reinterpret_cast<bf16x8*>(g.C2 + row * g.ldc2 + c + j * 16) = o2;
+					if constexpr (SW) {
+						if (g.C2) {  // the activation again, for a stash that dropped it
+							bf16x8 oa;
+#pragma unroll
+							for (int t = 0; t < 8; t++) oa[t] = (bf16_t)swiglu_f((float)p[i][j / 2][t], (float)u[i][j / 2][t]);
+							*reinterpret_cast<bf16x8*>(g.C2 + row * g.ldc2 + c + j * 16) = oa;
+						}
+					}
+				}
+		} else if constexpr (EPI == EPI_BF16 || EPI == EPI_BF16_RESID) {
 			static_assert(CF % 2 == 0, "slabs are stored in pairs");
 			const int c = col0 + 16 * (g4 & 1) + 8 * (g4 >> 1);
 			bf16x8 rs[EPI == EPI_BF16_RESID ? RF : 1][CF / 2];
@@ -381,12 +489,43 @@ int gemm_bf16_ring(int a_t, int b_t, int M, int N, int K, const void* A, int64_t
                    int64_t ldr, int k_splits, int bm, int bn, hipStream_t stream) {
 	ELF_REQUIRE(M % 64 == 0 && N % 64 == 0 && K % dma::BKS == 0, "gemm (ring tile): sizes must be multiples of 64");
 	ELF_REQUIRE(gemm_reaches(a_t ? dma::BKS : bm, lda) && gemm_reaches(b_t ? dma::BKS : bn, ldb), "gemm (ring tile): leading dimension too large (%lld, %lld)", (long long)lda, (long long)ldb);
-	ring::Args g{(const bf16_t*)A, (const bf16_t*)B, C, (const bf16_t*)R, lda, ldb, ldc, ldr, M, N, K, 0, 0, k_splits, 0};
+	ring::Args g{(const bf16_t*)A, (const bf16_t*)B, C, (const bf16_t*)R, lda, ldb, ldc, ldr, M, N, K, 0, 0, k_splits, 0, nullptr, 0, nullptr, 0, 0, 0};
 	if (bm == 128 && bn == 128) return ring::launch_layout<128, 128>(g, a_t, b_t, epi, stream);
 	if (bm == 64 && bn == 128) return ring::launch_layout<64, 128>(g, a_t, b_t, epi, stream);
 	if (bm == 128 && bn == 64) return ring::launch_layout<128, 64>(g, a_t, b_t, epi, stream);
 	if (bm == 64 && bn == 64) return ring::launch_layout<64, 64>(g, a_t, b_t, epi, stream);
 	set_error("gemm (ring tile): unknown tile %dx%d", bm, bn);
+	return -1;
+}
+
+namespace ring {
+template <bool BT, int EPI>
+static int launch_act(const Args& g, hipStream_t stream) {
+	return g.K <= RING_SHORT_K ? launch<64, 64, false, BT, EPI, true>(g, stream) : launch<64, 64, false, BT, EPI, false>(g, stream);
+}
+}  // namespace ring
+
+int gemm_ring_act(int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb, void* C, int64_t ldc, int epi, const void* R, int64_t ldr,
+                  hipStream_t stream, void* C2, int64_t ldc2, const void* rope_cs, int rope_S, int rope_cols, int rope_D) {
+	const bool bt = epi == EPI_BF16_SWIGLU_BWD || epi == EPI_BF16_GELU_BWD;
+	ELF_REQUIRE(M > 0 && N > 0 && M % 64 == 0 && N % 64 == 0 && K > 0 && K % dma::BKS == 0, "gemm (ring tile): sizes must be multiples of 64");
+	// the rows of a pair are addressed with 32-bit byte offsets from the tile's first row
+	const int brows = epi == EPI_BF16_SWIGLU ? N / 2 + 64 : epi == EPI_BF16_ROPE ? rope_D : 64;
+	ELF_REQUIRE(gemm_reaches(64, lda) && gemm_reaches(brows, ldb), "gemm (ring tile): leading dimension too large (%lld, %lld)", (long long)lda, (long long)ldb);
+	ELF_REQUIRE(epi != EPI_BF16_SWIGLU || N % 128 == 0, "gemm (ring tile): the SwiGLU epilogue needs F to be a multiple of 64");
+	ELF_REQUIRE(epi != EPI_BF16_ROPE || (rope_cs && rope_S > 0 && (rope_D == 64 || rope_D == 128) && N % rope_D == 0 && rope_cols % rope_D == 0),
+	            "gemm (ring tile): the RoPE epilogue needs a table and whole heads of 64 or 128 columns");
+	ELF_REQUIRE((C2 || (epi != EPI_BF16_SWIGLU && epi != EPI_BF16_GELU)) && (R || !bt), "gemm (ring tile): an epilogue's operand is missing");
+	ring::Args g{(const bf16_t*)A, (const bf16_t*)B, C, (const bf16_t*)R, lda, ldb, ldc, ldr, M, N, K, M / 64, N / 64, 1, 0,
+	             (bf16_t*)C2, ldc2, (const float2*)rope_cs, rope_S, rope_cols, rope_D};
+	switch (epi) {
+		case EPI_BF16_SWIGLU: return ring::launch_act<false, EPI_BF16_SWIGLU>(g, stream);
+		case EPI_BF16_ROPE: return ring::launch_act<false, EPI_BF16_ROPE>(g, stream);
+		case EPI_BF16_GELU: return ring::launch_act<false, EPI_BF16_GELU>(g, stream);
+		case EPI_BF16_GELU_BWD: return ring::launch_act<true, EPI_BF16_GELU_BWD>(g, stream);
+		case EPI_BF16_SWIGLU_BWD: return ring::launch_act<true, EPI_BF16_SWIGLU_BWD>(g, stream);
+	}
+	set_error("gemm (ring tile): unknown epilogue %d", epi);
 	return -1;
 }
 

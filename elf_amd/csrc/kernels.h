@@ -23,6 +23,9 @@ enum GemmEpilogue {
 	EPI_BF16_ROPE = 6,
 	// both operands reduction-major, 256x256 direct-to-LDS tiles without a K split (see gemm_dw_final):
 	EPI_F32_ACC_SCALE = 7,  // C(fp32) = (C + acc) * scale, C2(bf16) = bf16 of that
+	// 64x64 ring tiles only, like EPI_BF16_SWIGLU, _SWIGLU_BWD and _ROPE there (gemm_ring_act):
+	EPI_BF16_GELU = 8,      // k-contiguous operands: C(bf16) = acc, C2(bf16) = gelu of the rounded acc
+	EPI_BF16_GELU_BWD = 9,  // k-contiguous A: R = the pre-activation, acc rounded to bf16 = d: C(bf16) = d gelu'(R)
 };
 
 int gemm_bf16(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb,
@@ -44,6 +47,10 @@ inline bool gemm_reaches(int rows, int64_t ld) { return (int64_t)(rows - 1) * ld
 constexpr int RING_SHORT_K = 256;
 int gemm_bf16_ring(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb, void* C, int64_t ldc, int epi, const void* R,
                    int64_t ldr, int k_splits, int bm, int bn, hipStream_t stream);
+// Its 64x64 tiles with the epilogue of an activation or a rotary embedding (arguments as for gemm_bf16_dma; everything dense
+// enough and 16-byte aligned; B is k-contiguous for EPI_BF16_SWIGLU, _GELU and _ROPE, n-contiguous for the backwards).
+int gemm_ring_act(int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb, void* C, int64_t ldc, int epi, const void* R, int64_t ldr,
+                  hipStream_t stream, void* C2 = nullptr, int64_t ldc2 = 0, const void* rope_cs = nullptr, int rope_S = 0, int rope_cols = 0, int rope_D = 0);
 
 // The weight gradient of the step's last micro-batch with the step's gradient scale folded in: acc [M, N] (fp32, dense)
 // = (acc + dY^T X) * scale and grad_bf16 [M, N] = bf16(acc), with dY [K, M] and X [K, N] (both reduction-major).  One
@@ -90,10 +97,10 @@ int gemm_turn_giveups(uint64_t* out);
 
 enum Activation { ACT_GELU = 0, ACT_SWIGLU = 1 };
 // Up-projection of the MLP with its activation: pre = A W^T (A [M, K], W [N, K], N = F for GELU and 2F =
-// [gate rows; up rows] for SwiGLU), out [M, F] = gelu(pre) or silu(pre[:, :F]) * pre[:, F:].  SwiGLU runs
-// as one kernel (activation in the GEMM epilogue) when the shape fits the direct-to-LDS tiles; otherwise,
-// and for GELU (whose erf costs as much in the epilogue as in a kernel of its own), the GEMM is followed
-// by the activation kernel.  Both ways give the same bits.
+// [gate rows; up rows] for SwiGLU), out [M, F] = gelu(pre) or silu(pre[:, :F]) * pre[:, F:].  One kernel (activation
+// in the GEMM epilogue) where that is faster: SwiGLU on the direct-to-LDS tiles, both on 64x64 tiles of the smallest
+// products (on larger ones GELU's erf costs as much in the epilogue as in a kernel of its own); otherwise the GEMM is
+// followed by the activation kernel.  Both ways give the same bits.
 int gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, const void* W, int64_t ldw, void* pre,
                   int64_t ldpre, void* out, int64_t ldout, hipStream_t stream);
 
@@ -107,6 +114,9 @@ int gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, cons
 bool gemm_swiglu_bwd_fused(int M, int F, int K);
 int gemm_swiglu_bwd_bf16(int M, int F, int K, const void* dY, int64_t lddy, const void* W, int64_t ldw, const void* gu,
                          int64_t ldgu, void* dgu, int64_t lddgu, void* scratch, hipStream_t stream, void* act = nullptr, int64_t ldact = 0);
+// The same for the GELU of a GPT block's MLP: dpre [M, F] = d gelu'(pre) for d = dY W, all buffers dense; scratch as above.
+bool gemm_gelu_bwd_fused(int M, int F, int K);
+int gemm_gelu_bwd_bf16(int M, int F, int K, const void* dY, const void* W, const void* pre, void* dpre, void* scratch, hipStream_t stream);
 
 enum NormKind { NORM_RMS = 0, NORM_LAYER = 1 };
 

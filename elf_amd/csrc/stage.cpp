@@ -430,6 +430,14 @@ static int run_backward(Stage* s, MbState& m, const void* dy, void* dx, bool gra
 			ELF_TRY(gemm_swiglu_bwd_bf16(T, F, d, dyin, d, p.w[P_W2], F, bs.b[B_GU].p, s->ffn_in, bs.b[B_DGU].p, s->ffn_in, nullptr, st,
 			                             form_a ? bs.b[B_A].p : nullptr, F));
 			ELF_TRY(gemm_bf16(0, 1, T, d, s->ffn_in, bs.b[B_DGU].p, s->ffn_in, p.w[P_W1], d, d_h.p, d, EPI_BF16, nullptr, 0, 0, 0, st));
+		} else if (!s->llama && !pre && gemm_gelu_bwd_fused(T, F, d) && ((uintptr_t)dyin % 16) == 0) {
+			const bool form_a = reform && bs.b[B_A].dropped;
+			ELF_TRY(gemm_gelu_bwd_bf16(T, F, d, dyin, p.w[P_W2], bs.b[B_GU].p, bs.b[B_DGU].p, nullptr, st));
+			if (form_a) {
+				ELF_TRY(buf_alloc(s, bs, B_A));
+				ELF_TRY(gelu_fwd(bs.b[B_GU].p, bs.b[B_A].p, (int64_t)T * F, st));
+			}
+			ELF_TRY(gemm_bf16(0, 1, T, d, F, bs.b[B_DGU].p, F, p.w[P_W1], d, d_h.p, d, EPI_BF16, nullptr, 0, 0, 0, st));
 		} else {
 			PoolTmp d_a(s->pool, (size_t)T * F * 2);
 			if (!d_a.p) return -3;

@@ -79,8 +79,8 @@ int elf_gemm_dw_group(int n, const elf_dw_problem* problems, int K, float scale,
 /* The MLP's up-projection with its activation: pre = A W^T with A [M, K] and W [N, K], both k contiguous;
  * act 0 (GELU): N = F, out[M, F] = gelu(pre); act 1 (SwiGLU): N = 2F, W = [gate rows; up rows],
  * pre[M, 2F] = [g | u], out[M, F] = silu(g) * u.  pre is kept because the backward needs it.  SwiGLU is
- * computed in the GEMM epilogue (one kernel, the pre-activation never re-read) or, as always for GELU, by elf_gemm_bf16
- * (epilogue 0) followed by elf_gelu_fwd / elf_swiglu_fwd, whichever is faster.  The one kernel runs every M and F of at least
+ * computed in the GEMM epilogue (one kernel, the pre-activation never re-read) or by elf_gemm_bf16 (epilogue 0) followed by
+ * elf_gelu_fwd / elf_swiglu_fwd, whichever is faster (GELU: one kernel for the smallest products only).  The one kernel runs every M and F of at least
  * 128 (sizes multiples of 64, leading dimensions of 8, 16-byte aligned operands): there the rows of pre and out may lie
  * further apart than 2 F and F, and it is then taken.  Same bits either way.
  * Replaces: fc1 + nn.GELU() of the GPT block's MLP (benchmarks/models/simple.py:44-52) run through

@@ -220,6 +220,24 @@ def test_gemm_tiles_between_128_and_256_rows(K, M, N, Kd):
 	assert torch.equal(K.gemm_swiglu_bwd(a, wt, g), K.gemm_swiglu_bwd(a, wt, g, fused=False))
 
 
+@pytest.mark.parametrize("M,F,Kd", [(64, 64, 256), (128, 192, 320), (512, 768, 512), (1024, 640, 256), (320, 448, 1088)])
+def test_small_products_with_their_activation_in_one_kernel(K, M, F, Kd):
+	"""Products that go to 64x64 tiles with the activation, its backward or the rotary embedding in the epilogue (both rings of
+	slices): the bits of the plain product followed by the pass of its own."""
+	a, w, w2 = _randn(M, Kd, seed=81), _randn(F, Kd, seed=82, scale=0.1), _randn(2 * F, Kd, seed=83, scale=0.1)
+	pre, act = K.gemm_act(a, w, K.ACT_GELU)
+	assert torch.equal(pre, K.gemm(a, w, tile_cfg=12)) and torch.equal(act, K.gelu_fwd(pre))
+	gu, act = K.gemm_act(a, w2, K.ACT_SWIGLU)
+	assert torch.equal(gu, K.gemm(a, w2, tile_cfg=12)) and torch.equal(act, K.swiglu_fwd(gu))
+	g, wt = _randn(M, 2 * F, seed=84), w.t().contiguous()
+	assert torch.equal(K.gemm_swiglu_bwd(a, wt, g), K.swiglu_bwd(K.gemm(a, wt, b_t=True, tile_cfg=12), g))
+	for D in (64, 128):
+		if 2 * F % D == 0:
+			cs, heads = K.rope_table(64, D, 5e5), 2 * F // D
+			for n_rot in (0, heads // 2, heads):
+				assert torch.equal(K.gemm_rope(a, w2, cs, 64, n_rot, D), K.gemm_rope(a, w2, cs, 64, n_rot, D, fused=False) if n_rot else K.gemm(a, w2, tile_cfg=12)), (D, n_rot)
+
+
 @pytest.mark.parametrize("shape", [(64, 64, 15424), (256, 704, 14080), (512, 384, 10112), (1536, 192, 12608), (64, 5632, 13696), (128, 256, 192)])
 def test_small_weight_gradients_are_split_along_the_tokens(K, shape):
 	"""Outputs too small for the chip with long reductions: the choice left open runs about as fast as the best of a few explicit
