@@ -17,7 +17,7 @@ namespace dma {
 //    of its split tiles with the `splits` workgroups of a tile side by side: the 32 tiles an XCD holds at a time are
 //    neighbours that share their operand slabs in its L2 (taken in launch order, neighbouring tiles of a 3-row problem
 //    land on different XCDs and every slab is fetched by all eight).
-constexpr int GROUP_MAX = 16;
+constexpr int GROUP_MAX = DW_GROUP_MAX;
 struct GroupArgs {
 	int n, compact;
 	int tiles, tail, splits;  // compact: all tiles of the launch, how many of the last are split, and how many ways
@@ -189,6 +189,16 @@ int gemm_dw_group(int n, const DwProblem* pr, int K, float scale, hipStream_t st
 		splits = 256 / rem < 8 ? 256 / rem : 8;
 		while (splits > 1 && nk / splits < 16) splits--;
 		if (splits > 1) tail = rem;
+	}
+	// Little work: where the layers make no more than a round of 128x128 tiles, these are done sooner than a few 256x256 ones (us,
+	// without and with the splits of the latter; fitted to launches over 128 to 8192 tokens).  Two blocks of a 512-wide Llama stage
+	// over 512 tokens 23.7 -> 12.7 us, of a 256-wide GPT stage 21.4 -> 10.8, one over 2048 tokens 33.5 -> 18.4; with two rounds it
+	// is one or the other (four layers of 768 over 1024 tokens 33.8 and 29.4, eight of 512 33.5 and 34.7).
+	int64_t small = 0;
+	for (int i = 0; i < n; i++) small += (int64_t)((pr[i].M + 127) / 128) * ((pr[i].N + 127) / 128);
+	if (small <= 256 && nk * 0.35f + 7.5f < (float)((nk + splits - 1) / splits) * 1.05f + 12.f + 2.f * (splits - 1)) {
+		ProfScope prof(PROF_GEMM, flops, stream);
+		return gemm_ring_dw_group(n, pr, K, scale, stream);
 	}
 	dma::GroupArgs ga{};
 	ga.n = n;

@@ -37,6 +37,7 @@ struct Args {
 	int64_t ldc2;
 	const float2* rope_cs;
 	int rope_S, rope_cols, rope_D;
+	float scale;  // EPI_F32_ACC_SCALE
 };
 
 // Turn counters of split tiles, one per tile and wave (the scheme of gemm_dma.hip: split s adds when the counter holds this
@@ -74,8 +75,9 @@ __device__ __forceinline__ void pair_slabs(f32x4& lo, f32x4& hi) {
 	}
 }
 
+// One workgroup: tile `pid`, K range `ksplit` of g.k_splits.
 template <int BM, int BN, bool AT, bool BT, int EPI, bool SHORT>
-__global__ __launch_bounds__(256) void gemm_ring_kernel(Args g) {
+__device__ __forceinline__ void gemm_ring_tile(const Args& g, const int pid, const int ksplit) {
 	using Sh = Shape<BM, BN, SHORT>;
 	constexpr int NST = Sh::NST, A_BYTES = Sh::A_BYTES, B_BYTES = Sh::B_BYTES, LOADS_A = Sh::LOADS_A, LOADS_B = Sh::LOADS_B, P = Sh::LOADS;
 	constexpr int WM = BM / 2, WN = BN / 2, RF = WM / 16, CF = WN / 16, NM = RF * CF, NR = RF + CF;
@@ -88,16 +90,6 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(Args g) {
 	const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 	const int wr = wave >> 1, wc = wave & 1;
 
-	// Workgroup w runs on XCD w % 8: every XCD takes a contiguous run of tiles (the splits of a tile side by side), walked in
-	// groups of eight tile rows that share their columns' slabs of B in its L2.
-	const int ntiles = g.tiles_m * g.tiles_n;
-	int ksplit, pid;
-	{
-		const int chunk = (ntiles + 7) >> 3, x = blockIdx.x & 7, slot = blockIdx.x >> 3;
-		ksplit = slot % g.k_splits;
-		pid = x * chunk + slot / g.k_splits;
-		if (slot / g.k_splits >= chunk || pid >= ntiles) return;
-	}
 	int m0, n0;
 	{
 		constexpr int GROUP_M = 8;
@@ -399,6 +391,7 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(Args g) {
 					*reinterpret_cast<bf16x8*>(reinterpret_cast<bf16_t*>(g.C) + (int64_t)(row0 + i * 16) * g.ldc + c + j * 16) = o;
 				}
 		} else {
+			constexpr bool ACCUM = EPI == EPI_F32_ACC || EPI == EPI_F32_ACC_SCALE;
 			float* const cp = reinterpret_cast<float*>(g.C) + (int64_t)row0 * g.ldc + col0 + 4 * g4;
 			if (EPI == EPI_F32_ACC && g.k_splits > 1) {
 #pragma unroll
@@ -408,8 +401,8 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(Args g) {
 #pragma unroll
 						for (int t = 0; t < 4; t++) unsafeAtomicAdd(cp + (int64_t)i * 16 * g.ldc + j * 16 + t, acc[i][j][t]);
 			} else {
-				f32x4 cv[EPI == EPI_F32_ACC ? RF : 1][CF];
-				if constexpr (EPI == EPI_F32_ACC) {  // every load of the wave's share before the first store
+				f32x4 cv[ACCUM ? RF : 1][CF];
+				if constexpr (ACCUM) {  // every load of the wave's share before the first store
 #pragma unroll
 					for (int i = 0; i < RF; i++)
 #pragma unroll
@@ -419,7 +412,14 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(Args g) {
 				for (int i = 0; i < RF; i++)
 #pragma unroll
 					for (int j = 0; j < CF; j++) {
-						if constexpr (EPI == EPI_F32_ACC) acc[i][j] += cv[i][j];
+						if constexpr (ACCUM) acc[i][j] += cv[i][j];
+						if constexpr (EPI == EPI_F32_ACC_SCALE) {  // as in gemm_dma_tile: the bits of scale_grads
+							acc[i][j] *= g.scale;
+							bf16x4 o;
+#pragma unroll
+							for (int t = 0; t < 4; t++) o[t] = (bf16_t)acc[i][j][t];
+							*reinterpret_cast<bf16x4*>(g.C2 + (int64_t)(row0 + i * 16) * g.ldc2 + col0 + 4 * g4 + j * 16) = o;
+						}
 						*reinterpret_cast<f32x4*>(cp + (int64_t)i * 16 * g.ldc + j * 16) = acc[i][j];
 					}
 			}
@@ -429,6 +429,41 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(Args g) {
 		if (g.k_splits > 1) pass_turn();
 	}
 	wait_vmcnt<0>();  // the loads past the end of K land in LDS too
+}
+
+template <int BM, int BN, bool AT, bool BT, int EPI, bool SHORT>
+__global__ __launch_bounds__(256) void gemm_ring_kernel(Args g) {
+	// Workgroup w runs on XCD w % 8: every XCD takes a contiguous run of tiles (the splits of a tile side by side), walked in
+	// groups of eight tile rows that share their columns' slabs of B in its L2.
+	const int ntiles = g.tiles_m * g.tiles_n;
+	int ksplit, pid;
+	{
+		const int chunk = (ntiles + 7) >> 3, x = blockIdx.x & 7, slot = blockIdx.x >> 3;
+		ksplit = slot % g.k_splits;
+		pid = x * chunk + slot / g.k_splits;
+		if (slot / g.k_splits >= chunk || pid >= ntiles) return;
+	}
+	gemm_ring_tile<BM, BN, AT, BT, EPI, SHORT>(g, pid, ksplit);
+}
+
+// The weight gradients of a stage's layers in one launch, as gemm_dw_group_kernel of gemm_dma.hip, for stages so small that its
+// 256x256 tiles leave most of the chip idle: the 128x128 tiles of all problems are one sequence, of which every XCD takes a
+// contiguous eighth.  What bounds it: one tile's chain (ring fill, slices, read-modify-write),
+// 12.7 us for two blocks of a 512-wide Llama stage over 512 tokens against 23.7 on 60 tiles of 256x256 (see gemm_dw_group()).
+struct GroupArgs {
+	int n, tiles;
+	int first[DW_GROUP_MAX];  // problem p's first tile in the sequence
+	Args a[DW_GROUP_MAX];
+};
+template <int EPI>
+__global__ __launch_bounds__(256) void gemm_ring_dw_group_kernel(GroupArgs ga) {
+	const int chunk = (ga.tiles + 7) >> 3, x = blockIdx.x & 7, slot = blockIdx.x >> 3, t = x * chunk + slot;
+	if (slot >= chunk || t >= ga.tiles) return;
+	int p = 0;
+	for (int i = 1; i < ga.n; i++)
+		if (t >= ga.first[i]) p = i;
+	p = __builtin_amdgcn_readfirstlane(p);
+	gemm_ring_tile<128, 128, true, true, EPI, false>(ga.a[p], t - ga.first[p], 0);
 }
 
 template <int BM, int BN, bool AT, bool BT, int EPI, bool SHORT>
@@ -489,7 +524,7 @@ int gemm_bf16_ring(int a_t, int b_t, int M, int N, int K, const void* A, int64_t
                    int64_t ldr, int k_splits, int bm, int bn, hipStream_t stream) {
 	ELF_REQUIRE(M % 64 == 0 && N % 64 == 0 && K % dma::BKS == 0, "gemm (ring tile): sizes must be multiples of 64");
 	ELF_REQUIRE(gemm_reaches(a_t ? dma::BKS : bm, lda) && gemm_reaches(b_t ? dma::BKS : bn, ldb), "gemm (ring tile): leading dimension too large (%lld, %lld)", (long long)lda, (long long)ldb);
-	ring::Args g{(const bf16_t*)A, (const bf16_t*)B, C, (const bf16_t*)R, lda, ldb, ldc, ldr, M, N, K, 0, 0, k_splits, 0, nullptr, 0, nullptr, 0, 0, 0};
+	ring::Args g{(const bf16_t*)A, (const bf16_t*)B, C, (const bf16_t*)R, lda, ldb, ldc, ldr, M, N, K, 0, 0, k_splits, 0, nullptr, 0, nullptr, 0, 0, 0, 0.f};
 	if (bm == 128 && bn == 128) return ring::launch_layout<128, 128>(g, a_t, b_t, epi, stream);
 	if (bm == 64 && bn == 128) return ring::launch_layout<64, 128>(g, a_t, b_t, epi, stream);
 	if (bm == 128 && bn == 64) return ring::launch_layout<128, 64>(g, a_t, b_t, epi, stream);
@@ -517,7 +552,7 @@ int gemm_ring_act(int M, int N, int K, const void* A, int64_t lda, const void* B
 	            "gemm (ring tile): the RoPE epilogue needs a table and whole heads of 64 or 128 columns");
 	ELF_REQUIRE((C2 || (epi != EPI_BF16_SWIGLU && epi != EPI_BF16_GELU)) && (R || !bt), "gemm (ring tile): an epilogue's operand is missing");
 	ring::Args g{(const bf16_t*)A, (const bf16_t*)B, C, (const bf16_t*)R, lda, ldb, ldc, ldr, M, N, K, M / 64, N / 64, 1, 0,
-	             (bf16_t*)C2, ldc2, (const float2*)rope_cs, rope_S, rope_cols, rope_D};
+	             (bf16_t*)C2, ldc2, (const float2*)rope_cs, rope_S, rope_cols, rope_D, 0.f};
 	switch (epi) {
 		case EPI_BF16_SWIGLU: return ring::launch_act<false, EPI_BF16_SWIGLU>(g, stream);
 		case EPI_BF16_ROPE: return ring::launch_act<false, EPI_BF16_ROPE>(g, stream);
@@ -527,6 +562,30 @@ int gemm_ring_act(int M, int N, int K, const void* A, int64_t lda, const void* B
 	}
 	set_error("gemm (ring tile): unknown epilogue %d", epi);
 	return -1;
+}
+
+// Arguments are validated by gemm_dw_group() before it dispatches here.
+int gemm_ring_dw_group(int n, const DwProblem* pr, int K, float scale, hipStream_t stream) {
+	ring::GroupArgs ga{};
+	ga.n = n;
+	for (int i = 0; i < n; i++) {
+		const DwProblem& q = pr[i];
+		ring::Args& a = ga.a[i];
+		a = ring::Args{(const bf16_t*)q.dY, (const bf16_t*)q.X, q.acc, nullptr, q.lddy, q.ldx, q.N, 0, q.M, q.N, K, (q.M + 127) / 128, (q.N + 127) / 128, 1, 0,
+		               (bf16_t*)q.grad_bf16, q.N, nullptr, 0, 0, 0, scale};
+		ga.first[i] = ga.tiles;
+		ga.tiles += a.tiles_m * a.tiles_n;
+	}
+	using Sh = ring::Shape<128, 128, false>;
+	auto kern = scale != 0.f ? ring::gemm_ring_dw_group_kernel<EPI_F32_ACC_SCALE> : ring::gemm_ring_dw_group_kernel<EPI_F32_ACC>;
+	static bool attr_set[2] = {};
+	if (bool& set = attr_set[scale != 0.f]; !set) {
+		ELF_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, Sh::SMEM));
+		set = true;
+	}
+	ELF_LAUNCH(kern, dim3(8 * ((ga.tiles + 7) / 8)), dim3(256), (Sh::SMEM), stream, ga);
+	ELF_CHECK_HIP(hipGetLastError());
+	return 0;
 }
 
 }  // namespace elf

@@ -75,6 +75,8 @@ struct DwProblem {
 	void* grad_bf16;  // may be null when scale == 0
 	int M, N;
 };
+constexpr int DW_GROUP_MAX = 16;
+int gemm_ring_dw_group(int n, const DwProblem* problems, int K, float scale, hipStream_t stream);  // on 128x128 ring tiles
 bool gemm_dw_groupable(int M, int N, int K, const void* dY, int64_t lddy, const void* X, int64_t ldx, const void* acc);
 int gemm_dw_group(int n, const DwProblem* problems, int K, float scale, hipStream_t stream);
 

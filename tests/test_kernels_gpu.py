@@ -238,6 +238,26 @@ def test_small_products_with_their_activation_in_one_kernel(K, M, F, Kd):
 				assert torch.equal(K.gemm_rope(a, w2, cs, 64, n_rot, D), K.gemm_rope(a, w2, cs, 64, n_rot, D, fused=False) if n_rot else K.gemm(a, w2, tile_cfg=12)), (D, n_rot)
 
 
+@pytest.mark.parametrize("Kd", [64, 320, 512, 1088])
+@pytest.mark.parametrize("shapes", [[(256, 256)], [(512, 768), (1536, 512), (512, 512), (1024, 512)], [(256, 1024)] * 16])
+def test_weight_gradients_of_small_stages_in_one_launch(K, shapes, Kd):
+	"""Groups of no more than a round of 128x128 tiles (one problem of the smallest size, one to sixteen, K slices fewer and more
+	than the ring holds): the bits of a launch per layer without a K split, and of that followed by the gradient scale."""
+	dy = [_randn(Kd, M, seed=91 + i) for i, (M, N) in enumerate(shapes)]
+	x = [_randn(Kd, N, seed=191 + i) for i, (M, N) in enumerate(shapes)]
+	start = [torch.randn(M, N, device="cuda", generator=torch.Generator(device="cuda").manual_seed(291 + i)) for i, (M, N) in enumerate(shapes)]
+	want = [s.clone() for s in start]
+	for d, a, w in zip(dy, x, want):
+		K.gemm(d, a, a_t=True, b_t=True, out=w, epilogue=K.EPI_F32_ACC, tile_cfg=12, k_splits=1)
+	got = [s.clone() for s in start]
+	K.gemm_dw_group(list(zip(dy, x, got)))
+	assert all(torch.equal(g, w) for g, w in zip(got, want))
+	got, bf = [s.clone() for s in start], [torch.empty(M, N, dtype=torch.bfloat16, device="cuda") for M, N in shapes]
+	K.gemm_dw_group(list(zip(dy, x, got, bf)), scale=0.375)
+	for g, b, w in zip(got, bf, want):
+		assert torch.equal(g, w * 0.375) and torch.equal(b, (w * 0.375).to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("shape", [(64, 64, 15424), (256, 704, 14080), (512, 384, 10112), (1536, 192, 12608), (64, 5632, 13696), (128, 256, 192)])
 def test_small_weight_gradients_are_split_along_the_tokens(K, shape):
 	"""Outputs too small for the chip with long reductions: the choice left open runs about as fast as the best of a few explicit
