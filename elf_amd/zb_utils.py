@@ -40,7 +40,9 @@ class LinearDX(torch.autograd.Function):
 		ctx.save_for_backward(input.detach())  # marks the input as needed by the backward, so that torch.utils.checkpoint recomputes it
 		x = _as_rows(input)
 		if bias is not None:
-			y = kernels.gemm(x, weight, epilogue=kernels.EPI_BF16_RESID, residual=bias, residual_ld=0)
+			# one dense row of N values as it lies (the views take 3 us); expand refuses any other size but 1
+			row = bias if bias.numel() == weight.shape[0] and bias.is_contiguous() else bias.reshape(1, -1).expand(1, weight.shape[0]).contiguous()
+			y = kernels.gemm(x, weight, epilogue=kernels.EPI_BF16_RESID, residual=row, residual_ld=0)
 		else:
 			y = kernels.gemm(x, weight)
 		return y.view(*input.shape[:-1], weight.shape[0])
