@@ -6,7 +6,8 @@
 //   dW       dW += dY^T . X  A = dY [K,M] m-contiguous ("T"), B = X  [K,N] n-contiguous ("T")
 // (reference semantics: elf/zb_utils.py:20 forward, :34-37 dX, :235-244 dW accumulate).
 //
-// The kernels are in gemm_dma.hip (256x256 and 128x256 tiles) and gemm_ring.hip (128x128 .. 64x64 tiles); all of them
+// The kernels are in gemm_dma_tile.h and gemm_dma_pers.hip (128 to 256 rows by 256 columns) and gemm_ring.hip (128x128 .. 64x64
+// tiles); all of them
 // add the products of an output in the same order, so the choice of a tile never changes its bits (a split of K does).
 #include <atomic>
 
@@ -286,8 +287,7 @@ int gemm_rope_bf16(int M, int N, int K, const void* A, int64_t lda, const void* 
 static bool swiglu_bwd_fits(int M, int F, int K) { return M >= 256 && F >= 256 && M % 64 == 0 && F % 64 == 0 && K % 64 == 0; }
 // The tile it runs on.  The epilogue reads and writes four of d, g, u and their two gradients at 256 tiles a time: 20 us more per
 // round of 256-row tiles than the plain one, and 4 us a launch (without these 3072 x 2304 x 768 took 33 us fused, 30.6 apart;
-// with 12 us for the whole round 1024 x 3072 x 64 took 25 us
-// fused, 13 apart, and 8448 x 512 x 512 32 and 20).
+// with 12 us for the whole round 1024 x 3072 x 64 took 25 us fused, 13 apart, and 8448 x 512 x 512 32 and 20).
 static Plan swiglu_bwd_tile(int M, int F, int K) {
 	Plan best;
 	auto weigh = [&](TileTime t) {

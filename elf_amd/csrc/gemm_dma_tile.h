@@ -1,4 +1,4 @@
-// 256x256 (and 128x256) bf16 MFMA GEMM tile kernel with direct global->LDS loads, for gfx950.
+// bf16 MFMA GEMM tile kernel (128 to 256 rows by 256 columns) with direct global->LDS loads, for gfx950.
 //
 // The contraction of gemm_bf16.hip (C (+)= sum_k A(m,k) B(n,k); "R" operands are
 // k-contiguous, "T" operands reduction-major), different data movement:

@@ -1,16 +1,16 @@
 // bf16 MFMA GEMM on small tiles (128x128, 64x128, 128x64, 64x64) with a deep ring of K slices in LDS, for gfx950.
 //
-// Same contraction, layouts and order of products along K as gemm_dma.hip (v_mfma_f32_16x16x32_bf16, 64 wide K slices in
+// Same contraction, layouts and order of products along K as gemm_dma_tile.h (v_mfma_f32_16x16x32_bf16, 64 wide K slices in
 // ascending order), so a tile's bits do not depend on which of the kernels computed it.  These are the tiles of products
-// too small to fill the chip with 256- or 128-row tiles of gemm_dma.hip: a workgroup then has few K slices and every trip to
+// too small to fill the chip with the 256-column tiles of gemm_dma_tile.h: a workgroup then has few K slices and every trip to
 // memory shows.  The ring holds as many slices as LDS takes (eight of the 64x64 tile, four of the 128x128 one), all fetched
 // before the first product; from then on a slice is fetched as soon as its predecessor in the same stage has been read.
 //
 // Bound: the 64 B/clk path into LDS (a slice of the 128x128 tile is 512 cycles of it and 512 of MFMA, of the 64x64 tile 256
 // against 128) and LDS reads; results leave from registers, two neighbouring column slabs exchanged between lane groups so
 // that a lane stores 16 bytes.  The activations and the rotary embedding of the smallest products ride in the epilogue of the
-// 64x64 tile (gemm_ring_act: what bounds these is the number of launches).  Against the register-staged tiles (global -> VGPR -> LDS, two stages) that these replace, cold
-// operands: 1920 x 1600 x 1600 23.1 -> 19.9 us, 2112 x 832 x 4288 50 -> 31, 512 x 512 x 1536 14.2 -> 7.9; weight
+// 64x64 tile (gemm_ring_act: what bounds these is the number of launches).
+// Against the register-staged tiles (global -> VGPR -> LDS, two stages) that these replace, cold operands: 1920 x 1600 x 1600 23.1 -> 19.9 us, 2112 x 832 x 4288 50 -> 31, 512 x 512 x 1536 14.2 -> 7.9; weight
 // gradients: 1600 x 1600 x 1920 36.7 -> 25.6, 832 x 4288 x 2112 50 -> 29, 768 x 768 x 4096 31 -> 22.
 #include "common.h"
 #include "gemm_tile.h"
