@@ -962,6 +962,10 @@ using namespace attn;
 // taken apart as well, which spares the chain the fixed part of its second tile and needs no partial sums.  The whole call, before
 // -> after (us): 2 x 256 tokens, 4 / 2 heads of 128 32.4 -> 22.5; 3 x 640, 25 heads of 64 63.9 -> 56.4; 4 x 512, 12 heads of 64
 // 48.9 -> 38.5; 896 tokens, 32 / 8 heads of 128 66.5 -> 60.9.
+// Causal with one key tile (128 tokens): a walk has four steps a head, what a step and a split cost beside the fixed part shows.
+// Constants of its own, fitted to every sharing of 250 such shapes (the one that is picked takes 0.2 % longer than the best on
+// average, 5 % at most; with those of longer walks 1.8 and 16 %).  The whole call, whole -> as shared now (us): 2 x 128 tokens, 4 heads of 64
+// 18.9 -> 16.7; 3 x 128, 48 / 16 heads of 128 34.8 -> 31.2; 7 x 128, 36 / 12 heads of 128 stay whole: 37.8, three ways 40.6.
 struct Splits {
 	int h = 1, q = 1;
 	bool paired = true;
@@ -971,7 +975,10 @@ static int64_t dkv_part_bytes(const Splits& sp, int B, int S, int Hkv, int D) { 
 // single key tiles.
 static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal, int64_t room) {
 	const int nkt = S / 128, G = Hq / Hkv;
-	const float slots = D == 128 ? 256.f : 512.f, step = D == 128 ? 1.2f : 1.1f, fixed = 8.f;
+	const bool one = causal && nkt == 1;
+	const float slots = D == 128 ? 256.f : 512.f, step = one ? 1.6f : D == 128 ? 1.2f : 1.1f, fixed = 8.f;
+	// a split: what it adds by itself, per split, and the partial sums at so many bytes a us; it has to be that much better than less sharing
+	const float split = one ? 0.f : 2.f, per_split = one ? 0.4f : 0.f, rate = one ? 4e6f : 5e6f, margin = one ? 1.f : 0.95f;
 	Splits best;
 	// From 2^18 query rows (2 x 4096 tokens of 32 heads) up walks stay whole.  With eight kv heads or more and several sequences such
 	// launches fill the chip; one sequence of 4096 tokens with 64 / 8 heads (128 walks for 256 compute units) does not, and sharing
@@ -991,8 +998,8 @@ static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal, int6
 				if (dkv_part_bytes(Splits{h, q}, B, S, Hkv, D) > room) continue;
 				const float rounds = ceilf((float)(walks * ns) / slots);
 				if (!paired && rounds > 1.f) continue;
-				const float us = rounds * (fixed + (float)(G / h) * ((tiles + q - 1) / q) * step) + (ns > 1 ? 2.f + (float)ns * B * S * Hkv * D * 16 / 5e6f : 0.f);
-				if (us < best_us * (ns > 1 ? 0.95f : 1.f)) best_us = us, best = Splits{h, q, paired != 0};
+				const float us = rounds * (fixed + (float)(G / h) * ((tiles + q - 1) / q) * step) + (ns > 1 ? split + ns * per_split + (float)ns * B * S * Hkv * D * 16 / rate : 0.f);
+				if (us < best_us * (ns > 1 ? margin : 1.f)) best_us = us, best = Splits{h, q, paired != 0};
 			}
 		}
 	}

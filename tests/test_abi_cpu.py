@@ -90,6 +90,15 @@ def test_attention_workspace_of_a_larger_shape_serves_the_smaller_ones(lib, D, c
 	assert lib.elf_attn_bwd_workspace_bytes(2, 4096, 8, D, 0) > lib.elf_attn_bwd_workspace_bytes(2, 4096, 8, D, 1)
 
 
+@pytest.mark.parametrize("shape,ways", [((2, 128, 4, 4, 64), 4), ((7, 128, 1, 1, 64), 4), ((1, 128, 8, 8, 128), 2), ((3, 128, 48, 16, 128), 3), ((3, 128, 75, 25, 64), 3), ((7, 128, 36, 12, 128), 1)])
+def test_attention_backward_shares_the_walks_of_one_key_tile(lib, shape, ways):
+	"""Causal sequences of 128: the sharing that the whole call was measured to be fastest with (us, whole and shared: 18.9 and 16.7,
+	19.0 and 16.4, 21.5 and 19.2, 34.8 and 31.2, 32.5 and 29.4, 37.8 and 40.6)."""
+	B, S, Hq, Hkv, D = shape
+	more = lib.elf_attn_bwd_shared_workspace_bytes(*shape, 1) - lib.elf_attn_bwd_workspace_bytes(B, S, Hq, D, 1)
+	assert more == (ways * 8 * B * S * Hkv * D if ways > 1 else 0)
+
+
 def test_attention_backward_refuses_a_workspace_that_is_too_small(lib):
 	n = lib.elf_attn_bwd_workspace_bytes(1, 128, 4, 64, 1)
 	rc = lib.elf_attn_bwd_shared(*[16] * 10, n - 1, *[64 * 12] * 8, 1, 128, 4, 4, 64, 1, 0.125, None, None)
