@@ -964,7 +964,7 @@ using namespace attn;
 // 48.9 -> 38.5; 896 tokens, 32 / 8 heads of 128 66.5 -> 60.9.
 // Causal with one key tile (128 tokens): a walk has four steps a head, what a step and a split cost beside the fixed part shows.
 // Constants of its own, fitted to every sharing of 250 such shapes (the one that is picked takes 0.2 % longer than the best on
-// average, 5 % at most; with those of longer walks 1.8 and 16 %).  The whole call, whole -> as shared now (us): 2 x 128 tokens, 4 heads of 64
+// average, 7 % at most; with those of longer walks 1.8 and 16 %).  The whole call, whole -> as shared now (us): 2 x 128 tokens, 4 heads of 64
 // 18.9 -> 16.7; 3 x 128, 48 / 16 heads of 128 34.8 -> 31.2; 7 x 128, 36 / 12 heads of 128 stay whole: 37.8, three ways 40.6.
 struct Splits {
 	int h = 1, q = 1;
@@ -985,8 +985,12 @@ static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal, int6
 	// has not been measured there.
 	if ((int64_t)B * S * Hq >= 1 << 18) return best;
 	float best_us = 1e30f;
+	bool shared_pairs = false;
 	for (int paired = 1; paired >= (causal && nkt > 1 ? 0 : 1); paired--) {
-		if (!paired) best_us += fixed;  // that of a pair's second tile, which all sharings of pairs have alike
+		if (!paired) {
+			best_us += fixed;  // that of a pair's second tile, which all sharings of pairs have alike
+			shared_pairs = best.h * best.q > 1;
+		}
 		const bool two = causal && paired && nkt > 1;  // key tiles one after the other
 		const int64_t walks = (int64_t)B * Hkv * (two ? (nkt + 1) / 2 : nkt);
 		const int tiles = two ? (nkt + 1) * 4 : nkt * 4;  // query tiles of the longest walk and head (a pair of key tiles has nkt + 1 of four)
@@ -999,7 +1003,11 @@ static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal, int6
 				const float rounds = ceilf((float)(walks * ns) / slots);
 				if (!paired && rounds > 1.f) continue;
 				const float us = rounds * (fixed + (float)(G / h) * ((tiles + q - 1) / q) * step) + (ns > 1 ? split + ns * per_split + (float)ns * B * S * Hkv * D * 16 / rate : 0.f);
-				if (us < best_us * (ns > 1 ? margin : 1.f)) best_us = us, best = Splits{h, q, paired != 0};
+				// Over 40 shapes that were shared as pairs a whole walk per tile is as fast where its estimate is 3 us above that of the
+				// shared pair, not 8.  Without this 8 x 1408 tokens, 6 / 2 heads of 128 took 187 us, 161 as pairs shared three ways;
+				// 10 x 512, 12 / 4 heads of 128 85.5 and 82.3.
+				const float lead = shared_pairs && ns == 1 ? fixed - 3.f : 0.f;
+				if (us + lead < best_us * (ns > 1 ? margin : 1.f)) best_us = us, best = Splits{h, q, paired != 0};
 			}
 		}
 	}
