@@ -43,6 +43,7 @@ int elf_gemm_rope_bf16(int M, int N, int K, const void* A, int64_t lda, const vo
                        int n_rot_heads, int D, void* stream) {
 	return elf::gemm_rope_bf16(M, N, K, A, lda, W, ldw, C, ldc, cs, S, n_rot_heads, D, S_(stream));
 }
+int elf_gemm_way(int product, int M, int N, int K, int D) { return elf::gemm_way(product, M, N, K, D); }
 int elf_norm_fwd(int kind, const void* x, const void* gamma, const void* beta, void* y, void* stats, int T, int d,
                  float eps, void* stream) {
 	return elf::norm_fwd(kind, x, gamma, beta, y, stats, T, d, eps, S_(stream));

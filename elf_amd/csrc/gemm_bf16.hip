@@ -48,8 +48,12 @@ int gemm_turn_giveups(uint64_t* out) {
 // 128-row ones make twice the rounds (without them the best tile takes 2.9 % longer on average): before -> after (us)
 //   2688 x 4096 x 28672 (a Llama-3-8B block's input gradient over 3 x 896 tokens) 504 on 176 tiles of 256 rows, 463 on 224 of 192;
 //   2688 x 4096 x 14336 with a residual 266 -> 231, 1920 x 4800 x 1600 32.1 on 152 tiles, 28.0 on 228 of 160,
-//   8192 x 2304 x 768 37.4 on 288 tiles of 256 rows, 31.1 on 468 of 160, 4096 x 5504 x 2048 with the SwiGLU backward 131 on 352
+//   8192 x 2304 x 768 42.4 on 288 tiles of 256 rows, 40.2 on 387 of 192, 4096 x 5504 x 2048 with the SwiGLU backward 131 on 352
 //   tiles of 256 rows, 117 on 484 of 192; 1920 x 1600 x 1600 stays on 195 tiles of 128x128 (14.6; 24 on 84 of 160 rows).
+// 160-row tiles fetch 30 % more operand bytes a product than 256-row ones (192: 17 %), which a stream at the power limit pays for in
+// its other kernels.  For K of at most 1024 they are taken where the launch is one round: with the QKV product on 468 of them
+// (39.0 us alone) a GPT-2-small stage took 8.06 ms where it takes 7.97 with 192 rows, on boxes that clock low; 7.69 and 7.70 on others.
+// For a longer K 192 rows take 5 to 10 % longer, and a Llama-3-8B block of 2688 tokens is as fast with either.
 struct TileTime {
 	int bm, bn;
 	float slice, round, launch;
@@ -94,7 +98,8 @@ static Plan plan_tiles(int M, int N, int K, bool mid = true, float ring_extra = 
 	}
 	for (const TileTime& t : TILES_BF16) weigh(t);
 	if (mid)
-		for (const TileTime& t : TILES_MID) weigh(t);
+		for (const TileTime& t : TILES_MID)
+			if (t.bm > 160 || K > 1024 || (int64_t)((M + 159) / 160) * ((N + 255) / 256) <= 256) weigh(t);
 	return best;
 }
 
@@ -205,6 +210,20 @@ int gemm_bf16(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda,
 	return gemm_bf16_ring(a_t, b_t, M, N, K, A, lda, B, ldb, C, ldc, epi, R, ldr, k_splits, bm, bn, stream);
 }
 
+// The way of an up-projection with its activation: a 256-column tile (SwiGLU), a 64x64 ring tile, bm = 0: two passes.
+static Plan act_plan(int act, int M, int F, int K, bool dense) {
+	const int N = act == ACT_SWIGLU ? 2 * F : F;
+	Plan best;
+	best.us = plan_tiles(M, N, K).us + pass_us((act == ACT_SWIGLU ? 6.0 : 4.0) * M * F);
+	if (act == ACT_SWIGLU) {
+		const Plan p = plan_tiles(M, N, K, true, dense ? pass_us(6.0 * M * F) : NO_RING, SWIGLU_FWD_US);
+		best.us = p.us;
+		if (p.dma()) best = p;
+	}
+	const float small = dense ? small_us(M, N, K, act == ACT_SWIGLU ? SMALL_SWIGLU_US : SMALL_GELU_US) : 1e30f;
+	return small < best.us ? Plan{64, 64, 1, small} : best;
+}
+
 int gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, const void* W, int64_t ldw, void* pre,
                   int64_t ldpre, void* out, int64_t ldout, hipStream_t stream) {
 	ELF_REQUIRE(act == ACT_GELU || act == ACT_SWIGLU, "gemm_act: unknown activation %d", act);
@@ -212,27 +231,18 @@ int gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, cons
 	const int N = act == ACT_SWIGLU ? 2 * F : F;
 	// the SwiGLU epilogue pairs 64 gate with 64 up columns per wave, so a 256-column tile covers 128 outputs; it reaches the up rows
 	// with 32-bit byte offsets from the gate rows
-	int bm = 0;
-	bool small = false;
+	Plan p;
 	if (M % 64 == 0 && F % 64 == 0 && K % 64 == 0 && lda % 8 == 0 && ldw % 8 == 0 && ldpre >= N && ldout >= F && ldpre % 8 == 0 && ldout % 8 == 0 && ((uintptr_t)A % 16) == 0 &&
-	    ((uintptr_t)W % 16) == 0 && ((uintptr_t)pre % 16) == 0 && ((uintptr_t)out % 16) == 0 && lda >= K && ldw >= K && gemm_reaches(256, lda) && (int64_t)(F + 256) * ldw * 2 < (int64_t(1) << 31)) {
-		const bool dense = ldpre == N && ldout == F;  // rows that lie further apart only the fused kernel of the large tiles writes
-		float us = plan_tiles(M, N, K).us + pass_us((act == ACT_SWIGLU ? 6.0 : 4.0) * M * F);
-		if (act == ACT_SWIGLU) {
-			const Plan p = plan_tiles(M, N, K, true, dense ? pass_us(6.0 * M * F) : NO_RING, SWIGLU_FWD_US);
-			bm = p.dma() ? p.bm : 0;
-			us = p.us;
-		}
-		small = dense && small_us(M, N, K, act == ACT_SWIGLU ? SMALL_SWIGLU_US : SMALL_GELU_US) < us;
-	}
-	if (small) {
+	    ((uintptr_t)W % 16) == 0 && ((uintptr_t)pre % 16) == 0 && ((uintptr_t)out % 16) == 0 && lda >= K && ldw >= K && gemm_reaches(256, lda) && (int64_t)(F + 256) * ldw * 2 < (int64_t(1) << 31))
+		p = act_plan(act, M, F, K, ldpre == N && ldout == F);  // rows that lie further apart only the fused kernel of the large tiles writes
+	if (p.bm == 64) {
 		ProfScope prof(PROF_GEMM, 2.0 * M * N * K, stream);
 		return gemm_ring_act(M, N, K, A, lda, W, ldw, pre, ldpre, act == ACT_SWIGLU ? EPI_BF16_SWIGLU : EPI_BF16_GELU, nullptr, 0, stream, out, ldout);
 	}
-	if (bm) {
+	if (p.bm) {
 		ProfScope prof(PROF_GEMM, 2.0 * M * N * K, stream);
 		return gemm_bf16_dma(0, 0, M, N, K, A, lda, W, ldw, pre, ldpre, EPI_BF16_SWIGLU, nullptr, 0, 1, 0,
-		                     bm, stream, out, ldout);
+		                     p.bm, stream, out, ldout);
 	}
 	ELF_REQUIRE(ldpre == N && ldout == F, "gemm_act: the unfused path needs dense outputs");
 	if (int rc = gemm_bf16(0, 0, M, N, K, A, lda, W, ldw, pre, ldpre, EPI_BF16, nullptr, 0, 0, 0, stream)) return rc;
@@ -353,6 +363,26 @@ int gemm_gelu_bwd_bf16(int M, int F, int K, const void* dY, const void* W, const
 	ELF_REQUIRE(scratch, "gemm_gelu_bwd: this shape needs a scratch buffer of M x F bf16");
 	if (int rc = gemm_bf16(0, 1, M, F, K, dY, K, W, F, scratch, F, EPI_BF16, nullptr, 0, 0, 0, stream)) return rc;
 	return gelu_bwd(scratch, pre, dpre, (int64_t)M * F, stream);
+}
+
+int gemm_way(int product, int M, int N, int K, int D) {
+	Plan p;
+	if (M < 64 || N < 64 || K < 64 || M % 64 || N % 64 || K % 64) return 0;
+	switch (product) {
+		case GEMM_WAY_FORWARD: case GEMM_WAY_INPUT_GRADIENT: p = plan_tiles(M, N, K); break;
+		case GEMM_WAY_GELU: p = act_plan(ACT_GELU, M, N, K, true); break;
+		case GEMM_WAY_SWIGLU: p = act_plan(ACT_SWIGLU, M, N, K, true); break;
+		case GEMM_WAY_GELU_BWD: if (gemm_gelu_bwd_fused(M, N, K)) p = Plan{64, 64}; break;
+		case GEMM_WAY_SWIGLU_BWD: {
+			const int way = swiglu_bwd_way(M, N, K);
+			if (way != WAY_APART) p = way == WAY_SMALL ? Plan{64, 64} : swiglu_bwd_tile(M, N, K);
+			break;
+		}
+		case GEMM_WAY_ROPE:
+			if (const int rows = rope_tile_rows(M, N, K, D)) p = Plan{rows, rows == 64 ? 64 : 256};
+			break;
+	}
+	return p.bm << 16 | p.bn;
 }
 
 }  // namespace elf

@@ -97,6 +97,10 @@ uint32_t next_turn_tag();
 // from two device counters).
 int gemm_turn_giveups(uint64_t* out);
 
+// The tile (rows << 16 | columns) that dense, aligned operands of a product take, 0: the epilogue's work in a pass of its own.
+enum GemmWay { GEMM_WAY_FORWARD = 0, GEMM_WAY_INPUT_GRADIENT, GEMM_WAY_GELU, GEMM_WAY_SWIGLU, GEMM_WAY_GELU_BWD, GEMM_WAY_SWIGLU_BWD, GEMM_WAY_ROPE };
+int gemm_way(int product, int M, int N, int K, int D);
+
 enum Activation { ACT_GELU = 0, ACT_SWIGLU = 1 };
 // Up-projection of the MLP with its activation: pre = A W^T (A [M, K], W [N, K], N = F for GELU and 2F =
 // [gate rows; up rows] for SwiGLU), out [M, F] = gelu(pre) or silu(pre[:, :F]) * pre[:, F:].  One kernel (activation

@@ -108,6 +108,12 @@ int elf_gemm_swiglu_bwd_bf16(int M, int F, int K, const void* dY, int64_t lddy, 
  *           (elf/zb_utils.py:20); no reference module for the rotary embedding. */
 int elf_gemm_rope_bf16(int M, int N, int K, const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc,
                        const void* cs, int S, int n_rot_heads, int D, void* stream);
+/* Which way the calls above take with dense, aligned operands and no tile asked for: rows << 16 | columns of the tile, 0 where
+ * the epilogue's work is a pass of its own (or a size is no multiple of 64).  product: 0 forward and 1 input gradient of
+ * elf_gemm_bf16 (epilogues 0 and 1), 2 GELU and 3 SwiGLU of elf_gemm_act_bf16 (N = F), 4 the same choice for the GELU backward
+ * inside a stage, 5 elf_gemm_swiglu_bwd_bf16 (N = F), 6 elf_gemm_rope_bf16 (heads of width D).  Host only; for tests and tuning, no
+ * counterpart in the reference. */
+int elf_gemm_way(int product, int M, int N, int K, int D);
 
 /* ---------------------------------------------------------------------------------------------
  * Bandwidth-bound stage ops.  bf16 row-major tensors, fp32 math, one rounding on store.
