@@ -389,6 +389,9 @@ __device__ __forceinline__ void gemm_ring_tile(const Args& g, const int pid, con
 						o[t] = (bf16_t)v;
 					}
 					*reinterpret_cast<bf16x8*>(reinterpret_cast<bf16_t*>(g.C) + (int64_t)(row0 + i * 16) * g.ldc + c + j * 16) = o;
+					// a slab leaves before the next is read: left alone the scheduler may keep all stores for the end, 0.2 us of a
+					// tile's 4 to 5 (128x64, K = 64: 128 x 9344 4.33 -> 4.50 us that way; a d = 256 GPT stage 2.80 -> 2.83 ms)
+					__builtin_amdgcn_sched_barrier(0);
 				}
 		} else {
 			constexpr bool ACCUM = EPI == EPI_F32_ACC || EPI == EPI_F32_ACC_SCALE;
