@@ -26,6 +26,7 @@ _SIGNATURES = {
 	"elf_norm_bwd_workspace_floats": (c_int64, [c_int, c_int]),
 	"elf_norm_bwd": (c_int, [c_int, _P, _P, _P, _P, _P, _P, _P, _P, _P, c_int, c_int, _P]),
 	"elf_gemm_rope_bf16": (c_int, [c_int, c_int, c_int, _P, c_int64, _P, c_int64, _P, c_int64, _P, c_int, c_int, c_int, _P]),
+	"elf_gemm_gelu_bwd_bf16": (c_int, [c_int, c_int, c_int, _P, _P, _P, _P, _P, _P]),
 	"elf_gemm_way": (c_int, [c_int] * 5),
 	"elf_colsum_workspace_floats": (c_int64, [c_int64, c_int]),
 	"elf_colsum_bf16": (c_int, [_P, c_int64, _P, c_int64, c_int, _P, _P]),

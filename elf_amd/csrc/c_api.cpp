@@ -38,6 +38,11 @@ int elf_gemm_swiglu_bwd_bf16(int M, int F, int K, const void* dY, int64_t lddy, 
 	return elf::gemm_swiglu_bwd_bf16(M, F, K, dY, lddy, W, ldw, gu, ldgu, dgu, lddgu, scratch, (hipStream_t)stream);
 }
 
+int elf_gemm_gelu_bwd_bf16(int M, int F, int K, const void* dY, const void* W, const void* pre, void* dpre, void* scratch, void* stream) {
+	ELF_REQUIRE(scratch, "gemm_gelu_bwd: a scratch buffer of M x F bf16 is needed");
+	return elf::gemm_gelu_bwd_bf16(M, F, K, dY, W, pre, dpre, scratch, (hipStream_t)stream);
+}
+
 #define S_(x) ((hipStream_t)(x))
 int elf_gemm_rope_bf16(int M, int N, int K, const void* A, int64_t lda, const void* W, int64_t ldw, void* C, int64_t ldc, const void* cs, int S,
                        int n_rot_heads, int D, void* stream) {

@@ -339,8 +339,9 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 	// the queue for ~1000 cycles with its MFMAs behind it.  With two waves per SIMD the wave also raises
 	// its issue priority for the length of the half-step: the one feeding the matrix pipe goes first.
 	// Reduction-major operands in this loop: the two transpose-read addresses of every fragment are computed
-	// once (k32 half 0 of stage 0); the k32 half and the stage are compile-time here (the loop is unrolled
-	// by two slices) and go into the instructions' offset fields, so the loop has no address arithmetic.
+	// once (k32 half 0 of stage 0); the k32 half and the stage are compile-time here (the loop is unrolled by
+	// PERIOD slices, three or six) and go into the instructions' offset fields.  Those hold 16 bits: stage 2 of B lies 64 and
+	// 80 KiB up and costs an add per read, a third of B's reads.
 	uint32_t ta[AT ? RF : 1][2], tb[BT ? 8 : 1][2];
 	{
 		if constexpr (AT)
@@ -667,8 +668,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_dma_kernel(Args g) {
 
 template <int NW, int RF, bool AT, bool BT, int EPI, bool EDGE>
 static int launch_sized(const Args& a, hipStream_t stream) {
-	// the ring + the target of the loads past the end of K (as many KiB as a wave issues loads per
-	// operand); the epilogue needs a 32 x 136 fp32 strip per wave
+	// the ring (the loads past the end of K go into its stages too) or, where that is more, the epilogue's 32 x 136 fp32 strip per wave
 	using Sh = Shape<NW, RF>;
 	constexpr int ring = Sh::RING_BYTES, epi = NW * 32 * 136 * 4;
 	constexpr int smem = ring > epi ? ring : epi;

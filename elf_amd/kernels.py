@@ -141,6 +141,36 @@ def gemm_swiglu_bwd(dy, w2, gu, fused=True):
 	return dgu
 
 
+def gemm_gelu_bwd(dy, w2, pre, fused=True):
+	"""dpre [M, F]: gradient of pre for d = dy @ w2 (dy [M, K], w2 [K, F]); ``fused=False`` forces the GEMM + activation-backward
+	pair (same bits)."""
+	for t, n in ((dy, "dy"), (w2, "w2"), (pre, "pre")):
+		_need(t, torch.bfloat16, "gemm_gelu_bwd." + n)
+		if not t.is_contiguous():
+			raise _lib.ElfStageError(f"gemm_gelu_bwd.{n}: must be dense")
+	M, K = dy.shape
+	F = w2.shape[1]
+	if w2.shape[0] != K or tuple(pre.shape) != (M, F):
+		raise _lib.ElfStageError(f"gemm_gelu_bwd: shapes {tuple(dy.shape)}, {tuple(w2.shape)}, {tuple(pre.shape)} do not fit")
+	if not fused:
+		return gelu_bwd(gemm(dy, w2, b_t=True), pre)
+	dpre = torch.empty_like(pre)
+	scratch = torch.empty_like(pre)
+	rc = _lib.load().elf_gemm_gelu_bwd_bf16(M, F, K, _ptr(dy), _ptr(w2), _ptr(pre), _ptr(dpre), _ptr(scratch), _stream())
+	_lib.check(rc, "elf_gemm_gelu_bwd_bf16")
+	return dpre
+
+
+# products of gemm_way
+WAY_FORWARD, WAY_INPUT_GRADIENT, WAY_GELU, WAY_SWIGLU, WAY_GELU_BWD, WAY_SWIGLU_BWD, WAY_ROPE = range(7)
+
+
+def gemm_way(product, M, N, K, D=64):
+	"""(rows, columns) of the tile that dense operands of a product take, (0, 0) where the epilogue's work is a pass of its own."""
+	way = _lib.load().elf_gemm_way(product, M, N, K, D)
+	return way >> 16, way & 0xFFFF
+
+
 def norm_fwd(kind, x, gamma, beta=None, eps=1e-5):
 	_need(x, torch.bfloat16, "norm.x")
 	T, d = x.shape

@@ -97,6 +97,10 @@ int elf_gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, 
  *           silu(gate) * up; no reference module for SwiGLU. */
 int elf_gemm_swiglu_bwd_bf16(int M, int F, int K, const void* dY, int64_t lddy, const void* W, int64_t ldw,
                              const void* gu, int64_t ldgu, void* dgu, int64_t lddgu, void* scratch, void* stream);
+/* The same for the GELU of a GPT block's MLP: dpre[M, F] = d gelu'(pre) for d = dY W, every buffer dense.  One kernel for the
+ * smallest products, else elf_gemm_bf16(0, 1, ...) into scratch [M, F] followed by elf_gelu_bwd.  Same bits either way.
+ * Replaces: LinearDX.backward of fc2 (elf/zb_utils.py:29-41) followed by autograd's backward of nn.GELU(). */
+int elf_gemm_gelu_bwd_bf16(int M, int F, int K, const void* dY, const void* W, const void* pre, void* dpre, void* scratch, void* stream);
 
 /* The attention block's packed q | k | v projection with the rotary embedding of its q and k heads:
  * C[M, N] = A W^T (A [M, K], W [N, K], both k contiguous) rounded to bf16, then the rotation of elf_rope_apply
@@ -110,8 +114,8 @@ int elf_gemm_rope_bf16(int M, int N, int K, const void* A, int64_t lda, const vo
                        const void* cs, int S, int n_rot_heads, int D, void* stream);
 /* Which way the calls above take with dense, aligned operands and no tile asked for: rows << 16 | columns of the tile, 0 where
  * the epilogue's work is a pass of its own (or a size is no multiple of 64).  product: 0 forward and 1 input gradient of
- * elf_gemm_bf16 (epilogues 0 and 1), 2 GELU and 3 SwiGLU of elf_gemm_act_bf16 (N = F), 4 the same choice for the GELU backward
- * inside a stage, 5 elf_gemm_swiglu_bwd_bf16 (N = F), 6 elf_gemm_rope_bf16 (heads of width D).  Host only; for tests and tuning, no
+ * elf_gemm_bf16 (epilogues 0 and 1), 2 GELU and 3 SwiGLU of elf_gemm_act_bf16 (N = F), 4 elf_gemm_gelu_bwd_bf16 and
+ * 5 elf_gemm_swiglu_bwd_bf16 (N = F), 6 elf_gemm_rope_bf16 (heads of width D).  Host only; for tests and tuning, no
  * counterpart in the reference. */
 int elf_gemm_way(int product, int M, int N, int K, int D);
 

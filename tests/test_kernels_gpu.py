@@ -126,12 +126,13 @@ def test_gemm_k_split_is_bit_reproducible(K, dims, ks):
 	assert ((runs[0] - one).norm() / one.norm()).item() <= 1e-5
 
 
-@pytest.mark.parametrize("shape", [(256, 256, 128), (512, 768, 256), (4096, 1280, 1152), (8192, 4096, 1024), (2048, 28672, 256)])
+@pytest.mark.parametrize("shape", [(256, 256, 128), (512, 768, 256), (4096, 1280, 1152), (8192, 4096, 1024), (2048, 28672, 256), (4352, 4352, 320), (4352, 8704, 448)])
 def test_persistent_forward_gemm_equals_the_tile_kernel_bit_for_bit(K, monkeypatch, shape):
 	"""Forward GEMMs on 256x256 tiles run as persistent workgroups that walk several tiles and store from registers
 	(operands swapped on the MFMA, permuted weight rows); the one-tile-per-workgroup kernel with its LDS-staged epilogue
 	(ELF_NO_PERSISTENT_GEMM=1) forms the same products in the same order: equal bits for every epilogue, from one tile
-	per workgroup (1, 6 tiles) to several with a ragged last round (80, 512, 896 tiles), also against fp32 torch."""
+	per workgroup (1, 6 tiles) to several with a ragged last round (80, 512, 896 tiles; 289 and 578 with an odd number of K slices: the
+	ring starts every other tile in its other half), also against fp32 torch."""
 	M, N, Kd = shape
 	a, w, r, bias = _randn(M, Kd, seed=61), _randn(N, Kd, seed=62, scale=0.05), _randn(M, N, seed=63), _randn(1, N, seed=64)
 	F = N // 2
@@ -199,9 +200,10 @@ def test_gemm_bits_do_not_depend_on_the_tile(K):
 
 @pytest.mark.parametrize("M,N,Kd", [(2112, 3968, 320), (2624, 4160, 320), (2624, 4160, 448), (4096, 3072, 2048), (896, 14336, 512)])
 def test_gemm_tiles_between_128_and_256_rows(K, M, N, Kd):
-	"""Sizes for which the tile rule takes 160, 192 and 224 rows (for one of the epilogues at least), with moved last tiles that end
-	inside a wave's 32-row strip, and fewer and more K slices than a turn of the ring: the bits of the 64x64 tile for every
-	epilogue (all tiles add the products in the same order), nothing written outside the output."""
+	"""Sizes around those of the tiles of 160, 192 and 224 rows (the last takes 256-row ones; which takes which is pinned in
+	test_gemm_every_epilogue_of_the_tiles_between_128_and_256_rows), with moved last tiles that end inside a wave's 32-row strip, and
+	fewer and more K slices than a turn of the ring: the bits of the 64x64 tile for every epilogue (all tiles add the products in
+	the same order), nothing written outside the output."""
 	a, w, r, bias = _randn(M, Kd, seed=71), _randn(N, Kd, seed=72, scale=0.05), _randn(M, N, seed=73), _randn(1, N, seed=74)
 	for kw, b in ((dict(), w), (dict(b_t=True), w.t().contiguous())):
 		want = K.gemm(a, b, tile_cfg=12, **kw)
@@ -218,6 +220,91 @@ def test_gemm_tiles_between_128_and_256_rows(K, M, N, Kd):
 		assert torch.equal(gu, K.gemm(a, w, tile_cfg=12)) and torch.equal(act, K.swiglu_fwd(gu))
 	g, wt = _randn(M, 2 * N, seed=75), w.t().contiguous()
 	assert torch.equal(K.gemm_swiglu_bwd(a, wt, g), K.gemm_swiglu_bwd(a, wt, g, fused=False))
+
+
+MID_TILES = [  # rows of the tile, product, M, N, K: moved last tiles in rows, in columns or both, 5, 7 and more K slices
+	*[(160, w, *s) for w in ("forward", "dx", "rope") for s in ((6592, 1088, 320), (6656, 1088, 448), (1216, 6656, 512))],
+	*[(192, w, *s) for w in ("forward", "dx", "rope") for s in ((6784, 1344, 320), (6784, 1344, 448), (1792, 5632, 512))],
+	*[(224, w, *s) for w in ("forward", "dx", "rope") for s in ((6976, 1600, 2048), (6976, 1600, 2112), (1984, 6144, 2048))],
+	(160, "swiglu", 576, 6592, 320), (160, "swiglu", 576, 6592, 448), (160, "swiglu", 576, 6656, 512),
+	(192, "swiglu", 832, 5440, 320), (192, "swiglu", 832, 5568, 448), (192, "swiglu", 704, 6656, 512),
+	(224, "swiglu", 832, 6592, 2048), (224, "swiglu", 832, 6592, 2112), (224, "swiglu", 832, 6656, 2048),
+	(160, "swiglu_bwd", 6784, 1088, 320), (160, "swiglu_bwd", 5504, 1344, 448), (160, "swiglu_bwd", 1216, 6656, 512),
+	(192, "swiglu_bwd", 6784, 1344, 320), (192, "swiglu_bwd", 6784, 1344, 448), (192, "swiglu_bwd", 1792, 5632, 512),
+	(224, "swiglu_bwd", 6976, 1600, 1088), (224, "swiglu_bwd", 4864, 2368, 1536), (224, "swiglu_bwd", 2368, 5120, 1088),
+]
+
+
+@pytest.mark.parametrize("rows,product,M,N,Kd", MID_TILES)
+def test_gemm_every_epilogue_of_the_tiles_between_128_and_256_rows(K, rows, product, M, N, Kd):
+	"""Every epilogue on tiles of 160, 192 and 224 rows (the rule is asked first whether the size goes there): the bits of the
+	64x64 tile followed by the pass of its own, nothing written outside a plain output."""
+	D = 128 if N % 128 == 0 else 64
+	way = {"forward": K.WAY_FORWARD, "dx": K.WAY_INPUT_GRADIENT, "rope": K.WAY_ROPE, "swiglu": K.WAY_SWIGLU, "swiglu_bwd": K.WAY_SWIGLU_BWD}[product]
+	assert K.gemm_way(way, M, N, Kd, D) == (rows, 256)
+	a, w = _randn(M, Kd, seed=76), _randn(2 * N if product == "swiglu" else N, Kd, seed=77, scale=0.05)
+	if product in ("forward", "dx"):
+		kw, b = (dict(), w) if product == "forward" else (dict(b_t=True), w.t().contiguous())
+		big = torch.full((M + 64, N + 64), 7.0, dtype=torch.bfloat16, device="cuda")
+		K.gemm(a, b, out=big[:M, :N], **kw)
+		assert torch.equal(big[:M, :N], K.gemm(a, b, tile_cfg=12, **kw)) and (big[M:] == 7).all() and (big[:, N:] == 7).all()
+		for res in (dict(residual=_randn(M, N, seed=78)), dict(residual=_randn(1, N, seed=79), residual_ld=0)):
+			assert torch.equal(K.gemm(a, b, epilogue=K.EPI_BF16_RESID, **res, **kw), K.gemm(a, b, epilogue=K.EPI_BF16_RESID, tile_cfg=12, **res, **kw))
+	elif product == "rope":
+		cs, n_rot = K.rope_table(64, D, 5e5), N // D // 2
+		assert torch.equal(K.gemm_rope(a, w, cs, 64, n_rot, D), K.rope_apply_(K.gemm(a, w, tile_cfg=12), cs, 64, n_rot, D))
+	elif product == "swiglu":
+		gu, act = K.gemm_act(a, w, K.ACT_SWIGLU)
+		assert torch.equal(gu, K.gemm(a, w, tile_cfg=12)) and torch.equal(act, K.swiglu_fwd(gu))
+	else:
+		g, wt = _randn(M, 2 * N, seed=75), w.t().contiguous()
+		assert torch.equal(K.gemm_swiglu_bwd(a, wt, g), K.swiglu_bwd(K.gemm(a, wt, b_t=True, tile_cfg=12), g))
+
+
+def _guarded(*shape):
+	"""A dense bf16 tensor with 4096 marked elements before and behind it, and the whole."""
+	n = int(torch.Size(shape).numel())
+	whole = torch.full((n + 8192,), 7.0, dtype=torch.bfloat16, device="cuda")
+	return whole[4096 : 4096 + n].view(*shape), whole
+
+
+@pytest.mark.parametrize("M,F,Kd", [(64, 64, 256), (64, 192, 320), (512, 1024, 256), (512, 768, 512), (320, 448, 1088)])
+def test_epilogues_of_the_64x64_tile(K, M, F, Kd):
+	"""The activations, their backwards and the rotary embedding on 64x64 tiles (the rule is asked first), on the ring of two slices (K = 256)
+	and with fewer and more slices than the long one holds: the bits of the product followed by the pass of its own, nothing
+	written before or behind an output."""
+	from elf_amd import _lib
+
+	lib, p, st = _lib.load(), lambda t: t.data_ptr(), _lib.raw_stream()
+	a, w, w2, wt = _randn(M, Kd, seed=81), _randn(F, Kd, seed=82, scale=0.1), _randn(2 * F, Kd, seed=83, scale=0.1), _randn(Kd, F, seed=85, scale=0.1)
+	for way, n in ((K.WAY_GELU, F), (K.WAY_GELU_BWD, F), (K.WAY_SWIGLU, F), (K.WAY_SWIGLU_BWD, F), (K.WAY_ROPE, 2 * F)):
+		assert K.gemm_way(way, M, n, Kd) == (64, 64), way
+	plain, d = K.gemm(a, w, tile_cfg=12), K.gemm(a, wt, b_t=True, tile_cfg=12)
+	pre, gu = _randn(M, F, seed=86), _randn(M, 2 * F, seed=84)
+
+	def check(outs, want, call):
+		views, wholes = zip(*[_guarded(*o) for o in outs])
+		_lib.check(call(*views), "call")
+		for v, whole, x in zip(views, wholes, want):
+			assert torch.equal(v, x)
+			assert (whole[:4096] == 7).all() and (whole[-4096:] == 7).all()
+
+	check([(M, F), (M, F)], [plain, K.gelu_fwd(plain)], lambda o, o2: lib.elf_gemm_act_bf16(K.ACT_GELU, M, F, Kd, p(a), Kd, p(w), Kd, p(o), F, p(o2), F, st))
+	plain2 = K.gemm(a, w2, tile_cfg=12)
+	check([(M, 2 * F), (M, F)], [plain2, K.swiglu_fwd(plain2)], lambda o, o2: lib.elf_gemm_act_bf16(K.ACT_SWIGLU, M, F, Kd, p(a), Kd, p(w2), Kd, p(o), 2 * F, p(o2), F, st))
+	scratch = torch.empty_like(pre)
+	check([(M, F)], [K.gelu_bwd(d, pre)], lambda o: lib.elf_gemm_gelu_bwd_bf16(M, F, Kd, p(a), p(wt), p(pre), p(o), p(scratch), st))
+	check([(M, 2 * F)], [K.swiglu_bwd(d, gu)], lambda o: lib.elf_gemm_swiglu_bwd_bf16(M, F, Kd, p(a), Kd, p(wt), F, p(gu), 2 * F, p(o), 2 * F, p(scratch), st))
+	cs, heads = K.rope_table(64, 64, 5e5), 2 * F // 64
+	want = K.rope_apply_(plain2.clone(), cs, 64, heads // 2, 64)
+	check([(M, 2 * F)], [want], lambda o: lib.elf_gemm_rope_bf16(M, 2 * F, Kd, p(a), Kd, p(w2), Kd, p(o), 2 * F, p(cs), 64, heads // 2, 64, st))
+
+
+@pytest.mark.parametrize("M,F,Kd", [(256, 512, 64), (1024, 4096, 512), (2048, 3072, 768)])
+def test_gelu_backward_of_larger_products_is_a_pass_of_its_own(K, M, F, Kd):
+	dy, w2, pre = _randn(M, Kd, seed=87), _randn(Kd, F, seed=88, scale=0.1), _randn(M, F, seed=89)
+	assert K.gemm_way(K.WAY_GELU_BWD, M, F, Kd) == (0, 0)
+	assert torch.equal(K.gemm_gelu_bwd(dy, w2, pre), K.gemm_gelu_bwd(dy, w2, pre, fused=False))
 
 
 @pytest.mark.parametrize("M,F,Kd", [(64, 64, 256), (128, 192, 320), (512, 768, 512), (1024, 640, 256), (320, 448, 1088)])
