@@ -53,7 +53,8 @@ int gemm_turn_giveups(uint64_t* out) {
 // 160-row tiles fetch 30 % more operand bytes a product than 256-row ones (192: 17 %), which a stream at the power limit pays for in
 // its other kernels.  For K of at most 1024 they are taken where the launch is one round: with the QKV product on 468 of them
 // (39.0 us alone) a GPT-2-small stage took 8.06 ms where it takes 7.97 with 192 rows, on boxes that clock low; 7.69 and 7.70 on others.
-// For a longer K 192 rows take 5 to 10 % longer, and a Llama-3-8B block of 2688 tokens is as fast with either.
+// For a longer K 192 rows take 5 to 10 % longer, and a Llama-3-8B block of 2688 tokens is as fast with either; with the rotary or SwiGLU
+// epilogue the other tiles cost a stage more than that (three Llama blocks of 512 over 2 x 7680 tokens 7.31 ms, 7.35 with 256 rows).
 struct TileTime {
 	int bm, bn;
 	float slice, round, launch;
@@ -99,7 +100,7 @@ static Plan plan_tiles(int M, int N, int K, bool mid = true, float ring_extra = 
 	for (const TileTime& t : TILES_BF16) weigh(t);
 	if (mid)
 		for (const TileTime& t : TILES_MID)
-			if (t.bm > 160 || K > 1024 || (int64_t)((M + 159) / 160) * ((N + 255) / 256) <= 256) weigh(t);
+			if (t.bm > 160 || K > 1024 || epi_extra > 0.f || (int64_t)((M + 159) / 160) * ((N + 255) / 256) <= 256) weigh(t);
 	return best;
 }
 

@@ -126,17 +126,19 @@ def test_gemm_refuses_rows_too_far_apart_for_its_offsets(lib):
 
 
 def test_gemm_of_short_reductions_takes_tiles_of_160_rows_for_a_single_round_only(lib):
-	"""The QKV product of a GPT-2-small stage (8192 x 2304 x 768), 468 tiles of 160 rows, is on 192; 1920 x 4800 x 1600, 228 of them, stays.
-	Over several rounds no product with K of at most 1024 takes them, longer ones do."""
+	"""The QKV product of a GPT-2-small stage (8192 x 2304 x 768), 468 tiles of 160 rows, is on 192; 1920 x 4800 x 1600, 228 of them, stays,
+	and so does the SwiGLU product 15360 x 2 * 1664 x 512.  Over several rounds no plain product with K of at most 1024 takes them;
+	longer ones and those with an epilogue (3 SwiGLU, 6 RoPE) do."""
 	assert lib.elf_gemm_way(0, 8192, 2304, 768, 0) == 192 << 16 | 256
 	assert lib.elf_gemm_way(0, 1920, 4800, 1600, 0) == 160 << 16 | 256
+	assert lib.elf_gemm_way(3, 15360, 1664, 512, 0) == 160 << 16 | 256
 	rng, seen = random.Random(3), set()
 	for _ in range(8000):
 		M, N, K = (64 * int(2 ** rng.uniform(0, 7.5)) for _ in range(3))
 		for product, cols in ((0, N), (1, N), (3, 2 * N), (6, N)):
 			if lib.elf_gemm_way(product, M, N, K, 64) >> 16 == 160:
 				seen.add((product, K <= 1024, -(-M // 160) * -(-cols // 256) <= 256))
-	assert seen == {(p, short, one) for p in (0, 1, 3, 6) for short in (False, True) for one in (False, True) if one or not short}
+	assert seen == {(p, short, one) for p in (0, 1, 3, 6) for short in (False, True) for one in (False, True) if one or p > 1 or not short}
 
 
 def test_stage_create_rejects_bad_configs(lib):
