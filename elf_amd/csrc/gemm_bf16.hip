@@ -52,7 +52,7 @@ int gemm_turn_giveups(uint64_t* out) {
 //   tiles of 256 rows, 117 on 484 of 192; 1920 x 1600 x 1600 stays on 195 tiles of 128x128 (14.6; 24 on 84 of 160 rows).
 // 160-row tiles fetch 30 % more operand bytes a product than 256-row ones (192: 17 %), which a stream at the power limit pays for in
 // its other kernels.  For K of at most 1024 they are taken where the launch is one round: with the QKV product on 468 of them
-// (39.0 us alone) a GPT-2-small stage took 8.06 ms where it takes 7.97 with 192 rows, on boxes that clock low; 7.69 and 7.70 on others.
+// (39.0 us alone) a GPT-2-small stage took 8.06 ms where it takes 7.97 with 192 rows, on parts that clock low; 7.69 and 7.70 on others.
 // For a longer K 192 rows take 5 to 10 % longer, and a Llama-3-8B block of 2688 tokens is as fast with either; with the rotary or SwiGLU
 // epilogue the other tiles cost a stage more than that (three Llama blocks of 512 over 2 x 7680 tokens 7.31 ms, 7.35 with 256 rows).
 struct TileTime {
