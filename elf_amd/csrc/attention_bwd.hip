@@ -1,15 +1,15 @@
 // Attention backward kernels (see attention_common.h for the layout conventions).
-#include "attention_common.h"
+#include "attention_bwd_common.h"
 #include <type_traits>
 
 namespace elf {
 namespace attn {
 
 // ------------------------------------------------------------------------------------------
-// delta[b,h,s] = sum_d dO * O and nlse2[b,h,s] = -lse * log2(e).  D/8 lanes share one (token, head)
+// ndelta[b,h,s] = -sum_d dO * O and nlse2[b,h,s] = -lse * log2(e).  D/8 lanes share one (token, head)
 // row, 16 bytes each, so a wave covers 4 (D = 128) or 8 (D = 64) rows per step.
 __global__ __launch_bounds__(256) void attn_delta_kernel(const bf16_t* __restrict__ dO, const bf16_t* __restrict__ O,
-                                                         const float* __restrict__ lse, float* __restrict__ delta,
+                                                         const float* __restrict__ lse, float* __restrict__ ndelta,
                                                          float* __restrict__ nlse2, int64_t ldd, int64_t ldo, int B, int S,
                                                          int Hq, int D) {
 	const int lpr = D / 8;  // lanes per row: 8 or 16
@@ -27,199 +27,8 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(const bf16_t* __restric
 		for (int o = lpr >> 1; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
 		if (sub == 0) {
 			const int64_t b = tok / S, sp = tok % S;
-			delta[(b * Hq + h) * S + sp] = s;
+			ndelta[(b * Hq + h) * S + sp] = -s;
 			nlse2[(b * Hq + h) * S + sp] = -lse[(b * Hq + h) * S + sp] * LOG2E;
-		}
-	}
-}
-
-struct AttnBwdArgs {
-	const bf16_t* q;
-	const bf16_t* k;
-	const bf16_t* v;
-	const bf16_t* dO;
-	const float* nlse2;  // -lse * log2(e)
-	const float* delta;
-	bf16_t* dq_part;  // per key tile partial dQ, see part_row0()
-	bf16_t* dk;
-	bf16_t* dv;
-	int64_t ldq, ldk, ldv, lddo, lddk, lddv;
-	int B, S, Hq, Hkv;
-	float scale;
-	// non-null: the q and k heads carry a rotary embedding whose backward (the inverse rotation) is applied to
-	// dQ and dK before they are stored; (cos, sin) table [S, D / 2] of rope_table()
-	const float2* rope_cs;
-	// A pass's walk (query heads of the group x query tiles) shared by h_splits x q_splits workgroups, each of which leaves its
-	// dK and dV as fp32 partial sums in dkv_part ([split][dK, dV][token][Hkv * D]) for the reduction kernel; 1 x 1: they are
-	// stored as they are.  See split_walk().
-	int h_splits, q_splits;
-	float* dkv_part;
-	int paired;  // causal: a workgroup takes two key tiles one after the other (see attn_bwd_kernel); 0: one
-};
-
-// The walk of one workgroup: query heads [h0, h0 + nh) and, per head, query tiles [q_lo, q_hi) of a pass.
-struct Walk {
-	int pair, b, hk, split, h0, nh;
-	__device__ __forceinline__ void tiles(const AttnBwdArgs& a, int qt_first, int nqt, int& q_lo, int& q_hi) const {
-		const int qs = split % a.q_splits, len = nqt - qt_first;
-		q_lo = qt_first + len * qs / a.q_splits;
-		q_hi = qt_first + len * (qs + 1) / a.q_splits;
-	}
-};
-__device__ __forceinline__ Walk locate_walk(const AttnBwdArgs& a, int npair) {
-	const int ns = a.h_splits * a.q_splits, per_group = npair * ns;
-	int rest = blockIdx.x % per_group, bh = blockIdx.x / per_group;
-	// all workgroups of a (batch, kv head) group on one XCD (workgroup w runs on XCD w % 8)
-	const int ngroups = (int)(gridDim.x / per_group);
-	if (ngroups % 8 == 0) {
-		const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-		bh = xcd + 8 * (slot / per_group);
-		rest = slot % per_group;
-	}
-	Walk w;
-	w.split = rest % ns;
-	w.pair = rest / ns;
-	w.hk = bh % a.Hkv, w.b = bh / a.Hkv;
-	w.nh = a.Hq / a.Hkv / a.h_splits;
-	w.h0 = w.hk * (a.Hq / a.Hkv) + (w.split / a.q_splits) * w.nh;
-	return w;
-}
-
-// dQ partials.  Every 128-key tile contributes a [queries, Hq*D] partial dQ; the partials are written
-// with plain stores, each by exactly one workgroup, rounded to bf16 (like the P and dS operands of the
-// products they come from), and summed in fp32 in a fixed order by dq_reduce_kernel: no atomics, no
-// zero fill, and a result that does not depend on the order in which workgroups run.  (Adding the
-// tiles into one fp32 buffer with atomics costs a read-modify-write of a line that is never cache
-// resident per 32 lanes: 0.3 T lanes/s chip-wide, 0.68 of 1.81 ms at the Llama-3-8B shape.)
-// Layout per batch element: the slices of the key tiles one after the other; with a causal mask
-// slice kt only holds the queries q >= 128 kt, so it starts at row kt S - 128 kt (kt - 1) / 2 and
-// its row index is q - 128 kt.
-__host__ __device__ __forceinline__ int64_t part_row0(int kt, int S, bool causal) {
-	return causal ? (int64_t)kt * S - 64 * (int64_t)kt * (kt - 1) : (int64_t)kt * S;
-}
-__host__ __device__ __forceinline__ int64_t part_rows(int S, bool causal) { return part_row0(S / 128, S, causal); }
-
-// Tiles fetched straight into LDS (lds_dma.h) are unpadded; the 16-byte chunk index of a row is
-// XOR-swizzled with a function of the row chosen so that both access patterns are conflict
-// free: row-wise fragment reads (16 consecutive rows, same chunk) and transpose reads (a
-// half-wave takes 64 contiguous bytes from each of 4 consecutive rows).
-template <int D>
-struct BwdTile {
-	static constexpr int ROW_BYTES = D * 2;
-	static constexpr int CPR = D / 8;             // 16-byte chunks per row
-	static constexpr int RPI = 1024 / ROW_BYTES;  // rows per DMA wave instruction
-	__device__ static __forceinline__ int swz(int row) {
-		// D = 128 (16 chunks per row, a row spans all banks): bits [3:2] from row % 4 put four consecutive
-		// rows into four different 64-byte bank groups, bits [1:0] from row / 4 make 16 consecutive rows
-		// distinct.  D = 64 (8 chunks, two rows span all banks): the same for row pairs, bit-reversed.
-		return D == 128 ? (((row & 3) << 2) | ((row >> 2) & 3)) : ((((row >> 1) & 1) << 2) | (((row >> 2) & 1) << 1) | ((row >> 3) & 1));
-	}
-	// row-wise operand: rows row0 + lane%32, 8 consecutive columns from 16*ks + 8*(lane/32)
-	__device__ static __forceinline__ bf16x8 rows(const unsigned char* t, int row0, int ks, int lane) {
-		const int r = row0 + (lane & 31);
-		return *reinterpret_cast<const bf16x8*>(t + r * ROW_BYTES + (((2 * ks + (lane >> 5)) ^ swz(r)) << 4));
-	}
-	// transposed operand: column m0 + lane%32 at the rows {kA..kA+3, kA+second..+3}, kA = k0 + 4*(lane/32)
-	// (second = 8: accumulator row order) or kA = k0 + 8*(lane/32) (second = 4: natural order)
-	template <bool ACC_ORDER>
-	__device__ static __forceinline__ bf16x8 cols(const unsigned char* t, int k0, int m0, int lane) {
-		const int j = lane & 15;
-		const int kk = k0 + (ACC_ORDER ? 4 : 8) * (lane >> 5) + (j >> 2);
-		const int k2 = kk + (ACC_ORDER ? 8 : 4);
-		const int c = (m0 + 16 * ((lane & 31) >> 4) + 4 * (j & 3)) >> 3;
-		const unsigned char* p0 = t + kk * ROW_BYTES + ((c ^ swz(kk)) << 4) + (j & 1) * 8;
-		const unsigned char* p1 = t + k2 * ROW_BYTES + ((c ^ swz(k2)) << 4) + (j & 1) * 8;
-		s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 ELF_LDS*)(p0));
-		s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 ELF_LDS*)(p1));
-		return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-	}
-};
-
-// 4 bytes per lane from a per-lane global address to LDS at lds_byte_addr + lane * 4.
-__device__ __forceinline__ void dma4(const void* lane_addr, uint32_t lds_byte_addr) {
-	asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_byte_addr), "v"(lane_addr) : "memory", "m0");
-}
-
-// dS^T tile in LDS: [key][q] bf16 with 64-byte rows (32 queries); the 16-byte chunk index is
-// XOR-swizzled with (key >> 2) & 3 so that the 8-byte accumulator writes of 32 consecutive keys
-// and the transpose reads of 4 consecutive keys both spread over all banks.
-__device__ __forceinline__ int ds_t_offset(int key, int q) {  // q a multiple of 4
-	return key * 64 + (((q >> 3) ^ ((key >> 2) & 3)) << 4) + ((q >> 2) & 1) * 8;
-}
-// A operand from the dS^T tile: row q = lane%32, keys k0 + 8*(lane/32) .. +7
-__device__ __forceinline__ bf16x8 ds_t_frag(const unsigned char* t, int k0, int lane) {
-	const int j = lane & 15;
-	const int kk = k0 + 8 * (lane >> 5) + (j >> 2);
-	const int q = 16 * ((lane & 31) >> 4) + 4 * (j & 3);
-	s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 ELF_LDS*)(t + ds_t_offset(kk, q)));
-	s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 ELF_LDS*)(t + ds_t_offset(kk + 4, q)));
-	return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-}
-
-// dK^T / dV^T accumulators of one wave -> memory: register r of tile dt <-> d = dt*32 + (r/4)*8 + 4g + r%4, lane <-> key.
-// With a rotary embedding on the k heads, dK (scaled and rounded to bf16, as a separate RoPE pass over the stored
-// gradient would read it) is rotated back first; the partner of column d is d + D/2, same register of tile dt + DT/2.
-template <int D>
-__device__ __forceinline__ void store_dk_dv(const f32x16 (&acc_dk)[D / 32], const f32x16 (&acc_dv)[D / 32], bf16_t* dkp, bf16_t* dvp, float scale, int g,
-                                            const float2* cs_row) {
-	constexpr int DT = D / 32;
-#pragma unroll
-	for (int dt = 0; dt < DT; dt++) {
-#pragma unroll
-		for (int r4 = 0; r4 < 4; r4++) {
-			bf16x4 v4;
-#pragma unroll
-			for (int u = 0; u < 4; u++) v4[u] = (bf16_t)acc_dv[dt][r4 * 4 + u];
-			*reinterpret_cast<bf16x4*>(dvp + dt * 32 + r4 * 8 + 4 * g) = v4;
-		}
-	}
-	if (cs_row == nullptr) {
-#pragma unroll
-		for (int dt = 0; dt < DT; dt++) {
-#pragma unroll
-			for (int r4 = 0; r4 < 4; r4++) {
-				bf16x4 k4;
-#pragma unroll
-				for (int u = 0; u < 4; u++) k4[u] = (bf16_t)(acc_dk[dt][r4 * 4 + u] * scale);
-				*reinterpret_cast<bf16x4*>(dkp + dt * 32 + r4 * 8 + 4 * g) = k4;
-			}
-		}
-		return;
-	}
-#pragma unroll
-	for (int dt = 0; dt < DT / 2; dt++) {
-#pragma unroll
-		for (int r4 = 0; r4 < 4; r4++) {
-			const int i = dt * 32 + r4 * 8 + 4 * g;
-			const f32x4 t0 = *reinterpret_cast<const f32x4*>(cs_row + i), t1 = *reinterpret_cast<const f32x4*>(cs_row + i + 2);
-			bf16x4 lo4, hi4;
-#pragma unroll
-			for (int u = 0; u < 4; u++) {
-				const float lo = (float)(bf16_t)(acc_dk[dt][r4 * 4 + u] * scale), hi = (float)(bf16_t)(acc_dk[dt + DT / 2][r4 * 4 + u] * scale);
-				const float c = (u < 2 ? t0 : t1)[(u & 1) * 2], sn = (u < 2 ? t0 : t1)[(u & 1) * 2 + 1];
-				float rl, rh;
-				rope_rot(lo, hi, c, -sn, rl, rh);
-				lo4[u] = (bf16_t)rl;
-				hi4[u] = (bf16_t)rh;
-			}
-			*reinterpret_cast<bf16x4*>(dkp + i) = lo4;
-			*reinterpret_cast<bf16x4*>(dkp + i + D / 2) = hi4;
-		}
-	}
-}
-
-// The same accumulators as fp32 partial sums: dK at p, dV `stride` floats further on.
-template <int D>
-__device__ __forceinline__ void store_dkv_part(const f32x16 (&acc_dk)[D / 32], const f32x16 (&acc_dv)[D / 32], float* p, int64_t stride, int g) {
-#pragma unroll
-	for (int dt = 0; dt < D / 32; dt++) {
-#pragma unroll
-		for (int r4 = 0; r4 < 4; r4++) {
-			f32x4 k4, v4;
-#pragma unroll
-			for (int u = 0; u < 4; u++) k4[u] = acc_dk[dt][r4 * 4 + u], v4[u] = acc_dv[dt][r4 * 4 + u];
-			*reinterpret_cast<f32x4*>(p + dt * 32 + r4 * 8 + 4 * g) = k4;
-			*reinterpret_cast<f32x4*>(p + stride + dt * 32 + r4 * 8 + 4 * g) = v4;
 		}
 	}
 }
@@ -234,9 +43,10 @@ __device__ __forceinline__ void store_dkv_part(const f32x16 (&acc_dk)[D / 32], c
 // by its slice of K (held in registers as B operands) to get its slice of the dQ tile.  That
 // product runs one tile behind, so a tile costs one barrier; the slice goes to this key tile's
 // partial dQ buffer (bf16).  The softmax scale of dK and dQ is applied by the epilogue / the
-// reduction kernel.  With a causal mask key tile kt meets 1 - kt/nkt of the query tiles, so
-// a workgroup takes the tiles kt and nkt-1-kt one after the other: every workgroup then does
-// the same amount of work.  (Where there are workgroups to spare each takes one tile: split_walk().)
+// reduction kernel.  With a causal mask key tile kt meets 1 - kt/nkt of the query tiles: a workgroup
+// takes one tile, or (a.paired) the tiles kt and nkt-1-kt one after the other, which is the same work
+// for every workgroup: see split_walk().
+// Heads of 64 columns come here where passes over 256 keys (attention_bwd_wide.hip) do not pay.
 template <int D, bool CAUSAL>
 __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kernel(AttnBwdArgs a) {
 	using TL = BwdTile<D>;
@@ -245,7 +55,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kernel(AttnBwdA
 	constexpr int DT = D / 32;
 	constexpr int NQ = BKV / 16;  // fragments of the dQ product (all 128 keys); waves 0..DT-1 own one 32-column slice each
 	constexpr int K_BYTES = BKV * TL::ROW_BYTES, Q_BYTES = BQ * TL::ROW_BYTES;
-	constexpr int STAGE = 2 * Q_BYTES + 256;  // Q tile, dO tile, 32 nlse2 + 32 delta floats
+	constexpr int STAGE = 2 * Q_BYTES + 256;  // Q tile, dO tile, 32 nlse2 + 32 -delta floats
 	constexpr int DS_BYTES = BKV * BQ * 2;
 	constexpr int Q_LOADS = 8 / TL::RPI;  // DMA instructions per wave and tile (8 rows per wave)
 	extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
@@ -258,7 +68,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kernel(AttnBwdA
 	const int g = lane >> 5, kl = lane & 31;
 	const int nkt = a.S / BKV;
 	const int npair = CAUSAL && a.paired ? (nkt + 1) / 2 : nkt;
-	const Walk wk = locate_walk(a, npair);
+	const Walk wk = locate_walk(a, npair, CAUSAL);
 	const int pair = wk.pair, hk = wk.hk, b = wk.b;
 	const int64_t tok0 = (int64_t)b * a.S;
 	const int64_t HqD = (int64_t)a.Hq * D;
@@ -345,12 +155,12 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kernel(AttnBwdA
 		int ld_h = wk.h0, ld_qt = q_lo;
 		const bf16_t* ld_q;
 		const bf16_t* ld_do;
-		const float* ld_stat;  // lanes 0..31: nlse2 of the tile's queries, lanes 32..63: delta
+		const float* ld_stat;  // lanes 0..31: nlse2 of the tile's queries, lanes 32..63: -delta
 		auto seek = [&]() {
 			const int64_t row = tok0 + ld_qt * BQ;
 			ld_q = a.q + row * a.ldq + ld_h * D;
 			ld_do = a.dO + row * a.lddo + ld_h * D;
-			ld_stat = (lane < 32 ? a.nlse2 : a.delta) + ((int64_t)b * a.Hq + ld_h) * a.S + ld_qt * BQ + (lane & 31);
+			ld_stat = (lane < 32 ? a.nlse2 : a.ndelta) + ((int64_t)b * a.Hq + ld_h) * a.S + ld_qt * BQ + (lane & 31);
 		};
 		seek();
 		const uint32_t lds_stage = lds_addr(sStage) + wave * 8 * TL::ROW_BYTES;
@@ -385,7 +195,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kernel(AttnBwdA
 		// position of the current tile; dq_prev_tile = where the dQ tile of iteration it-1 goes
 		int cur_h = wk.h0, cur_qt = q_lo;
 		// rows of this key tile's slice: first query of the slice = key0 (causal) or 0
-		bf16_t* const part = a.dq_part + ((int64_t)b * part_rows(a.S, CAUSAL) + part_row0(kt_idx, a.S, CAUSAL) - qt_first * BQ) * HqD;
+		bf16_t* const part = a.dq_part + ((int64_t)b * part_rows(a.S, CAUSAL, BKV) + part_row0(kt_idx, a.S, CAUSAL, BKV) - qt_first * BQ) * HqD;
 		bf16_t* dq_prev_tile = part + (int64_t)(q_lo * BQ) * HqD + cur_h * D;
 
 		for (int it = 0; it < n_iter; it++) {
@@ -471,7 +281,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kernel(AttnBwdA
 			for (int r4 = 0; r4 < 4; r4++) {
 				const f32x4 d4 = *reinterpret_cast<const f32x4*>(sLse + 32 + r4 * 8 + 4 * g);
 #pragma unroll
-				for (int t = 0; t < 4; t++) ds[r4 * 4 + t] = p[r4 * 4 + t] * (dp[r4 * 4 + t] - d4[t]);
+				for (int t = 0; t < 4; t++) ds[r4 * 4 + t] = p[r4 * 4 + t] * (dp[r4 * 4 + t] + d4[t]);
 			}
 			const bf16x8 dsf[2] = {pack8(ds), pack8(ds + 8)};
 			// accumulator rows of register r: q = (r/4)*8 + 4g + r%4 -> four 8-byte groups per lane
@@ -526,8 +336,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void attn_bwd_kernel(AttnBwdA
 // register file).  Nothing else fills its issue gaps, so the schedule is explicit: Q / dO tiles in a three-stage
 // ring fetched two steps ahead, every fragment read issued one product ahead of its use into two buffers
 // that alternate roles, and every MFMA pinned between its share of the reads and of the vector work.
-// 2690 against 3650 cycles per tile; in the stream (between GEMMs) the call takes 1.04 against 1.13 ms.  At
-// head_dim 64 the plain kernel above keeps two waves per SIMD, which this schedule's live ranges would cost.
+// 2690 against 3650 cycles per tile; in the stream (between GEMMs) the call takes 1.04 against 1.13 ms.
 template <int D, bool CAUSAL>
 __global__ __launch_bounds__(256) void attn_bwd_kernel_lone(AttnBwdArgs a) {
 	using TL = BwdTile<D>;
@@ -536,7 +345,7 @@ __global__ __launch_bounds__(256) void attn_bwd_kernel_lone(AttnBwdArgs a) {
 	constexpr int DT = D / 32;
 	constexpr int NQ = BKV / 16;  // fragments of the dQ product (all 128 keys); waves 0..DT-1 own one 32-column slice each
 	constexpr int K_BYTES = BKV * TL::ROW_BYTES, Q_BYTES = BQ * TL::ROW_BYTES;
-	constexpr int STAGE = 2 * Q_BYTES + 256;  // Q tile, dO tile, 32 nlse2 + 32 delta floats
+	constexpr int STAGE = 2 * Q_BYTES + 256;  // Q tile, dO tile, 32 nlse2 + 32 -delta floats
 	constexpr int NSTAGE = 3;                 // tiles are fetched two steps ahead
 	constexpr int DS_BYTES = BKV * BQ * 2;
 	constexpr int Q_LOADS = 8 / TL::RPI;  // DMA instructions per wave and tile (8 rows per wave)
@@ -550,7 +359,7 @@ __global__ __launch_bounds__(256) void attn_bwd_kernel_lone(AttnBwdArgs a) {
 	const int g = lane >> 5, kl = lane & 31;
 	const int nkt = a.S / BKV;
 	const int npair = CAUSAL && a.paired ? (nkt + 1) / 2 : nkt;
-	const Walk wk = locate_walk(a, npair);
+	const Walk wk = locate_walk(a, npair, CAUSAL);
 	const int pair = wk.pair, hk = wk.hk, b = wk.b;
 	const int64_t tok0 = (int64_t)b * a.S;
 	const int64_t HqD = (int64_t)a.Hq * D;
@@ -633,12 +442,12 @@ __global__ __launch_bounds__(256) void attn_bwd_kernel_lone(AttnBwdArgs a) {
 		int ld_h = wk.h0, ld_qt = q_lo;
 		const bf16_t* ld_q;
 		const bf16_t* ld_do;
-		const float* ld_stat;  // lanes 0..31: nlse2 of the tile's queries, lanes 32..63: delta
+		const float* ld_stat;  // lanes 0..31: nlse2 of the tile's queries, lanes 32..63: -delta
 		auto seek = [&]() {
 			const int64_t row = tok0 + ld_qt * BQ;
 			ld_q = a.q + row * a.ldq + ld_h * D;
 			ld_do = a.dO + row * a.lddo + ld_h * D;
-			ld_stat = (lane < 32 ? a.nlse2 : a.delta) + ((int64_t)b * a.Hq + ld_h) * a.S + ld_qt * BQ + (lane & 31);
+			ld_stat = (lane < 32 ? a.nlse2 : a.ndelta) + ((int64_t)b * a.Hq + ld_h) * a.S + ld_qt * BQ + (lane & 31);
 		};
 		seek();
 		const uint32_t lds_stage = lds_addr(sStage) + wave * 8 * TL::ROW_BYTES;
@@ -674,7 +483,7 @@ __global__ __launch_bounds__(256) void attn_bwd_kernel_lone(AttnBwdArgs a) {
 		// position of the current tile; dq_prev_tile = where the dQ tile of iteration it-1 goes
 		int cur_h = wk.h0, cur_qt = q_lo;
 		// rows of this key tile's slice: first query of the slice = key0 (causal) or 0
-		bf16_t* const part = a.dq_part + ((int64_t)b * part_rows(a.S, CAUSAL) + part_row0(kt_idx, a.S, CAUSAL) - qt_first * BQ) * HqD;
+		bf16_t* const part = a.dq_part + ((int64_t)b * part_rows(a.S, CAUSAL, BKV) + part_row0(kt_idx, a.S, CAUSAL, BKV) - qt_first * BQ) * HqD;
 		bf16_t* dq_prev_tile = part + (int64_t)(q_lo * BQ) * HqD + cur_h * D;
 
 		// One step = one (head, 32-query tile).  Two fragment buffers alternate roles so that every LDS
@@ -769,7 +578,7 @@ __global__ __launch_bounds__(256) void attn_bwd_kernel_lone(AttnBwdArgs a) {
 				acc_dv[i % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(Y[i], pf[i / DT], acc_dv[i % DT], 0, 0, 0);
 				if (i < NF / 2) {
 #pragma unroll
-					for (int r = i * (32 / NF); r < (i + 1) * (32 / NF); r++) ds[r] = p[r] * (dp[r] - d4[r >> 2][r & 3]);
+					for (int r = i * (32 / NF); r < (i + 1) * (32 / NF); r++) ds[r] = p[r] * (dp[r] + d4[r >> 2][r & 3]);
 				} else if (i < NF / 2 + 2) {
 					// accumulator rows of register r: q = (r/4)*8 + 4g + r%4 -> four 8-byte groups per lane
 					const int u = i - NF / 2;
@@ -845,7 +654,7 @@ struct DkvReduce {
 	int splits, Hkv, blocks;
 };
 __global__ __launch_bounds__(256) void dq_reduce_kernel(const bf16_t* __restrict__ part, bf16_t* __restrict__ dq, int B, int S, int cols,
-                                                        int64_t ld, float scale, int causal, int D, const float2* __restrict__ cs, DkvReduce dkv) {
+                                                        int64_t ld, float scale, int causal, int keys, int D, const float2* __restrict__ cs, DkvReduce dkv) {
 	const int dq_blocks = (int)gridDim.x - dkv.blocks;
 	if ((int)blockIdx.x >= dq_blocks) {
 		const int half = D / 2, cph = half / 8, ppr = dkv.Hkv * cph;  // chunk pairs per row
@@ -886,8 +695,8 @@ __global__ __launch_bounds__(256) void dq_reduce_kernel(const bf16_t* __restrict
 	const int half = D / 2, cph = half / 8;  // 8-column chunks per half head
 	const int ppr = cols / 16;               // chunk pairs per row
 	const int64_t n = (int64_t)B * S * ppr;
-	const int nkt = S / 128;
-	const int64_t rows_b = part_rows(S, causal);
+	const int nkt = (S + keys - 1) / keys;
+	const int64_t rows_b = part_rows(S, causal, keys);
 	for (int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; j < n; j += (int64_t)dq_blocks * blockDim.x) {
 		// last rows first: under a causal mask they sum the most partials, and the launch then ends on the short ones
 		const int64_t i = n - 1 - j;
@@ -895,12 +704,12 @@ __global__ __launch_bounds__(256) void dq_reduce_kernel(const bf16_t* __restrict
 		const int pr = (int)(i - row * ppr);
 		const int c = (pr / cph) * D + (pr % cph) * 8;
 		const int b = (int)(row / S), q = (int)(row - (int64_t)b * S);
-		const int ns = causal ? q / 128 + 1 : nkt;
+		const int ns = causal ? q / keys + 1 : nkt;
 		float lo[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, hi[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 		const bf16_t* pb = part + (int64_t)b * rows_b * cols + c;
 #pragma unroll 8
 		for (int kt = 0; kt < ns; kt++) {
-			const bf16_t* pr_row = pb + (part_row0(kt, S, causal) + q - (causal ? 128 * kt : 0)) * cols;
+			const bf16_t* pr_row = pb + (part_row0(kt, S, causal, keys) + q - (causal ? keys * kt : 0)) * cols;
 			// read once: no point in keeping the partials in the caches
 			const bf16x8 v = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(pr_row)), w = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(pr_row + half));
 #pragma unroll
@@ -952,38 +761,31 @@ int launch_bwd(const AttnBwdArgs& a, dim3 grid, hipStream_t stream) {
 using namespace attn;
 
 // How the walks of a launch are shared out.  A workgroup's walk over the query heads of its group and their query tiles is
-// serial (one 32-query tile per step), and B * Hkv * (key tile pairs) walks leave the chip idle where there are few of them:
-// then the heads of a group and, after those, the query tiles are split, as long as the estimate gets smaller.  Steps and the
-// fixed part of a walk (K / V rows in, first tiles in, dK / dV out) are in microseconds as measured; a split adds
-// 16 bytes per element of dK to write and to read again.  The whole call, before -> after (us): 2 x 2048 tokens, 16 / 4 heads
-// of 128 346 -> 160 (64 walks, heads split 4 ways); 3 x 896, 32 / 8 heads of 128 189 -> 134 (2 ways); 4096 tokens, 6 / 1 heads
-// of 128 886 -> 125 (6 x 2); 2 x 1024, 16 / 4 heads of 64 196 -> 59 (4 x 2).  Full launches stay whole: 2 x 4096, 32 / 8 heads
-// of 128 takes 1000 us whole and 1030 in two.  Causal: where even the key tiles by themselves fit the chip at once a pair is
-// taken apart as well, which spares the chain the fixed part of its second tile and needs no partial sums.  The whole call, before
-// -> after (us): 2 x 256 tokens, 4 / 2 heads of 128 32.4 -> 22.5; 3 x 640, 25 heads of 64 63.9 -> 56.4; 4 x 512, 12 heads of 64
-// 48.9 -> 38.5; 896 tokens, 32 / 8 heads of 128 66.5 -> 60.9.
-// Causal with one key tile (128 tokens): a walk has four steps a head, what a step and a split cost beside the fixed part shows.
-// Constants of its own, fitted to every sharing of 250 such shapes (the one that is picked takes 0.2 % longer than the best on
-// average, 7 % at most; with those of longer walks 1.8 and 16 %).  The whole call, whole -> as shared now (us): 2 x 128 tokens, 4 heads of 64
-// 18.9 -> 16.7; 3 x 128, 48 / 16 heads of 128 34.8 -> 31.2; 7 x 128, 36 / 12 heads of 128 stay whole: 37.8, three ways 40.6.
+// serial (one 32-query tile per step), and B * Hkv * (key tiles) walks leave the chip idle where there are few of them: then the
+// heads of a group and, after those, the query tiles are split, as long as the estimate gets smaller.  A split adds fp32 partial
+// sums of dK and dV to write and to read again.  Causal: a workgroup takes one key tile (the long walks are dispatched first, see
+// locate_walk()) or a light and a heavy one, where these make whole rounds.
 struct Splits {
 	int h = 1, q = 1;
 	bool paired = true;
+	bool wide = false;  // passes over 256 keys (attention_bwd_wide.hip)
 };
 static int64_t dkv_part_bytes(const Splits& sp, int B, int S, int Hkv, int D) { return sp.h * sp.q > 1 ? (int64_t)sp.h * sp.q * 2 * B * S * Hkv * D * 4 : 0; }
-// room: bytes there are for the partial sums.  Splits are tried in ascending order of what they need, first of pairs and then of
-// single key tiles.
-static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal, int64_t room) {
+
+// Heads of 64 columns, short sequences in a launch that does not fill the chip: workgroups of 128 keys, two on a compute unit.
+// Constants in microseconds as measured.  Causal with one key tile (128 tokens): a walk has four steps a head, what a step and a
+// split cost beside the fixed part shows.  Constants of its own, fitted to every sharing of 250 such shapes (the one that is picked
+// takes 0.2 % longer than the best on average, 7 % at most; with those of longer walks 1.8 and 16 %).  The whole call, whole -> as
+// shared now (us): 2 x 128 tokens, 4 heads of 64 18.9 -> 16.7; 3 x 128, 48 / 16 heads of 128 34.8 -> 31.2; 7 x 128, 36 / 12 heads
+// of 128 stay whole: 37.8, three ways 40.6.
+static Splits split_short(int B, int S, int Hq, int Hkv, int D, bool causal, int64_t room) {
 	const int nkt = S / 128, G = Hq / Hkv;
 	const bool one = causal && nkt == 1;
 	const float slots = D == 128 ? 256.f : 512.f, step = one ? 1.6f : D == 128 ? 1.2f : 1.1f, fixed = 8.f;
 	// a split: what it adds by itself, per split, and the partial sums at so many bytes a us; it has to be that much better than less sharing
 	const float split = one ? 0.f : 2.f, per_split = one ? 0.4f : 0.f, rate = one ? 4e6f : 5e6f, margin = one ? 1.f : 0.95f;
 	Splits best;
-	// From 2^18 query rows (2 x 4096 tokens of 32 heads) up walks stay whole.  With eight kv heads or more and several sequences such
-	// launches fill the chip; one sequence of 4096 tokens with 64 / 8 heads (128 walks for 256 compute units) does not, and sharing
-	// has not been measured there.
-	if ((int64_t)B * S * Hq >= 1 << 18) return best;
+	if ((int64_t)B * S * Hq >= 1 << 18) return best;  // these fill the chip
 	float best_us = 1e30f;
 	bool shared_pairs = false;
 	for (int paired = 1; paired >= (causal && nkt > 1 ? 0 : 1); paired--) {
@@ -1003,11 +805,51 @@ static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal, int6
 				const float rounds = ceilf((float)(walks * ns) / slots);
 				if (!paired && rounds > 1.f) continue;
 				const float us = rounds * (fixed + (float)(G / h) * ((tiles + q - 1) / q) * step) + (ns > 1 ? split + ns * per_split + (float)ns * B * S * Hkv * D * 16 / rate : 0.f);
-				// Over 40 shapes that were shared as pairs a whole walk per tile is as fast where its estimate is 3 us above that of the
-				// shared pair, not 8.  Without this 8 x 1408 tokens, 6 / 2 heads of 128 took 187 us, 161 as pairs shared three ways;
-				// 10 x 512, 12 / 4 heads of 128 85.5 and 82.3.
 				const float lead = shared_pairs && ns == 1 ? fixed - 3.f : 0.f;
 				if (us + lead < best_us * (ns > 1 ? margin : 1.f)) best_us = us, best = Splits{h, q, paired != 0};
+			}
+		}
+	}
+	return best;
+}
+
+// room: bytes there are for the partial sums.
+//
+// One workgroup on a compute unit (heads of 128 columns, and of 64 on passes over 256 keys).  The longest walk, or the average filling of the
+// chip and half a walk's fixed part where there are several rounds; constants in microseconds fitted to every sharing of 189 shapes of heads of 128 and
+// 232 of 64 from 512 tokens up: what is picked takes 0.1 and 0.5 % longer than the best.  Against pairs of key tiles in any case but where all single
+// tiles fit the chip at once, and the 128-key kernel for heads of 64, these shapes take 0.96 and 0.80 of the time.  The whole call,
+// before -> after (us): 8 x 1408 tokens, 6 / 2 heads of 128 161 -> 140 (single tiles, heads split 3 ways); 3 x 896, 32 / 8 heads of 128 134 -> 118;
+// 4096 tokens, 64 / 8 heads of 128 1424 -> 1012 (128 whole pairs before, shared 2 ways now); 8 x 1024, 12 heads of 64 101 -> 65, not causal
+// 130 -> 103; 8192 tokens, 16 heads of 64 559 -> 360.  Pairs that make whole rounds stay: 4 x 4096, 32 / 8 heads of 128 2020, single tiles 2053.
+static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal, int64_t room) {
+	const int G = Hq / Hkv;
+	// Heads of 64 columns: a pass of 256 keys has twice the fixed part of one of 128.  Below 896 tokens it pays where there is work for the
+	// chip (heads x key tiles of 128), below 512 if the passes fit at once or the 128-key ones do not either (us, 128 and 256 keys): 3 x 384
+	// tokens, 31 heads, causal 40 and 33, 3 x 256, 16 heads 22 and 23, 5 x 384, 26 heads 42 and 57; 3 x 512, 8 heads 30 and 33, 16 heads
+	// 37 and 36; 512 tokens, 7 heads, causal 22 and 23, 2 x 512, 6 / 1 heads, causal 33 and 30.
+	const int64_t work = (int64_t)B * Hq * (S / 128), tiles128 = (int64_t)B * Hkv * (S / 128), tiles256 = (int64_t)B * Hkv * ((S + 255) / 256);
+	const bool wide = D == 64 && S >= 256 && (S >= 896 || (S >= 512 && work >= (causal ? 48 : 120)) || (work >= 256 && (tiles256 <= 256 || tiles128 > 512)));
+	if (S < 256 || (D == 64 && !wide)) return split_short(B, S, Hq, Hkv, D, causal, room);
+	const int keys = wide ? 256 : 128, n = (S + keys - 1) / keys, tile = keys / 32, Q = S / 32;  // key tiles; query tiles of a key tile, of a sequence
+	const float slots = 256.f, step = wide ? 1.f : 1.05f, fixed = wide ? 4.f : 9.f;
+	const float split = wide ? 0.4f : 1.4f, per_split = wide ? 0.3f : 0.35f, rate = wide ? 4.8e6f : 8.5e6f, margin = 0.96f;
+	Splits best;
+	float best_us = 1e30f;
+	for (int paired = 1; paired >= (causal && n > 1 ? 0 : 1); paired--) {
+		for (int h = 1; h <= G; h++) {
+			if (G % h) continue;
+			for (int q = 1; q <= 4; q *= 2) {
+				if (q > 1 && h < G) continue;
+				const int ns = h * q;
+				if (dkv_part_bytes(Splits{h, q}, B, S, Hkv, D) > room) continue;
+				const float walks = (float)B * Hkv * ns, per = (float)(G / h) / q * step;
+				float us;
+				if (causal && paired && n > 1) us = ceilf(walks * ((n + 1) / 2) / slots) * (2.f * fixed + per * (2 * Q - tile * (n - 1)));
+				else if (!causal || n == 1) us = ceilf(walks * n / slots) * (fixed + per * Q);
+				else us = fmaxf(fixed + per * Q, walks * n <= slots ? 0.f : walks * (n * fixed + per * ((float)n * Q - tile * 0.5f * n * (n - 1))) / slots + 0.5f * fixed);
+				if (ns > 1) us = (us + split + ns * per_split + (float)ns * B * S * Hkv * D * 16 / rate) / margin;
+				if (us < best_us) best_us = us, best = Splits{h, q, paired != 0, wide};
 			}
 		}
 	}
@@ -1017,7 +859,7 @@ static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal, int6
 // bf16 dQ partials of every key tile + delta + scaled log-sum-exp: what a backward whose walks stay whole needs.  It grows with
 // each of its arguments, so a buffer for the largest of a caller's shapes serves the smaller ones.
 int64_t attn_bwd_workspace_bytes(int B, int S, int Hq, int D, int causal) {
-	return (int64_t)B * part_rows(S, causal != 0) * Hq * D * 2 + 2 * (int64_t)B * S * Hq * 4;
+	return (int64_t)B * part_rows(S, causal != 0, 128) * Hq * D * 2 + 2 * (int64_t)B * S * Hq * 4;
 }
 
 // With the partial sums of the walks this shape shares: 2 x 2048 tokens, 16 / 4 heads of 128 143 + 67 MB; 2 x 4096, 32 / 8 heads
@@ -1047,22 +889,23 @@ int attn_bwd(const void* q, const void* k, const void* v, const void* o, const v
 	ProfScope prof(PROF_ATTN_BWD, (causal ? 4.0 : 8.0) * B * Hq * (double)S * S * D, stream);
 	const int64_t T = (int64_t)B * S;
 	bf16_t* dq_part = (bf16_t*)workspace;
-	float* delta = (float*)(dq_part + (int64_t)B * part_rows(S, causal != 0) * Hq * D);
-	float* nlse2 = delta + T * Hq;
+	float* ndelta = (float*)(dq_part + (int64_t)B * part_rows(S, causal != 0, 128) * Hq * D);
+	float* nlse2 = ndelta + T * Hq;
 	{
 		const int64_t rows = T * Hq, per_block = 256 / (D / 8);
 		const int64_t want = (rows + per_block - 1) / per_block;
 		ELF_LAUNCH(attn_delta_kernel, dim3((unsigned)(want < 8192 ? want : 8192)), dim3(256), 0, stream, (const bf16_t*)dO,
-	                   (const bf16_t*)o, (const float*)lse, delta, nlse2, lddo, ldo, B, S, Hq, D);
+	                   (const bf16_t*)o, (const float*)lse, ndelta, nlse2, lddo, ldo, B, S, Hq, D);
 	}
 	const Splits sp = split_walk(B, S, Hq, Hkv, D, causal != 0, workspace_bytes - whole);
 	float* dkv_part = sp.h * sp.q > 1 ? nlse2 + T * Hq : nullptr;
-	AttnBwdArgs a{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)dO, nlse2, delta, dq_part,
+	AttnBwdArgs a{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)dO, nlse2, ndelta, dq_part,
 	              (bf16_t*)dk, (bf16_t*)dv, ldq, ldk, ldv, lddo, lddk, lddv, B, S, Hq, Hkv, scale, (const float2*)rope_cs, sp.h, sp.q, dkv_part, sp.paired};
-	const int nkt = S / 128;
+	const int nkt = sp.wide ? (S + 255) / 256 : S / 128;
 	const dim3 grid((unsigned)((int64_t)B * Hkv * (causal && sp.paired ? (nkt + 1) / 2 : nkt) * sp.h * sp.q)), block(256);
 	int rc;
-	if (D == 128) rc = causal ? launch_bwd<128, true>(a, grid, stream) : launch_bwd<128, false>(a, grid, stream);
+	if (sp.wide) rc = launch_bwd_wide(a, causal != 0, grid, stream);
+	else if (D == 128) rc = causal ? launch_bwd<128, true>(a, grid, stream) : launch_bwd<128, false>(a, grid, stream);
 	else rc = causal ? launch_bwd<64, true>(a, grid, stream) : launch_bwd<64, false>(a, grid, stream);
 	if (rc) return rc;
 	const int64_t n16 = T * (Hq * D / 16);
@@ -1073,7 +916,7 @@ int attn_bwd(const void* q, const void* k, const void* v, const void* o, const v
 		dkv.blocks = (int)(want < 4096 ? want : 4096);
 	}
 	ELF_LAUNCH(dq_reduce_kernel, dim3((unsigned)(blocks < 16384 ? blocks : 16384) + dkv.blocks), dim3(256), 0, stream, dq_part, (bf16_t*)dq, B, S,
-	                   Hq * D, lddq, scale, causal, D, (const float2*)rope_cs, dkv);
+	                   Hq * D, lddq, scale, causal, sp.wide ? 256 : 128, D, (const float2*)rope_cs, dkv);
 	ELF_CHECK_HIP(hipGetLastError());
 	return 0;
 }

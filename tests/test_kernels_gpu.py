@@ -821,6 +821,25 @@ def test_attention_backward_with_walks_shared_by_workgroups(K, cfg):
 	assert sizes == sorted(sizes)
 
 
+@pytest.mark.parametrize("cfg", [(1, 896, 4, 4, 64, False), (2, 1152, 4, 2, 64, True), (9, 256, 16, 16, 64, True), (6, 384, 20, 4, 64, False), (1, 2048, 3, 3, 64, True), (3, 1024, 48, 8, 64, True)])
+def test_attention_backward_of_64_columns_over_256_keys_a_pass(K, cfg):
+	"""Heads of 64 columns take 256 keys a pass from 896 tokens up, shorter ones where they fill the chip: sequences that 256 divides
+	and odd multiples of 128 (half of the last pass lies past the end), one pass and many, walks whole, split by heads and by
+	queries, more workgroups than compute units.  Bounds of the 128-key kernels above: the same bf16 roundings, half as many of dQ."""
+	B, S, Hq, Hkv, D, causal = cfg
+	T = B * S
+	qkv, do = _randn(T, (Hq + 2 * Hkv) * D, seed=59), _randn(T, Hq * D, seed=60)
+	o_ref, _, dqkv_ref = _attn_ref(qkv, B, S, Hq, Hkv, D, causal, do)
+	o, lse = K.attn_fwd(qkv, B, S, Hq, Hkv, D, causal)
+	dqkv = K.attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal)
+	for name, sl in (("dq", slice(0, Hq * D)), ("dk", slice(Hq * D, (Hq + Hkv) * D)), ("dv", slice((Hq + Hkv) * D, None))):
+		_close(dqkv[:, sl], dqkv_ref[:, sl], rel_fro=1.5e-2, what=f"attn {name} {cfg}")
+	assert torch.equal(dqkv, K.attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal))
+	cs = K.rope_table(S, D, 5e5)
+	fused = K.attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal, rope_cs=cs)
+	assert torch.equal(fused, K.rope_apply_(dqkv.clone(), cs, S, Hq + Hkv, D, backward=True))
+
+
 @pytest.mark.parametrize("cfg", [(1, 128, 8, 2, 128, True), (3, 256, 4, 2, 128, True), (4, 512, 12, 12, 64, True), (1, 1152, 6, 3, 64, True), (1, 640, 12, 2, 128, True)])
 def test_attention_backward_with_a_workgroup_per_key_tile(K, cfg):
 	"""Causal, key tiles (one, two, an odd number) that all fit the chip at once: each goes to a workgroup of its own, with and
