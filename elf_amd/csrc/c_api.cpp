@@ -26,6 +26,15 @@ int elf_gemm_dw_group(int n, const elf_dw_problem* problems, int K, float scale,
 	return elf::gemm_dw_group(n, reinterpret_cast<const elf::DwProblem*>(problems), K, scale, (hipStream_t)stream);
 }
 
+static_assert(sizeof(elf_linear_w) == sizeof(elf::LinearW) && offsetof(elf_linear_w, bias_acc) == offsetof(elf::LinearW, bias) && offsetof(elf_linear_w, N) == offsetof(elf::LinearW, N),
+              "elf_linear_w and elf::LinearW differ");
+int64_t elf_linear_w_workspace_floats(int n, const elf_linear_w* layers, int T) {
+	return elf::colsum_group_workspace_floats(layers ? n : 0, reinterpret_cast<const elf::LinearW*>(layers), T);
+}
+int elf_linear_w_pass(int n, const elf_linear_w* layers, int T, float* workspace, void* stream) {
+	return elf::linear_w_pass(n, reinterpret_cast<const elf::LinearW*>(layers), T, workspace, (hipStream_t)stream);
+}
+
 int elf_gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, const void* W, int64_t ldw,
                       void* pre, int64_t ldpre, void* out, int64_t ldout, void* stream) {
 	return elf::gemm_act_bf16(act, M, F, K, A, lda, W, ldw, pre, ldpre, out, ldout, (hipStream_t)stream);

@@ -211,6 +211,77 @@ int gemm_bf16(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda,
 	return gemm_bf16_ring(a_t, b_t, M, N, K, A, lda, B, ldb, C, ldc, epi, R, ldr, k_splits, bm, bn, stream);
 }
 
+// Whether the weight gradients of several layers are done sooner in one launch of gemm_dw_group (256x256 tiles, or 128x128 ones where
+// these make no more than a round) than in a launch each on the best tile, and that launch costs 2 us.  Of 29 pairs of layers over 128
+// to 7000 tokens (us, apart and together): 2112 tokens, 4288 x 1600 and 832 x 4288 62.6 and 57.8; 1792, 1536 x 5184 and 3328 x 1536 70 and 58;
+// 5312, 1216 x 896 and 1536 x 1216 72 and 40; 256, 2112 x 1024 and 384 x 2112 14.4 and 10.4.  More than a round of tiles stays apart (4544,
+// 5824 x 7232 and 1792 x 5824 441 and 470), and a split of the tiles has to pay for its adds, 10 us a split (2048, 3520 x 256 and 1984 x
+// 3520 48 and 75).
+static bool group_pays(int n, const DwProblem* pr, int K) {
+	float apart = 2.f * (n - 1);
+	int64_t tiles = 0, small = 0;
+	for (int i = 0; i < n; i++) {
+		apart += plan_weight_gradient(pr[i].M, pr[i].N, K).us;
+		tiles += (int64_t)((pr[i].M + 255) / 256) * ((pr[i].N + 255) / 256);
+		small += (int64_t)((pr[i].M + 127) / 128) * ((pr[i].N + 127) / 128);
+	}
+	const TileTime &t256 = TILES_F32[0], &t128 = TILES_F32[2];
+	const int nk = K / BK;
+	int splits = 1;  // of the last round's tiles, as gemm_dw_group splits them
+	if (const int rem = (int)(tiles % 256); rem != 0 && rem <= 128) {
+		splits = 256 / rem < 8 ? 256 / rem : 8;
+		while (splits > 1 && nk / splits < 16) splits--;
+	}
+	const float last = (nk + splits - 1) / splits * t256.slice + t256.round + 10.f * (splits - 1);
+	if (tiles > 256) return false;
+	float group = last;
+	if (small <= 256) group = fminf(group, nk * t128.slice + t128.round);
+	return group < 0.97f * apart;
+}
+
+int linear_w_pass(int n, const LinearW* layers, int T, float* workspace, hipStream_t stream) {
+	ELF_REQUIRE(n > 0 && layers && T > 0, "linear_w_pass: no layers or no tokens");
+	ELF_REQUIRE(T % BK == 0, "linear_w_pass: the tokens must be a multiple of %d (T=%d)", BK, T);
+	bool biased = false;
+	for (int i = 0; i < n; i++) {
+		const LinearW& l = layers[i];
+		ELF_REQUIRE(l.dY && l.X && l.acc && l.M > 0 && l.N > 0 && l.M % 64 == 0 && l.N % 64 == 0 && l.lddy % 8 == 0 && l.ldx % 8 == 0 && l.lddy >= l.M && l.ldx >= l.N &&
+		                ((uintptr_t)l.dY % 16) == 0 && ((uintptr_t)l.X % 16) == 0,
+		            "linear_w_pass: layer %d (M=%d N=%d) has a null operand, sizes that are no multiples of 64 or misaligned rows", i, l.M, l.N);
+		biased = biased || l.bias;
+	}
+	ELF_REQUIRE(!biased || workspace, "linear_w_pass: bias sums need a workspace");
+	DwProblem group[DW_GROUP_MAX];
+	int ng = 0;
+	auto alone = [&](const DwProblem& q) { return gemm_bf16(1, 1, q.M, q.N, T, q.dY, q.lddy, q.X, q.ldx, q.acc, q.N, EPI_F32_ACC, nullptr, 0, 0, 0, stream); };
+	auto flush = [&]() -> int {
+		const int m = ng;
+		ng = 0;
+		if (m > 1 && group_pays(m, group, T)) return gemm_dw_group(m, group, T, 0.f, stream);
+		for (int i = 0; i < m; i++)
+			if (int rc = alone(group[i])) return rc;
+		return 0;
+	};
+	for (int i = 0; i < n; i++) {
+		const LinearW& l = layers[i];
+		const DwProblem q{l.dY, l.lddy, l.X, l.ldx, l.acc, nullptr, l.M, l.N};
+		bool again = false;  // an accumulator that an earlier layer of the launch adds to as well: one after the other
+		for (int j = 0; j < ng; j++) again = again || (q.acc < group[j].acc + (int64_t)group[j].M * group[j].N && group[j].acc < q.acc + (int64_t)q.M * q.N);
+		if (again || ng == DW_GROUP_MAX) {
+			if (int rc = flush()) return rc;
+		}
+		if (gemm_dw_groupable(l.M, l.N, T, l.dY, l.lddy, l.X, l.ldx, l.acc)) {
+			group[ng++] = q;
+		} else {
+			// (behind what is waiting: it may add to the same accumulator)
+			if (int rc = flush()) return rc;
+			if (int rc = alone(q)) return rc;
+		}
+	}
+	if (int rc = flush()) return rc;
+	return biased ? colsum_group(n, layers, T, workspace, stream) : 0;
+}
+
 // The way of an up-projection with its activation: a 256-column tile (SwiGLU), a 64x64 ring tile, bm = 0: two passes.
 static Plan act_plan(int act, int M, int F, int K, bool dense) {
 	const int N = act == ACT_SWIGLU ? 2 * F : F;

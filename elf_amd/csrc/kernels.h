@@ -80,6 +80,21 @@ int gemm_ring_dw_group(int n, const DwProblem* problems, int K, float scale, hip
 bool gemm_dw_groupable(int M, int N, int K, const void* dY, int64_t lddy, const void* X, int64_t ldx, const void* acc);
 int gemm_dw_group(int n, const DwProblem* problems, int K, float scale, hipStream_t stream);
 
+// The parameter gradients of linear layers over the same T tokens: acc [M, N] += dY^T X, bias [M] (optional) += column sums of dY.
+// Weight gradients share launches where that is the faster way, bias sums two; layers whose accumulators overlap follow each other.
+struct LinearW {
+	const void* dY;
+	int64_t lddy;
+	const void* X;
+	int64_t ldx;
+	float* acc;
+	float* bias;
+	int M, N;
+};
+int linear_w_pass(int n, const LinearW* layers, int T, float* workspace, hipStream_t stream);
+int64_t colsum_group_workspace_floats(int n, const LinearW* layers, int T);
+int colsum_group(int n, const LinearW* layers, int T, float* workspace, hipStream_t stream);  // the bias sums alone
+
 // The attention block's packed q | k | v projection with the rotary embedding of the q and k heads: C [M, N] =
 // A W^T rounded to bf16, then rope_apply's rotation on the first n_rot_heads heads of width D (cs: the table of
 // rope_table for sequence length S; row r is at position r mod S).  One kernel (rotation in the GEMM epilogue, the

@@ -17,7 +17,7 @@ from torch.utils.checkpoint import checkpoint
 
 from .. import _lib
 from ..scheduling import OpOptions
-from ..zb_utils import LayerDW, replace_layer_with_layer_dw
+from ..zb_utils import LayerDW, LinearDW, replace_layer_with_layer_dw
 from .block import StageBlockBase
 
 logger = logging.getLogger("block")
@@ -126,9 +126,12 @@ class AutogradStageBlock(StageBlockBase):
 
 	def backward_params(self, mb_id, **options):
 		with self._timed(f"backward_params({self.id}:{mb_id})"):
-			for m in self._layers_dw():
-				if not m.is_empty("grad_output"):
+			ready = [m for m in self._layers_dw() if not m.is_empty("grad_output")]
+			plain = [m for m in ready if type(m).backward is LinearDW.backward and "backward" not in m.__dict__]
+			for m in ready:
+				if m not in plain:
 					m.backward(mb_id)
+			LinearDW.backward_together(plain, mb_id)
 
 	def recompute_forward(self, mb_id, **options):
 		inputs = [var.get(var.saved, mb_id) for var in self.input_variables]

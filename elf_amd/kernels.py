@@ -81,6 +81,38 @@ def gemm_dw_group(problems, *, scale=0.0):
 	_lib.check(rc, "elf_gemm_dw_group")
 
 
+class _LinearW(ctypes.Structure):
+	"""``elf_linear_w`` of include/elf_stage.h."""
+
+	_fields_ = [("dY", ctypes.c_void_p), ("lddy", ctypes.c_int64), ("X", ctypes.c_void_p), ("ldx", ctypes.c_int64), ("acc", ctypes.c_void_p),
+	            ("bias_acc", ctypes.c_void_p), ("M", ctypes.c_int), ("N", ctypes.c_int)]
+
+
+def linear_w_pass(layers):
+	"""The parameter gradients of linear layers over the same tokens.  ``layers``: tuples ``(dy [T, M] bf16, x [T, N] bf16,
+	acc [M, N] fp32, bias_acc [M] fp32 or None)``, dense accumulators: ``acc += dy.T @ x``, ``bias_acc += dy.sum(0)``."""
+	arr = (_LinearW * len(layers))()
+	T = layers[0][0].shape[0]
+	for q, (dy, x, acc, bias) in zip(arr, layers):
+		_need(dy, torch.bfloat16, "linear_w_pass.dy")
+		_need(x, torch.bfloat16, "linear_w_pass.x")
+		_need(acc, torch.float32, "linear_w_pass.acc")
+		M, N = dy.shape[1], x.shape[1]
+		if dy.shape[0] != T or x.shape[0] != T:
+			raise _lib.ElfStageError(f"linear_w_pass: every layer sums over the same {T} rows")
+		if tuple(acc.shape) != (M, N) or not acc.is_contiguous():
+			raise _lib.ElfStageError(f"linear_w_pass: the accumulator must be dense [{M}, {N}]")
+		if bias is not None:
+			_need(bias, torch.float32, "linear_w_pass.bias_acc")
+			if bias.numel() != M or not bias.is_contiguous():
+				raise _lib.ElfStageError(f"linear_w_pass: the bias accumulator must be dense [{M}]")
+		q.dY, q.lddy, q.X, q.ldx, q.acc, q.bias_acc, q.M, q.N = dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), acc.data_ptr(), _ptr(bias), M, N
+	lib = _lib.load()
+	floats = lib.elf_linear_w_workspace_floats(len(layers), arr, T)
+	ws = torch.empty(floats, dtype=torch.float32, device=layers[0][0].device) if floats else None
+	_lib.check(lib.elf_linear_w_pass(len(layers), arr, T, _ptr(ws), _stream()), "elf_linear_w_pass")
+
+
 def gemm_turn_giveups():
 	"""Waves of split-K GEMM launches on the current device that added out of turn since the library was loaded."""
 	n = ctypes.c_uint64()

@@ -25,7 +25,9 @@ __all__ = ["LinearDX", "LayerDW", "LinearDW", "MappingDW", "replace_layer_with_l
 
 
 def _as_rows(t):
-	"""[..., C] -> contiguous [rows, C] view (a copy only if the layout forces one)."""
+	"""[..., C] -> contiguous [rows, C] (a copy only if the layout forces one)."""
+	if t.dim() == 2 and t.is_contiguous():
+		return t
 	t2 = t.reshape(-1, t.shape[-1])
 	return t2 if t2.is_contiguous() else t2.contiguous()
 
@@ -45,7 +47,7 @@ class LinearDX(torch.autograd.Function):
 			y = kernels.gemm(x, weight, epilogue=kernels.EPI_BF16_RESID, residual=row, residual_ld=0)
 		else:
 			y = kernels.gemm(x, weight)
-		return y.view(*input.shape[:-1], weight.shape[0])
+		return y if input.dim() == 2 else y.view(*input.shape[:-1], weight.shape[0])
 
 	@staticmethod
 	def backward(ctx, grad_output):
@@ -53,7 +55,7 @@ class LinearDX(torch.autograd.Function):
 		linear._accumulate_grad_output(grad_output)
 		go = _as_rows(grad_output)
 		grad_input = kernels.gemm(go, linear.weight.detach(), b_t=True)  # dY [T, out] x W [out, in] with W read as it lies
-		return grad_input.view(*grad_output.shape[:-1], linear.weight.shape[1]), None, None, None
+		return (grad_input if grad_output.dim() == 2 else grad_input.view(*grad_output.shape[:-1], linear.weight.shape[1])), None, None, None
 
 
 class LayerDW:
@@ -169,6 +171,26 @@ class LinearDW(LayerDW, nn.Linear):
 			kernels.colsum_(go, self._main_grad(self.bias))
 		self.ctx["grad_output"][mb_id] = None
 		self.ctx["input"][mb_id] = None
+
+
+	@staticmethod
+	def backward_together(layers, mb_id):
+		"""W of several layers: what ``backward`` does for each, the layers over the same number of tokens in one call of the library
+		(weight gradients and bias sums then share launches).  What such a call does not take goes through ``backward``."""
+		by_tokens = {}
+		for m in layers:
+			grad_output, inputs, acc = m.ctx["grad_output"][mb_id], m.ctx["input"][mb_id], m._main_grad(m.weight)
+			bias = m._main_grad(m.bias) if m.bias is not None else None
+			if not all(g is None or (g.dtype == torch.float32 and g.is_contiguous()) for g in (acc, bias)) or grad_output.dtype != torch.bfloat16 or inputs.dtype != torch.bfloat16:
+				m.backward(mb_id)
+				continue
+			go, inp = _as_rows(grad_output), _as_rows(inputs)
+			by_tokens.setdefault(go.shape[0], []).append((m, (go, inp, acc, bias)))
+		for group in by_tokens.values():
+			kernels.linear_w_pass([layer for _, layer in group])
+			for m, _ in group:
+				m.ctx["grad_output"][mb_id] = None
+				m.ctx["input"][mb_id] = None
 
 
 LinearDW.register_dx_function(LinearDX)

@@ -76,6 +76,27 @@ typedef struct elf_dw_problem {
 } elf_dw_problem;
 int elf_gemm_dw_group(int n, const elf_dw_problem* problems, int K, float scale, void* stream);
 
+/* The parameter gradients of several linear layers over the same T tokens: for layer i acc[M, N] (fp32, dense) += dY^T X with
+ * dY [T, M] (leading dim lddy) and X [T, N] (leading dim ldx), and, where bias_acc is not NULL, bias_acc[M] += the column sums
+ * of dY.  What n calls of elf_gemm_bf16(1, 1, ..., epilogue 2) and elf_colsum_bf16 compute; the weight gradients share a launch
+ * where that is the faster way (their sums over T may then be split differently, in a fixed order either way), the bias sums share
+ * two, with elf_colsum_bf16's bits.  Layers whose accumulators overlap are taken one after the other.  workspace:
+ * elf_linear_w_workspace_floats() floats (NULL without biases).  M, N, T multiples of 64, leading dimensions of 8, dY and X
+ * 16-byte aligned.
+ * Replaces: the loop over LayerDW modules of PipelineBlock.backward_params (elf/execution/block.py:384-389) with
+ *           LinearDW.backward (elf/zb_utils.py:235-252). */
+typedef struct elf_linear_w {
+	const void* dY;
+	int64_t lddy;
+	const void* X;
+	int64_t ldx;
+	float* acc;
+	float* bias_acc;
+	int M, N;
+} elf_linear_w;
+int64_t elf_linear_w_workspace_floats(int n, const elf_linear_w* layers, int T);
+int elf_linear_w_pass(int n, const elf_linear_w* layers, int T, float* workspace, void* stream);
+
 /* The MLP's up-projection with its activation: pre = A W^T with A [M, K] and W [N, K], both k contiguous;
  * act 0 (GELU): N = F, out[M, F] = gelu(pre); act 1 (SwiGLU): N = 2F, W = [gate rows; up rows],
  * pre[M, 2F] = [g | u], out[M, F] = silu(g) * u.  pre is kept because the backward needs it.  SwiGLU is

@@ -931,6 +931,40 @@ def test_colsum_is_exact_to_rounding_and_repeatable(K, T, N, ld):
 	assert ((runs[0].double() - want).abs().max() / want.abs().max()).item() <= 1e-5
 
 
+@pytest.mark.parametrize("T,shapes", [
+	(2112, [(4288, 1600, True), (832, 4288, True)]),                          # one launch of 256x256 tiles, the last ones split
+	(512, [(512, 512, True), (1536, 512, False), (512, 768, True)]),          # one launch of 128x128 tiles
+	(64, [(64, 128, True), (256, 64, True)]),                                 # narrower than 256: one launch each
+	(192, [(320, 256, False), (64, 64, True), (256, 320, False)] * 6),        # more layers than a launch takes, mixed
+])
+def test_parameter_gradients_of_a_list_of_layers(K, T, shapes):
+	"""Weight and bias gradients of several layers in one call, on top of what the accumulators hold: against fp64 sums (fp32 sums of
+	T products: T * 2^-24 of their magnitude, far below the bound), bias sums the bits of a call each, equal bits from run to run; two
+	layers that share their parameters both count."""
+	layers, want = [], []
+	for i, (M, N, bias) in enumerate(shapes):
+		dy, x = _randn(T, M, seed=300 + i), _randn(T, N, seed=400 + i)
+		acc = torch.randn(M, N, device="cuda", generator=torch.Generator(device="cuda").manual_seed(500 + i))
+		b = torch.randn(M, device="cuda", generator=torch.Generator(device="cuda").manual_seed(600 + i)) if bias else None
+		layers.append((dy, x, acc, b))
+		want.append((acc.double() + dy.double().t() @ x.double(), K.colsum_(dy, b.clone()) if bias else None))
+	runs = []
+	for _ in range(2):
+		run = [(dy, x, acc.clone(), None if b is None else b.clone()) for dy, x, acc, b in layers]
+		K.linear_w_pass(run)
+		runs.append(run)
+	for a, b, (w, wb) in zip(*runs, want):
+		assert torch.equal(a[2], b[2])
+		assert float((a[2].double() - w).norm() / w.norm()) <= 1e-5
+		assert wb is None or (torch.equal(a[3], wb) and torch.equal(b[3], wb))
+	dy, x, acc, b = layers[0]
+	twice, bias = acc.clone(), torch.zeros(dy.shape[1], device="cuda")
+	K.linear_w_pass([(dy, x, twice, bias), (dy, x, twice, bias)])
+	w = acc.double() + 2 * (dy.double().t() @ x.double())
+	assert float((twice.double() - w).norm() / w.norm()) <= 1e-5
+	assert torch.allclose(bias.double(), 2 * dy.double().sum(0), rtol=1e-4, atol=1e-3)
+
+
 def test_split_k_on_one_stream_never_gives_up_its_turn_and_wide_splits_are_refused(K):
 	"""Back-to-back split-K launches on one stream keep their turns (the counter of waves that added out of turn does not
 	move, which is what bit-reproducible weight gradients rest on), and a split count that would not fit the 8 bits the
