@@ -13,7 +13,10 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libelf_stage.so")
 
+TORCH_LIB_PATH = os.path.join(_HERE, "libelf_torch.so")
+
 _lib = None
+_torch_allocated = None
 
 # name -> (restype, argtypes); kept in one table so that tests can check the exported symbols
 # against the header.
@@ -102,6 +105,19 @@ def load():
 		fn.restype, fn.argtypes = restype, argtypes
 	_lib = lib
 	return lib
+
+
+def torch_allocated(device):
+	"""(allocated, peak) bytes of PyTorch's caching allocator on ``device`` through libelf_torch.so, or None without that library."""
+	global _torch_allocated
+	if _torch_allocated is None:
+		if not os.path.exists(TORCH_LIB_PATH):
+			return None
+		fn = ctypes.CDLL(TORCH_LIB_PATH).elf_torch_allocated
+		fn.restype, fn.argtypes = c_int, [c_int, _P]
+		_torch_allocated = fn
+	out = (c_int64 * 2)()
+	return (out[0], out[1]) if _torch_allocated(device, out) == 0 else None
 
 
 def check(rc, what=""):
