@@ -47,6 +47,7 @@ _SIGNATURES = {
 	"elf_embedding_fwd": (c_int, [_P, _P, _P, c_int64, c_int, c_int, _P]),
 	"elf_embedding_bwd": (c_int, [_P, _P, _P, c_int64, c_int, c_int, _P]),
 	"elf_cross_entropy": (c_int, [_P, c_int64, _P, c_int64, c_int64, c_int64, c_float, _P, _P, _P, c_int64, _P]),
+	"elf_cross_entropy_loss": (c_int, [_P, c_int64, c_int, _P, c_int64, c_int64, c_int64, c_float, c_int, _P, _P, _P, c_int64, _P, _P]),
 	"elf_cross_entropy_dense": (c_int, [_P, _P, c_int64, c_int64, c_int64, c_float, _P, _P, _P, _P]),
 	"elf_scale_by_bf16": (c_int, [_P, _P, _P, c_int64, _P]),
 	"elf_cross_entropy_reduce": (c_int, [_P, _P, c_int64, c_int64, _P, _P]),

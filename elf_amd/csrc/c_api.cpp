@@ -107,6 +107,10 @@ int elf_cross_entropy(const void* logits, int64_t ld, const void* target, int64_
                       const void* dev_div, void* row_loss, void* dlogits, int64_t ld_out, void* stream) {
 	return elf::cross_entropy(logits, ld, target, rows, V, ignore_index, scale, dev_div, row_loss, dlogits, ld_out, S_(stream));
 }
+int elf_cross_entropy_loss(const void* logits, int64_t ld, int dense, const void* target, int64_t rows, int64_t V, int64_t ignore_index, float scale, int mean,
+                           void* row_loss, void* loss, void* dlogits, int64_t ld_out, void* scratch2, void* stream) {
+	return elf::cross_entropy_loss(logits, ld, dense != 0, target, rows, V, ignore_index, scale, mean != 0, row_loss, loss, dlogits, ld_out, scratch2, S_(stream));
+}
 int elf_cross_entropy_dense(const void* logits, const void* target, int64_t rows, int64_t V, int64_t ignore_index, float scale, const void* dev_div,
                             void* row_loss, void* dlogits, void* stream) {
 	return elf::cross_entropy_dense(logits, target, rows, V, ignore_index, scale, dev_div, row_loss, dlogits, S_(stream));

@@ -186,9 +186,12 @@ int embedding_fwd(const void* ids, const void* table, void* out, int64_t T, int 
 int embedding_bwd(const void* ids, const void* dx, void* dtable_f32, int64_t T, int d, int V, hipStream_t s);
 // Cross-entropy over bf16 logits [rows, V] (row stride ld), loss and gradient in one pass; target int64 [rows].
 int cross_entropy(const void* logits, int64_t ld, const void* target, int64_t rows, int64_t V, int64_t ignore_index, float scale,
-                  const void* dev_div, void* row_loss, void* dlogits, int64_t ld_out, hipStream_t s);
+                  const void* dev_div, void* row_loss, void* dlogits, int64_t ld_out, hipStream_t s, bool count = false);
 int cross_entropy_dense(const void* logits, const void* target, int64_t rows, int64_t V, int64_t ignore_index, float scale, const void* dev_div,
-                        void* row_loss, void* dlogits, hipStream_t s);
+                        void* row_loss, void* dlogits, hipStream_t s, bool count = false);
+// (count: the gradient is divided by the live rows, which the kernel counts itself)
+int cross_entropy_loss(const void* logits, int64_t ld, bool dense, const void* target, int64_t rows, int64_t V, int64_t ignore_index, float scale, bool mean,
+                       void* row_loss, void* loss, void* dlogits, int64_t ld_out, void* scratch2, hipStream_t s);
 int scale_by_bf16(const void* x, const void* g_f32, void* y, int64_t n, hipStream_t s);
 int cross_entropy_reduce(const void* row_loss, const void* target, int64_t rows, int64_t ignore_index, void* out2, hipStream_t s);
 

@@ -21,6 +21,8 @@ constexpr float LOG2E_F = 1.4426950408889634f;
 // which a softmax term that small may do).
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+constexpr int64_t STREAM_ELEMS = int64_t(1) << 25;  // arrays from this size on go past the caches
+
 struct LossArgs {
 	const bf16_t* x;
 	int64_t ld;
@@ -30,6 +32,7 @@ struct LossArgs {
 	int64_t ignore_index;
 	float scale;
 	const float* dev_div;  // optional device scalar the gradient is divided by
+	int count;             // != 0: the gradient is divided by the number of live rows, which every wave counts (G = 64 only)
 	float* row_loss;       // optional
 	bf16_t* dx;            // optional
 	int64_t ld_out;
@@ -62,6 +65,11 @@ __device__ __forceinline__ float row_loss_of(const LossArgs& a, int64_t row, int
 	return m + logf(s) - (float)a.x[row * a.ld + tgt];
 }
 
+// Launches of at most this many rows of at most COUNT_COLS columns count the live rows themselves, each wave under the loads of its own
+// row, instead of reading what a launch before them counted (4 us): 512 x 1000, loss and gradient 17.8 us -> 14.5.  Not wider ones: the
+// registers are full there, and with 2048 rows of 50304 columns the count took longer than that launch.
+constexpr int COUNT_ROWS = 2048, COUNT_COLS = 64 * 8 * 8;
+
 // G threads per row, C 16-byte chunks (8 logits) per thread: rows of up to G * C * 8 columns, read once into registers,
 // reduced there, and their gradient written from the same registers.  Bound: HBM (4 bytes per logit) and, close behind, the two
 // exponentials per logit.  Rows beyond 16384 columns used to be read twice by 256 threads, the second time from a cache that
@@ -73,7 +81,9 @@ __device__ __forceinline__ float row_loss_of(const LossArgs& a, int64_t row, int
 // neighbouring rows (or with what lies behind the last column), are read and written element by element by lanes 0 and 1.
 // Rows that lie apart have their last chunk to themselves: it is taken whole and masked (element by element 301 x 1350 took 5.7 us,
 // 4.2 masked; 36 x 1014 5.0 and 3.7).
-template <int G, int C, bool DENSE>
+// STREAM: the logits are read past the caches, so that these hold the gradient for who reads it next.  Loss, gradient and its product with the
+// incoming one, 4096 x 32000 186 -> 171 us, 1024 x 128256 213 -> 195, 2048 x 50257 161 -> 157; the gradient written past them as well 190, 205 and 167.
+template <int G, int C, bool DENSE, bool STREAM>
 __global__ __launch_bounds__(G < 256 ? 256 : G, G >= 256 ? 64 / C : 1) void cross_entropy_kernel(LossArgs a) {
 	constexpr int BLOCK = G < 256 ? 256 : G;
 	constexpr int ROWS = BLOCK / G;
@@ -96,7 +106,17 @@ __global__ __launch_bounds__(G < 256 ? 256 : G, G >= 256 ? 64 / C : 1) void cros
 #pragma unroll
 	for (int j = 0; j < C; j++) {
 		const int c = j * G + lane;
-		if (c >= cbeg && c < cend) reg[j] = *reinterpret_cast<const bf16x8*>(xr + (int64_t)c * 8);
+		if (c >= cbeg && c < cend) {
+			const bf16x8* p = reinterpret_cast<const bf16x8*>(xr + (int64_t)c * 8);
+			reg[j] = STREAM ? __builtin_nontemporal_load(p) : *p;
+		}
+	}
+	float live = 0.f;
+	if constexpr (G == 64) {
+		if (a.count) {
+			for (int64_t r = lane; r < a.rows; r += 64) live += a.target[r] != a.ignore_index ? 1.f : 0.f;
+			live = wave_sum(live);
+		}
 	}
 	if (ec >= 0) {
 		for (int i = elo; i < ehi; i++) m = fmaxf(m, (float)xr[(int64_t)ec * 8 + i]);
@@ -133,7 +153,7 @@ __global__ __launch_bounds__(G < 256 ? 256 : G, G >= 256 ? 64 / C : 1) void cros
 	const int64_t tgt = a.target[row];
 	if (a.row_loss && lane == 0) a.row_loss[row] = row_loss_of(a, row, tgt, m, s);
 	if (!a.dx) return;
-	const float g = tgt != a.ignore_index ? grad_scale(a) : 0.f;
+	const float g = tgt != a.ignore_index ? G == 64 && a.count ? a.scale / live : grad_scale(a) : 0.f;
 	bf16_t* const dr = a.dx + (row * a.ld_out - rot);
 	const int tchunk = tgt >= 0 && tgt < a.V ? (int)((tgt + rot) >> 3) : -1, tcol = (int)((tgt + rot) & 7);
 	// softmax * |g| of the wide rows = exp2(x*log2e - (m + log2(s) - log2|g|)), its sign by an exclusive or: no product per
@@ -265,9 +285,11 @@ __global__ __launch_bounds__(G) void cross_entropy_stream_kernel(LossArgs a) {
 }
 
 // out[0] = sum of row_loss (skipped when row_loss is null), out[1] = number of rows whose target is
-// not ignore_index.  One workgroup, fixed summation order: the same inputs give the same bits.
+// not ignore_index; loss (optional) = out[0], or out[0] / out[1] if mean.  One workgroup, fixed summation order: the same inputs
+// give the same bits.
 __global__ __launch_bounds__(1024) void cross_entropy_reduce_kernel(const float* __restrict__ row_loss, const int64_t* __restrict__ target,
-                                                                    int64_t rows, int64_t ignore_index, float* __restrict__ out) {
+                                                                    int64_t rows, int64_t ignore_index, float* __restrict__ out,
+                                                                    float* __restrict__ loss, int mean) {
 	__shared__ float red[16];
 	float s = 0.f, n = 0.f;
 	for (int64_t r = threadIdx.x; r < rows; r += 1024) {
@@ -277,8 +299,11 @@ __global__ __launch_bounds__(1024) void cross_entropy_reduce_kernel(const float*
 	s = group_reduce<1024, false>(s, red);
 	n = group_reduce<1024, false>(n, red);
 	if (threadIdx.x == 0) {
-		if (row_loss) out[0] = s;
-		out[1] = n;
+		if (out) {
+			if (row_loss) out[0] = s;
+			out[1] = n;
+		}
+		if (loss) *loss = mean ? s / n : s;
 	}
 }
 
@@ -286,7 +311,9 @@ template <int G, int C, bool DENSE>
 void launch_rows(const LossArgs& a, hipStream_t s) {
 	constexpr int BLOCK = G < 256 ? 256 : G;
 	constexpr int ROWS = BLOCK / G;
-	ELF_LAUNCH((cross_entropy_kernel<G, C, DENSE>), dim3((unsigned)((a.rows + ROWS - 1) / ROWS)), dim3(BLOCK), 0, s, a);
+	const dim3 grid((unsigned)((a.rows + ROWS - 1) / ROWS));
+	if (a.rows * a.V >= STREAM_ELEMS) ELF_LAUNCH((cross_entropy_kernel<G, C, DENSE, true>), grid, dim3(BLOCK), 0, s, a);
+	else ELF_LAUNCH((cross_entropy_kernel<G, C, DENSE, false>), grid, dim3(BLOCK), 0, s, a);
 }
 
 // The narrowest group of threads whose registers hold a row of `width` columns; false: none does.
@@ -306,7 +333,6 @@ bool launch_resident(const LossArgs& a, int64_t width, hipStream_t s) {
 // thread.  Bound: HBM.  STREAM: past the caches, for arrays these do not hold; 4096 x 128256 464 us -> 352 (4.5 -> 6.0 TB/s; walked
 // with a grid of 8192 workgroups before), 1024 x 151936 125 -> 89, 2048 x 50257 69 -> 60.  16 MB take 7.5 us either way, and stay
 // in the caches for who reads the gradient next.
-constexpr int64_t STREAM_ELEMS = int64_t(1) << 25;
 template <int U, bool STREAM>
 __global__ __launch_bounds__(256) void scale_by_kernel(const bf16_t* __restrict__ x, const float* __restrict__ g, bf16_t* __restrict__ y, int64_t n) {
 	const float f = (float)(bf16_t)*g;
@@ -338,7 +364,7 @@ void launch_scale_by(const bf16_t* x, const float* g, bf16_t* y, int64_t n, hipS
 }  // namespace
 
 int cross_entropy(const void* logits, int64_t ld, const void* target, int64_t rows, int64_t V, int64_t ignore_index, float scale,
-                  const void* dev_div, void* row_loss, void* dlogits, int64_t ld_out, hipStream_t s) {
+                  const void* dev_div, void* row_loss, void* dlogits, int64_t ld_out, hipStream_t s, bool count) {
 	ELF_REQUIRE(logits && target && rows > 0 && V > 0 && V < (1ll << 30), "cross_entropy: bad argument");
 	ELF_REQUIRE(rows < (1ll << 31), "cross_entropy: too many rows");
 	ELF_REQUIRE(ld % 8 == 0 && ld >= V && ((uintptr_t)logits & 15) == 0,
@@ -347,7 +373,7 @@ int cross_entropy(const void* logits, int64_t ld, const void* target, int64_t ro
 	if (dlogits)
 		ELF_REQUIRE(ld_out % 8 == 0 && ld_out >= V && ((uintptr_t)dlogits & 15) == 0,
 		            "cross_entropy: gradient rows must start on 16-byte boundaries (row stride %lld must be a multiple of 8 and >= V)", (long long)ld_out);
-	LossArgs a{(const bf16_t*)logits, ld, (const int64_t*)target, rows, (int)V, ignore_index, scale, (const float*)dev_div,
+	LossArgs a{(const bf16_t*)logits, ld, (const int64_t*)target, rows, (int)V, ignore_index, scale, (const float*)dev_div, count,
 	           (float*)row_loss, (bf16_t*)dlogits, dlogits ? ld_out : 0};
 	const int64_t width = dlogits && ld_out > V ? ld_out : V;
 	ProfScope prof(PROF_LOSS, (dlogits ? 4.0 : 2.0) * rows * V, s);
@@ -362,13 +388,13 @@ int cross_entropy(const void* logits, int64_t ld, const void* target, int64_t ro
 }
 
 int cross_entropy_dense(const void* logits, const void* target, int64_t rows, int64_t V, int64_t ignore_index, float scale, const void* dev_div,
-                        void* row_loss, void* dlogits, hipStream_t s) {
+                        void* row_loss, void* dlogits, hipStream_t s, bool count) {
 	ELF_REQUIRE(logits && target && rows > 0 && rows < (1ll << 31) && V > 0, "cross_entropy_dense: bad argument");
 	ELF_REQUIRE(V <= 1024 * 16 * 8 - 7, "cross_entropy_dense: rows of at most %d columns (V=%lld)", 1024 * 16 * 8 - 7, (long long)V);
 	ELF_REQUIRE(row_loss || dlogits, "cross_entropy_dense: nothing to compute (no row_loss and no dlogits)");
 	ELF_REQUIRE(((uintptr_t)logits & 1) == 0 && (!dlogits || ((uintptr_t)logits & 15) == ((uintptr_t)dlogits & 15)),
 	            "cross_entropy_dense: logits and their gradient must lie alike modulo 16 bytes");
-	LossArgs a{(const bf16_t*)logits, V, (const int64_t*)target, rows, (int)V, ignore_index, scale, (const float*)dev_div, (float*)row_loss, (bf16_t*)dlogits, V};
+	LossArgs a{(const bf16_t*)logits, V, (const int64_t*)target, rows, (int)V, ignore_index, scale, (const float*)dev_div, count, (float*)row_loss, (bf16_t*)dlogits, V};
 	ProfScope prof(PROF_LOSS, (dlogits ? 4.0 : 2.0) * rows * V, s);
 	launch_resident<true>(a, V + 7, s);  // a row may cover one chunk more than V / 8
 	ELF_CHECK_HIP(hipGetLastError());
@@ -388,7 +414,23 @@ int scale_by_bf16(const void* x, const void* g_f32, void* y, int64_t n, hipStrea
 int cross_entropy_reduce(const void* row_loss, const void* target, int64_t rows, int64_t ignore_index, void* out2, hipStream_t s) {
 	ELF_REQUIRE(target && out2 && rows > 0, "cross_entropy_reduce: bad argument");
 	ELF_LAUNCH(cross_entropy_reduce_kernel, dim3(1), dim3(1024), 0, s, (const float*)row_loss, (const int64_t*)target, rows,
-	                   ignore_index, (float*)out2);
+	                   ignore_index, (float*)out2, nullptr, 0);
+	ELF_CHECK_HIP(hipGetLastError());
+	return 0;
+}
+
+int cross_entropy_loss(const void* logits, int64_t ld, bool dense, const void* target, int64_t rows, int64_t V, int64_t ignore_index, float scale, bool mean,
+                       void* row_loss, void* loss, void* dlogits, int64_t ld_out, void* scratch2, hipStream_t s) {
+	ELF_REQUIRE(row_loss && loss && scratch2, "cross_entropy_loss: null pointer");
+	const bool divide = mean && dlogits, count = divide && rows <= COUNT_ROWS && (dense ? V + 7 : ld_out > V ? ld_out : V) <= COUNT_COLS;
+	float* const out2 = (float*)scratch2;
+	if (divide && !count)
+		if (int rc = cross_entropy_reduce(nullptr, target, rows, ignore_index, out2, s)) return rc;
+	const void* div = divide && !count ? out2 + 1 : nullptr;
+	if (int rc = dense ? cross_entropy_dense(logits, target, rows, V, ignore_index, scale, div, row_loss, dlogits, s, count)
+	                   : cross_entropy(logits, ld, target, rows, V, ignore_index, scale, div, row_loss, dlogits, ld_out, s, count))
+		return rc;
+	ELF_LAUNCH(cross_entropy_reduce_kernel, dim3(1), dim3(1024), 0, s, (const float*)row_loss, (const int64_t*)target, rows, ignore_index, (float*)nullptr, (float*)loss, (int)mean);
 	ELF_CHECK_HIP(hipGetLastError());
 	return 0;
 }

@@ -49,10 +49,12 @@ def _check_target(target, rows):
 _DENSE_MAX = 1024 * 16 * 8 - 7  # widest row elf_cross_entropy_dense holds in registers
 
 
-def _run(pred, target, *, ignore_index, scale, mean, want_grad, padded=True):
-	"""(row_loss fp32 [rows], out2 = [sum, count] fp32, grad or None).  The gradient is [rows, ld_out] bf16 with ``ld_out`` a
-	multiple of 64, or, unless ``padded``, [rows, V] where V is a multiple of 8 or the logits are one dense block: rows that start
-	at any address are then read in place (50257 columns: the padded copy of the logits took half of a loss's time)."""
+def _run(pred, target, *, ignore_index, scale, reduction, want_grad, padded=True):
+	"""(loss, grad or None).  The gradient is [rows, ld_out] bf16 with ``ld_out`` a multiple of 64, or, unless ``padded``, [rows, V]
+	where V is a multiple of 8 or the logits are one dense block: rows that start at any address are then read in place (50257
+	columns: the padded copy of the logits took half of a loss's time)."""
+	if reduction not in ("sum", "mean", "none"):
+		raise ValueError(f"{reduction} is not a valid value for reduction")
 	V = pred.shape[-1]
 	dense = V % 8 != 0 and not (want_grad and padded) and pred.dtype == torch.bfloat16 and pred.is_cuda and pred.is_contiguous() and not pred.is_neg() and pred.data_ptr() % 16 == 0 and 0 < V <= _DENSE_MAX
 	src, ld = (pred, V) if dense else _rows_view(pred, V)
@@ -61,38 +63,22 @@ def _run(pred, target, *, ignore_index, scale, mean, want_grad, padded=True):
 	lib, stream = _lib.load(), _stream()
 	dev = pred.device
 	row_loss = torch.empty(rows, dtype=torch.float32, device=dev)
-	out2 = torch.empty(2, dtype=torch.float32, device=dev)
-	grad, ld_out, div = None, 0, None
-	if mean:  # the gradient divides by the number of live rows, which only depends on the target
-		_lib.check(lib.elf_cross_entropy_reduce(None, target.data_ptr(), rows, ignore_index, out2.data_ptr(), stream), "elf_cross_entropy_reduce")
-		div = out2[1:]
+	grad, ld_out, dx = None, 0, None
 	if want_grad:
 		ld_out = V if dense or (V % 8 == 0 and not padded) else -(-V // _PAD) * _PAD
 		grad = torch.empty(rows, ld_out, dtype=torch.bfloat16, device=dev)
+		dx = grad.data_ptr()
+	if reduction != "none":
+		loss, scratch = torch.empty((), dtype=torch.float32, device=dev), torch.empty(2, dtype=torch.float32, device=dev)
+		rc = lib.elf_cross_entropy_loss(src.data_ptr(), ld, dense, target.data_ptr(), rows, V, ignore_index, scale, reduction == "mean",
+			row_loss.data_ptr(), loss.data_ptr(), dx, ld_out, scratch.data_ptr(), stream)
+		_lib.check(rc, "elf_cross_entropy_loss")
+		return loss, grad
 	if dense:
-		_lib.check(
-			lib.elf_cross_entropy_dense(src.data_ptr(), target.data_ptr(), rows, V, ignore_index, scale, div.data_ptr() if div is not None else None,
-				row_loss.data_ptr(), grad.data_ptr() if grad is not None else None, stream),
-			"elf_cross_entropy_dense",
-		)
+		_lib.check(lib.elf_cross_entropy_dense(src.data_ptr(), target.data_ptr(), rows, V, ignore_index, scale, None, row_loss.data_ptr(), dx, stream), "elf_cross_entropy_dense")
 	else:
-		_lib.check(
-			lib.elf_cross_entropy(src.data_ptr(), ld, target.data_ptr(), rows, V, ignore_index, scale, div.data_ptr() if div is not None else None,
-				row_loss.data_ptr(), grad.data_ptr() if grad is not None else None, ld_out, stream),
-			"elf_cross_entropy",
-		)
-	_lib.check(lib.elf_cross_entropy_reduce(row_loss.data_ptr(), target.data_ptr(), rows, ignore_index, out2.data_ptr(), stream), "elf_cross_entropy_reduce")
-	return row_loss, out2, grad
-
-
-def _reduced(row_loss, out2, reduction, shape):
-	if reduction == "sum":
-		return out2[0].clone()
-	if reduction == "mean":
-		return out2[0] / out2[1]
-	if reduction == "none":
-		return row_loss.view(shape)
-	raise ValueError(f"{reduction} is not a valid value for reduction")
+		_lib.check(lib.elf_cross_entropy(src.data_ptr(), ld, target.data_ptr(), rows, V, ignore_index, scale, None, row_loss.data_ptr(), dx, ld_out, stream), "elf_cross_entropy")
+	return row_loss.view(pred.shape[:-1]), grad
 
 
 _has_storage, _wrapped, _dispatch_modes = torch._C._has_storage, torch._C._functorch.is_functorch_wrapped_tensor, torch._C._len_torch_dispatch_stack
@@ -109,9 +95,9 @@ def _plain(t):
 class _CrossEntropy(torch.autograd.Function):
 	@staticmethod
 	def forward(ctx, pred, target, reduction, ignore_index):
-		row_loss, out2, grad = _run(pred, target, ignore_index=ignore_index, scale=1.0, mean=reduction == "mean", want_grad=ctx.needs_input_grad[0], padded=False)
-		ctx.grad, ctx.shape, ctx.per_row = grad, pred.shape, reduction == "none"
-		return _reduced(row_loss, out2, reduction, pred.shape[:-1])
+		loss, ctx.grad = _run(pred, target, ignore_index=ignore_index, scale=1.0, reduction=reduction, want_grad=ctx.needs_input_grad[0], padded=False)
+		ctx.shape, ctx.per_row = pred.shape, reduction == "none"
+		return loss
 
 	@staticmethod
 	def backward(ctx, g):
@@ -132,8 +118,7 @@ def cross_entropy(pred, target, reduction="mean", ignore_index=-100):
 	bf16 GPU logits ``[..., V]`` and int64 class indices ``[...]``; differentiable w.r.t. ``pred``."""
 	if pred.requires_grad and torch.is_grad_enabled():
 		return _CrossEntropy.apply(pred, target, reduction, ignore_index)
-	row_loss, out2, _ = _run(pred, target, ignore_index=ignore_index, scale=1.0, mean=reduction == "mean", want_grad=False)
-	return _reduced(row_loss, out2, reduction, pred.shape[:-1])
+	return _run(pred, target, ignore_index=ignore_index, scale=1.0, reduction=reduction, want_grad=False)[0]
 
 
 def _loss_and_grad(pred, target, reduction="sum", ignore_index=-100, scale=1.0):
@@ -143,9 +128,9 @@ def _loss_and_grad(pred, target, reduction="sum", ignore_index=-100, scale=1.0):
 	in place."""
 	if reduction not in ("sum", "mean"):
 		raise ValueError("loss_and_grad needs a scalar loss: reduction must be 'sum' or 'mean'")
-	row_loss, out2, grad = _run(pred, target, ignore_index=ignore_index, scale=scale, mean=reduction == "mean", want_grad=True)
+	loss, grad = _run(pred, target, ignore_index=ignore_index, scale=scale, reduction=reduction, want_grad=True)
 	V = pred.shape[-1]
-	return _reduced(row_loss, out2, reduction, None), grad.view(*pred.shape[:-1], -1)[..., :V]
+	return loss, grad.view(*pred.shape[:-1], -1)[..., :V]
 
 
 cross_entropy.loss_and_grad = _loss_and_grad

@@ -229,6 +229,11 @@ int elf_cross_entropy_dense(const void* logits, const void* target, int64_t rows
  * loss multiplied by the gradient that arrives at it. */
 int elf_scale_by_bf16(const void* x, const void* g_f32, void* y, int64_t n, void* stream);
 int elf_cross_entropy_reduce(const void* row_loss, const void* target, int64_t rows, int64_t ignore_index, void* out2, void* stream);
+/* The whole of a reduced loss: elf_cross_entropy (dense != 0: elf_cross_entropy_dense) with row_loss and, where dlogits is not
+ * NULL, the gradient of the sum or, mean != 0, of the mean over the rows that are not ignored, times scale; and loss (fp32) = that
+ * sum or mean, unscaled.  scratch2: two floats.  The bits of those calls and elf_cross_entropy_reduce's. */
+int elf_cross_entropy_loss(const void* logits, int64_t ld, int dense, const void* target, int64_t rows, int64_t V, int64_t ignore_index,
+                           float scale, int mean, void* row_loss, void* loss, void* dlogits, int64_t ld_out, void* scratch2, void* stream);
 
 /* ---------------------------------------------------------------------------------------------
  * Attention on the packed projection layout: q/k/v/o are column slices of [T, ld*] bf16 buffers,
