@@ -66,6 +66,11 @@ static constexpr TileTime TILES_MID[] = {{224, 256, 1.01f, 11.1f, 0.f}, {192, 25
 // K of at most RING_SHORT_K: the small tiles on the ring of two slices
 static constexpr TileTime TILES_SHORT[] = {{256, 256, 1.293f, 7.15f, 2.5f}, {128, 256, 0.996f, 4.9f, 0.44f}, {128, 128, 0.388f, 1.94f, 3.5f},
                                                   {64, 128, 0.285f, 0.93f, 3.7f}, {128, 64, 0.325f, 1.0f, 2.4f}, {64, 64, 0.184f, 0.55f, 2.9f}};
+// 32x32 tiles, K beyond RING_SHORT_K and up to it: a k-contiguous A, bf16 outputs, no more tiles than compute units.  A slice of the 64x64
+// tile is 16 KB through a compute unit's path into LDS, one of these 8, and four times as many units take part.  GPU time alone, 64x64 ->
+// 32x32 (us): 512 x 512 x 1536 7.4 -> 4.8 (B reduction-major 7.7 -> 6.0), 512 x 512 x 512 4.2 -> 3.4, 512 x 256 x 1024 5.1 -> 3.9, 128 x
+// 256 x 64 2.8 -> 2.6; with two rounds of them 1024 x 512 x 1024 5.8 and 5.6 (reduction-major 6.1 and 6.6), 768 x 768 x 768 5.3 and 6.9.
+static constexpr TileTime TILE_TINY = {32, 32, 0.11f, 1.2f, 1.3f}, TILE_TINY_SHORT = {32, 32, 0.1f, 0.5f, 2.9f};
 // weight gradients: both operands reduction-major, fp32 read-modify-write of the output
 static constexpr TileTime TILES_F32[] = {{256, 256, 1.3f, 22.f, 0.f}, {128, 256, 0.757f, 12.9f, 0.f}, {128, 128, 0.537f, 9.9f, 0.f},
                                                 {64, 128, 0.442f, 5.9f, 0.f}, {128, 64, 0.416f, 7.5f, 0.f}, {64, 64, 0.26f, 4.f, 0.f}};
@@ -82,10 +87,11 @@ static float tile_us(const TileTime& t, int M, int N, int slices, int k_splits =
 	return rounds * ((slices + k_splits - 1) / k_splits * t.slice + t.round) + t.launch;
 }
 
-// The tile of a bf16 output with the smallest estimate.  mid: the tiles between 128 and 256 rows are to be had.  For an epilogue
+// The tile of a bf16 output with the smallest estimate.  mid: the tiles between 128 and 256 rows are to be had, tiny: those of 32x32
+// (left out where a product and a pass are weighed against a fused epilogue, which saves more than those tiles do).  For an epilogue
 // that only the 256-column tiles have: epi_extra, its time per round of 256x256 tiles, and ring_extra, the time of the pass of its
 // own that the small ring tiles need instead.
-static Plan plan_tiles(int M, int N, int K, bool mid = true, float ring_extra = 0.f, float epi_extra = 0.f) {
+static Plan plan_tiles(int M, int N, int K, bool mid = true, float ring_extra = 0.f, float epi_extra = 0.f, bool tiny = false) {
 	Plan best;
 	auto weigh = [&](TileTime t) {
 		if (M < t.bm || N < t.bn) return;
@@ -93,6 +99,7 @@ static Plan plan_tiles(int M, int N, int K, bool mid = true, float ring_extra = 
 		const float us = tile_us(t, M, N, K / BK) + (t.bn == 256 ? 0.f : ring_extra);
 		if (us < best.us) best = Plan{t.bm, t.bn, 1, us};
 	};
+	if (tiny && (int64_t)(M / 32) * (N / 32) <= 256) weigh(K <= RING_SHORT_K ? TILE_TINY_SHORT : TILE_TINY);
 	if (K <= RING_SHORT_K) {
 		for (const TileTime& t : TILES_SHORT) weigh(t);
 		return best;
@@ -193,7 +200,8 @@ int gemm_bf16(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda,
 	if (bm == 0) {
 		Plan p;
 		if (epi != EPI_F32_ACC) {
-			p = plan_tiles(M, N, K, !a_t && (epi == EPI_BF16 || epi == EPI_BF16_RESID));
+			const bool bf16_out = !a_t && (epi == EPI_BF16 || epi == EPI_BF16_RESID);
+			p = plan_tiles(M, N, K, bf16_out, 0.f, 0.f, bf16_out);
 		} else if (k_splits > 0) {
 			p = plan_weight_gradient(M, N, K, 1);
 		} else if (M >= 256 && N >= 256 && (int64_t)((M + 255) / 256) * ((N + 255) / 256) >= 192 && K >= 4096) {
@@ -441,7 +449,7 @@ int gemm_way(int product, int M, int N, int K, int D) {
 	Plan p;
 	if (M < 64 || N < 64 || K < 64 || M % 64 || N % 64 || K % 64) return 0;
 	switch (product) {
-		case GEMM_WAY_FORWARD: case GEMM_WAY_INPUT_GRADIENT: p = plan_tiles(M, N, K); break;
+		case GEMM_WAY_FORWARD: case GEMM_WAY_INPUT_GRADIENT: p = plan_tiles(M, N, K, true, 0.f, 0.f, true); break;
 		case GEMM_WAY_GELU: p = act_plan(ACT_GELU, M, N, K, true); break;
 		case GEMM_WAY_SWIGLU: p = act_plan(ACT_SWIGLU, M, N, K, true); break;
 		case GEMM_WAY_GELU_BWD: if (gemm_gelu_bwd_fused(M, N, K)) p = Plan{64, 64}; break;

@@ -1,4 +1,4 @@
-// bf16 MFMA GEMM on small tiles (128x128, 64x128, 128x64, 64x64) with a deep ring of K slices in LDS, for gfx950.
+// bf16 MFMA GEMM on small tiles (128x128, 64x128, 128x64, 64x64, 32x32) with a deep ring of K slices in LDS, for gfx950.
 //
 // Same contraction, layouts and order of products along K as gemm_dma_tile.h (v_mfma_f32_16x16x32_bf16, 64 wide K slices in
 // ascending order), so a tile's bits do not depend on which of the kernels computed it.  These are the tiles of products
@@ -54,7 +54,8 @@ static __device__ unsigned int turn_giveups;
 template <int BM, int BN, bool SHORT>
 struct Shape {
 	static constexpr int A_BYTES = BM * BKS * 2, B_BYTES = BN * BKS * 2, STAGE_BYTES = A_BYTES + B_BYTES;
-	static constexpr int NST = SHORT ? 2 : BM == 64 && BN == 64 ? 8 : BM == 128 && BN == 128 ? 4 : 6;  // 128 .. 144 KiB of slices
+	// 128 .. 144 KiB of slices (of the 32x32 tile 64, as many of them as of the 64x64 one; 32 KiB of it if SHORT)
+	static constexpr int NST = SHORT ? BM == 32 ? 4 : 2 : BM <= 64 && BN <= 64 ? 8 : BM == 128 && BN == 128 ? 4 : 6;
 	static constexpr int LOADS_A = A_BYTES / 4096, LOADS_B = B_BYTES / 4096, LOADS = LOADS_A + LOADS_B;  // 1 KiB pieces per wave and slice
 	static constexpr int SMEM = NST * STAGE_BYTES + (LOADS_A > LOADS_B ? LOADS_A : LOADS_B) * 1024;
 };
@@ -367,6 +368,18 @@ __device__ __forceinline__ void gemm_ring_tile(const Args& g, const int pid, con
 					}
 				}
 		} else if constexpr (EPI == EPI_BF16 || EPI == EPI_BF16_RESID) {
+			if constexpr (CF == 1) {  // 32x32 tiles: one 16-column slab, four columns per lane
+				static_assert(RF == 1, "one slab");
+				bf16x4 rs{}, o;
+				if constexpr (EPI == EPI_BF16_RESID) rs = *reinterpret_cast<const bf16x4*>(g.R + (int64_t)row0 * g.ldr + col0 + 4 * g4);
+#pragma unroll
+				for (int t = 0; t < 4; t++) {
+					float v = acc[0][0][t];
+					if constexpr (EPI == EPI_BF16_RESID) v += (float)rs[t];
+					o[t] = (bf16_t)v;
+				}
+				*reinterpret_cast<bf16x4*>(reinterpret_cast<bf16_t*>(g.C) + (int64_t)row0 * g.ldc + col0 + 4 * g4) = o;
+			} else {
 			static_assert(CF % 2 == 0, "slabs are stored in pairs");
 			const int c = col0 + 16 * (g4 & 1) + 8 * (g4 >> 1);
 			bf16x8 rs[EPI == EPI_BF16_RESID ? RF : 1][CF / 2];
@@ -393,6 +406,7 @@ __device__ __forceinline__ void gemm_ring_tile(const Args& g, const int pid, con
 					// tile's 4 to 5 (128x64, K = 64: 128 x 9344 4.33 -> 4.50 us that way; a d = 256 GPT stage 2.80 -> 2.83 ms)
 					__builtin_amdgcn_sched_barrier(0);
 				}
+			}
 		} else {
 			constexpr bool ACCUM = EPI == EPI_F32_ACC || EPI == EPI_F32_ACC_SCALE;
 			float* const cp = reinterpret_cast<float*>(g.C) + (int64_t)row0 * g.ldc + col0 + 4 * g4;
@@ -500,6 +514,13 @@ static int launch_epi(const Args& g, int epi, hipStream_t stream) {
 	return -1;
 }
 
+// 32x32 tiles: bf16 outputs with a k-contiguous A
+template <bool BT>
+static int launch_tiny(const Args& g, int epi, hipStream_t stream) {
+	if (epi == EPI_BF16) return g.K <= RING_SHORT_K ? launch<32, 32, false, BT, EPI_BF16, true>(g, stream) : launch<32, 32, false, BT, EPI_BF16, false>(g, stream);
+	return g.K <= RING_SHORT_K ? launch<32, 32, false, BT, EPI_BF16_RESID, true>(g, stream) : launch<32, 32, false, BT, EPI_BF16_RESID, false>(g, stream);
+}
+
 template <int BM, int BN>
 static int launch_layout(Args& g, int a_t, int b_t, int epi, hipStream_t stream) {
 	ELF_REQUIRE(g.M >= BM && g.N >= BN, "gemm (ring tile): M at least %d and N at least %d", BM, BN);
@@ -532,6 +553,10 @@ int gemm_bf16_ring(int a_t, int b_t, int M, int N, int K, const void* A, int64_t
 	if (bm == 64 && bn == 128) return ring::launch_layout<64, 128>(g, a_t, b_t, epi, stream);
 	if (bm == 128 && bn == 64) return ring::launch_layout<128, 64>(g, a_t, b_t, epi, stream);
 	if (bm == 64 && bn == 64) return ring::launch_layout<64, 64>(g, a_t, b_t, epi, stream);
+	if (bm == 32 && bn == 32) {
+		g.tiles_m = M / 32, g.tiles_n = N / 32, g.k_splits = 1;
+		if (!a_t && (epi == EPI_BF16 || epi == EPI_BF16_RESID)) return b_t ? ring::launch_tiny<true>(g, epi, stream) : ring::launch_tiny<false>(g, epi, stream);
+	}
 	set_error("gemm (ring tile): unknown tile %dx%d", bm, bn);
 	return -1;
 }

@@ -34,6 +34,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 // (two k rows span the banks): the same for pairs of rows
 template <int ROWS = 256>
 __device__ __forceinline__ int t_swz(int k) {
+	if constexpr (ROWS == 32) return ((k >> 3) & 1) << 1;  // (four k rows span the banks: rows k and k + 8 take different halves)
 	if constexpr (ROWS == 64) return (((k >> 1) & 1) << 2) ^ (((k >> 3) & 1) << 1);
 	return ((k & (ROWS == 256 ? 7 : 3)) << 2) ^ (((k >> 3) & 1) << 1);
 }

@@ -965,6 +965,27 @@ def test_parameter_gradients_of_a_list_of_layers(K, T, shapes):
 	assert torch.allclose(bias.double(), 2 * dy.double().sum(0), rtol=1e-4, atol=1e-3)
 
 
+@pytest.mark.parametrize("M,N", [(64, 64), (512, 512), (128, 2048), (64, 4096)])
+@pytest.mark.parametrize("Kd", [64, 256, 320, 1024, 3136])
+@pytest.mark.parametrize("b_t", [False, True])
+def test_products_on_32x32_tiles_have_the_bits_of_larger_ones(K, M, N, Kd, b_t):
+	"""Products of at most 256 tiles of 32x32: one tile and a full round of them, K of one slice, of the short ring's last and the deep
+	ring's first, of many.  A tile adds its products in the order of K whatever its size: the bits of the 64x64 tile, without and with a
+	residual and a bias, in rows of its own width and further apart."""
+	a = _randn(M, Kd, seed=700)
+	b = _randn(Kd, N, seed=701) if b_t else _randn(N, Kd, seed=701)
+	res, bias = _randn(M, N, seed=702), _randn(1, N, seed=703)
+	assert K.gemm_way(K.WAY_INPUT_GRADIENT if b_t else K.WAY_FORWARD, M, N, Kd) == (32, 32)
+	for kw in ({}, {"epilogue": K.EPI_BF16_RESID, "residual": res}, {"epilogue": K.EPI_BF16_RESID, "residual": bias, "residual_ld": 0}):
+		want = K.gemm(a, b, b_t=b_t, tile_cfg=12, **kw)
+		assert torch.equal(K.gemm(a, b, b_t=b_t, **kw), want)
+		wide = torch.full((M, N + 24), 7.0, dtype=torch.bfloat16, device="cuda")
+		K.gemm(a, b, b_t=b_t, out=wide[:, 3 : N + 3], **kw)
+		assert torch.equal(wide[:, 3 : N + 3], want) and float((wide[:, :3] - 7).abs().max()) == 0 and float((wide[:, N + 3 :] - 7).abs().max()) == 0
+	ref = a.double() @ (b.double() if b_t else b.double().t())
+	_close(K.gemm(a, b, b_t=b_t), ref.float(), what="32x32 tile")
+
+
 def test_split_k_on_one_stream_never_gives_up_its_turn_and_wide_splits_are_refused(K):
 	"""Back-to-back split-K launches on one stream keep their turns (the counter of waves that added out of turn does not
 	move, which is what bit-reproducible weight gradients rest on), and a split count that would not fit the 8 bits the
