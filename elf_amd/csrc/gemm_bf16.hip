@@ -63,6 +63,12 @@ static constexpr TileTime TILES_BF16[] = {{256, 256, 1.18f, 6.f, 0.f}, {128, 256
                                           {128, 64, 0.341f, 1.9f, 1.f}, {64, 64, 0.213f, 1.5f, 1.3f}};
 // the tiles between 128 and 256 rows (k-contiguous A and bf16 outputs only)
 static constexpr TileTime TILES_MID[] = {{224, 256, 1.01f, 11.1f, 0.f}, {192, 256, 0.938f, 6.5f, 0.f}, {160, 256, 0.854f, 6.2f, 0.f}};
+// 128x192: a k-contiguous A, bf16 outputs, no more tiles than compute units.  Outputs of which 128x256 tiles leave compute units idle (64 x 3
+// of them for 8192 x 768) and 128x128 ones make a second round.  Best tile before -> now, k-contiguous B / reduction-major B (us): 8192 x 768 x
+// 768 14.6 -> 13.7 / 15.0 -> 14.6, x 3072 42.3 -> 38.8 / 41.5 -> 39.1, 896 x 6208 x 4160 66.6 -> 61.3 / 64.4 -> 60.3, 2560 x 1664 x 320 9.3 ->
+// 8.4 / 9.8 -> 8.8.  More than a round of them gained nothing on 25 sizes (15 % more operand bytes a product than 128x256), and
+// 256x192 tiles nothing on 59 of 60.
+static constexpr TileTime TILE_192 = {128, 192, 0.68f, 5.1f, 0.f};
 // K of at most RING_SHORT_K: the small tiles on the ring of two slices
 static constexpr TileTime TILES_SHORT[] = {{256, 256, 1.293f, 7.15f, 2.5f}, {128, 256, 0.996f, 4.9f, 0.44f}, {128, 128, 0.388f, 1.94f, 3.5f},
                                                   {64, 128, 0.285f, 0.93f, 3.7f}, {128, 64, 0.325f, 1.0f, 2.4f}, {64, 64, 0.184f, 0.55f, 2.9f}};
@@ -78,7 +84,7 @@ static constexpr TileTime TILES_F32[] = {{256, 256, 1.3f, 22.f, 0.f}, {128, 256,
 struct Plan {
 	int bm = 0, bn = 0, k_splits = 1;
 	float us = 1e30f;
-	bool dma() const { return bn == 256; }
+	bool dma() const { return bn >= 192; }
 };
 
 static float tile_us(const TileTime& t, int M, int N, int slices, int k_splits = 1) {
@@ -87,11 +93,11 @@ static float tile_us(const TileTime& t, int M, int N, int slices, int k_splits =
 	return rounds * ((slices + k_splits - 1) / k_splits * t.slice + t.round) + t.launch;
 }
 
-// The tile of a bf16 output with the smallest estimate.  mid: the tiles between 128 and 256 rows are to be had, tiny: those of 32x32
-// (left out where a product and a pass are weighed against a fused epilogue, which saves more than those tiles do).  For an epilogue
+// The tile of a bf16 output with the smallest estimate.  mid: the tiles between 128 and 256 rows are to be had, plain: those of
+// 32x32 and 128x192 (left out where a product and a pass are weighed against a fused epilogue, which saves more than those tiles do).  For an epilogue
 // that only the 256-column tiles have: epi_extra, its time per round of 256x256 tiles, and ring_extra, the time of the pass of its
 // own that the small ring tiles need instead.
-static Plan plan_tiles(int M, int N, int K, bool mid = true, float ring_extra = 0.f, float epi_extra = 0.f, bool tiny = false) {
+static Plan plan_tiles(int M, int N, int K, bool mid = true, float ring_extra = 0.f, float epi_extra = 0.f, bool plain = false) {
 	Plan best;
 	auto weigh = [&](TileTime t) {
 		if (M < t.bm || N < t.bn) return;
@@ -99,12 +105,13 @@ static Plan plan_tiles(int M, int N, int K, bool mid = true, float ring_extra = 
 		const float us = tile_us(t, M, N, K / BK) + (t.bn == 256 ? 0.f : ring_extra);
 		if (us < best.us) best = Plan{t.bm, t.bn, 1, us};
 	};
-	if (tiny && (int64_t)(M / 32) * (N / 32) <= 256) weigh(K <= RING_SHORT_K ? TILE_TINY_SHORT : TILE_TINY);
+	if (plain && (int64_t)(M / 32) * (N / 32) <= 256) weigh(K <= RING_SHORT_K ? TILE_TINY_SHORT : TILE_TINY);
 	if (K <= RING_SHORT_K) {
 		for (const TileTime& t : TILES_SHORT) weigh(t);
 		return best;
 	}
 	for (const TileTime& t : TILES_BF16) weigh(t);
+	if (plain && (int64_t)((M + 127) / 128) * ((N + 191) / 192) <= 256) weigh(TILE_192);
 	if (mid)
 		for (const TileTime& t : TILES_MID)
 			if (t.bm > 160 || K > 1024 || epi_extra > 0.f || (int64_t)((M + 159) / 160) * ((N + 255) / 256) <= 256) weigh(t);
@@ -215,7 +222,7 @@ int gemm_bf16(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda,
 	}
 	if (epi != EPI_F32_ACC) k_splits = 1;
 	if (bm == 256 && k_splits <= 0) dw_split_plan(M, N, K, &k_splits, &tail_tiles);
-	if (bn == 256) return gemm_bf16_dma(a_t, b_t, M, N, K, A, lda, B, ldb, C, ldc, epi, R, ldr, k_splits < 1 ? 1 : k_splits, tail_tiles, bm, stream);
+	if (bn >= 192) return gemm_bf16_dma(a_t, b_t, M, N, K, A, lda, B, ldb, C, ldc, epi, R, ldr, k_splits < 1 ? 1 : k_splits, tail_tiles, bm, stream, nullptr, 0, nullptr, 0, 0, 0, 1.f, bn);
 	return gemm_bf16_ring(a_t, b_t, M, N, K, A, lda, B, ldb, C, ldc, epi, R, ldr, k_splits, bm, bn, stream);
 }
 

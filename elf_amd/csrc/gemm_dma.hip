@@ -111,11 +111,13 @@ int dma_turn_giveups(uint64_t* out) {
 // Arguments are validated by gemm_bf16() before it dispatches here.
 int gemm_bf16_dma(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb, void* C,
                   int64_t ldc, int epi, const void* R, int64_t ldr, int k_splits, int tail_tiles, int bm, hipStream_t stream,
-                  void* C2, int64_t ldc2, const void* rope_cs, int rope_S, int rope_cols, int rope_D, float scale) {
+                  void* C2, int64_t ldc2, const void* rope_cs, int rope_S, int rope_cols, int rope_D, float scale, int bn) {
 	ELF_REQUIRE(bm == 256 || bm == 128 || (!a_t && gemm_mid_rows(bm)), "gemm (dma tile): 256- or 128-row tiles, 160, 192 or 224 rows with a k-contiguous A");
-	ELF_REQUIRE(M >= bm && N >= dma::BN && M % 64 == 0 && N % 64 == 0 && K % dma::BKS == 0, "gemm (dma tile): M at least %d, N at least 256, all sizes multiples of 64", bm);
-	const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + dma::BN - 1) / dma::BN, ntiles = tiles_m * tiles_n;
-	ELF_REQUIRE(gemm_reaches(a_t ? dma::BKS : bm, lda) && gemm_reaches(b_t ? dma::BKS : dma::BN, ldb), "gemm (dma tile): leading dimension too large (%lld, %lld)", (long long)lda, (long long)ldb);
+	ELF_REQUIRE(bn == dma::BN || (bn == 192 && !a_t && bm == 128 && (epi == EPI_BF16 || epi == EPI_BF16_RESID)),
+	            "gemm (dma tile): 256 columns, 192 with 128 rows of a k-contiguous A and a bf16 output");
+	ELF_REQUIRE(M >= bm && N >= bn && M % 64 == 0 && N % 64 == 0 && K % dma::BKS == 0, "gemm (dma tile): M at least %d, N at least %d, all sizes multiples of 64", bm, bn);
+	const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + bn - 1) / bn, ntiles = tiles_m * tiles_n;
+	ELF_REQUIRE(gemm_reaches(a_t ? dma::BKS : bm, lda) && gemm_reaches(b_t ? dma::BKS : bn, ldb), "gemm (dma tile): leading dimension too large (%lld, %lld)", (long long)lda, (long long)ldb);
 	// a tile's columns are taken in heads: the last one may only move back by whole heads
 	ELF_REQUIRE(epi != EPI_BF16_ROPE || N % rope_D == 0, "gemm (dma tile): the RoPE epilogue needs N to be a multiple of the head width");
 	ELF_REQUIRE(epi != EPI_BF16_SWIGLU || (C2 && !a_t && !b_t), "gemm (dma tile): the SwiGLU epilogue needs k-contiguous operands and a second output");
@@ -144,13 +146,13 @@ int gemm_bf16_dma(int a_t, int b_t, int M, int N, int K, const void* A, int64_t 
 	// k-contiguous A (forward, dX): four waves with 128x128 wave tiles; both operands reduction-major (dW): eight
 	// waves with 64x128 wave tiles (with two transpose reads per fragment on both operands the lone wave wins on
 	// some shapes by 2-3 % and loses on most by 1-10 %)
-	if (!a_t && b_t) return dma::launch_rt(bm, a, epi, stream);
-	if (!a_t && bm == 256 && K / dma::BKS >= 2 && (epi == EPI_BF16 || epi == EPI_BF16_RESID || epi == EPI_BF16_SWIGLU) && !getenv("ELF_NO_PERSISTENT_GEMM")) {
+	if (!a_t && b_t) return dma::launch_rt(bm, bn, a, epi, stream);
+	if (!a_t && bm == 256 && bn == 256 && K / dma::BKS >= 2 && (epi == EPI_BF16 || epi == EPI_BF16_RESID || epi == EPI_BF16_SWIGLU) && !getenv("ELF_NO_PERSISTENT_GEMM")) {
 		// forward shapes: persistent workgroups, register epilogue (the QKV projection with its rotary epilogue stays on the
 		// one-tile kernel: with the table fetches in a lone wave's register epilogue the persistent form ran 3 % slower)
 		return dma::launch_pers(a, epi, stream);
 	}
-	if (!a_t) return dma::launch_rr(bm, a, epi, stream);
+	if (!a_t) return dma::launch_rr(bm, bn, a, epi, stream);
 	if (bm == 128) return dma::launch_tt<4, 4>(a, epi, stream);
 	if (int rc = dma::launch_tt<8, 4>(a, epi, stream)) return rc;
 	if (epi == EPI_F32_ACC_SCALE && a.tail_tiles > 0) {

@@ -47,7 +47,7 @@ __device__ __forceinline__ void mfma_init(f32x4& acc, const bf16x8& a, const bf1
 template <int EPI, bool EDGE>
 __global__ __launch_bounds__(256) void gemm_pers_kernel(Args g) {
 	using Sh = Shape<4, 8>;
-	constexpr int BM = 256, RF = 8, A_BYTES = Sh::A_BYTES, NSA = Sh::NSA, NSB = Sh::NSB;
+	constexpr int BM = 256, RF = 8, A_BYTES = Sh::A_BYTES, B_BYTES = Sh::B_BYTES, NSA = Sh::NSA, NSB = Sh::NSB;
 	constexpr int LOADS_A = Sh::LOADS_A, LOADS_B = Sh::LOADS_B;
 	constexpr bool PAIRED = EPI == EPI_BF16_SWIGLU;
 	static_assert(NSA == 2 && NSB == 3 && LOADS_A == 8 && LOADS_B == 8, "ring of two slices of A and three of B, 32 KiB each");

@@ -33,7 +33,18 @@ static int launch_mid(const Args& a, int epi, hipStream_t stream) {
 	return -1;
 }
 
-int launch_rt(int bm, const Args& a, int epi, hipStream_t stream) {
+// 128 rows and 192 columns: always clipped as well
+static int launch_192(const Args& a, int epi, hipStream_t stream) {
+	switch (epi) {
+		case EPI_BF16: return launch_sized<4, 4, false, true, EPI_BF16, true, 192>(a, stream);
+		case EPI_BF16_RESID: return launch_sized<4, 4, false, true, EPI_BF16_RESID, true, 192>(a, stream);
+	}
+	set_error("gemm: epilogue %d has no 192-column tile", epi);
+	return -1;
+}
+
+int launch_rt(int bm, int tn, const Args& a, int epi, hipStream_t stream) {
+	if (tn == 192) return launch_192(a, epi, stream);
 	switch (bm) {
 		case 128: return launch_epi<4>(a, epi, stream);
 		case 160: return launch_mid<5>(a, epi, stream);

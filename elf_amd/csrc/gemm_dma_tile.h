@@ -24,14 +24,15 @@ namespace elf {
 
 namespace dma {
 
-constexpr int BN = 256;
+constexpr int BN = 256;  // columns of a tile (192 where a kernel says so)
 constexpr int PERS_WORKGROUPS = 256;  // one per compute unit: the persistent kernel's grid
-constexpr int B_BYTES = BN * BKS * 2;  // 32 KiB per stage
 
 // Shape of one workgroup: NW waves arranged (NW / 2) x 2, each owning RF x 8 accumulator tiles of
-// 16 x 16, so the workgroup tile is BM x 256 with BM = (NW / 2) * RF * 16.
-template <int NW, int RF>
+// 16 x 16 (6 of them across in a tile of 192 columns), so the workgroup tile is BM x TN with BM = (NW / 2) * RF * 16.
+template <int NW, int RF, int TN = BN>
 struct Shape {
+	static constexpr int B_BYTES = TN * BKS * 2;
+	static constexpr int CH = TN / 64;  // 16-column slabs of a wave in either column half
 	static constexpr int BM = (NW / 2) * RF * 16;
 	static constexpr int STRIPS = (RF + 1) / 2;  // 32-row strips of a wave in the epilogue (the last of an odd RF has 16 rows)
 	static constexpr int A_BYTES = BM * BKS * 2;
@@ -137,11 +138,11 @@ __device__ __forceinline__ void mfma_acc(f32x4& acc, const bf16x8& a, const bf16
 
 
 // Origin (m0, n0) of tile `pid` of the launch: see "Tile assignment" in gemm_dma_kernel for the two walks.
-template <int BM>
+template <int BM, int TN = BN>
 __device__ __forceinline__ void tile_origin(const Args& g, int pid, int& m0, int& n0) {
 	if (g.walk == 2) {  // tiles in plain order, down the rows first (the launch places them on the XCDs itself)
 		m0 = (pid % g.tiles_m) * BM;
-		n0 = (pid / g.tiles_m) * BN;
+		n0 = (pid / g.tiles_m) * TN;
 		return;
 	}
 	const int ntiles = g.tiles_m * g.tiles_n;
@@ -162,7 +163,7 @@ __device__ __forceinline__ void tile_origin(const Args& g, int pid, int& m0, int
 		const bool pair = 2 * band + 1 < nsb_m;
 		const int sbm = 2 * band + (pair ? within & 1 : 0), sbn = pair ? within >> 1 : within;
 		m0 = (sbm * 8 + (jj & 7)) * BM;
-		n0 = (sbn * 4 + (jj >> 3)) * BN;
+		n0 = (sbn * 4 + (jj >> 3)) * TN;
 	} else {
 		if ((ntiles & 7) == 0) pid = (pid & 7) * (ntiles >> 3) + (pid >> 3);
 		constexpr int GROUP_M = 8;
@@ -170,7 +171,7 @@ __device__ __forceinline__ void tile_origin(const Args& g, int pid, int& m0, int
 		const int first_m = (pid / per_group) * GROUP_M;
 		const int gsz = min(g.tiles_m - first_m, GROUP_M);
 		m0 = (first_m + (pid % per_group) % gsz) * BM;
-		n0 = ((pid % per_group) / gsz) * BN;
+		n0 = ((pid % per_group) / gsz) * TN;
 	}
 }
 
@@ -178,10 +179,10 @@ __device__ __forceinline__ void tile_origin(const Args& g, int pid, int& m0, int
 // its neighbour does not (it needs M >= BM, N >= 256).  Every operand load stays inside the matrix without a bounds check
 // in the K loop, and the partly empty tile multiplies rows its neighbour multiplies as well instead of padding.  (M, N
 // multiples of 64: what is skipped are whole 32-row strips and whole 64-column halves.)
-template <int BM>
+template <int BM, int TN = BN>
 __device__ __forceinline__ void clip_tile(const Args& g, int& m0, int& n0) {
 	m0 = min(m0, g.M - BM);
-	n0 = min(n0, g.N - BN);
+	n0 = min(n0, g.N - TN);
 }
 
 // Tile, K range and turn counter of workgroup `bid` of the problem `g` (the block index of a launch with one problem).
@@ -211,10 +212,12 @@ __device__ __forceinline__ void locate_tile(const Args& g, const int bid, int& p
 // One workgroup: tile `pid` of the problem `g`, K range `ksplit` of `splits`; a split tile's turn counters are those of
 // `turn_slot`.
 // EDGE: M or N is no multiple of the tile (see clip_tile).
-template <int NW, int RF, bool AT, bool BT, int EPI, bool EDGE>
+template <int NW, int RF, bool AT, bool BT, int EPI, bool EDGE, int TN = BN>
 __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, const int ksplit, const int splits, const int turn_slot) {
-	using Sh = Shape<NW, RF>;
-	constexpr int BM = Sh::BM, A_BYTES = Sh::A_BYTES, STRIPS = Sh::STRIPS;
+	using Sh = Shape<NW, RF, TN>;
+	constexpr int BM = Sh::BM, A_BYTES = Sh::A_BYTES, B_BYTES = Sh::B_BYTES, STRIPS = Sh::STRIPS;
+	constexpr int CH = Sh::CH, WCOLS = TN / 2;  // columns of a wave
+	static_assert(TN == BN || EPI == EPI_BF16 || EPI == EPI_BF16_RESID, "the other epilogues are written for 256 columns");
 	constexpr int LOADS_A = Sh::LOADS_A, LOADS_B = Sh::LOADS_B, NSA = Sh::NSA, NSB = Sh::NSB;
 	constexpr bool PAIRED = EPI == EPI_BF16_SWIGLU;
 	static_assert(!PAIRED || !BT, "the paired row order is defined for a k-contiguous B");
@@ -235,11 +238,11 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 	//    the gate/up projection, 28672 x 4096 at K = 8192, A = 470 MB: 5-7 % faster).  A last, partly filled
 	//    round shares each 8 x 4 block between several XCDs.
 	int m0, n0;
-	tile_origin<BM>(g, pid, m0, n0);
+	tile_origin<BM, TN>(g, pid, m0, n0);
 	m0 = __builtin_amdgcn_readfirstlane(m0);
 	n0 = __builtin_amdgcn_readfirstlane(n0);
 	const int m_lo = m0, n_lo = n0;  // first row and column this tile stores
-	if constexpr (EDGE) clip_tile<BM>(g, m0, n0);
+	if constexpr (EDGE) clip_tile<BM, TN>(g, m0, n0);
 
 	const int nk_total = g.K / BKS;
 	const int nk_per = (nk_total + splits - 1) / splits;
@@ -276,7 +279,7 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 	const int64_t b_step = BT ? (int64_t)BKS * g.ldb : BKS;
 	uint32_t aoff[LOADS_A], boff[LOADS_B];
 	lane_offsets<AT, LOADS_A, false, BM>(wave, lane, g.lda, aoff);
-	lane_offsets<BT, LOADS_B, PAIRED>(wave, lane, g.ldb, boff, g.N / 2);
+	lane_offsets<BT, LOADS_B, PAIRED, TN>(wave, lane, g.ldb, boff, g.N / 2);
 
 	// this wave's first 1 KiB piece of each operand in stage 0
 	const uint32_t lds_a = lds_addr(smem) + wave * (LOADS_A * 1024);
@@ -297,11 +300,11 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 
 	// 16x16 accumulator tiles: RF down, 8 across (the 16x16x32 MFMA moves half as many accumulator
 	// registers per FLOP as the 32x32x16 one, and sustains a higher clock under the power limit)
-	f32x4 acc[RF][8];
+	f32x4 acc[RF][2 * CH];
 #pragma unroll
 	for (int i = 0; i < RF; i++)
 #pragma unroll
-		for (int j = 0; j < 8; j++)
+		for (int j = 0; j < 2 * CH; j++)
 #pragma unroll
 			for (int r = 0; r < 4; r++) acc[i][j][r] = 0.f;
 
@@ -311,7 +314,7 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 	// kt+1 sits before the LAST half-step of slice kt: by then every wave has read all of slice kt (its
 	// last fragments are in registers), so the same barrier frees its stages: the fetch of A's next slice for that
 	// stage goes out in the last half-step, that of B's in the first two of slice kt+1.
-	static_assert(pieces_have_slots(RF * 4, LOADS_A) && pieces_have_slots(RF * 4, LOADS_B / 2), "a half-step has too few even MFMA slots for its loads");
+	static_assert(pieces_have_slots(RF * CH, LOADS_A) && pieces_have_slots(RF * CH, LOADS_B / 2), "a half-step has too few even MFMA slots for its loads");
 	// slices 0 .. NSB-2 of B and 0 .. NSA-1 of A; slice 0 has to have landed
 	static_for<NSB>([&](auto sc) {
 		constexpr int S = decltype(sc)::value;
@@ -321,7 +324,7 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 	wait_vmcnt<(NSA - 1) * LOADS_A + (NSB - 2) * LOADS_B>();
 	__syncthreads();
 
-	bf16x8 fa[2][RF], fb[2][4];
+	bf16x8 fa[2][RF], fb[2][CH];
 	auto load_a = [&](int buf, int step, int kq) {
 		const unsigned char* sa = smem + (step % NSA) * A_BYTES;
 #pragma unroll
@@ -330,9 +333,9 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 	auto load_b = [&](int buf, int step, int kq, int h) {
 		const unsigned char* sb = smem + NSA * A_BYTES + (step % NSB) * B_BYTES;
 #pragma unroll
-		for (int j = 0; j < 4; j++) fb[buf][j] = frag<BT>(sb, wc * 128 + (h * 4 + j) * 16, kq, lane);
+		for (int j = 0; j < CH; j++) fb[buf][j] = frag<BT, TN>(sb, wc * WCOLS + (h * CH + j) * 16, kq, lane);
 	};
-	// One half-step: RF * 4 MFMAs with the fragment reads of the next half-step (one read per two MFMAs, B
+	// One half-step: RF * CH MFMAs with the fragment reads of the next half-step (one read per two MFMAs, or as many as it takes, B
 	// slabs first: they are needed first) and, in two of the four half-steps, half of this wave's loads of a
 	// slice dealt between them one at a time.  A lone wave per SIMD has nothing else to fill its issue
 	// gaps, and a wave that issues its loads in one burst (64 KiB per slice through a 64 B/clk path) sits in
@@ -342,7 +345,7 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 	// once (k32 half 0 of stage 0); the k32 half and the stage are compile-time here (the loop is unrolled by
 	// PERIOD slices, three or six) and go into the instructions' offset fields.  Those hold 16 bits: stage 2 of B lies 64 and
 	// 80 KiB up and costs an add per read, a third of B's reads.
-	uint32_t ta[AT ? RF : 1][2], tb[BT ? 8 : 1][2];
+	uint32_t ta[AT ? RF : 1][2], tb[BT ? 2 * CH : 1][2];
 	{
 		if constexpr (AT)
 #pragma unroll
@@ -354,8 +357,8 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 			}
 		if constexpr (BT)
 #pragma unroll
-			for (int i = 0; i < 8; i++) {
-				frag_t_offsets(wc * 128 + i * 16, lane, tb[i]);
+			for (int i = 0; i < 2 * CH; i++) {
+				frag_t_offsets<TN>(wc * WCOLS + i * 16, lane, tb[i]);
 				tb[i][0] += lds_addr(smem) + NSA * A_BYTES, tb[i][1] += lds_addr(smem) + NSA * A_BYTES;
 				asm volatile("" : "+v"(tb[i][0]), "+v"(tb[i][1]));
 			}
@@ -363,26 +366,29 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 	auto half_step = [&](int abuf, int bbuf, auto hc, int pb_buf, auto pb_stage, int pb_kq, int pb_h, bool pa, int pa_buf, auto pa_stage, int pa_kq,
 	                     const Loads& ld, auto dealt) {
 		// dealt: which loads go out in this half-step (0: none, 1: a slice of A, 2 and 3: the halves of a slice of B)
-		constexpr int DEALT = decltype(dealt)::value, NP = DEALT == 0 ? 0 : DEALT == 1 ? LOADS_A : LOADS_B / 2, H = decltype(hc)::value, NM = RF * 4;
+		constexpr int DEALT = decltype(dealt)::value, NP = DEALT == 0 ? 0 : DEALT == 1 ? LOADS_A : LOADS_B / 2, H = decltype(hc)::value, NM = RF * CH;
 		constexpr int SA = decltype(pa_stage)::value, SB = decltype(pb_stage)::value;
 		const unsigned char* sa = smem + SA * A_BYTES;
 		const unsigned char* sb = smem + NSA * A_BYTES + SB * B_BYTES;
 		if constexpr (NW == 8) __builtin_amdgcn_s_setprio(1);
 		static_for<NM>([&](auto nc) {
-			constexpr int n = decltype(nc)::value, i = n / 4, j = n % 4;
-			mfma_acc(acc[i][H * 4 + j], fa[abuf][i], fb[bbuf][j]);
-			if constexpr (n % 2 == 1) {
-				constexpr int r = n / 2;
-				if constexpr (r < 4) {
-					if constexpr (BT) fb[pb_buf][r] = frag_t_at(tb[pb_h * 4 + r], (uint32_t)(SB * B_BYTES + pb_kq * (32 * 512)));
-					else fb[pb_buf][r] = frag<BT>(sb, wc * 128 + (pb_h * 4 + r) * 16, pb_kq, lane);
-				} else if constexpr (r - 4 < RF) {
+			constexpr int n = decltype(nc)::value, i = n / CH, j = n % CH;
+			mfma_acc(acc[i][H * CH + j], fa[abuf][i], fb[bbuf][j]);
+			// reads [r0, r1) ride behind this MFMA: one behind every odd one, or, where those are too few (64 x 96 wave tiles), evenly dealt
+			constexpr bool ODD = NM / 2 >= CH + RF;
+			constexpr int r0 = ODD ? n / 2 : n * (CH + RF) / NM, r1 = ODD ? (n % 2 == 1 ? n / 2 + 1 : n / 2) : (n + 1) * (CH + RF) / NM;
+			static_for<r1 - r0>([&](auto rc) {
+				constexpr int r = r0 + decltype(rc)::value;
+				if constexpr (r < CH) {
+					if constexpr (BT) fb[pb_buf][r] = frag_t_at(tb[pb_h * CH + r], (uint32_t)(SB * B_BYTES + pb_kq * (32 * TN * 2)));
+					else fb[pb_buf][r] = frag<BT, TN>(sb, wc * WCOLS + (pb_h * CH + r) * 16, pb_kq, lane);
+				} else if constexpr (r - CH < RF) {
 					if (pa) {
-						if constexpr (AT) fa[pa_buf][r - 4] = frag_t_at(ta[r - 4], (uint32_t)(SA * A_BYTES + pa_kq * (32 * BM * 2)));
-						else fa[pa_buf][r - 4] = frag<AT, BM>(sa, wr * (RF * 16) + (r - 4) * 16, pa_kq, lane);
+						if constexpr (AT) fa[pa_buf][r - CH] = frag_t_at(ta[r - CH], (uint32_t)(SA * A_BYTES + pa_kq * (32 * BM * 2)));
+						else fa[pa_buf][r - CH] = frag<AT, BM>(sa, wr * (RF * 16) + (r - CH) * 16, pa_kq, lane);
 					}
 				}
-			}
+			});
 			constexpr int piece = NP == 0 ? -1 : piece_in_slot(n, NM, NP);
 			if constexpr (piece >= 0) {
 				if constexpr (DEALT == 1) piece_a(ld, std::integral_constant<int, piece>{});
@@ -449,12 +455,12 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 #pragma unroll
 		for (int ii = 0; ii < 2; ii++)
 #pragma unroll
-			for (int j = 0; j < 8; j++)
+			for (int j = 0; j < 2 * CH; j++)
 #pragma unroll
 				for (int r = 0; r < 4; r++)
 					if (ii * 16 < rows) ws[(ii * 16 + row_l + r) * PITCH + j * 16 + col_l] = acc[i * 2 + ii < RF ? i * 2 + ii : 0][j][r];
 		const int grow0 = m0 + wr * (RF * 16) + i * 32;
-		const int gcol0 = n0 + wc * 128;
+		const int gcol0 = n0 + wc * WCOLS;
 		if (EDGE && grow0 + (ROW_CLIP ? rows - 16 : 0) < m_lo) continue;  // the neighbouring tile's rows (the same strips for every K split of a tile)
 		const int c_lo = EDGE ? n_lo - gcol0 : 0;  // columns of the wave's 128 below c_lo are the neighbouring tile's
 		if constexpr (EPI == EPI_BF16_SWIGLU) {
@@ -565,7 +571,7 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 		} else if constexpr (EPI == EPI_BF16 || EPI == EPI_BF16_RESID) {
 			// the strip's residual values first, all loads in flight together: read inside the loop below each
 			// one would be awaited (a full trip to HBM) before the store that follows it in program order
-			if (EDGE && (lane & 15) * 8 < c_lo) continue;
+			if ((EDGE && (lane & 15) * 8 < c_lo) || (WCOLS < 128 && (lane & 15) * 8 >= WCOLS)) continue;
 			bf16x8 rs[EPI == EPI_BF16_RESID ? 8 : 1];
 			if constexpr (EPI == EPI_BF16_RESID) {
 #pragma unroll
@@ -659,20 +665,20 @@ __device__ __forceinline__ void gemm_dma_tile(const Args& g, const int pid, cons
 	}
 }
 
-template <int NW, int RF, bool AT, bool BT, int EPI, bool EDGE>
+template <int NW, int RF, bool AT, bool BT, int EPI, bool EDGE, int TN = BN>
 __global__ __launch_bounds__(NW * 64) void gemm_dma_kernel(Args g) {
 	int pid, ksplit, splits, turn_slot;
 	locate_tile(g, (int)blockIdx.x, pid, ksplit, splits, turn_slot);
-	gemm_dma_tile<NW, RF, AT, BT, EPI, EDGE>(g, pid, ksplit, splits, turn_slot);
+	gemm_dma_tile<NW, RF, AT, BT, EPI, EDGE, TN>(g, pid, ksplit, splits, turn_slot);
 }
 
-template <int NW, int RF, bool AT, bool BT, int EPI, bool EDGE>
+template <int NW, int RF, bool AT, bool BT, int EPI, bool EDGE, int TN = BN>
 static int launch_sized(const Args& a, hipStream_t stream) {
 	// the ring (the loads past the end of K go into its stages too) or, where that is more, the epilogue's 32 x 136 fp32 strip per wave
-	using Sh = Shape<NW, RF>;
+	using Sh = Shape<NW, RF, TN>;
 	constexpr int ring = Sh::RING_BYTES, epi = NW * 32 * 136 * 4;
 	constexpr int smem = ring > epi ? ring : epi;
-	auto kern = gemm_dma_kernel<NW, RF, AT, BT, EPI, EDGE>;
+	auto kern = gemm_dma_kernel<NW, RF, AT, BT, EPI, EDGE, TN>;
 	static bool attr_set = false;
 	if (!attr_set) {
 		ELF_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
@@ -690,8 +696,9 @@ static int launch(const Args& a, hipStream_t stream) {
 
 // Tiles of bm rows with a k-contiguous A, by the layout of B (gemm_dma_rr.hip, gemm_dma_rt.hip), and the persistent kernel for
 // EPI_BF16, EPI_BF16_RESID and EPI_BF16_SWIGLU (gemm_dma_pers.hip).
-int launch_rr(int bm, const Args& a, int epi, hipStream_t stream);
-int launch_rt(int bm, const Args& a, int epi, hipStream_t stream);
+// (tn: 256 columns, or 192 with 128 rows, EPI_BF16 and EPI_BF16_RESID)
+int launch_rr(int bm, int tn, const Args& a, int epi, hipStream_t stream);
+int launch_rt(int bm, int tn, const Args& a, int epi, hipStream_t stream);
 int launch_pers(const Args& a, int epi, hipStream_t stream);
 int rr_turn_giveups(uint64_t* sum);
 int rt_turn_giveups(uint64_t* sum);

@@ -34,6 +34,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 // (two k rows span the banks): the same for pairs of rows
 template <int ROWS = 256>
 __device__ __forceinline__ int t_swz(int k) {
+	if constexpr (ROWS == 192) return (((k >> 1) & 1) << 1) | (((k >> 3) & 1) << 2);  // (rows k and k + 2 start at the same bank)
 	if constexpr (ROWS == 32) return ((k >> 3) & 1) << 1;  // (four k rows span the banks: rows k and k + 8 take different halves)
 	if constexpr (ROWS == 64) return (((k >> 1) & 1) << 2) ^ (((k >> 3) & 1) << 1);
 	return ((k & (ROWS == 256 ? 7 : 3)) << 2) ^ (((k >> 3) & 1) << 1);
@@ -52,8 +53,8 @@ __device__ __forceinline__ void lane_offsets(int wave, int lane, int64_t ld, uin
 			const int64_t grow = PAIRED ? (row >> 7) * 64 + (row & 63) + ((row >> 6) & 1) * pair_rows : row;
 			off[i] = (uint32_t)((grow * ld + ((slot ^ ((row >> 1) & 7)) << 3)) * 2);
 		} else {
-			constexpr int CPR = ROWS / 8;  // 16-byte chunks per k row; a 1 KiB piece holds 64 / CPR k rows
-			const int krow = q * (64 / CPR) + lane / CPR, slot = lane % CPR;
+			constexpr int CPR = ROWS / 8;  // 16-byte chunks per k row; a 1 KiB piece holds 64 of them
+			const int krow = (q * 64 + lane) / CPR, slot = (q * 64 + lane) % CPR;
 			off[i] = (uint32_t)((krow * ld + ((slot ^ t_swz<ROWS>(krow)) << 3)) * 2);
 		}
 	}

@@ -38,7 +38,7 @@ int gemm_bf16(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda,
 int gemm_bf16_dma(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda, const void* B, int64_t ldb, void* C,
                   int64_t ldc, int epi, const void* R, int64_t ldr, int k_splits, int tail_tiles, int bm, hipStream_t stream,
                   void* C2 = nullptr, int64_t ldc2 = 0, const void* rope_cs = nullptr, int rope_S = 0, int rope_cols = 0, int rope_D = 0,
-                  float scale = 1.f);
+                  float scale = 1.f, int bn = 256);
 // The tile kernels address an operand with unsigned 32-bit byte offsets from the tile's first row: whether these reach the last of
 // `rows` rows (of a k-contiguous operand the tile's, of a reduction-major one the 64 of a K slice).
 inline bool gemm_reaches(int rows, int64_t ld) { return (int64_t)(rows - 1) * ld * 2 + 512 <= (int64_t(1) << 32); }

@@ -986,6 +986,23 @@ def test_products_on_32x32_tiles_have_the_bits_of_larger_ones(K, M, N, Kd, b_t):
 	_close(K.gemm(a, b, b_t=b_t), ref.float(), what="32x32 tile")
 
 
+@pytest.mark.parametrize("b_t", [False, True])
+@pytest.mark.parametrize("M, N, Kd", [(8192, 768, 768), (896, 6208, 4160), (2560, 1664, 320), (8128, 768, 1088)])
+def test_products_on_128x192_tiles_have_the_bits_of_smaller_ones(K, M, N, Kd, b_t):
+	"""Products of one round of 128x192 tiles: whole ones, a last column of tiles moved back by 64 and by 128 columns, a last row moved
+	back, K of few slices and of a number that is no multiple of the ring.  The bits of the 64x64 tile, as above."""
+	a = _randn(M, Kd, seed=710)
+	b = _randn(Kd, N, seed=711) if b_t else _randn(N, Kd, seed=711)
+	res, bias = _randn(M, N, seed=712), _randn(1, N, seed=713)
+	assert K.gemm_way(K.WAY_INPUT_GRADIENT if b_t else K.WAY_FORWARD, M, N, Kd) == (128, 192)
+	for kw in ({}, {"epilogue": K.EPI_BF16_RESID, "residual": res}, {"epilogue": K.EPI_BF16_RESID, "residual": bias, "residual_ld": 0}):
+		want = K.gemm(a, b, b_t=b_t, tile_cfg=12, **kw)
+		assert torch.equal(K.gemm(a, b, b_t=b_t, **kw), want)
+		wide = torch.full((M, N + 24), 7.0, dtype=torch.bfloat16, device="cuda")
+		K.gemm(a, b, b_t=b_t, out=wide[:, 3 : N + 3], **kw)
+		assert torch.equal(wide[:, 3 : N + 3], want) and float((wide[:, :3] - 7).abs().max()) == 0 and float((wide[:, N + 3 :] - 7).abs().max()) == 0
+
+
 def test_split_k_on_one_stream_never_gives_up_its_turn_and_wide_splits_are_refused(K):
 	"""Back-to-back split-K launches on one stream keep their turns (the counter of waves that added out of turn does not
 	move, which is what bit-reproducible weight gradients rest on), and a split count that would not fit the 8 bits the
