@@ -775,7 +775,8 @@ static int64_t dkv_part_bytes(const Splits& sp, int B, int S, int Hkv, int D) { 
 // Heads of 64 columns, short sequences in a launch that does not fill the chip: workgroups of 128 keys, two on a compute unit.
 // Constants in microseconds as measured.  Causal with one key tile (128 tokens): a walk has four steps a head, what a step and a
 // split cost beside the fixed part shows.  Constants of its own, fitted to every sharing of 250 such shapes (the one that is picked
-// takes 0.2 % longer than the best on average, 7 % at most; with those of longer walks 1.8 and 16 %).  The whole call, whole -> as
+// takes 0.2 % longer than the best on average, 7 % at most; with those of longer walks 1.8 and 16 %).  (Where one_kernel_pays() nothing is
+// shared, the workspace query asks for the room all the same.)  The whole call, whole -> as
 // shared now (us): 2 x 128 tokens, 4 heads of 64 18.9 -> 16.7; 3 x 128, 48 / 16 heads of 128 34.8 -> 31.2; 7 x 128, 36 / 12 heads
 // of 128 stay whole: 37.8, three ways 40.6.
 static Splits split_short(int B, int S, int Hq, int Hkv, int D, bool causal, int64_t room) {
@@ -811,6 +812,21 @@ static Splits split_short(int B, int S, int Hq, int Hkv, int D, bool causal, int
 		}
 	}
 	return best;
+}
+
+// 128 tokens: one kernel for the whole call (attention_bwd_one.hip) or -delta, walks and sums in three.  A workgroup of the one kernel has a compute
+// unit to itself and takes the query heads of its group in turn (4.3 us each for heads of 64, 7.3 of 128; 6 and 7 us besides), the walks
+// are shared.  Whole call of every sort of group on 2 to 1600 workgroups, three kernels -> one (us, causal / not):
+//   one head of 64 a group: 16 groups 16.8 -> 10.8 / 16.1 -> 11.0, 240 24.8 -> 13.3 / 20.6 -> 13.8, 272 29.8 -> 23.4 / 25.3 -> 24.2, 800 59.1 -> 49.8 / 48.8 -> 51.4
+//   one of 128: 16 20.3 -> 15.7 / 20.6 -> 17.1, 240 32.2 -> 22.7 / 31.3 -> 26.0, 800 94.8 -> 79.1 / 91.9 -> 90.3
+//   four of 64: 32 24.4 and 24.5 / 21.6 and 25.1, 96 35.8 -> 26.4 / 30.4 -> 27.1, 320 63.8 -> 55.7 / 58.0 and 58.3
+//   four of 128: 64 37.6 and 41.5 / 41.3 and 45.3, 96 47.4 -> 43.6 / 46.2 and 48.1, 256 67.3 -> 57.3 / 66.8 and 64.4
+//   eight: 64 groups of 64 38.0 and 45.2, 128 58.2 -> 48.4 / 52.5 and 50.3; of 128 128 75.5 and 79.3, 320 173.5 and 179.9
+static bool one_kernel_pays(int B, int S, int Hq, int Hkv, int D, bool causal) {
+	const int64_t groups = (int64_t)B * Hkv, G = Hq / Hkv;
+	if (S != 128 || G > 8 || groups < (causal && D == 64 ? 16 : 32) * (G - 1)) return false;
+	if (causal) return groups <= 256 || G <= 4;
+	return D == 64 ? groups <= 256 : G == 1 || (G == 2 && groups <= 256);
 }
 
 // room: bytes there are for the partial sums.
@@ -888,6 +904,11 @@ int attn_bwd(const void* q, const void* k, const void* v, const void* o, const v
 	ELF_REQUIRE(((uintptr_t)o % 16) == 0 && ((uintptr_t)dO % 16) == 0, "attn_bwd: o and dO must be 16-byte aligned");
 	ProfScope prof(PROF_ATTN_BWD, (causal ? 4.0 : 8.0) * B * Hq * (double)S * S * D, stream);
 	const int64_t T = (int64_t)B * S;
+	if (one_kernel_pays(B, S, Hq, Hkv, D, causal != 0)) {
+		const AttnBwdArgs a{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)dO, nullptr, nullptr, nullptr,
+		                    (bf16_t*)dk, (bf16_t*)dv, ldq, ldk, ldv, lddo, lddk, lddv, B, S, Hq, Hkv, scale, (const float2*)rope_cs, 1, 1, nullptr, 0};
+		return launch_bwd_one(a, D, causal != 0, (const bf16_t*)o, (const float*)lse, (bf16_t*)dq, ldo, lddq, stream);
+	}
 	bf16_t* dq_part = (bf16_t*)workspace;
 	float* ndelta = (float*)(dq_part + (int64_t)B * part_rows(S, causal != 0, 128) * Hq * D);
 	float* nlse2 = ndelta + T * Hq;

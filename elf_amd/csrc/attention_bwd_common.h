@@ -137,56 +137,60 @@ __device__ __forceinline__ bf16x8 ds_t_frag(const unsigned char* t, int k0, int 
 	return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-// dK^T / dV^T accumulators of one wave -> memory: register r of tile dt <-> d = dt*32 + (r/4)*8 + 4g + r%4, lane <-> key.
-// With a rotary embedding on the k heads, dK (scaled and rounded to bf16, as a separate RoPE pass over the stored
+// dK^T, dV^T and dQ^T accumulators of one wave -> memory: register r of tile dt <-> d = dt*32 + (r/4)*8 + 4g + r%4, lane <-> token; p: the
+// token's row at the tile's first column.
+__device__ __forceinline__ void store_tile(const f32x16& acc, bf16_t* p, float scale, int g) {
+#pragma unroll
+	for (int r4 = 0; r4 < 4; r4++) {
+		bf16x4 o;
+#pragma unroll
+		for (int u = 0; u < 4; u++) o[u] = (bf16_t)(acc[r4 * 4 + u] * scale);
+		*reinterpret_cast<bf16x4*>(p + r4 * 8 + 4 * g) = o;
+	}
+}
+// With a rotary embedding on the heads, the gradient (scaled and rounded to bf16, as a separate RoPE pass over the stored
 // gradient would read it) is rotated back first; the partner of column d is d + D/2, same register of tile dt + DT/2.
+template <int D>
+__device__ __forceinline__ void store_tiles_rotated(const f32x16& acc_lo, const f32x16& acc_hi, bf16_t* p, float scale, int g, const float2* cs) {
+#pragma unroll
+	for (int r4 = 0; r4 < 4; r4++) {
+		const int i = r4 * 8 + 4 * g;
+		const f32x4 t0 = *reinterpret_cast<const f32x4*>(cs + i), t1 = *reinterpret_cast<const f32x4*>(cs + i + 2);
+		bf16x4 lo4, hi4;
+#pragma unroll
+		for (int u = 0; u < 4; u++) {
+			const float lo = (float)(bf16_t)(acc_lo[r4 * 4 + u] * scale), hi = (float)(bf16_t)(acc_hi[r4 * 4 + u] * scale);
+			const float c = (u < 2 ? t0 : t1)[(u & 1) * 2], sn = (u < 2 ? t0 : t1)[(u & 1) * 2 + 1];
+			float rl, rh;
+			rope_rot(lo, hi, c, -sn, rl, rh);
+			lo4[u] = (bf16_t)rl;
+			hi4[u] = (bf16_t)rh;
+		}
+		*reinterpret_cast<bf16x4*>(p + i) = lo4;
+		*reinterpret_cast<bf16x4*>(p + i + D / 2) = hi4;
+	}
+}
+template <int D>
+__device__ __forceinline__ void store_dk(const f32x16 (&acc)[D / 32], bf16_t* p, float scale, int g, const float2* cs_row) {
+	constexpr int DT = D / 32;
+	if (cs_row == nullptr) {
+#pragma unroll
+		for (int dt = 0; dt < DT; dt++) store_tile(acc[dt], p + dt * 32, scale, g);
+	} else {
+#pragma unroll
+		for (int dt = 0; dt < DT / 2; dt++) store_tiles_rotated<D>(acc[dt], acc[dt + DT / 2], p + dt * 32, scale, g, cs_row + dt * 32);
+	}
+}
+template <int D>
+__device__ __forceinline__ void store_dv(const f32x16 (&acc)[D / 32], bf16_t* p, int g) {
+#pragma unroll
+	for (int dt = 0; dt < D / 32; dt++) store_tile(acc[dt], p + dt * 32, 1.f, g);
+}
 template <int D>
 __device__ __forceinline__ void store_dk_dv(const f32x16 (&acc_dk)[D / 32], const f32x16 (&acc_dv)[D / 32], bf16_t* dkp, bf16_t* dvp, float scale, int g,
                                             const float2* cs_row) {
-	constexpr int DT = D / 32;
-#pragma unroll
-	for (int dt = 0; dt < DT; dt++) {
-#pragma unroll
-		for (int r4 = 0; r4 < 4; r4++) {
-			bf16x4 v4;
-#pragma unroll
-			for (int u = 0; u < 4; u++) v4[u] = (bf16_t)acc_dv[dt][r4 * 4 + u];
-			*reinterpret_cast<bf16x4*>(dvp + dt * 32 + r4 * 8 + 4 * g) = v4;
-		}
-	}
-	if (cs_row == nullptr) {
-#pragma unroll
-		for (int dt = 0; dt < DT; dt++) {
-#pragma unroll
-			for (int r4 = 0; r4 < 4; r4++) {
-				bf16x4 k4;
-#pragma unroll
-				for (int u = 0; u < 4; u++) k4[u] = (bf16_t)(acc_dk[dt][r4 * 4 + u] * scale);
-				*reinterpret_cast<bf16x4*>(dkp + dt * 32 + r4 * 8 + 4 * g) = k4;
-			}
-		}
-		return;
-	}
-#pragma unroll
-	for (int dt = 0; dt < DT / 2; dt++) {
-#pragma unroll
-		for (int r4 = 0; r4 < 4; r4++) {
-			const int i = dt * 32 + r4 * 8 + 4 * g;
-			const f32x4 t0 = *reinterpret_cast<const f32x4*>(cs_row + i), t1 = *reinterpret_cast<const f32x4*>(cs_row + i + 2);
-			bf16x4 lo4, hi4;
-#pragma unroll
-			for (int u = 0; u < 4; u++) {
-				const float lo = (float)(bf16_t)(acc_dk[dt][r4 * 4 + u] * scale), hi = (float)(bf16_t)(acc_dk[dt + DT / 2][r4 * 4 + u] * scale);
-				const float c = (u < 2 ? t0 : t1)[(u & 1) * 2], sn = (u < 2 ? t0 : t1)[(u & 1) * 2 + 1];
-				float rl, rh;
-				rope_rot(lo, hi, c, -sn, rl, rh);
-				lo4[u] = (bf16_t)rl;
-				hi4[u] = (bf16_t)rh;
-			}
-			*reinterpret_cast<bf16x4*>(dkp + i) = lo4;
-			*reinterpret_cast<bf16x4*>(dkp + i + D / 2) = hi4;
-		}
-	}
+	store_dv<D>(acc_dv, dvp, g);
+	store_dk<D>(acc_dk, dkp, scale, g, cs_row);
 }
 
 // The same accumulators as fp32 partial sums: dK at p, dV `stride` floats further on.
@@ -207,6 +211,8 @@ __device__ __forceinline__ void store_dkv_part(const f32x16 (&acc_dk)[D / 32], c
 
 // attention_bwd_wide.hip: passes over 256 keys, heads of 64 columns
 int launch_bwd_wide(const AttnBwdArgs& a, bool causal, dim3 grid, hipStream_t stream);
+// attention_bwd_one.hip: sequences of 128 tokens, the whole call
+int launch_bwd_one(const AttnBwdArgs& a, int D, bool causal, const bf16_t* o, const float* lse, bf16_t* dq, int64_t ldo, int64_t lddq, hipStream_t stream);
 
 }  // namespace attn
 }  // namespace elf

@@ -19,7 +19,8 @@
 // query tiles (32 queries at a time) of every query head in the group; dS^T goes through LDS,
 // each wave multiplies it with its slice of K one tile later and stores its part of the key
 // tile's partial dQ; a second kernel adds the partials of all key tiles in a fixed order.  (Heads of
-// 64 columns and sequences that are not short: 256 keys, 64 per wave, attention_bwd_wide.hip.)
+// 64 columns and sequences that are not short: 256 keys, 64 per wave, attention_bwd_wide.hip;
+// sequences of 128 tokens: the whole call in one kernel, attention_bwd_one.hip.)
 #pragma once
 #include "common.h"
 #include "kernels.h"

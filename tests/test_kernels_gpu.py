@@ -858,6 +858,25 @@ def test_attention_backward_with_a_workgroup_per_key_tile(K, cfg):
 	assert torch.equal(fused, K.rope_apply_(dqkv.clone(), cs, S, Hq + Hkv, D, backward=True))
 
 
+@pytest.mark.parametrize("cfg", [(1, 1, 1, 64, False), (3, 5, 5, 64, True), (2, 3, 3, 128, False), (1, 2, 2, 128, True), (9, 32, 32, 64, True), (9, 32, 32, 128, True), (8, 6, 2, 64, False),
+                                 (16, 6, 3, 64, True), (17, 4, 2, 128, False), (14, 64, 8, 64, True)])
+def test_attention_backward_of_128_tokens_in_one_kernel(K, cfg):
+	"""One key tile: a head a workgroup and groups of two to eight, one workgroup, more than compute units, the fewest groups
+	of a size that come here.  Bounds, repeated bits and rotation as above (dQ has one rounding less)."""
+	B, Hq, Hkv, D, causal = cfg
+	S, T = 128, B * 128
+	qkv, do = _randn(T, (Hq + 2 * Hkv) * D, seed=61), _randn(T, Hq * D, seed=62)
+	o_ref, _, dqkv_ref = _attn_ref(qkv, B, S, Hq, Hkv, D, causal, do)
+	o, lse = K.attn_fwd(qkv, B, S, Hq, Hkv, D, causal)
+	dqkv = K.attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal)
+	for name, sl in (("dq", slice(0, Hq * D)), ("dk", slice(Hq * D, (Hq + Hkv) * D)), ("dv", slice((Hq + Hkv) * D, None))):
+		_close(dqkv[:, sl], dqkv_ref[:, sl], rel_fro=1.5e-2, what=f"attn {name} {cfg}")
+	assert torch.equal(dqkv, K.attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal))
+	cs = K.rope_table(S, D, 5e5)
+	fused = K.attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal, rope_cs=cs)
+	assert torch.equal(fused, K.rope_apply_(dqkv.clone(), cs, S, Hq + Hkv, D, backward=True))
+
+
 @pytest.mark.parametrize("cfg", [(1, 4096, 4, 4, 64, False), (2, 2048, 8, 4, 64, False), (1, 896, 8, 1, 128, True)])
 @pytest.mark.parametrize("ways", [None, 1, 2, 3, 64])
 def test_attention_backward_stays_inside_its_workspace(K, cfg, ways):
