@@ -6,9 +6,10 @@
 //   dW       dW += dY^T . X  A = dY [K,M] m-contiguous ("T"), B = X  [K,N] n-contiguous ("T")
 // (reference semantics: elf/zb_utils.py:20 forward, :34-37 dX, :235-244 dW accumulate).
 //
-// The kernels are in gemm_dma_tile.h and gemm_dma_pers.hip (128 to 256 rows by 256 columns) and gemm_ring.hip (128x128 .. 64x64
+// The kernels are in gemm_dma_tile.h and gemm_dma_pers.hip (128 to 256 rows by 256 columns, 128x192) and gemm_ring.hip (128x128 .. 32x32
 // tiles); all of them
 // add the products of an output in the same order, so the choice of a tile never changes its bits (a split of K does).
+#include <algorithm>
 #include <atomic>
 
 #include "common.h"
@@ -218,7 +219,8 @@ int gemm_bf16(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda,
 		}
 		bm = p.bm, bn = p.bn;
 		if (epi == EPI_F32_ACC && k_splits <= 0) k_splits = p.k_splits;
-		if (!gemm_reaches(a_t ? BK : bm, lda) || !gemm_reaches(b_t ? BK : bn, ldb)) bm = bn = 64;  // rows 16 MB apart and more
+		// rows 16 MB apart and more (those that 64 rows of are out of reach are refused, a 32x32 tile or not)
+		if (!gemm_reaches(a_t ? BK : std::max(bm, 64), lda) || !gemm_reaches(b_t ? BK : std::max(bn, 64), ldb)) bm = bn = 64;
 	}
 	if (epi != EPI_F32_ACC) k_splits = 1;
 	if (bm == 256 && k_splits <= 0) dw_split_plan(M, N, K, &k_splits, &tail_tiles);
