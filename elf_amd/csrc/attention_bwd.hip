@@ -822,6 +822,9 @@ static Splits split_short(int B, int S, int Hq, int Hkv, int D, bool causal, int
 //   four of 64: 32 24.4 and 24.5 / 21.6 and 25.1, 96 35.8 -> 26.4 / 30.4 -> 27.1, 320 63.8 -> 55.7 / 58.0 and 58.3
 //   four of 128: 64 37.6 and 41.5 / 41.3 and 45.3, 96 47.4 -> 43.6 / 46.2 and 48.1, 256 67.3 -> 57.3 / 66.8 and 64.4
 //   eight: 64 groups of 64 38.0 and 45.2, 128 58.2 -> 48.4 / 52.5 and 50.3; of 128 128 75.5 and 79.3, 320 173.5 and 179.9
+//
+// It addresses all 128 rows of Q, dO and (heads of 128) V with 32-bit byte offsets, where the three kernels take 32 rows of Q and dO and
+// read V through 64-bit pointers: rows that far apart stay with those.  (128 rows of K are what either needs.)
 static bool one_kernel_pays(int B, int S, int Hq, int Hkv, int D, bool causal) {
 	const int64_t groups = (int64_t)B * Hkv, G = Hq / Hkv;
 	if (S != 128 || G > 8 || groups < (causal && D == 64 ? 16 : 32) * (G - 1)) return false;
@@ -886,6 +889,13 @@ int64_t attn_bwd_shared_workspace_bytes(int B, int S, int Hq, int Hkv, int D, in
 	return whole + dkv_part_bytes(split_walk(B, S, Hq, Hkv, D, causal != 0, INT64_MAX), B, S, Hkv, D);
 }
 
+AttnBwdWay attn_bwd_way(int64_t ldq, int64_t ldv, int64_t lddo, int B, int S, int Hq, int Hkv, int D, int causal, int64_t workspace_bytes) {
+	const bool reached = gemm_reaches(128, ldq) && gemm_reaches(128, lddo) && (D == 64 || gemm_reaches(128, ldv));
+	if (reached && one_kernel_pays(B, S, Hq, Hkv, D, causal != 0)) return AttnBwdWay{0, 1, 1, 0};
+	const Splits sp = split_walk(B, S, Hq, Hkv, D, causal != 0, workspace_bytes - attn_bwd_workspace_bytes(B, S, Hq, D, causal));
+	return AttnBwdWay{sp.wide ? 256 : 128, sp.h, sp.q, causal && sp.paired && S > (sp.wide ? 256 : 128)};
+}
+
 int attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* dO, const void* lse, void* dq,
              void* dk, void* dv, void* workspace, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo, int64_t lddo,
              int64_t lddq, int64_t lddk, int64_t lddv, int B, int S, int Hq, int Hkv, int D, int causal, float scale,
@@ -904,7 +914,8 @@ int attn_bwd(const void* q, const void* k, const void* v, const void* o, const v
 	ELF_REQUIRE(((uintptr_t)o % 16) == 0 && ((uintptr_t)dO % 16) == 0, "attn_bwd: o and dO must be 16-byte aligned");
 	ProfScope prof(PROF_ATTN_BWD, (causal ? 4.0 : 8.0) * B * Hq * (double)S * S * D, stream);
 	const int64_t T = (int64_t)B * S;
-	if (one_kernel_pays(B, S, Hq, Hkv, D, causal != 0)) {
+	const AttnBwdWay way = attn_bwd_way(ldq, ldv, lddo, B, S, Hq, Hkv, D, causal, workspace_bytes);
+	if (way.keys == 0) {
 		const AttnBwdArgs a{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)dO, nullptr, nullptr, nullptr,
 		                    (bf16_t*)dk, (bf16_t*)dv, ldq, ldk, ldv, lddo, lddk, lddv, B, S, Hq, Hkv, scale, (const float2*)rope_cs, 1, 1, nullptr, 0};
 		return launch_bwd_one(a, D, causal != 0, (const bf16_t*)o, (const float*)lse, (bf16_t*)dq, ldo, lddq, stream);
@@ -918,26 +929,25 @@ int attn_bwd(const void* q, const void* k, const void* v, const void* o, const v
 		ELF_LAUNCH(attn_delta_kernel, dim3((unsigned)(want < 8192 ? want : 8192)), dim3(256), 0, stream, (const bf16_t*)dO,
 	                   (const bf16_t*)o, (const float*)lse, ndelta, nlse2, lddo, ldo, B, S, Hq, D);
 	}
-	const Splits sp = split_walk(B, S, Hq, Hkv, D, causal != 0, workspace_bytes - whole);
-	float* dkv_part = sp.h * sp.q > 1 ? nlse2 + T * Hq : nullptr;
+	float* dkv_part = way.h_splits * way.q_splits > 1 ? nlse2 + T * Hq : nullptr;
 	AttnBwdArgs a{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)dO, nlse2, ndelta, dq_part,
-	              (bf16_t*)dk, (bf16_t*)dv, ldq, ldk, ldv, lddo, lddk, lddv, B, S, Hq, Hkv, scale, (const float2*)rope_cs, sp.h, sp.q, dkv_part, sp.paired};
-	const int nkt = sp.wide ? (S + 255) / 256 : S / 128;
-	const dim3 grid((unsigned)((int64_t)B * Hkv * (causal && sp.paired ? (nkt + 1) / 2 : nkt) * sp.h * sp.q)), block(256);
+	              (bf16_t*)dk, (bf16_t*)dv, ldq, ldk, ldv, lddo, lddk, lddv, B, S, Hq, Hkv, scale, (const float2*)rope_cs, way.h_splits, way.q_splits, dkv_part, way.paired};
+	const int nkt = (S + way.keys - 1) / way.keys;
+	const dim3 grid((unsigned)((int64_t)B * Hkv * (way.paired ? (nkt + 1) / 2 : nkt) * way.h_splits * way.q_splits)), block(256);
 	int rc;
-	if (sp.wide) rc = launch_bwd_wide(a, causal != 0, grid, stream);
+	if (way.keys == 256) rc = launch_bwd_wide(a, causal != 0, grid, stream);
 	else if (D == 128) rc = causal ? launch_bwd<128, true>(a, grid, stream) : launch_bwd<128, false>(a, grid, stream);
 	else rc = causal ? launch_bwd<64, true>(a, grid, stream) : launch_bwd<64, false>(a, grid, stream);
 	if (rc) return rc;
 	const int64_t n16 = T * (Hq * D / 16);
 	const int64_t blocks = (n16 + 255) / 256;
-	DkvReduce dkv{dkv_part, (bf16_t*)dk, (bf16_t*)dv, lddk, lddv, sp.h * sp.q, Hkv, 0};
+	DkvReduce dkv{dkv_part, (bf16_t*)dk, (bf16_t*)dv, lddk, lddv, way.h_splits * way.q_splits, Hkv, 0};
 	if (dkv_part) {
 		const int64_t want = (2 * T * Hkv * (D / 16) + 255) / 256;
 		dkv.blocks = (int)(want < 4096 ? want : 4096);
 	}
 	ELF_LAUNCH(dq_reduce_kernel, dim3((unsigned)(blocks < 16384 ? blocks : 16384) + dkv.blocks), dim3(256), 0, stream, dq_part, (bf16_t*)dq, B, S,
-	                   Hq * D, lddq, scale, causal, sp.wide ? 256 : 128, D, (const float2*)rope_cs, dkv);
+	                   Hq * D, lddq, scale, causal, way.keys, D, (const float2*)rope_cs, dkv);
 	ELF_CHECK_HIP(hipGetLastError());
 	return 0;
 }

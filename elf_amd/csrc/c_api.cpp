@@ -140,6 +140,12 @@ int elf_attn_bwd_rope(const void* q, const void* k, const void* v, const void* o
 	                     Hkv, D, causal, scale, S_(stream), cs, elf::attn_bwd_workspace_bytes(B, S, Hq, D, causal));
 }
 
+int elf_attn_bwd_way(int64_t workspace_bytes, int64_t ldq, int64_t ldv, int64_t lddo, int B, int S, int Hq, int Hkv, int D, int causal, int* way) {
+	ELF_REQUIRE(way && B > 0 && S > 0 && S % 128 == 0 && Hkv > 0 && Hq > 0 && Hq % Hkv == 0 && (D == 64 || D == 128), "attn_bwd_way: a shape that the backward refuses");
+	const elf::AttnBwdWay w = elf::attn_bwd_way(ldq, ldv, lddo, B, S, Hq, Hkv, D, causal, workspace_bytes);
+	way[0] = w.keys, way[1] = w.h_splits, way[2] = w.q_splits, way[3] = w.paired;
+	return 0;
+}
 int64_t elf_attn_bwd_shared_workspace_bytes(int B, int S, int Hq, int Hkv, int D, int causal) { return elf::attn_bwd_shared_workspace_bytes(B, S, Hq, Hkv, D, causal); }
 int elf_attn_bwd_shared(const void* q, const void* k, const void* v, const void* o, const void* dO, const void* lse, void* dq,
                         void* dk, void* dv, void* workspace, int64_t workspace_bytes, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo,

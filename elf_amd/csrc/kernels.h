@@ -200,6 +200,12 @@ int attn_fwd(const void* q, const void* k, const void* v, void* o, void* lse, in
              int64_t ldo, int B, int S, int Hq, int Hkv, int D, int causal, float scale, hipStream_t stream);
 int64_t attn_bwd_workspace_bytes(int B, int S, int Hq, int D, int causal);
 int64_t attn_bwd_shared_workspace_bytes(int B, int S, int Hq, int Hkv, int D, int causal);
+// The way attn_bwd takes: keys of a workgroup's pass, 0: the whole call in one kernel (128 tokens); the ways a group's query heads and their
+// queries are shared; paired: key tiles two by two (causal).
+struct AttnBwdWay {
+	int keys, h_splits, q_splits, paired;
+};
+AttnBwdWay attn_bwd_way(int64_t ldq, int64_t ldv, int64_t lddo, int B, int S, int Hq, int Hkv, int D, int causal, int64_t workspace_bytes);
 // workspace_bytes: what lies at `workspace`, at least attn_bwd_workspace_bytes(); what it holds beyond that is used for the
 // partial sums of shared walks, and a launch shares its walks only as far as they fit.
 int attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* dO, const void* lse, void* dq,

@@ -322,6 +322,18 @@ def attn_fwd(qkv, B, S, Hq, Hkv, D, causal, scale=None):
 	return o, lse
 
 
+def attn_bwd_way(B, S, Hq, Hkv, D, causal, ld=None, workspace=None):
+	"""(keys of a pass, ways the query heads of a group are shared, ways their queries are, pairs of key tiles) of ``attn_bwd``; 0 keys: the
+	whole call in one kernel.  ``ld``: the row strides of q, v and dO (packed rows if left out), ``workspace``: bytes."""
+	lib = _lib.load()
+	row = (Hq + 2 * Hkv) * D
+	way = (ctypes.c_int * 4)()
+	if workspace is None:
+		workspace = lib.elf_attn_bwd_shared_workspace_bytes(B, S, Hq, Hkv, D, int(causal))
+	_lib.check(lib.elf_attn_bwd_way(workspace, *(ld or (row, row, Hq * D)), B, S, Hq, Hkv, D, int(causal), way), "elf_attn_bwd_way")
+	return way[0], way[1], way[2], bool(way[3])
+
+
 def attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal, scale=None, rope_cs=None):
 	"""Returns dqkv packed like qkv.  ``rope_cs``: the q and k heads of ``qkv`` are rotated (``rope_apply_`` with this
 	table); dq and dk then come out with the rotation's backward applied."""

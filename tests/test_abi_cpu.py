@@ -215,3 +215,24 @@ def test_pinned_pool_matches_policy_model(seed):
 		assert p.free(addr)
 	assert all(len(s) == 1 and s[0][0] == 0 for s in p.free_segments())
 	assert all((s[0][1] & (s[0][1] - 1)) == 0 for s in p.free_segments()), "parent sizes are powers of two"
+
+
+def _attn_way(lib, shape, causal, ld=None, workspace=None):
+	from elf_amd import kernels
+
+	return kernels.attn_bwd_way(*shape, causal, ld=ld, workspace=workspace)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+def test_attention_backward_of_128_tokens_whose_rows_lie_far_apart_stays_out_of_one_kernel(lib, D, causal):
+	"""The one kernel reaches 128 rows of Q and dO, and of V with heads of 128, with 32-bit byte offsets; the three kernels reach 32 rows of
+	Q and dO and any of V."""
+	shape, dense = (1, 128, 2, 2, D), 6 * D
+	near, far = (((1 << 32) - 512) // 2 // 127) & ~7, 1 << 25
+	assert 127 * near * 2 + 512 <= 1 << 32 < 127 * (near + 8) * 2 + 512
+	assert _attn_way(lib, shape, causal, ld=(near, near, near))[0] == 0
+	for ld in ((near + 8, dense, dense), (dense, dense, near + 8), (far, dense, dense), (dense, dense, far)):
+		assert _attn_way(lib, shape, causal, ld=ld)[0] == 128
+	for ldv in (near + 8, far):
+		assert _attn_way(lib, shape, causal, ld=(dense, ldv, dense))[0] == (0 if D == 64 else 128)

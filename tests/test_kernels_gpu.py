@@ -877,6 +877,38 @@ def test_attention_backward_of_128_tokens_in_one_kernel(K, cfg):
 	assert torch.equal(fused, K.rope_apply_(dqkv.clone(), cs, S, Hq + Hkv, D, backward=True))
 
 
+def _attn_bwd_separate(B, S, Hq, Hkv, D, causal, q, k, v, o, do, lse, rope_cs=None):
+	"""dq, dk and dv of operands in buffers of their own ([B * S, heads * D] with any row stride)."""
+	from elf_amd import _lib
+
+	lib, T = _lib.load(), B * S
+	n = lib.elf_attn_bwd_shared_workspace_bytes(B, S, Hq, Hkv, D, int(causal))
+	ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+	dq, dk, dv = (torch.empty(T, h * D, dtype=torch.bfloat16, device="cuda") for h in (Hq, Hkv, Hkv))
+	rc = lib.elf_attn_bwd_shared(*(t.data_ptr() for t in (q, k, v, o, do, lse, dq, dk, dv, ws)), n, *(t.stride(0) for t in (q, k, v, o, do, dq, dk, dv)),
+	                             B, S, Hq, Hkv, D, int(causal), 1 / math.sqrt(D), rope_cs.data_ptr() if rope_cs is not None else None, torch.cuda.current_stream().cuda_stream)
+	_lib.check(rc, "elf_attn_bwd_shared")
+	return dq, dk, dv
+
+
+@pytest.mark.parametrize("D,causal", [(64, True), (128, False)])
+@pytest.mark.parametrize("far", ["q", "v", "do"])
+def test_attention_backward_of_128_tokens_whose_rows_lie_far_apart(K, D, causal, far):
+	"""Rows of 2^24 + 2^20 elements: row 121 lies 4 GiB from the first, further than a 32-bit byte offset reaches.  Against fp32 autograd,
+	within the bounds of dense rows."""
+	B, S, H, ld = 1, 128, 2, (1 << 24) + (1 << 20)
+	qkv, do = _randn(S, 3 * H * D, seed=63), _randn(S, H * D, seed=64)
+	o_ref, _, ref = _attn_ref(qkv, B, S, H, H, D, causal, do)
+	o, lse = K.attn_fwd(qkv, B, S, H, H, D, causal)
+	ops = dict(zip("qkv", (t.contiguous() for t in qkv.split(H * D, dim=1))), do=do)
+	rows = torch.empty(127 * ld + H * D, dtype=torch.bfloat16, device="cuda").as_strided((S, H * D), (ld, 1))
+	rows.copy_(ops[far])
+	ops[far] = rows
+	got = _attn_bwd_separate(B, S, H, H, D, causal, ops["q"], ops["k"], ops["v"], o, ops["do"], lse)
+	for name, g, r in zip(("dq", "dk", "dv"), got, ref.split(H * D, dim=1)):
+		_close(g, r, rel_fro=1.5e-2, what=f"attn {name} with {far} rows far apart")
+
+
 @pytest.mark.parametrize("cfg", [(1, 4096, 4, 4, 64, False), (2, 2048, 8, 4, 64, False), (1, 896, 8, 1, 128, True)])
 @pytest.mark.parametrize("ways", [None, 1, 2, 3, 64])
 def test_attention_backward_stays_inside_its_workspace(K, cfg, ways):
