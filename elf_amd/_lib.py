@@ -62,7 +62,7 @@ _SIGNATURES = {
 	"elf_prof_collect": (c_int, [c_int, POINTER(c_double), POINTER(c_double)]),
 	"elf_prof_launches": (c_int64, [c_int, POINTER(c_double)]),
 	"elf_attn_bwd_shared_workspace_bytes": (c_int64, [c_int] * 6),
-	"elf_attn_bwd_way": (c_int, [c_int64] * 4 + [c_int] * 6 + [POINTER(c_int)]),
+	"elf_attn_bwd_way": (c_int, [c_int64, _P] + [c_int64] * 3 + [c_int] * 6 + [POINTER(c_int)]),
 	"elf_attn_bwd_shared": (c_int, [_P] * 10 + [c_int64] * 9 + [c_int] * 6 + [c_float, _P, _P]),
 	"elf_attn_bwd": (c_int, [_P] * 10 + [c_int64] * 8 + [c_int] * 6 + [c_float, _P]),
 	"elf_attn_bwd_rope": (c_int, [_P] * 10 + [c_int64] * 8 + [c_int] * 6 + [c_float, _P, _P]),

@@ -824,7 +824,8 @@ static Splits split_short(int B, int S, int Hq, int Hkv, int D, bool causal, int
 //   eight: 64 groups of 64 38.0 and 45.2, 128 58.2 -> 48.4 / 52.5 and 50.3; of 128 128 75.5 and 79.3, 320 173.5 and 179.9
 //
 // It addresses all 128 rows of Q, dO and (heads of 128) V with 32-bit byte offsets, where the three kernels take 32 rows of Q and dO and
-// read V through 64-bit pointers: rows that far apart stay with those.  (128 rows of K are what either needs.)
+// read V through 64-bit pointers: rows that far apart stay with those.  So do V's of 128 columns a head that are not 16-byte aligned: the one
+// kernel brings them into LDS as it does Q, K and dO.  (128 rows of K are what either needs.)
 static bool one_kernel_pays(int B, int S, int Hq, int Hkv, int D, bool causal) {
 	const int64_t groups = (int64_t)B * Hkv, G = Hq / Hkv;
 	if (S != 128 || G > 8 || groups < (causal && D == 64 ? 16 : 32) * (G - 1)) return false;
@@ -889,8 +890,8 @@ int64_t attn_bwd_shared_workspace_bytes(int B, int S, int Hq, int Hkv, int D, in
 	return whole + dkv_part_bytes(split_walk(B, S, Hq, Hkv, D, causal != 0, INT64_MAX), B, S, Hkv, D);
 }
 
-AttnBwdWay attn_bwd_way(int64_t ldq, int64_t ldv, int64_t lddo, int B, int S, int Hq, int Hkv, int D, int causal, int64_t workspace_bytes) {
-	const bool reached = gemm_reaches(128, ldq) && gemm_reaches(128, lddo) && (D == 64 || gemm_reaches(128, ldv));
+AttnBwdWay attn_bwd_way(const void* v, int64_t ldq, int64_t ldv, int64_t lddo, int B, int S, int Hq, int Hkv, int D, int causal, int64_t workspace_bytes) {
+	const bool reached = gemm_reaches(128, ldq) && gemm_reaches(128, lddo) && (D == 64 || (gemm_reaches(128, ldv) && ((uintptr_t)v % 16) == 0));
 	if (reached && one_kernel_pays(B, S, Hq, Hkv, D, causal != 0)) return AttnBwdWay{0, 1, 1, 0};
 	const Splits sp = split_walk(B, S, Hq, Hkv, D, causal != 0, workspace_bytes - attn_bwd_workspace_bytes(B, S, Hq, D, causal));
 	return AttnBwdWay{sp.wide ? 256 : 128, sp.h, sp.q, causal && sp.paired && S > (sp.wide ? 256 : 128)};
@@ -914,7 +915,7 @@ int attn_bwd(const void* q, const void* k, const void* v, const void* o, const v
 	ELF_REQUIRE(((uintptr_t)o % 16) == 0 && ((uintptr_t)dO % 16) == 0, "attn_bwd: o and dO must be 16-byte aligned");
 	ProfScope prof(PROF_ATTN_BWD, (causal ? 4.0 : 8.0) * B * Hq * (double)S * S * D, stream);
 	const int64_t T = (int64_t)B * S;
-	const AttnBwdWay way = attn_bwd_way(ldq, ldv, lddo, B, S, Hq, Hkv, D, causal, workspace_bytes);
+	const AttnBwdWay way = attn_bwd_way(v, ldq, ldv, lddo, B, S, Hq, Hkv, D, causal, workspace_bytes);
 	if (way.keys == 0) {
 		const AttnBwdArgs a{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)dO, nullptr, nullptr, nullptr,
 		                    (bf16_t*)dk, (bf16_t*)dv, ldq, ldk, ldv, lddo, lddk, lddv, B, S, Hq, Hkv, scale, (const float2*)rope_cs, 1, 1, nullptr, 0};

@@ -140,9 +140,9 @@ int elf_attn_bwd_rope(const void* q, const void* k, const void* v, const void* o
 	                     Hkv, D, causal, scale, S_(stream), cs, elf::attn_bwd_workspace_bytes(B, S, Hq, D, causal));
 }
 
-int elf_attn_bwd_way(int64_t workspace_bytes, int64_t ldq, int64_t ldv, int64_t lddo, int B, int S, int Hq, int Hkv, int D, int causal, int* way) {
+int elf_attn_bwd_way(int64_t workspace_bytes, const void* v, int64_t ldq, int64_t ldv, int64_t lddo, int B, int S, int Hq, int Hkv, int D, int causal, int* way) {
 	ELF_REQUIRE(way && B > 0 && S > 0 && S % 128 == 0 && Hkv > 0 && Hq > 0 && Hq % Hkv == 0 && (D == 64 || D == 128), "attn_bwd_way: a shape that the backward refuses");
-	const elf::AttnBwdWay w = elf::attn_bwd_way(ldq, ldv, lddo, B, S, Hq, Hkv, D, causal, workspace_bytes);
+	const elf::AttnBwdWay w = elf::attn_bwd_way(v, ldq, ldv, lddo, B, S, Hq, Hkv, D, causal, workspace_bytes);
 	way[0] = w.keys, way[1] = w.h_splits, way[2] = w.q_splits, way[3] = w.paired;
 	return 0;
 }

@@ -205,7 +205,7 @@ int64_t attn_bwd_shared_workspace_bytes(int B, int S, int Hq, int Hkv, int D, in
 struct AttnBwdWay {
 	int keys, h_splits, q_splits, paired;
 };
-AttnBwdWay attn_bwd_way(int64_t ldq, int64_t ldv, int64_t lddo, int B, int S, int Hq, int Hkv, int D, int causal, int64_t workspace_bytes);
+AttnBwdWay attn_bwd_way(const void* v, int64_t ldq, int64_t ldv, int64_t lddo, int B, int S, int Hq, int Hkv, int D, int causal, int64_t workspace_bytes);
 // workspace_bytes: what lies at `workspace`, at least attn_bwd_workspace_bytes(); what it holds beyond that is used for the
 // partial sums of shared walks, and a launch shares its walks only as far as they fit.
 int attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* dO, const void* lse, void* dq,

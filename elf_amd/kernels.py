@@ -322,15 +322,16 @@ def attn_fwd(qkv, B, S, Hq, Hkv, D, causal, scale=None):
 	return o, lse
 
 
-def attn_bwd_way(B, S, Hq, Hkv, D, causal, ld=None, workspace=None):
+def attn_bwd_way(B, S, Hq, Hkv, D, causal, ld=None, workspace=None, v=None):
 	"""(keys of a pass, ways the query heads of a group are shared, ways their queries are, pairs of key tiles) of ``attn_bwd``; 0 keys: the
-	whole call in one kernel.  ``ld``: the row strides of q, v and dO (packed rows if left out), ``workspace``: bytes."""
+	whole call in one kernel.  ``ld``: the row strides of q, v and dO (packed rows if left out), ``workspace``: bytes,
+	``v``: its address."""
 	lib = _lib.load()
 	row = (Hq + 2 * Hkv) * D
 	way = (ctypes.c_int * 4)()
 	if workspace is None:
 		workspace = lib.elf_attn_bwd_shared_workspace_bytes(B, S, Hq, Hkv, D, int(causal))
-	_lib.check(lib.elf_attn_bwd_way(workspace, *(ld or (row, row, Hq * D)), B, S, Hq, Hkv, D, int(causal), way), "elf_attn_bwd_way")
+	_lib.check(lib.elf_attn_bwd_way(workspace, v, *(ld or (row, row, Hq * D)), B, S, Hq, Hkv, D, int(causal), way), "elf_attn_bwd_way")
 	return way[0], way[1], way[2], bool(way[3])
 
 

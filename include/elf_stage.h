@@ -280,9 +280,9 @@ int elf_attn_bwd_shared(const void* q, const void* k, const void* v, const void*
                         int Hq, int Hkv, int D, int causal, float scale, const void* cs, void* stream);
 /* Which way these calls take with a workspace of that size (elf_attn_bwd: elf_attn_bwd_workspace_bytes()): way[0] keys of a workgroup's
  * pass, 128 or 256, or 0: the whole call in one kernel; way[1] and way[2] how many ways the query heads of a group and their
- * queries are shared; way[3] 1: a causal pass takes a light and a heavy key tile.  Host only; for tests and tuning, no
- * counterpart in the reference. */
-int elf_attn_bwd_way(int64_t workspace_bytes, int64_t ldq, int64_t ldv, int64_t lddo, int B, int S, int Hq, int Hkv, int D, int causal,
+ * queries are shared; way[3] 1: a causal pass takes a light and a heavy key tile.  Of v only the alignment counts, nothing is
+ * read.  Host only; for tests and tuning, no counterpart in the reference. */
+int elf_attn_bwd_way(int64_t workspace_bytes, const void* v, int64_t ldq, int64_t ldv, int64_t lddo, int B, int S, int Hq, int Hkv, int D, int causal,
                      int* way);
 
 /* ---------------------------------------------------------------------------------------------

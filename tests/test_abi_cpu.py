@@ -217,10 +217,10 @@ def test_pinned_pool_matches_policy_model(seed):
 	assert all((s[0][1] & (s[0][1] - 1)) == 0 for s in p.free_segments()), "parent sizes are powers of two"
 
 
-def _attn_way(lib, shape, causal, ld=None, workspace=None):
+def _attn_way(lib, shape, causal, ld=None, workspace=None, v=None):
 	from elf_amd import kernels
 
-	return kernels.attn_bwd_way(*shape, causal, ld=ld, workspace=workspace)
+	return kernels.attn_bwd_way(*shape, causal, ld=ld, workspace=workspace, v=v)
 
 
 @pytest.mark.parametrize("D", [64, 128])
@@ -236,3 +236,12 @@ def test_attention_backward_of_128_tokens_whose_rows_lie_far_apart_stays_out_of_
 		assert _attn_way(lib, shape, causal, ld=ld)[0] == 128
 	for ldv in (near + 8, far):
 		assert _attn_way(lib, shape, causal, ld=(dense, ldv, dense))[0] == (0 if D == 64 else 128)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_attention_backward_of_a_misaligned_v_stays_out_of_one_kernel(lib, D):
+	"""Heads of 128: the one kernel brings V into LDS in 16-byte pieces, which the kernels of longer sequences do with Q, K and dO only."""
+	shape = (1, 128, 2, 2, D)
+	assert _attn_way(lib, shape, True, v=1 << 20)[0] == 0
+	for off in (2, 4, 8):
+		assert _attn_way(lib, shape, True, v=(1 << 20) + off)[0] == (0 if D == 64 else 128)

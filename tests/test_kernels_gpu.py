@@ -909,6 +909,24 @@ def test_attention_backward_of_128_tokens_whose_rows_lie_far_apart(K, D, causal,
 		_close(g, r, rel_fro=1.5e-2, what=f"attn {name} with {far} rows far apart")
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("off", [0, 4])
+def test_attention_backward_of_128_tokens_with_v_in_a_buffer_of_its_own(K, D, off):
+	"""V on a 16-byte boundary and 8 bytes past one, in rows of its own width."""
+	B, S, H = 3, 128, 2
+	T = B * S
+	qkv, do = _randn(T, 3 * H * D, seed=65), _randn(T, H * D, seed=66)
+	o_ref, _, ref = _attn_ref(qkv, B, S, H, H, D, True, do)
+	o, lse = K.attn_fwd(qkv, B, S, H, H, D, True)
+	q, k, v = qkv.split(H * D, dim=1)
+	own = torch.empty(T * H * D + 8, dtype=torch.bfloat16, device="cuda")[off : off + T * H * D].view(T, H * D)
+	own.copy_(v)
+	assert K.attn_bwd_way(B, S, H, H, D, True, v=own.data_ptr())[0] == (128 if D == 128 and off else 0)
+	got = _attn_bwd_separate(B, S, H, H, D, True, q, k, own, o, do, lse)
+	for name, g, r in zip(("dq", "dk", "dv"), got, ref.split(H * D, dim=1)):
+		_close(g, r, rel_fro=1.5e-2, what=f"attn {name} with v {2 * off} bytes past a boundary")
+
+
 @pytest.mark.parametrize("cfg", [(1, 4096, 4, 4, 64, False), (2, 2048, 8, 4, 64, False), (1, 896, 8, 1, 128, True)])
 @pytest.mark.parametrize("ways", [None, 1, 2, 3, 64])
 def test_attention_backward_stays_inside_its_workspace(K, cfg, ways):
