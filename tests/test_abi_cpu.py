@@ -245,3 +245,14 @@ def test_attention_backward_of_a_misaligned_v_stays_out_of_one_kernel(lib, D):
 	assert _attn_way(lib, shape, True, v=1 << 20)[0] == 0
 	for off in (2, 4, 8):
 		assert _attn_way(lib, shape, True, v=(1 << 20) + off)[0] == (0 if D == 64 else 128)
+
+
+@pytest.mark.parametrize("given,both", [((), True), (("TORCH_DIR=/nonexistent",), False), (("PYTHON=false",), False)])
+def test_the_stage_library_builds_without_pytorch(given, both):
+	"""The default target, dry run: where the interpreter has no PyTorch, or one without headers, nothing of libelf_torch.so is asked for."""
+	import subprocess
+	import sys
+
+	out = subprocess.run(["make", "-n", "-B", "-C", os.path.join(ROOT, "elf_amd", "csrc"), *(given or (f"PYTHON={sys.executable}",))], capture_output=True, text=True)
+	assert out.returncode == 0 and "-o ../libelf_stage.so" in out.stdout
+	assert ("allocator.cpp" in out.stdout) == both
