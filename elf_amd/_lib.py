@@ -5,6 +5,7 @@ There is no fallback: if the shared object is missing, loading raises.
 """
 
 import ctypes
+import logging
 import os
 from ctypes import c_int, c_int64, c_float, c_double, c_void_p, c_char_p, POINTER
 
@@ -15,8 +16,10 @@ LIB_PATH = os.path.join(_HERE, "libelf_stage.so")
 
 TORCH_LIB_PATH = os.path.join(_HERE, "libelf_torch.so")
 
+logger = logging.getLogger("lib")
+
 _lib = None
-_torch_allocated = None
+_torch_allocated = None  # not looked for yet; False: not to be had
 
 # name -> (restype, argtypes); kept in one table so that tests can check the exported symbols
 # against the header.
@@ -109,15 +112,32 @@ def load():
 	return lib
 
 
+def _torch_reader():
+	"""libelf_torch.so's reading of PyTorch's caching allocator, or False where the library is missing, does not load or was built for another
+	PyTorch than this one."""
+	if not os.path.exists(TORCH_LIB_PATH):
+		return False
+	try:
+		lib = ctypes.CDLL(TORCH_LIB_PATH)
+		lib.elf_torch_built_for.restype = c_char_p
+		built_for, fn = lib.elf_torch_built_for().decode(), lib.elf_torch_allocated
+	except (OSError, AttributeError) as e:
+		logger.warning("%s is not used: %s", TORCH_LIB_PATH, e)
+		return False
+	if built_for != torch.__version__:
+		logger.warning("%s is not used: built for PyTorch %s, this is %s", TORCH_LIB_PATH, built_for, torch.__version__)
+		return False
+	fn.restype, fn.argtypes = c_int, [c_int, _P]
+	return fn
+
+
 def torch_allocated(device):
 	"""(allocated, peak) bytes of PyTorch's caching allocator on ``device`` through libelf_torch.so, or None without that library."""
 	global _torch_allocated
 	if _torch_allocated is None:
-		if not os.path.exists(TORCH_LIB_PATH):
-			return None
-		fn = ctypes.CDLL(TORCH_LIB_PATH).elf_torch_allocated
-		fn.restype, fn.argtypes = c_int, [c_int, _P]
-		_torch_allocated = fn
+		_torch_allocated = _torch_reader()
+	if _torch_allocated is False:
+		return None
 	out = (c_int64 * 2)()
 	return (out[0], out[1]) if _torch_allocated(device, out) == 0 else None
 

@@ -4,6 +4,9 @@
 
 #include <cstdint>
 
+// The PyTorch whose headers this was built against: the figures lie where that one keeps them.
+extern "C" const char* elf_torch_built_for() { return ELF_TORCH_VERSION; }
+
 // out[0] = bytes allocated on `device` now, out[1] = the peak.  -1: the allocator knows no such device.
 extern "C" int elf_torch_allocated(int device, int64_t* out) {
 	try {

@@ -256,3 +256,23 @@ def test_the_stage_library_builds_without_pytorch(given, both):
 	out = subprocess.run(["make", "-n", "-B", "-C", os.path.join(ROOT, "elf_amd", "csrc"), *(given or (f"PYTHON={sys.executable}",))], capture_output=True, text=True)
 	assert out.returncode == 0 and "-o ../libelf_stage.so" in out.stdout
 	assert ("allocator.cpp" in out.stdout) == both
+
+
+def test_an_unusable_torch_library_leaves_the_figures_to_pytorch(monkeypatch, tmp_path):
+	"""Missing, no library at all, without the symbols, built for another PyTorch: looked for once, and the caller gets None."""
+	import torch
+
+	from elf_amd import _lib
+
+	assert _lib._torch_reader(), "the library that was built here is usable"
+	bad = tmp_path / "libelf_torch.so"
+	bad.write_bytes(b"no library")
+	for path, version in ((str(tmp_path / "none.so"), None), (str(bad), None), (_lib.LIB_PATH, None), (_lib.TORCH_LIB_PATH, "0.0.0")):
+		with monkeypatch.context() as m:
+			m.setattr(_lib, "TORCH_LIB_PATH", path)
+			m.setattr(_lib, "_torch_allocated", None)
+			if version:
+				m.setattr(torch, "__version__", version)
+			assert _lib.torch_allocated(0) is None
+			m.setattr(_lib, "_torch_reader", lambda: pytest.fail("looked for again"))
+			assert _lib.torch_allocated(0) is None

@@ -132,6 +132,20 @@ def test_memory_figures_of_one_allocator_query():
 	del held
 
 
+def test_memory_figures_where_the_torch_library_does_not_load(monkeypatch, tmp_path):
+	from elf_amd import _lib
+	from elf_amd.execution import engine as E
+
+	bad = tmp_path / "libelf_torch.so"
+	bad.write_bytes(b"no library")
+	held = torch.empty(1 << 20, dtype=torch.uint8, device="cuda")
+	monkeypatch.setattr(_lib, "TORCH_LIB_PATH", str(bad))
+	monkeypatch.setattr(_lib, "_torch_allocated", None)
+	for _ in range(2):
+		assert E._mem() == (torch.cuda.memory_allocated(), torch.cuda.max_memory_allocated())
+	del held
+
+
 def test_steps_in_a_row_hand_over_their_own_outputs():
 	"""Six steps on six batches without a wait in between: the host is never more than two steps' output copies ahead, and every
 	step's outputs and loss are those the same step gives alone."""
