@@ -176,12 +176,13 @@ class LinearDW(LayerDW, nn.Linear):
 	@staticmethod
 	def backward_together(layers, mb_id):
 		"""W of several layers: what ``backward`` does for each, the layers over the same number of tokens in one call of the library
-		(weight gradients and bias sums then share launches).  What such a call does not take goes through ``backward``."""
+		(weight gradients and bias sums then share launches).  What such a call does not take goes through ``backward``, and so do layers whose
+		stash has to be copied to dense rows: one copy is alive at a time."""
 		by_tokens = {}
 		for m in layers:
 			grad_output, inputs, acc = m.ctx["grad_output"][mb_id], m.ctx["input"][mb_id], m._main_grad(m.weight)
 			bias = m._main_grad(m.bias) if m.bias is not None else None
-			if not all(g is None or (g.dtype == torch.float32 and g.is_contiguous()) for g in (acc, bias)) or grad_output.dtype != torch.bfloat16 or inputs.dtype != torch.bfloat16:
+			if not all(g is None or (g.dtype == torch.float32 and g.is_contiguous()) for g in (acc, bias)) or not all(t.dtype == torch.bfloat16 and t.is_contiguous() for t in (grad_output, inputs)):
 				m.backward(mb_id)
 				continue
 			go, inp = _as_rows(grad_output), _as_rows(inputs)
