@@ -127,7 +127,7 @@ class AutogradStageBlock(StageBlockBase):
 	def backward_params(self, mb_id, **options):
 		with self._timed(f"backward_params({self.id}:{mb_id})"):
 			ready = [m for m in self._layers_dw() if not m.is_empty("grad_output")]
-			plain = [m for m in ready if type(m).backward is LinearDW.backward and "backward" not in m.__dict__]
+			plain = [m for m in ready if type(m).backward is LinearDW._own_backward and "backward" not in m.__dict__]
 			for m in ready:
 				if m not in plain:
 					m.backward(mb_id)

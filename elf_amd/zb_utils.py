@@ -172,6 +172,7 @@ class LinearDW(LayerDW, nn.Linear):
 		self.ctx["grad_output"][mb_id] = None
 		self.ctx["input"][mb_id] = None
 
+	_own_backward = backward  # what backward_together stands for: a method put in its place, on the class too, is asked layer by layer
 
 	@staticmethod
 	def backward_together(layers, mb_id):

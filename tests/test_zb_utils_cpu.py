@@ -126,3 +126,7 @@ def test_w_pass_asks_a_backward_that_is_not_linear_dws_own(monkeypatch):
 	monkeypatch.setattr(wrapped, "backward", lambda mb: (asked.append("object"), zb_utils.LinearDW.backward(wrapped, mb)))
 	_w_pass([_stashed(cls=Own), wrapped, _stashed()])
 	assert asked == ["class", "object"] and k.asked == ["one", "one", 1]
+	own = zb_utils.LinearDW.backward
+	monkeypatch.setattr(zb_utils.LinearDW, "backward", lambda self, mb: (asked.append("patched"), own(self, mb)))
+	_w_pass([_stashed(), _stashed()])
+	assert asked[2:] == ["patched", "patched"]
