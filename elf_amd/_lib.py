@@ -58,6 +58,7 @@ _SIGNATURES = {
 	"elf_attn_bwd_workspace_bytes": (c_int64, [c_int, c_int, c_int, c_int, c_int]),
 	"elf_gemm_turn_giveups": (c_int, [POINTER(ctypes.c_uint64)]),
 	"elf_linear_w_workspace_floats": (c_int64, [c_int, _P, c_int]),
+	"elf_linear_w_way": (c_int, [c_int, _P, c_int]),
 	"elf_linear_w_pass": (c_int, [c_int, _P, c_int, _P, _P]),
 	"elf_gemm_dw_group": (c_int, [c_int, _P, c_int, c_float, _P]),
 	"elf_hbm_probe": (c_int, [c_int, _P, _P, c_int64, _P]),

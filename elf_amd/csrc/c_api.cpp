@@ -35,6 +35,8 @@ int elf_linear_w_pass(int n, const elf_linear_w* layers, int T, float* workspace
 	return elf::linear_w_pass(n, reinterpret_cast<const elf::LinearW*>(layers), T, workspace, (hipStream_t)stream);
 }
 
+int elf_linear_w_way(int n, const elf_linear_w* layers, int T) { return elf::linear_w_way(n, reinterpret_cast<const elf::LinearW*>(layers), T); }
+
 int elf_gemm_act_bf16(int act, int M, int F, int K, const void* A, int64_t lda, const void* W, int64_t ldw,
                       void* pre, int64_t ldpre, void* out, int64_t ldout, void* stream) {
 	return elf::gemm_act_bf16(act, M, F, K, A, lda, W, ldw, pre, ldpre, out, ldout, (hipStream_t)stream);

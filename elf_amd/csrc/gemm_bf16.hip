@@ -228,32 +228,37 @@ int gemm_bf16(int a_t, int b_t, int M, int N, int K, const void* A, int64_t lda,
 	return gemm_bf16_ring(a_t, b_t, M, N, K, A, lda, B, ldb, C, ldc, epi, R, ldr, k_splits, bm, bn, stream);
 }
 
-// Whether the weight gradients of several layers are done sooner in one launch of gemm_dw_group (256x256 tiles, or 128x128 ones where
-// these make no more than a round) than in a launch each on the best tile, and that launch costs 2 us.  Of 29 pairs of layers over 128
-// to 7000 tokens (us, apart and together): 2112 tokens, 4288 x 1600 and 832 x 4288 62.6 and 57.8; 1792, 1536 x 5184 and 3328 x 1536 70 and 58;
-// 5312, 1216 x 896 and 1536 x 1216 72 and 40; 256, 2112 x 1024 and 384 x 2112 14.4 and 10.4.  More than a round of tiles stays apart (4544,
-// 5824 x 7232 and 1792 x 5824 441 and 470), and a split of the tiles has to pay for its adds, 10 us a split (2048, 3520 x 256 and 1984 x
-// 3520 48 and 75).
+// Whether the weight gradients of several layers are done sooner in one launch of gemm_dw_group, the way that takes them, than in a launch
+// each on the best tile, and 2 us for that launch.  Constants in microseconds, fitted to 649 lists of 2 to 16 layers of at most a
+// round of 256x256 tiles over 64 to 8192 tokens, operands past the caches; on 450 others no list that goes together takes 3 % longer than
+// apart, and three that would be 4 to 6 % faster together stay apart.  us, apart and together: 2112 tokens, 4288 x 1600 and 832 x 4288 70 and 59; 1792,
+// 1536 x 5184 and 3328 x 1536 75 and 60; 5312, 1216 x 896 and 1536 x 1216 88 and 57; 256, 2112 x 1024 and 384 x 2112 15.4 and 10.8.
+// Staying apart: 8192, 1536 x 1536 and 1536 x 256 96 and 123; 3008, 1344 x 384 and 4544 x 1344 68 and 79; 2048, 4096 x 960 and 960 x 2560 56
+// and 66; lists of more than a round, 4544 tokens, 5824 x 7232 and 1792 x 5824 465 and 480.
 static bool group_pays(int n, const DwProblem* pr, int K) {
+	const DwGroupWay way = gemm_dw_group_way(n, pr, K);
+	if (way.tiles > 256) return false;
 	float apart = 2.f * (n - 1);
-	int64_t tiles = 0, small = 0;
-	for (int i = 0; i < n; i++) {
-		apart += plan_weight_gradient(pr[i].M, pr[i].N, K).us;
-		tiles += (int64_t)((pr[i].M + 255) / 256) * ((pr[i].N + 255) / 256);
-		small += (int64_t)((pr[i].M + 127) / 128) * ((pr[i].N + 127) / 128);
-	}
-	const TileTime &t256 = TILES_F32[0], &t128 = TILES_F32[2];
+	for (int i = 0; i < n; i++) apart += plan_weight_gradient(pr[i].M, pr[i].N, K).us;
 	const int nk = K / BK;
-	int splits = 1;  // of the last round's tiles, as gemm_dw_group splits them
-	if (const int rem = (int)(tiles % 256); rem != 0 && rem <= 128) {
-		splits = 256 / rem < 8 ? 256 / rem : 8;
-		while (splits > 1 && nk / splits < 16) splits--;
+	const float fill = way.tiles / 256.f;
+	float group = nk * 0.45f + 9.9f;
+	if (!way.small) {
+		group = (nk + way.splits - 1) / way.splits * (0.8f + 0.8f * fill) + 18.f;
+		if (way.splits > 1) group += 6.f * (way.splits - 1) + 30.f * way.splits * fill;  // the parts of a tile add one after the other
 	}
-	const float last = (nk + splits - 1) / splits * t256.slice + t256.round + 10.f * (splits - 1);
-	if (tiles > 256) return false;
-	float group = last;
-	if (small <= 256) group = fminf(group, nk * t128.slice + t128.round);
 	return group < 0.97f * apart;
+}
+
+int linear_w_way(int n, const LinearW* layers, int T) {
+	ELF_REQUIRE(n > 0 && n <= DW_GROUP_MAX && layers && T > 0 && T % BK == 0, "linear_w_way: 1..%d layers over a multiple of %d tokens", DW_GROUP_MAX, BK);
+	DwProblem pr[DW_GROUP_MAX];
+	for (int i = 0; i < n; i++) {
+		const LinearW& l = layers[i];
+		if (!gemm_dw_groupable(l.M, l.N, T, l.dY, l.lddy, l.X, l.ldx, l.acc)) return 0;
+		pr[i] = DwProblem{l.dY, l.lddy, l.X, l.ldx, l.acc, nullptr, l.M, l.N};
+	}
+	return n == 1 || !group_pays(n, pr, T) ? 0 : gemm_dw_group_way(n, pr, T).small ? 128 : 256;
 }
 
 int linear_w_pass(int n, const LinearW* layers, int T, float* workspace, hipStream_t stream) {

@@ -167,9 +167,33 @@ bool gemm_dw_groupable(int M, int N, int K, const void* dY, int64_t lddy, const 
 	       ((uintptr_t)dY % 16) == 0 && ((uintptr_t)X % 16) == 0 && ((uintptr_t)acc % 16) == 0;
 }
 
+DwGroupWay gemm_dw_group_way(int n, const DwProblem* pr, int K) {
+	DwGroupWay w;
+	int64_t small = 0;
+	for (int i = 0; i < n; i++) {
+		w.tiles += (int64_t)((pr[i].M + 255) / 256) * ((pr[i].N + dma::BN - 1) / dma::BN);
+		small += (int64_t)((pr[i].M + 127) / 128) * ((pr[i].N + 127) / 128);
+	}
+	// Whole tiles, one workgroup each, except in the launch's last round: when that round would fill at most half of the
+	// chip, its tiles (the last ones of the last problems) are split along K so that proportionally shorter workgroups
+	// fill it - at least 16 K slices each, and no more than 8 ways (the splits of a tile add with atomics, one after the
+	// other: past that their adds cost more than the idle compute units).
+	const int nk = K / dma::BKS;
+	if (const int rem = (int)(w.tiles % 256); rem != 0 && rem <= 128 && rem <= dma::TURN_TILES) {
+		w.splits = 256 / rem < 8 ? 256 / rem : 8;
+		while (w.splits > 1 && nk / w.splits < 16) w.splits--;
+		if (w.splits > 1) w.tail = rem;
+	}
+	// Little work: where the layers make no more than a round of 128x128 tiles, these are done sooner than a few 256x256 ones (us,
+	// without and with the splits of the latter; fitted to launches over 128 to 8192 tokens).  Two blocks of a 512-wide Llama stage
+	// over 512 tokens 23.7 -> 12.7 us, of a 256-wide GPT stage 21.4 -> 10.8, one over 2048 tokens 33.5 -> 18.4; with two rounds it
+	// is one or the other (four layers of 768 over 1024 tokens 33.8 and 29.4, eight of 512 33.5 and 34.7).
+	w.small = small <= 256 && nk * 0.35f + 7.5f < (float)((nk + w.splits - 1) / w.splits) * 1.05f + 12.f + 2.f * (w.splits - 1);
+	return w;
+}
+
 int gemm_dw_group(int n, const DwProblem* pr, int K, float scale, hipStream_t stream) {
 	ELF_REQUIRE(n > 0 && n <= dma::GROUP_MAX && pr, "gemm_dw_group: 1..%d problems", dma::GROUP_MAX);
-	int64_t tiles = 0;
 	double flops = 0;
 	bool edge = false;
 	auto tiles_of = [](const DwProblem& q) { return ((q.M + 255) / 256) * ((q.N + dma::BN - 1) / dma::BN); };
@@ -177,31 +201,16 @@ int gemm_dw_group(int n, const DwProblem* pr, int K, float scale, hipStream_t st
 		ELF_REQUIRE(pr[i].dY && pr[i].X && pr[i].acc && gemm_dw_groupable(pr[i].M, pr[i].N, K, pr[i].dY, pr[i].lddy, pr[i].X, pr[i].ldx, pr[i].acc),
 		            "gemm_dw_group: problem %d (M=%d N=%d K=%d) needs M, N of at least 256, all sizes multiples of 64 and 16-byte aligned operands", i, pr[i].M, pr[i].N, K);
 		ELF_REQUIRE(scale == 0.f || (pr[i].grad_bf16 && ((uintptr_t)pr[i].grad_bf16 % 8) == 0), "gemm_dw_group: a scaling pass needs the bf16 gradient buffers");
-		tiles += tiles_of(pr[i]);
 		edge = edge || pr[i].M % 256 || pr[i].N % dma::BN;
 		flops += 2.0 * pr[i].M * pr[i].N * K;
 	}
-	// Whole tiles, one workgroup each, except in the launch's last round: when that round would fill at most half of the
-	// chip, its tiles (the last ones of the last problems) are split along K so that proportionally shorter workgroups
-	// fill it - at least 16 K slices each, and no more than 8 ways (the splits of a tile add with atomics, one after the
-	// other: past that their adds cost more than the idle compute units).
-	const int nk = K / dma::BKS;
-	int splits = 1, tail = 0;
-	if (const int rem = (int)(tiles % 256); rem != 0 && rem <= 128 && rem <= dma::TURN_TILES) {
-		splits = 256 / rem < 8 ? 256 / rem : 8;
-		while (splits > 1 && nk / splits < 16) splits--;
-		if (splits > 1) tail = rem;
-	}
-	// Little work: where the layers make no more than a round of 128x128 tiles, these are done sooner than a few 256x256 ones (us,
-	// without and with the splits of the latter; fitted to launches over 128 to 8192 tokens).  Two blocks of a 512-wide Llama stage
-	// over 512 tokens 23.7 -> 12.7 us, of a 256-wide GPT stage 21.4 -> 10.8, one over 2048 tokens 33.5 -> 18.4; with two rounds it
-	// is one or the other (four layers of 768 over 1024 tokens 33.8 and 29.4, eight of 512 33.5 and 34.7).
-	int64_t small = 0;
-	for (int i = 0; i < n; i++) small += (int64_t)((pr[i].M + 127) / 128) * ((pr[i].N + 127) / 128);
-	if (small <= 256 && nk * 0.35f + 7.5f < (float)((nk + splits - 1) / splits) * 1.05f + 12.f + 2.f * (splits - 1)) {
+	const DwGroupWay way = gemm_dw_group_way(n, pr, K);
+	if (way.small) {
 		ProfScope prof(PROF_GEMM, flops, stream);
 		return gemm_ring_dw_group(n, pr, K, scale, stream);
 	}
+	const int64_t tiles = way.tiles;
+	const int splits = way.splits, tail = way.tail;
 	dma::GroupArgs ga{};
 	ga.n = n;
 	ga.compact = 1;

@@ -79,6 +79,13 @@ constexpr int DW_GROUP_MAX = 16;
 int gemm_ring_dw_group(int n, const DwProblem* problems, int K, float scale, hipStream_t stream);  // on 128x128 ring tiles
 bool gemm_dw_groupable(int M, int N, int K, const void* dY, int64_t lddy, const void* X, int64_t ldx, const void* acc);
 int gemm_dw_group(int n, const DwProblem* problems, int K, float scale, hipStream_t stream);
+// How that launch is done: 128x128 tiles (small), or `tiles` 256x256 ones of which the last `tail` are split `splits` ways along K.
+struct DwGroupWay {
+	bool small = false;
+	int64_t tiles = 0;
+	int splits = 1, tail = 0;
+};
+DwGroupWay gemm_dw_group_way(int n, const DwProblem* problems, int K);
 
 // The parameter gradients of linear layers over the same T tokens: acc [M, N] += dY^T X, bias [M] (optional) += column sums of dY.
 // Weight gradients share launches where that is the faster way, bias sums two; layers whose accumulators overlap follow each other.
@@ -92,6 +99,7 @@ struct LinearW {
 	int M, N;
 };
 int linear_w_pass(int n, const LinearW* layers, int T, float* workspace, hipStream_t stream);
+int linear_w_way(int n, const LinearW* layers, int T);
 int64_t colsum_group_workspace_floats(int n, const LinearW* layers, int T);
 int colsum_group(int n, const LinearW* layers, int T, float* workspace, hipStream_t stream);  // the bias sums alone
 

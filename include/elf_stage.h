@@ -96,6 +96,9 @@ typedef struct elf_linear_w {
 } elf_linear_w;
 int64_t elf_linear_w_workspace_floats(int n, const elf_linear_w* layers, int T);
 int elf_linear_w_pass(int n, const elf_linear_w* layers, int T, float* workspace, void* stream);
+/* Which way that call takes the weight gradients of a list of at most 16 layers with accumulators apart: 0 a launch each, 128 or 256
+ * one launch of 128x128 or 256x256 tiles.  Host only; for tests and tuning, no counterpart in the reference. */
+int elf_linear_w_way(int n, const elf_linear_w* layers, int T);
 
 /* The MLP's up-projection with its activation: pre = A W^T with A [M, K] and W [N, K], both k contiguous;
  * act 0 (GELU): N = F, out[M, F] = gelu(pre); act 1 (SwiGLU): N = 2F, W = [gate rows; up rows],

@@ -276,3 +276,19 @@ def test_an_unusable_torch_library_leaves_the_figures_to_pytorch(monkeypatch, tm
 			assert _lib.torch_allocated(0) is None
 			m.setattr(_lib, "_torch_reader", lambda: pytest.fail("looked for again"))
 			assert _lib.torch_allocated(0) is None
+
+
+@pytest.mark.parametrize("T,shapes,way", [
+	(2112, [(4288, 1600), (832, 4288)], 256), (512, [(512, 512), (1536, 512), (512, 768)], 128), (256, [(2112, 1024), (384, 2112)], 128),
+	(8192, [(1536, 1536), (1536, 256)], 0), (3008, [(1344, 384), (4544, 1344)], 0), (2048, [(4096, 960), (960, 2560)], 0), (4096, [(2048, 2048), (2048, 2048)], 0),
+	(4544, [(5824, 7232), (1792, 5824)], 0), (2112, [(4288, 1600), (192, 4288)], 0), (512, [(512, 512)], 0),
+])
+def test_weight_gradients_share_a_launch_where_the_way_it_takes_is_faster(lib, T, shapes, way):
+	"""Lists that the one launch does sooner, on 256x256 and on 128x128 tiles, and lists that it would do later on the tiles it takes (measured:
+	123 us for 96, 79 for 68, 66 for 56, 102 for 94), that make more than a round of tiles or hold a layer no such launch takes."""
+	from elf_amd.kernels import _LinearW
+
+	layers = (_LinearW * len(shapes))()
+	for q, (M, N) in zip(layers, shapes):
+		q.dY, q.lddy, q.X, q.ldx, q.acc, q.M, q.N = 1 << 20, M, 1 << 20, N, 1 << 20, M, N
+	assert lib.elf_linear_w_way(len(shapes), layers, T) == way
