@@ -816,12 +816,14 @@ static Splits split_short(int B, int S, int Hq, int Hkv, int D, bool causal, int
 
 // 128 tokens: one kernel for the whole call (attention_bwd_one.hip) or -delta, walks and sums in three.  A workgroup of the one kernel has a compute
 // unit to itself and takes the query heads of its group in turn (4.3 us each for heads of 64, 7.3 of 128; 6 and 7 us besides), the walks
-// are shared.  Whole call of every sort of group on 2 to 1600 workgroups, three kernels -> one (us, causal / not):
-//   one head of 64 a group: 16 groups 16.8 -> 10.8 / 16.1 -> 11.0, 240 24.8 -> 13.3 / 20.6 -> 13.8, 272 29.8 -> 23.4 / 25.3 -> 24.2, 800 59.1 -> 49.8 / 48.8 -> 51.4
-//   one of 128: 16 20.3 -> 15.7 / 20.6 -> 17.1, 240 32.2 -> 22.7 / 31.3 -> 26.0, 800 94.8 -> 79.1 / 91.9 -> 90.3
-//   four of 64: 32 24.4 and 24.5 / 21.6 and 25.1, 96 35.8 -> 26.4 / 30.4 -> 27.1, 320 63.8 -> 55.7 / 58.0 and 58.3
-//   four of 128: 64 37.6 and 41.5 / 41.3 and 45.3, 96 47.4 -> 43.6 / 46.2 and 48.1, 256 67.3 -> 57.3 / 66.8 and 64.4
-//   eight: 64 groups of 64 38.0 and 45.2, 128 58.2 -> 48.4 / 52.5 and 50.3; of 128 128 75.5 and 79.3, 320 173.5 and 179.9
+// are shared.  Whole call, three kernels -> one, on operands past the caches (us, causal / not; on operands in them both take 4 to 15 % less):
+//   one head of 64 a group: 16 groups 18.3 -> 11.0 / 16.6 -> 11.3, 240 28.1 -> 16.6 / 23.7 -> 17.0, 272 34.6 -> 27.8 / 28.6 and 28.4, 800 68.4 -> 55.5 / 56.3 and 56.9
+//   one of 128: 16 21.2 -> 16.2 / 21.2 -> 17.5, 240 34.4 -> 26.1 / 33.3 -> 28.5, 800 104.4 -> 87.6 / 100.5 -> 95.9
+//   two of 128: 256 48.2 -> 38.6 / 47.2 -> 42.2, 512 85.4 -> 71.4 / 83.4 and 78.3; three: 256 58.6 -> 50.6 / 57.2 and 55.7, 264 83.6 -> 82.6 / 81.8 and 91.7
+//   four of 64: 64 31.2 -> 29.3 / 28.5 and 29.9, 96 37.7 -> 29.8 / 31.4 -> 30.7, 320 69.0 -> 61.1 / 60.8 and 62.7
+//   four of 128: 96 49.9 -> 49.1 / 48.5 and 53.1, 256 71.6 -> 63.3 / 70.2 and 68.8, 264 100.3 and 104.1, 288 101.8 and 105.9, 352 108.7 -> 107.6 / 105.4 and 117.8
+//   eight of 64: 112 58.5 -> 52.8 / 52.1 and 53.6, 224 85.2 -> 57.7 / 76.6 -> 58.8, 252 90.3 -> 57.9 / 80.9 -> 59.2
+//   eight of 128: 128 77.4 and 88.5 / 75.7 and 96.8, 224 105.0 -> 101.4 / 104.1 and 109.7, 252 112.8 -> 103.5 / 111.0 and 113.4, 272 161.6 and 180.9
 //
 // It addresses all 128 rows of Q, dO and (heads of 128) V with 32-bit byte offsets, where the three kernels take 32 rows of Q and dO and
 // read V through 64-bit pointers: rows that far apart stay with those.  So do V's of 128 columns a head that are not 16-byte aligned: the one
@@ -829,7 +831,7 @@ static Splits split_short(int B, int S, int Hq, int Hkv, int D, bool causal, int
 static bool one_kernel_pays(int B, int S, int Hq, int Hkv, int D, bool causal) {
 	const int64_t groups = (int64_t)B * Hkv, G = Hq / Hkv;
 	if (S != 128 || G > 8 || groups < (causal && D == 64 ? 16 : 32) * (G - 1)) return false;
-	if (causal) return groups <= 256 || G <= 4;
+	if (causal) return groups <= 256 || G < 4 || (G == 4 && (D == 64 || groups >= 320));
 	return D == 64 ? groups <= 256 : G == 1 || (G == 2 && groups <= 256);
 }
 

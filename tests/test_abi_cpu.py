@@ -292,3 +292,13 @@ def test_weight_gradients_share_a_launch_where_the_way_it_takes_is_faster(lib, T
 	for q, (M, N) in zip(layers, shapes):
 		q.dY, q.lddy, q.X, q.ldx, q.acc, q.M, q.N = 1 << 20, M, 1 << 20, N, 1 << 20, M, N
 	assert lib.elf_linear_w_way(len(shapes), layers, T) == way
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,D,causal,one", [
+	(32, 32, 8, 128, True, True), (33, 32, 8, 128, True, False), (38, 32, 8, 128, True, False), (40, 32, 8, 128, True, True), (33, 24, 8, 128, True, True), (33, 32, 8, 64, True, True),
+	(28, 64, 8, 128, True, True), (32, 64, 8, 128, True, True), (33, 64, 8, 128, True, False), (28, 64, 8, 64, False, True), (32, 64, 8, 128, False, False),
+])
+def test_attention_backward_of_128_tokens_takes_the_faster_way(lib, B, Hq, Hkv, D, causal, one):
+	"""One kernel or three, whichever was measured to be faster on operands past the caches: causal groups of four heads of 128 in a second
+	round that is not a quarter full stay with three (264 groups 100.3 us and 104.1)."""
+	assert (_attn_way(lib, (B, 128, Hq, Hkv, D), causal)[0] == 0) == one
