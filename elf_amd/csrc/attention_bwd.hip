@@ -920,7 +920,7 @@ int attn_bwd(const void* q, const void* k, const void* v, const void* o, const v
 	const AttnBwdWay way = attn_bwd_way(v, ldq, ldv, lddo, B, S, Hq, Hkv, D, causal, workspace_bytes);
 	if (way.keys == 0) {
 		const AttnBwdArgs a{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)dO, nullptr, nullptr, nullptr,
-		                    (bf16_t*)dk, (bf16_t*)dv, ldq, ldk, ldv, lddo, lddk, lddv, B, S, Hq, Hkv, scale, (const float2*)rope_cs, 1, 1, nullptr, 0};
+		                    (bf16_t*)dk, (bf16_t*)dv, ldq, ldk, ldv, lddo, lddk, lddv, B, S, Hq, Hkv, scale, (const float2*)rope_cs, 1, 1, nullptr, 0, 0};
 		return launch_bwd_one(a, D, causal != 0, (const bf16_t*)o, (const float*)lse, (bf16_t*)dq, ldo, lddq, stream);
 	}
 	bf16_t* dq_part = (bf16_t*)workspace;
@@ -933,10 +933,12 @@ int attn_bwd(const void* q, const void* k, const void* v, const void* o, const v
 	                   (const bf16_t*)o, (const float*)lse, ndelta, nlse2, lddo, ldo, B, S, Hq, D);
 	}
 	float* dkv_part = way.h_splits * way.q_splits > 1 ? nlse2 + T * Hq : nullptr;
-	AttnBwdArgs a{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)dO, nlse2, ndelta, dq_part,
-	              (bf16_t*)dk, (bf16_t*)dv, ldq, ldk, ldv, lddo, lddk, lddv, B, S, Hq, Hkv, scale, (const float2*)rope_cs, way.h_splits, way.q_splits, dkv_part, way.paired};
 	const int nkt = (S + way.keys - 1) / way.keys;
-	const dim3 grid((unsigned)((int64_t)B * Hkv * (way.paired ? (nkt + 1) / 2 : nkt) * way.h_splits * way.q_splits)), block(256);
+	const int64_t workgroups = (int64_t)B * Hkv * (way.paired ? (nkt + 1) / 2 : nkt) * way.h_splits * way.q_splits;
+	const int longest_first = causal && !way.paired && nkt > 1 && workgroups > 256;
+	AttnBwdArgs a{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (const bf16_t*)dO, nlse2, ndelta, dq_part,
+	              (bf16_t*)dk, (bf16_t*)dv, ldq, ldk, ldv, lddo, lddk, lddv, B, S, Hq, Hkv, scale, (const float2*)rope_cs, way.h_splits, way.q_splits, dkv_part, way.paired, longest_first};
+	const dim3 grid((unsigned)workgroups), block(256);
 	int rc;
 	if (way.keys == 256) rc = launch_bwd_wide(a, causal != 0, grid, stream);
 	else if (D == 128) rc = causal ? launch_bwd<128, true>(a, grid, stream) : launch_bwd<128, false>(a, grid, stream);

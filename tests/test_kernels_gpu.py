@@ -877,6 +877,34 @@ def test_attention_backward_of_128_tokens_in_one_kernel(K, cfg):
 	assert torch.equal(fused, K.rope_apply_(dqkv.clone(), cs, S, Hq + Hkv, D, backward=True))
 
 
+def _check_attn_bwd(K, cfg, way, seed):
+	"""The way a shape takes, then gradients against fp32 autograd, equal bits from run to run and the rotation undone as by a pass of its own."""
+	B, S, Hq, Hkv, D, causal = cfg
+	T = B * S
+	assert K.attn_bwd_way(*cfg) == way
+	qkv, do = _randn(T, (Hq + 2 * Hkv) * D, seed=seed), _randn(T, Hq * D, seed=seed + 1)
+	o_ref, _, dqkv_ref = _attn_ref(qkv, B, S, Hq, Hkv, D, causal, do)
+	o, lse = K.attn_fwd(qkv, B, S, Hq, Hkv, D, causal)
+	dqkv = K.attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal)
+	for name, sl in (("dq", slice(0, Hq * D)), ("dk", slice(Hq * D, (Hq + Hkv) * D)), ("dv", slice((Hq + Hkv) * D, None))):
+		_close(dqkv[:, sl], dqkv_ref[:, sl], rel_fro=1.5e-2, what=f"attn {name} {cfg}")
+	assert torch.equal(dqkv, K.attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal))
+	cs = K.rope_table(S, D, 5e5)
+	fused = K.attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal, rope_cs=cs)
+	assert torch.equal(fused, K.rope_apply_(dqkv.clone(), cs, S, Hq + Hkv, D, backward=True))
+
+
+@pytest.mark.parametrize("cfg,way", [
+	((8, 256, 1, 1, 128, True), (128, 1, 4, False)), ((9, 640, 8, 8, 128, True), (128, 1, 1, False)), ((11, 512, 7, 7, 128, True), (128, 1, 1, False)),
+	((8, 384, 8, 8, 64, True), (128, 1, 1, False)), ((9, 384, 9, 9, 64, True), (128, 1, 1, False)),
+	((1, 1152, 6, 3, 64, True), (256, 2, 4, False)), ((8, 1024, 16, 8, 64, True), (256, 1, 1, False)), ((9, 1024, 16, 8, 64, True), (256, 1, 1, False)),
+])
+def test_attention_backward_of_single_key_tiles_that_fit_at_once_or_do_not(K, cfg, way):
+	"""Causal launches of single key tiles, of each kernel: 64 to 256 workgroups (a group's tiles side by side) and 288 to 360 (the longest
+	walks first), groups in a multiple of eight (each on one XCD) and not."""
+	_check_attn_bwd(K, cfg, way, 67)
+
+
 def _attn_bwd_separate(B, S, Hq, Hkv, D, causal, q, k, v, o, do, lse, rope_cs=None):
 	"""dq, dk and dv of operands in buffers of their own ([B * S, heads * D] with any row stride)."""
 	from elf_amd import _lib
