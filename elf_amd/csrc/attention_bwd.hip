@@ -843,7 +843,10 @@ static bool one_kernel_pays(int B, int S, int Hq, int Hkv, int D, bool causal) {
 // tiles fit the chip at once, and the 128-key kernel for heads of 64, these shapes take 0.96 and 0.80 of the time.  The whole call,
 // before -> after (us): 8 x 1408 tokens, 6 / 2 heads of 128 161 -> 140 (single tiles, heads split 3 ways); 3 x 896, 32 / 8 heads of 128 134 -> 118;
 // 4096 tokens, 64 / 8 heads of 128 1424 -> 1012 (128 whole pairs before, shared 2 ways now); 8 x 1024, 12 heads of 64 101 -> 65, not causal
-// 130 -> 103; 8192 tokens, 16 heads of 64 559 -> 360.  Pairs that make whole rounds stay: 4 x 4096, 32 / 8 heads of 128 2020, single tiles 2053.
+// 130 -> 103; 8192 tokens, 16 heads of 64 559 -> 360.  Single tiles of 128 keys, a few more than fit: the last ones follow the shortest walks, which
+// short sequences feel (2.2 walks of the last key tile; of 436 shapes of 256 to 4096 tokens 3 instead of 9 take 3 % longer than the
+// sharing before these constants; 11 x 256, 12 / 2 heads of 128 shared 6 ways, 264 workgroups, 58, 3 ways 50; 2 x 384, 44 / 22 heads 61
+// shared 2 ways, whole 55).  Pairs that make whole rounds stay: 4 x 4096, 32 / 8 heads of 128 2020, single tiles 2053.
 static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal, int64_t room) {
 	const int G = Hq / Hkv;
 	// Heads of 64 columns: a pass of 256 keys has twice the fixed part of one of 128.  Below 896 tokens it pays where there is work for the
@@ -869,7 +872,8 @@ static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal, int6
 				float us;
 				if (causal && paired && n > 1) us = ceilf(walks * ((n + 1) / 2) / slots) * (2.f * fixed + per * (2 * Q - tile * (n - 1)));
 				else if (!causal || n == 1) us = ceilf(walks * n / slots) * (fixed + per * Q);
-				else us = fmaxf(fixed + per * Q, walks * n <= slots ? 0.f : walks * (n * fixed + per * ((float)n * Q - tile * 0.5f * n * (n - 1))) / slots + 0.5f * fixed);
+				else if (walks * n <= slots) us = fixed + per * Q;
+				else us = fmaxf(fmaxf(fixed + per * Q, (wide ? 0.f : 2.2f) * (fixed + per * tile)), walks * (n * fixed + per * ((float)n * Q - tile * 0.5f * n * (n - 1))) / slots + 0.5f * fixed);
 				if (ns > 1) us = (us + split + ns * per_split + (float)ns * B * S * Hkv * D * 16 / rate) / margin;
 				if (us < best_us) best_us = us, best = Splits{h, q, paired != 0, wide};
 			}

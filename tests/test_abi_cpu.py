@@ -302,3 +302,11 @@ def test_attention_backward_of_128_tokens_takes_the_faster_way(lib, B, Hq, Hkv, 
 	"""One kernel or three, whichever was measured to be faster on operands past the caches: causal groups of four heads of 128 in a second
 	round that is not a quarter full stay with three (264 groups 100.3 us and 104.1)."""
 	assert (_attn_way(lib, (B, 128, Hq, Hkv, D), causal)[0] == 0) == one
+
+
+@pytest.mark.parametrize("shape,way", [((2, 384, 44, 22, 128), (128, 1, 1, False)), ((18, 256, 16, 4, 128), (128, 1, 1, False)), ((11, 256, 12, 2, 128), (128, 3, 1, False)),
+                                       ((2, 384, 48, 6, 128), (128, 4, 1, False)), ((6, 256, 48, 12, 128), (128, 1, 1, False))])
+def test_attention_backward_shares_no_walks_into_a_second_round_that_is_nearly_empty(lib, shape, way):
+	"""Causal, heads of 128, a few single key tiles more than compute units: the sharing before is faster as measured (us, shared into 264 and 288
+	workgroups and as here: 61.2 and 55.4, 76.4 and 73.3, 58.2 and 50.0, 63.9 and 60.7, 77.6 and 73.1)."""
+	assert _attn_way(lib, shape, True) == way
