@@ -849,12 +849,15 @@ static bool one_kernel_pays(int B, int S, int Hq, int Hkv, int D, bool causal) {
 // shared 2 ways, whole 55).  Pairs that make whole rounds stay: 4 x 4096, 32 / 8 heads of 128 2020, single tiles 2053.
 static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal, int64_t room) {
 	const int G = Hq / Hkv;
-	// Heads of 64 columns: a pass of 256 keys has twice the fixed part of one of 128.  Below 896 tokens it pays where there is work for the
-	// chip (heads x key tiles of 128), below 512 if the passes fit at once or the 128-key ones do not either (us, 128 and 256 keys): 3 x 384
-	// tokens, 31 heads, causal 40 and 33, 3 x 256, 16 heads 22 and 23, 5 x 384, 26 heads 42 and 57; 3 x 512, 8 heads 30 and 33, 16 heads
-	// 37 and 36; 512 tokens, 7 heads, causal 22 and 23, 2 x 512, 6 / 1 heads, causal 33 and 30.
+	// Heads of 64 columns: a pass of 256 keys has twice the fixed part of one of 128.  Short sequences take it where there is work for the
+	// chip (heads x key tiles of 128), below 512 tokens if the passes fit at once or the 128-key ones do not either, long ones always (us, 128
+	// and 256 keys).  Causal: 3 x 384 tokens, 31 heads 40 and 33, 512, 7 heads 22 and 23, 2 x 512, 6 / 1 heads 33 and 30.  Not: 3 x 256,
+	// 16 heads 22 and 23, 5 x 384, 26 heads 42 and 57, 3 x 512, 8 heads 30 and 33, 640, 24 / 8 heads 33.6 and 35.9, 30 / 10 39.7 and 34.1, 1024,
+	// 2 heads 23.4 and 25.6, 2 x 1024, 4 / 1 heads 31.9 and 33.7, 5 x 896, 2 heads 33.7 and 30.5, 1280, 4 / 1 heads 33.3 and 34.0, 1536, 4 / 2 34.3 either
+	// way, 5 x 1536, 2 heads 48.7 and 40.1.
 	const int64_t work = (int64_t)B * Hq * (S / 128), tiles128 = (int64_t)B * Hkv * (S / 128), tiles256 = (int64_t)B * Hkv * ((S + 255) / 256);
-	const bool wide = D == 64 && S >= 256 && (S >= 896 || (S >= 512 && work >= (causal ? 48 : 120)) || (work >= 256 && (tiles256 <= 256 || tiles128 > 512)));
+	const bool worth = causal ? S >= 896 || (S >= 512 && work >= 48) : S >= 1408 || (S >= 896 && work >= 70) || (S >= 512 && work >= 150);
+	const bool wide = D == 64 && S >= 256 && (worth || (work >= 256 && (tiles256 <= 256 || tiles128 > 512)));
 	if (S < 256 || (D == 64 && !wide)) return split_short(B, S, Hq, Hkv, D, causal, room);
 	const int keys = wide ? 256 : 128, n = (S + keys - 1) / keys, tile = keys / 32, Q = S / 32;  // key tiles; query tiles of a key tile, of a sequence
 	const float slots = 256.f, step = wide ? 1.f : 1.05f, fixed = wide ? 4.f : 9.f;

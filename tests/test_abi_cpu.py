@@ -310,3 +310,11 @@ def test_attention_backward_shares_no_walks_into_a_second_round_that_is_nearly_e
 	"""Causal, heads of 128, a few single key tiles more than compute units: the sharing before is faster as measured (us, shared into 264 and 288
 	workgroups and as here: 61.2 and 55.4, 76.4 and 73.3, 58.2 and 50.0, 63.9 and 60.7, 77.6 and 73.1)."""
 	assert _attn_way(lib, shape, True) == way
+
+
+@pytest.mark.parametrize("shape,keys", [((1, 1024, 2, 2, 64), 128), ((2, 1024, 4, 1, 64), 128), ((1, 1280, 4, 1, 64), 128), ((1, 640, 24, 8, 64), 128), ((1, 896, 6, 6, 64), 128),
+                                        ((5, 896, 2, 2, 64), 256), ((1, 640, 30, 10, 64), 256), ((1, 1408, 1, 1, 64), 256), ((8, 1024, 12, 12, 64), 256)])
+def test_attention_backward_of_little_work_without_a_mask_stays_with_128_keys_a_pass(lib, shape, keys):
+	"""Heads of 64: passes over 256 keys where they were measured to be no slower (us, 128 and 256 keys: 23.4 and 25.6, 31.9 and 33.7, 33.3 and
+	34.0, 33.6 and 35.9, 27.4 and 28.1; 33.7 and 30.5, 39.7 and 34.1)."""
+	assert _attn_way(lib, shape, False)[0] == keys
