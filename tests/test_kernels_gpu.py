@@ -821,13 +821,14 @@ def test_attention_backward_with_walks_shared_by_workgroups(K, cfg):
 	assert sizes == sorted(sizes)
 
 
-@pytest.mark.parametrize("cfg", [(1, 896, 4, 4, 64, False), (2, 1152, 4, 2, 64, True), (9, 256, 16, 16, 64, True), (6, 384, 20, 4, 64, False), (1, 2048, 3, 3, 64, True), (3, 1024, 48, 8, 64, True)])
+@pytest.mark.parametrize("cfg", [(5, 896, 2, 2, 64, False), (2, 1152, 4, 2, 64, True), (9, 256, 16, 16, 64, True), (6, 384, 20, 4, 64, False), (1, 2048, 3, 3, 64, True), (3, 1024, 48, 8, 64, True)])
 def test_attention_backward_of_64_columns_over_256_keys_a_pass(K, cfg):
-	"""Heads of 64 columns take 256 keys a pass from 896 tokens up, shorter ones where they fill the chip: sequences that 256 divides
+	"""Heads of 64 columns take 256 keys a pass where the sequence is long or there is work for the chip: sequences that 256 divides
 	and odd multiples of 128 (half of the last pass lies past the end), one pass and many, walks whole, split by heads and by
 	queries, more workgroups than compute units.  Bounds of the 128-key kernels above: the same bf16 roundings, half as many of dQ."""
 	B, S, Hq, Hkv, D, causal = cfg
 	T = B * S
+	assert K.attn_bwd_way(*cfg)[0] == 256
 	qkv, do = _randn(T, (Hq + 2 * Hkv) * D, seed=59), _randn(T, Hq * D, seed=60)
 	o_ref, _, dqkv_ref = _attn_ref(qkv, B, S, Hq, Hkv, D, causal, do)
 	o, lse = K.attn_fwd(qkv, B, S, Hq, Hkv, D, causal)
@@ -858,13 +859,14 @@ def test_attention_backward_with_a_workgroup_per_key_tile(K, cfg):
 	assert torch.equal(fused, K.rope_apply_(dqkv.clone(), cs, S, Hq + Hkv, D, backward=True))
 
 
-@pytest.mark.parametrize("cfg", [(1, 1, 1, 64, False), (3, 5, 5, 64, True), (2, 3, 3, 128, False), (1, 2, 2, 128, True), (9, 32, 32, 64, True), (9, 32, 32, 128, True), (8, 6, 2, 64, False),
+@pytest.mark.parametrize("cfg", [(1, 1, 1, 64, False), (3, 5, 5, 64, True), (2, 3, 3, 128, False), (1, 2, 2, 128, True), (9, 32, 32, 64, True), (9, 32, 32, 128, True), (32, 6, 2, 64, False),
                                  (16, 6, 3, 64, True), (17, 4, 2, 128, False), (14, 64, 8, 64, True)])
 def test_attention_backward_of_128_tokens_in_one_kernel(K, cfg):
 	"""One key tile: a head a workgroup and groups of two to eight, one workgroup, more than compute units, the fewest groups
 	of a size that come here.  Bounds, repeated bits and rotation as above (dQ has one rounding less)."""
 	B, Hq, Hkv, D, causal = cfg
 	S, T = 128, B * 128
+	assert K.attn_bwd_way(B, S, Hq, Hkv, D, causal)[0] == 0
 	qkv, do = _randn(T, (Hq + 2 * Hkv) * D, seed=61), _randn(T, Hq * D, seed=62)
 	o_ref, _, dqkv_ref = _attn_ref(qkv, B, S, Hq, Hkv, D, causal, do)
 	o, lse = K.attn_fwd(qkv, B, S, Hq, Hkv, D, causal)
@@ -905,6 +907,17 @@ def test_attention_backward_of_single_key_tiles_that_fit_at_once_or_do_not(K, cf
 	_check_attn_bwd(K, cfg, way, 67)
 
 
+@pytest.mark.parametrize("cfg,way", [
+	((8, 2048, 32, 16, 64, True), (256, 1, 1, True)), ((8, 1920, 32, 8, 64, True), (256, 1, 1, True)), ((1, 3968, 16, 2, 64, True), (256, 8, 2, True)),
+	((13, 384, 60, 10, 64, True), (128, 1, 1, True)),
+])
+def test_attention_backward_of_pairs_of_key_tiles_of_64_columns(K, cfg, way):
+	"""Causal, a light and a heavy key tile one after the other in a workgroup: the second pass reuses the first one's LDS, takes a last tile
+	that is half past the end (1920 and 3968 tokens are odd multiples of 128), leaves partial dK and dV, and follows the middle tile of three,
+	which has no partner (384 tokens)."""
+	_check_attn_bwd(K, cfg, way, 69)
+
+
 def _attn_bwd_separate(B, S, Hq, Hkv, D, causal, q, k, v, o, do, lse, rope_cs=None):
 	"""dq, dk and dv of operands in buffers of their own ([B * S, heads * D] with any row stride)."""
 	from elf_amd import _lib
@@ -917,6 +930,57 @@ def _attn_bwd_separate(B, S, Hq, Hkv, D, causal, q, k, v, o, do, lse, rope_cs=No
 	                             B, S, Hq, Hkv, D, int(causal), 1 / math.sqrt(D), rope_cs.data_ptr() if rope_cs is not None else None, torch.cuda.current_stream().cuda_stream)
 	_lib.check(rc, "elf_attn_bwd_shared")
 	return dq, dk, dv
+
+
+_EACH_KERNEL = [((3, 128, 5, 5, 64, True), 0), ((2, 128, 3, 3, 128, False), 0), ((32, 128, 6, 2, 64, False), 0), ((2, 1152, 4, 2, 64, True), 256),
+                ((5, 896, 2, 2, 64, False), 256), ((8, 384, 2, 1, 64, True), 128), ((3, 256, 4, 2, 128, True), 128)]
+
+
+@pytest.mark.parametrize("cfg,keys", _EACH_KERNEL)
+def test_attention_backward_of_operands_in_buffers_of_their_own(K, cfg, keys):
+	"""Rows of q, k, v, o and dO with a stride of their own each: the bits of packed rows."""
+	B, S, Hq, Hkv, D, causal = cfg
+	T = B * S
+	assert K.attn_bwd_way(*cfg)[0] == keys
+	qkv, do = _randn(T, (Hq + 2 * Hkv) * D, seed=71), _randn(T, Hq * D, seed=72)
+	o, lse = K.attn_fwd(qkv, B, S, Hq, Hkv, D, causal)
+	want = K.attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal)
+	own = []
+	for i, t in enumerate((*qkv.split([Hq * D, Hkv * D, Hkv * D], dim=1), o, do)):
+		own.append(torch.full((T, t.shape[1] + 8 * (2 * i + 1)), float("nan"), dtype=torch.bfloat16, device="cuda")[:, : t.shape[1]])
+		own[-1].copy_(t)
+	got = _attn_bwd_separate(B, S, Hq, Hkv, D, causal, *own, lse)
+	assert torch.equal(torch.cat(got, dim=1), want)
+
+
+@pytest.mark.parametrize("cfg,keys", _EACH_KERNEL)
+@pytest.mark.parametrize("what", [float("inf"), float("nan")])
+def test_attention_backward_keeps_an_infinity_in_its_group(K, cfg, keys, what):
+	"""An infinity or NaN in one dO row of one head: every other group of heads and sequence has the bits it has without, and of that head's dQ
+	the rows of other queries too; that row's dQ is not finite, and no dV of a key it attends to is."""
+	B, S, Hq, Hkv, D, causal = cfg
+	T, G = B * S, Hq // Hkv
+	assert K.attn_bwd_way(*cfg)[0] == keys
+	qkv, do = _randn(T, (Hq + 2 * Hkv) * D, seed=73), _randn(T, Hq * D, seed=74)
+	o, lse = K.attn_fwd(qkv, B, S, Hq, Hkv, D, causal)
+	want = K.attn_bwd(qkv, o, do, lse, B, S, Hq, Hkv, D, causal)
+	row, head = S // 2 + 5, Hq - 1  # of sequence 0
+	bad = do.clone()
+	bad[row, head * D + 3] = what
+	got = K.attn_bwd(qkv, o, bad, lse, B, S, Hq, Hkv, D, causal)
+	assert torch.equal(got[S:], want[S:])
+	hk = head // G
+	clean = torch.ones(got.shape[1], dtype=torch.bool, device="cuda")
+	clean[head * D : (head + 1) * D] = False
+	for first in (Hq + hk, Hq + Hkv + hk):
+		clean[first * D : (first + 1) * D] = False
+	assert torch.equal(got[:S, clean], want[:S, clean])
+	others = torch.arange(S, device="cuda") != row
+	dq = slice(head * D, (head + 1) * D)
+	assert torch.equal(got[:S, dq][others], want[:S, dq][others])
+	assert not torch.isfinite(got[row, dq].float()).any()
+	dv = got[:S, (Hq + Hkv + hk) * D + 3].float()
+	assert not torch.isfinite(dv[: row + 1] if causal else dv).any()
 
 
 @pytest.mark.parametrize("D,causal", [(64, True), (128, False)])
