@@ -977,35 +977,43 @@ int add_bf16(const void* a, const void* b, void* out, int64_t n, hipStream_t s) 
 // Bias gradients of split linear layers (elf/zb_utils.py:247-252: go.sum(0) added to bias.grad in
 // LinearDW.backward): out[c] += sum_t x[t, c] in fp32, for every layer of a list in two launches.  A workgroup owns 256 columns and
 // one slice of the rows of a layer; its 8 row groups are folded through LDS and the slice's sums go to part[slice][c].  The second
-// kernel adds the slices in ascending order, one writer per column: equal bits from run to run.  Bound: launches (4.5 us each with a
-// layer of 2112 x 4288, 18 MB, alone; a list of two layers takes 9 us instead of 18).
+// kernel adds the slices in ascending order, one writer per column: equal bits from run to run.  Bound: launches, whose arguments lie in
+// host memory.  MAX: layers a launch has room for.  One layer (64 to 16384 rows) takes 4.3 to 4.9 us through the argument of one, 5.9 to 6.5 through
+// that of DW_GROUP_MAX (us, the two launches), which a list of two makes once instead of two calls of 4.5.
+struct ColsumLayer {
+	int first, first_fold;  // its first workgroup in either launch
+	int slices, N;
+	const bf16_t* x;
+	int64_t ld;
+	float* part;
+	float* out;
+};
+template <int MAX>
 struct ColsumArgs {
 	int n;
-	int first[DW_GROUP_MAX], first_fold[DW_GROUP_MAX];  // a layer's first workgroup in either launch
-	int slices[DW_GROUP_MAX], N[DW_GROUP_MAX];
-	const bf16_t* x[DW_GROUP_MAX];
-	int64_t ld[DW_GROUP_MAX], T;
-	float* part[DW_GROUP_MAX];
-	float* out[DW_GROUP_MAX];
+	int64_t T;
+	ColsumLayer layers[MAX];
 };
-__device__ __forceinline__ int colsum_layer(const int (&first)[DW_GROUP_MAX], int n) {
+template <int MAX>
+__device__ __forceinline__ ColsumLayer colsum_layer(const ColsumArgs<MAX>& a, int ColsumLayer::*first) {
+	if constexpr (MAX == 1) return a.layers[0];
 	int p = 0;
-	for (int i = 1; i < n; i++)
-		if ((int)blockIdx.x >= first[i]) p = i;
-	return __builtin_amdgcn_readfirstlane(p);
+	for (int i = 1; i < a.n; i++)
+		if ((int)blockIdx.x >= a.layers[i].*first) p = i;
+	return a.layers[__builtin_amdgcn_readfirstlane(p)];
 }
-__global__ __launch_bounds__(256) void colsum_kernel(ColsumArgs a) {
+template <int MAX>
+__global__ __launch_bounds__(256) void colsum_kernel(ColsumArgs<MAX> a) {
 	__shared__ float red[8][256];
-	const int p = colsum_layer(a.first, a.n), N = a.N[p], slices = a.slices[p];
-	const int bid = (int)blockIdx.x - a.first[p], block = bid / slices, slice = bid - block * slices;
+	const ColsumLayer l = colsum_layer(a, &ColsumLayer::first);
+	// neighbouring workgroups take neighbouring columns of the same rows
+	const int col_blocks = (l.N + 255) >> 8, bid = (int)blockIdx.x - l.first, slice = bid / col_blocks, block = bid - slice * col_blocks;
 	const int cl = threadIdx.x & 31, rg = threadIdx.x >> 5;
 	const int c0 = (block * 32 + cl) * 8;
-	const bf16_t* const x = a.x[p] + c0;
-	const int64_t ld = a.ld[p];
 	float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-	if (c0 < N) {
-		for (int64_t t = (int64_t)slice * 8 + rg; t < a.T; t += 8 * (int64_t)slices) {
-			const Chunk c = load8(x + t * ld);
+	if (c0 < l.N) {
+		for (int64_t t = (int64_t)slice * 8 + rg; t < a.T; t += 8 * (int64_t)l.slices) {
+			const Chunk c = load8(l.x + t * l.ld + c0);
 #pragma unroll
 			for (int j = 0; j < 8; j++) s[j] += c.v[j];
 		}
@@ -1014,22 +1022,29 @@ __global__ __launch_bounds__(256) void colsum_kernel(ColsumArgs a) {
 	for (int j = 0; j < 8; j++) red[rg][cl * 8 + j] = s[j];
 	__syncthreads();
 	const int c = block * 256 + threadIdx.x;
-	if (c < N) {
+	if (c < l.N) {
 		float t = 0.f;
 #pragma unroll
 		for (int r = 0; r < 8; r++) t += red[r][threadIdx.x];
-		a.part[p][(int64_t)slice * N + c] = t;
+		l.part[(int64_t)slice * l.N + c] = t;
 	}
 }
-__global__ __launch_bounds__(256) void colsum_fold_kernel(ColsumArgs a) {
-	const int p = colsum_layer(a.first_fold, a.n), N = a.N[p];
-	const int c = ((int)blockIdx.x - a.first_fold[p]) * 256 + threadIdx.x;
-	if (c >= N) return;
-	const float* const part = a.part[p] + c;
+template <int MAX>
+__global__ __launch_bounds__(256) void colsum_fold_kernel(ColsumArgs<MAX> a) {
+	const ColsumLayer l = colsum_layer(a, &ColsumLayer::first_fold);
+	const int c = ((int)blockIdx.x - l.first_fold) * 256 + threadIdx.x;
+	if (c >= l.N) return;
 	float t = 0.f;
 #pragma unroll 8
-	for (int sl = 0; sl < a.slices[p]; sl++) t += part[(int64_t)sl * N];
-	a.out[p][c] += t;
+	for (int sl = 0; sl < l.slices; sl++) t += l.part[(int64_t)sl * l.N + c];
+	l.out[c] += t;
+}
+template <int MAX>
+static int launch_colsum(const ColsumArgs<MAX>& a, int blocks, int folds, hipStream_t s) {
+	ELF_LAUNCH(colsum_kernel<MAX>, dim3((unsigned)blocks), dim3(256), 0, s, a);
+	ELF_LAUNCH(colsum_fold_kernel<MAX>, dim3((unsigned)folds), dim3(256), 0, s, a);
+	ELF_CHECK_HIP(hipGetLastError());
+	return 0;
 }
 static inline int colsum_slices(int64_t T, int N) {
 	const int col_blocks = (N + 255) / 256;
@@ -1046,45 +1061,36 @@ int64_t colsum_group_workspace_floats(int n, const LinearW* layers, int T) {
 	return sum;
 }
 int colsum_group(int n, const LinearW* layers, int T, float* workspace, hipStream_t s) {
-	ColsumArgs a{};
+	ColsumArgs<DW_GROUP_MAX> a{};
 	a.T = T;
 	int blocks = 0, folds = 0;
 	auto flush = [&]() -> int {
-		if (a.n) {
-			ELF_LAUNCH(colsum_kernel, dim3(blocks), dim3(256), 0, s, a);
-			ELF_LAUNCH(colsum_fold_kernel, dim3(folds), dim3(256), 0, s, a);
-			ELF_CHECK_HIP(hipGetLastError());
-		}
+		int rc = 0;
+		if (a.n == 1) rc = launch_colsum(ColsumArgs<1>{1, a.T, {a.layers[0]}}, blocks, folds, s);
+		else if (a.n) rc = launch_colsum(a, blocks, folds, s);
 		a.n = blocks = folds = 0;
-		return 0;
+		return rc;
 	};
 	for (int i = 0; i < n; i++) {
 		const LinearW& l = layers[i];
 		if (!l.bias) continue;
 		bool again = false;  // a bias that an earlier layer of the list adds to as well
-		for (int j = 0; j < a.n; j++) again = again || (l.bias < a.out[j] + a.N[j] && a.out[j] < l.bias + l.M);
+		for (int j = 0; j < a.n; j++) again = again || (l.bias < a.layers[j].out + a.layers[j].N && a.layers[j].out < l.bias + l.M);
 		if (again || a.n == DW_GROUP_MAX) {
 			if (int rc = flush()) return rc;
 		}
-		const int k = a.n++, col_blocks = (l.M + 255) / 256;
-		a.slices[k] = colsum_slices(T, l.M);
-		a.first[k] = blocks, a.first_fold[k] = folds;
-		a.N[k] = l.M, a.x[k] = (const bf16_t*)l.dY, a.ld[k] = l.lddy, a.part[k] = workspace, a.out[k] = l.bias;
-		workspace += (int64_t)a.slices[k] * l.M;
-		blocks += col_blocks * a.slices[k], folds += col_blocks;
+		const int col_blocks = (l.M + 255) / 256, slices = colsum_slices(T, l.M);
+		a.layers[a.n++] = ColsumLayer{blocks, folds, slices, l.M, (const bf16_t*)l.dY, l.lddy, workspace, l.bias};
+		workspace += (int64_t)slices * l.M;
+		blocks += col_blocks * slices, folds += col_blocks;
 	}
 	return flush();
 }
 int colsum_bf16(const void* x, int64_t ld, void* out_f32, int64_t T, int N, float* workspace, hipStream_t s) {
 	ELF_REQUIRE(x && out_f32 && workspace && T > 0 && N > 0 && N % 8 == 0 && ld % 8 == 0 && ld >= N,
 	            "colsum: null pointer, or N and the row stride are not multiples of 8 (T=%lld N=%d ld=%lld)", (long long)T, N, (long long)ld);
-	ColsumArgs a{};
-	const int col_blocks = (N + 255) / 256;
-	a.n = 1, a.T = T, a.slices[0] = colsum_slices(T, N), a.N[0] = N, a.x[0] = (const bf16_t*)x, a.ld[0] = ld, a.part[0] = workspace, a.out[0] = (float*)out_f32;
-	ELF_LAUNCH(colsum_kernel, dim3((unsigned)(col_blocks * a.slices[0])), dim3(256), 0, s, a);
-	ELF_LAUNCH(colsum_fold_kernel, dim3(col_blocks), dim3(256), 0, s, a);
-	ELF_CHECK_HIP(hipGetLastError());
-	return 0;
+	const int col_blocks = (N + 255) / 256, slices = colsum_slices(T, N);
+	return launch_colsum(ColsumArgs<1>{1, T, {{0, 0, slices, N, (const bf16_t*)x, ld, workspace, (float*)out_f32}}}, col_blocks * slices, col_blocks, s);
 }
 
 // ------------------------------------------------------------------------------------------
