@@ -66,9 +66,10 @@ __device__ __forceinline__ float row_loss_of(const LossArgs& a, int64_t row, int
 }
 
 // Launches of at most this many rows of at most COUNT_COLS columns count the live rows themselves, each wave under the loads of its own
-// row, instead of reading what a launch before them counted (4 us): 512 x 1000, loss and gradient 17.8 us -> 14.5.  Not wider ones: the
-// registers are full there, and with 2048 rows of 50304 columns the count took longer than that launch.
-constexpr int COUNT_ROWS = 2048, COUNT_COLS = 64 * 8 * 8;
+// row, instead of reading what a launch before them counted.  Loss, gradient and its product with the incoming one, counted before and
+// here (us): 64 x 1000 10.8 and 8.5, 512 x 1000 11.1 and 9.5, 1024 x 1000 11.9 and 11.2, 1024 x 4080 18.4 and 17.7, 1536 x 1000 13.1 and 13.3, 2048 x
+// 512 12.1 and 13.2, 2048 x 4080 26.1 and 29.5.  Not wider rows: the registers are full there.
+constexpr int COUNT_ROWS = 1024, COUNT_COLS = 64 * 8 * 8;
 
 // G threads per row, C 16-byte chunks (8 logits) per thread: rows of up to G * C * 8 columns, read once into registers,
 // reduced there, and their gradient written from the same registers.  Bound: HBM (4 bytes per logit) and, close behind, the two
