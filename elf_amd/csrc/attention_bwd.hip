@@ -788,12 +788,8 @@ static Splits split_short(int B, int S, int Hq, int Hkv, int D, bool causal, int
 	Splits best;
 	if ((int64_t)B * S * Hq >= 1 << 18) return best;  // these fill the chip
 	float best_us = 1e30f;
-	bool shared_pairs = false;
 	for (int paired = 1; paired >= (causal && nkt > 1 ? 0 : 1); paired--) {
-		if (!paired) {
-			best_us += fixed;  // that of a pair's second tile, which all sharings of pairs have alike
-			shared_pairs = best.h * best.q > 1;
-		}
+		if (!paired) best_us += fixed;  // that of a pair's second tile, which all sharings of pairs have alike
 		const bool two = causal && paired && nkt > 1;  // key tiles one after the other
 		const int64_t walks = (int64_t)B * Hkv * (two ? (nkt + 1) / 2 : nkt);
 		const int tiles = two ? (nkt + 1) * 4 : nkt * 4;  // query tiles of the longest walk and head (a pair of key tiles has nkt + 1 of four)
@@ -806,8 +802,7 @@ static Splits split_short(int B, int S, int Hq, int Hkv, int D, bool causal, int
 				const float rounds = ceilf((float)(walks * ns) / slots);
 				if (!paired && rounds > 1.f) continue;
 				const float us = rounds * (fixed + (float)(G / h) * ((tiles + q - 1) / q) * step) + (ns > 1 ? split + ns * per_split + (float)ns * B * S * Hkv * D * 16 / rate : 0.f);
-				const float lead = shared_pairs && ns == 1 ? fixed - 3.f : 0.f;
-				if (us + lead < best_us * (ns > 1 ? margin : 1.f)) best_us = us, best = Splits{h, q, paired != 0};
+				if (us < best_us * (ns > 1 ? margin : 1.f)) best_us = us, best = Splits{h, q, paired != 0};
 			}
 		}
 	}
