@@ -776,9 +776,10 @@ static int64_t dkv_part_bytes(const Splits& sp, int B, int S, int Hkv, int D) { 
 // Constants in microseconds as measured.  Causal with one key tile (128 tokens): a walk has four steps a head, what a step and a
 // split cost beside the fixed part shows.  Constants of its own, fitted to every sharing of 250 such shapes (the one that is picked
 // takes 0.2 % longer than the best on average, 7 % at most; with those of longer walks 1.8 and 16 %).  (Where one_kernel_pays() nothing is
-// shared, the workspace query asks for the room all the same.)  The whole call, whole -> as
-// shared now (us): 2 x 128 tokens, 4 heads of 64 18.9 -> 16.7; 3 x 128, 48 / 16 heads of 128 34.8 -> 31.2; 7 x 128, 36 / 12 heads
-// of 128 stay whole: 37.8, three ways 40.6.
+// shared; the workspace query, which does not see strides and addresses, asks for the room that calls need whose rows or V stay out of it.)  The whole call in
+// three kernels, whole -> as shared now (us): 2 x 128 tokens, 4 heads of 64 18.9 -> 16.7; 3 x 128, 48 / 16 heads of 128 34.8 -> 31.2; 7 x 128, 36 / 12 heads
+// of 128 stay whole: 37.8, three ways 40.6.  Heads of 64, 256 to 1280 tokens: what is picked takes 1.2 and (causal) 1.5 % longer than the best
+// sharing of 128-key passes over 75 and 79 shapes, 12 and 17 % at most.
 static Splits split_short(int B, int S, int Hq, int Hkv, int D, bool causal, int64_t room) {
 	const int nkt = S / 128, G = Hq / Hkv;
 	const bool one = causal && nkt == 1;

@@ -13,8 +13,9 @@ namespace attn {
 //   S = Q K^T, dP = dO V^T, P = exp2(S sc - lse), dS = P (dP - delta), dV^T += dO^T P, dK^T += Q^T dS | dQ^T = K^T dS^T
 // At the end the waves of a pair swap: w adds the two dK, w + 4 the two dV.
 // What bounds it is a chain: the tiles' way into LDS, two query tiles of five products a wave, dQ, the stores; four waves that take
-// four tiles each were as slow for one head of 64 and 4 us slower for one of 128.  4 x 128 tokens, 4 heads of 64, causal: 16.7 us in three kernels
-// (and two launches more), 10.6; 4 heads of 128 20.0 -> 15.5; 8 x 128, 32 heads of 64 25.9 -> 13.6.  dQ is rounded to bf16 once instead of
+// four tiles each were as slow for one head of 64 and 4 us slower for one of 128.  The call by itself, over and over on the same operands: 4 x
+// 128 tokens, 4 heads of 64, causal 16.7 us in three kernels (and two launches more), 10.6; 4 heads of 128 20.0 -> 15.5; 8 x 128, 32 heads of 64
+// 25.9 -> 13.6.  In the pass of a stage, between other kernels, the first takes 12.5 us of kernel.  dQ is rounded to bf16 once instead of
 // twice: its error against 64 bits is 0.0026 for 0.0031 with heads of 128, and the same with those of 64, whose scale is a power of two.
 template <int D, bool CAUSAL>
 __global__ __launch_bounds__(512) void attn_bwd_one_kernel(AttnBwdArgs a, const bf16_t* __restrict__ O, const float* __restrict__ lse, bf16_t* dq, int64_t ldo, int64_t lddq) {
@@ -52,7 +53,8 @@ __global__ __launch_bounds__(512) void attn_bwd_one_kernel(AttnBwdArgs a, const 
 #pragma unroll 1
 	for (int hh = 0; hh < G; hh++) {
 		const int h = hk * G + hh;
-		// (what a lane's addresses are made of, anew for every head and query tile: kept for the whole walk the addresses spill)
+		// (what a lane's addresses are made of, anew for every head and query tile: kept for the whole walk the addresses spill; without a mask
+		// and with heads of 128 eleven registers do all the same, 48 bytes a lane)
 		int ln = lane, id = tid;
 		asm volatile("" : "+v"(ln), "+v"(id));
 		// wave w moves rows [16w, 16w + 16) of a tile

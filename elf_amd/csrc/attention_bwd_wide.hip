@@ -36,8 +36,8 @@ __device__ __forceinline__ bf16x8 tr_frag(uint32_t lo_addr, uint32_t hi_addr, ui
 // A wave's share of dQ is 32 columns of 16 queries over all 256 keys: half as many partial sums as with 128 keys, to write, to read
 // back and to round.  -delta is what the dP products start from, which saves a subtraction per element.  The ring of tiles has four
 // stages and a step's code one of them, so that every LDS address is a constant of the lane and an offset field.
-// Main kernel and whole call, 128 -> 256 keys (us): 8192 tokens, 16 heads, causal 486 -> 327 (0.71 -> 1.05 PFLOP/s of the five products) and
-// 559 -> 360; 8 x 1024, 12 heads, not causal 128 -> 103 whole (1.5 rounds of workgroups).  A step takes 2330 cycles, 1280 of them
+// Main kernel and whole call, by itself and over and over, 128 -> 256 keys (us): 8192 tokens, 16 heads, causal 486 -> 327 (0.71 -> 1.05 PFLOP/s of the five products) and
+// 559 -> 360; 8 x 1024, 12 heads, not causal 128 -> 103 whole (1.5 rounds of workgroups; in a stage's pass the main kernel alone takes 96).  A step takes 2330 cycles, 1280 of them
 // MFMA; the instructions of a lone wave issue one at a time (1370), an exponential holds the vector pipe for four (another 380).
 // Dealing the exponentials evenly over the slots, with S two products earlier, or alternating the halves' products made no difference.
 // Keys past the end of the sequence (S an odd multiple of 128: waves 2 and 3 of the last pass) are computed on the last ones that
