@@ -63,9 +63,9 @@ def test_cross_entropy_loss_and_gradient(rows, V, ld):
 	_check_grad(xa.grad, xf.grad * (3.0 / live), 3.0 / live)
 
 
-@pytest.mark.parametrize("rows,V", [(1024, 1000), (1025, 1000), (1024, 4089), (1024, 4090), (1023, 4096), (2048, 1000), (66, 4097), (700, 48000)])
+@pytest.mark.parametrize("rows,V", [(2048, 1000), (2049, 1000), (2048, 4089), (2048, 4090), (2047, 4096), (66, 4097), (700, 48000)])
 def test_mean_where_the_loss_kernel_counts_the_live_rows_and_where_it_does_not(rows, V):
-	"""Up to 1024 rows of up to 4096 columns (a dense row may cover 7 more) every wave counts the rows that are not ignored, beyond
+	"""Up to 2048 rows of up to 4096 columns (a dense row may cover 7 more) every wave counts the rows that are not ignored, beyond
 	that a launch before it does; logits from 2^25 elements up are read past the caches.  Mean and gradient against fp32 of PyTorch."""
 	from elf_amd import losses
 
@@ -80,6 +80,12 @@ def test_mean_where_the_loss_kernel_counts_the_live_rows_and_where_it_does_not(r
 	_check_grad(xa.grad, xf.grad.cpu(), 1.0 / int((t != -100).sum()))
 	none = losses.cross_entropy(xg, torch.full_like(t, -100).cuda())
 	assert torch.isnan(none)  # no live row, as torch
+
+
+@pytest.mark.parametrize("rows,V", [(1024, 1000), (1025, 1000), (1024, 4089), (1024, 4090), (1023, 4096)])
+def test_mean_on_both_sides_of_1024_rows(rows, V):
+	"""The line up to which every wave counts the rows that are not ignored, at either end of the widths.  Bounds as above."""
+	test_mean_where_the_loss_kernel_counts_the_live_rows_and_where_it_does_not(rows, V)
 
 
 @pytest.mark.parametrize("rows,V,ld", [(9, 3, 8), (300, 1003, 1024), (37, 1230, 1232), (5, 4095, 4160), (7, 16381, 16384), (6, 20003, 20032), (3, 65533, 65536), (3, 100001, 100008)])
