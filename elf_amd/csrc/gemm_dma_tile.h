@@ -165,7 +165,11 @@ __device__ __forceinline__ void tile_origin(const Args& g, int pid, int& m0, int
 		m0 = (sbm * 8 + (jj & 7)) * BM;
 		n0 = (sbn * 4 + (jj >> 3)) * TN;
 	} else {
-		if ((ntiles & 7) == 0) pid = (pid & 7) * (ntiles >> 3) + (pid >> 3);
+		// (192 columns: also where 8 does not divide the tiles, the first XCDs then have one more.  These tiles take the place of ones of 256 columns, of
+		// which a product may have a multiple of 8, and with the neighbours of a slab on all XCDs each of them fetches all of B.  us on operands in
+		// the memory-side cache, 256 columns, 192 in plain order, 192 so: 768 x 8000 x 12544, B reduction-major 133, 174 and 122; 320 x 16320 x
+		// 2752 31.8, 51.2 and 35.0; 448 x 9728 x 1984, B reduction-major 24.5, 27.3 and 21.9)
+		if ((ntiles & 7) == 0 || TN != BN) pid = (pid & 7) * (ntiles >> 3) + min(pid & 7, ntiles & 7) + (pid >> 3);
 		constexpr int GROUP_M = 8;
 		const int per_group = GROUP_M * g.tiles_n;
 		const int first_m = (pid / per_group) * GROUP_M;

@@ -261,6 +261,18 @@ def test_gemm_every_epilogue_of_the_tiles_between_128_and_256_rows(K, rows, prod
 		assert torch.equal(K.gemm_swiglu_bwd(a, wt, g), K.swiglu_bwd(K.gemm(a, wt, b_t=True, tile_cfg=12), g))
 
 
+@pytest.mark.parametrize("product", ["forward", "dx"])
+@pytest.mark.parametrize("M,N,Kd", [(448, 9984, 512), (576, 8576, 512), (576, 8000, 512), (832, 5504, 512), (448, 9728, 512), (1088, 3968, 512), (576, 7232, 512), (576, 8128, 512)])
+def test_gemm_tiles_of_192_columns_in_any_number(K, product, M, N, Kd):
+	"""Tiles that 8 XCDs share with each remainder: every tile once, the bits of the 64x64 tile, nothing written outside the output."""
+	assert K.gemm_way(K.WAY_FORWARD if product == "forward" else K.WAY_INPUT_GRADIENT, M, N, Kd) == (128, 192)
+	a, w = _randn(M, Kd, seed=80), _randn(N, Kd, seed=81, scale=0.05)
+	kw, b = (dict(), w) if product == "forward" else (dict(b_t=True), w.t().contiguous())
+	big = torch.full((M + 64, N + 64), 7.0, dtype=torch.bfloat16, device="cuda")
+	K.gemm(a, b, out=big[:M, :N], **kw)
+	assert torch.equal(big[:M, :N], K.gemm(a, b, tile_cfg=12, **kw)) and (big[M:] == 7).all() and (big[:, N:] == 7).all()
+
+
 def _guarded(*shape):
 	"""A dense bf16 tensor with 4096 marked elements before and behind it, and the whole."""
 	n = int(torch.Size(shape).numel())
