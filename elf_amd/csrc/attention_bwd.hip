@@ -780,15 +780,16 @@ static int64_t dkv_part_bytes(const Splits& sp, int B, int S, int Hkv, int D) { 
 // three kernels, whole -> as shared now (us): 2 x 128 tokens, 4 heads of 64 18.9 -> 16.7; 3 x 128, 48 / 16 heads of 128 34.8 -> 31.2; 7 x 128, 36 / 12 heads
 // of 128 stay whole: 37.8, three ways 40.6.  Heads of 64, 256 to 1280 tokens: what is picked takes 1.2 and (causal) 1.5 % longer than the best
 // sharing of 128-key passes over 75 and 79 shapes, 12 and 17 % at most.
-static Splits split_short(int B, int S, int Hq, int Hkv, int D, bool causal, int64_t room) {
+static Splits split_short(int B, int S, int Hq, int Hkv, int D, bool causal, int64_t room, float* estimate = nullptr) {
 	const int nkt = S / 128, G = Hq / Hkv;
 	const bool one = causal && nkt == 1;
 	const float slots = D == 128 ? 256.f : 512.f, step = one ? 1.6f : D == 128 ? 1.2f : 1.1f, fixed = 8.f;
 	// a split: what it adds by itself, per split, and the partial sums at so many bytes a us; it has to be that much better than less sharing
 	const float split = one ? 0.f : 2.f, per_split = one ? 0.4f : 0.f, rate = one ? 4e6f : 5e6f, margin = one ? 1.f : 0.95f;
 	Splits best;
-	if ((int64_t)B * S * Hq >= 1 << 18) return best;  // these fill the chip
 	float best_us = 1e30f;
+	if (estimate) *estimate = best_us;
+	if ((int64_t)B * S * Hq >= 1 << 18) return best;  // these fill the chip
 	for (int paired = 1; paired >= (causal && nkt > 1 ? 0 : 1); paired--) {
 		if (!paired) best_us += fixed;  // that of a pair's second tile, which all sharings of pairs have alike
 		const bool two = causal && paired && nkt > 1;  // key tiles one after the other
@@ -807,6 +808,7 @@ static Splits split_short(int B, int S, int Hq, int Hkv, int D, bool causal, int
 			}
 		}
 	}
+	if (estimate) *estimate = best_us;
 	return best;
 }
 
@@ -877,6 +879,15 @@ static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal, int6
 				if (us < best_us) best_us = us, best = Splits{h, q, paired != 0, wide};
 			}
 		}
+	}
+	// Without a mask all walks are alike: 128-key tiles, two on a compute unit, that fit at once against 256-key ones, the last one perhaps half
+	// empty, whose second round is.  The two estimates are of kernels of their own, 1.38 is where both took the same time (us, 128 and 256 keys:
+	// 3 x 896, 24 heads 75.8 and 93.0, 11 x 1152, 5 heads 89.3 and 107, 6 x 640, 17 heads 62.6 and 74.9, 4 x 896, 68 / 17 245 and 264;
+	// below it 1 x 1152, 26 / 13 heads 59.4 and 58.4).  From 2048 tokens up the longer pass makes up for the round: 12 x 2688, 6 / 2 heads 530 and 488.
+	if (wide && !causal && S < 2048) {
+		float short_us;
+		const Splits sp = split_short(B, S, Hq, Hkv, D, causal, room, &short_us);
+		if (short_us * 1.38f < best_us) return sp;
 	}
 	return best;
 }
