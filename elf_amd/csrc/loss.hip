@@ -21,8 +21,6 @@ constexpr float LOG2E_F = 1.4426950408889634f;
 // which a softmax term that small may do).
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-constexpr int64_t STREAM_ELEMS = int64_t(1) << 25;  // arrays from this size on go past the caches
-
 struct LossArgs {
 	const bf16_t* x;
 	int64_t ld;
@@ -308,12 +306,23 @@ __global__ __launch_bounds__(1024) void cross_entropy_reduce_kernel(const float*
 	}
 }
 
+// Which logits are read past the caches: those that the memory-side cache does not hold, 2^27 of them, and from 84 M on in long rows, where
+// the gradient then finds more room: of 8192 columns and more if they start on 128-byte lines, otherwise of 32768.  Loss, gradient and product, with
+// what produces the logits before, as usual and past the caches (us): 3108 x 31552 206 and 188, 2680 x 46784 266 and 245, 4096 x 32000 273 and 254.  On
+// the other side of the lines, loss and padded gradient: 4959 x 10592 78 and 84, 5736 x 11824 99 and 109, 6641 x 10176 97 and 102; of 200 runs from
+// 2^25 up a third were 2 to 12 % slower past them.  Dense rows without a gradient only from 2^27 on: at 2^26 they take 3 % longer.
+template <bool DENSE>
+bool past_caches(const LossArgs& a) {
+	const int64_t n = a.rows * a.V, columns = !DENSE && a.ld % 64 == 0 && ((uintptr_t)a.x & 127) == 0 ? 8192 : 32768;
+	return n >= int64_t(1) << 27 || (n >= int64_t(5) << 24 && a.V >= columns && (!DENSE || a.dx));
+}
+
 template <int G, int C, bool DENSE>
 void launch_rows(const LossArgs& a, hipStream_t s) {
 	constexpr int BLOCK = G < 256 ? 256 : G;
 	constexpr int ROWS = BLOCK / G;
 	const dim3 grid((unsigned)((a.rows + ROWS - 1) / ROWS));
-	if (a.rows * a.V >= STREAM_ELEMS) ELF_LAUNCH((cross_entropy_kernel<G, C, DENSE, true>), grid, dim3(BLOCK), 0, s, a);
+	if (past_caches<DENSE>(a)) ELF_LAUNCH((cross_entropy_kernel<G, C, DENSE, true>), grid, dim3(BLOCK), 0, s, a);
 	else ELF_LAUNCH((cross_entropy_kernel<G, C, DENSE, false>), grid, dim3(BLOCK), 0, s, a);
 }
 
@@ -334,6 +343,7 @@ bool launch_resident(const LossArgs& a, int64_t width, hipStream_t s) {
 // thread.  Bound: HBM.  STREAM: past the caches, for arrays these do not hold; 4096 x 128256 464 us -> 352 (4.5 -> 6.0 TB/s; walked
 // with a grid of 8192 workgroups before), 1024 x 151936 125 -> 89, 2048 x 50257 69 -> 60.  16 MB take 7.5 us either way, and stay
 // in the caches for who reads the gradient next.
+constexpr int64_t STREAM_ELEMS = int64_t(1) << 25;
 template <int U, bool STREAM>
 __global__ __launch_bounds__(256) void scale_by_kernel(const bf16_t* __restrict__ x, const float* __restrict__ g, bf16_t* __restrict__ y, int64_t n) {
 	const float f = (float)(bf16_t)*g;

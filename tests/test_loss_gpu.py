@@ -82,6 +82,12 @@ def test_mean_where_the_loss_kernel_counts_the_live_rows_and_where_it_does_not(r
 	assert torch.isnan(none)  # no live row, as torch
 
 
+@pytest.mark.parametrize("rows,V", [(1800, 48000), (1800, 47999), (10239, 8192), (10240, 8192), (10250, 8191), (32800, 4096)])
+def test_mean_of_logits_that_are_read_past_the_caches(rows, V):
+	"""5 x 2^24 logits in long rows, 2^27 in narrower ones, and either side of these lines.  Bounds as above."""
+	test_mean_where_the_loss_kernel_counts_the_live_rows_and_where_it_does_not(rows, V)
+
+
 @pytest.mark.parametrize("rows,V", [(1024, 1000), (1025, 1000), (1024, 4089), (1024, 4090), (1023, 4096)])
 def test_mean_on_both_sides_of_1024_rows(rows, V):
 	"""The line up to which every wave counts the rows that are not ignored, at either end of the widths.  Bounds as above."""
