@@ -878,7 +878,7 @@ static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal, int6
 				if (ns > 1) us = (us + split + ns * per_split + (float)ns * B * S * Hkv * D * 16 / rate) / margin;
 				// partial sums of short walks in a launch of several rounds take a little more than that: of 80 shapes that this decides 30 were
 				// slower by more than 3 % than the sharing before these constants, none is now (us, without and with: 6 x 512, 16 / 2 heads of
-				// 128 83.3 and 75.7, 2 x 512, 48 / 12 77.6 and 73.9; 13 x 640, 2 / 1 45.6 and 48.2)
+				// 128 83.3 and 76.2, 2 x 512, 48 / 12 77.6 and 74.4; 13 x 640, 2 / 1 45.6 and 48.2)
 				if (causal && !paired && !wide && ns > 1 && n <= 6 && walks * n > slots) us *= 1.05f;
 				if (us < best_us) best_us = us, best = Splits{h, q, paired != 0, wide};
 			}
