@@ -887,11 +887,12 @@ static Splits split_walk(int B, int S, int Hq, int Hkv, int D, bool causal, int6
 	// Without a mask all walks are alike: 128-key tiles, two on a compute unit, that fit at once against 256-key ones, the last one perhaps half
 	// empty, whose second round is.  The two estimates are of kernels of their own, 1.38 is where both took the same time (us, 128 and 256 keys:
 	// 3 x 896, 24 heads 75.8 and 93.0, 11 x 1152, 5 heads 89.3 and 107, 6 x 640, 17 heads 62.6 and 74.9, 4 x 896, 68 / 17 245 and 264;
-	// below it 1 x 1152, 26 / 13 heads 59.4 and 58.4).  From 2048 tokens up the longer pass makes up for the round: 12 x 2688, 6 / 2 heads 530 and 488.
+	// below it 1 x 1152, 26 / 13 heads 59.4 and 58.4).  384 tokens, of whose three tiles of 128 the two of 256 keys leave a quarter empty, from 1.1
+	// on: 11 x 384, 25 heads 80.5 and 89.6, 9 x 384, 15 / 5 heads 48.3 and 54.2; 6 x 384, 48 / 12 heads, 1.09, 80.0 and 79.8.  From 2048 tokens up the longer pass makes up for the round: 12 x 2688, 6 / 2 heads 530 and 488.
 	if (wide && !causal && S < 2048) {
 		float short_us;
 		const Splits sp = split_short(B, S, Hq, Hkv, D, causal, room, &short_us);
-		if (short_us * 1.38f < best_us) return sp;
+		if (short_us * (S < 512 ? 1.1f : 1.38f) < best_us) return sp;
 	}
 	return best;
 }
