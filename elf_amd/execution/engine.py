@@ -70,6 +70,39 @@ def _mem():
 	return figures
 
 
+class _OutputCopies:
+	"""The copies of a step's outputs to pinned memory, on a stream of their own.  The allocator knows the outputs as the compute stream's: given
+	up while a copy still reads it, one would be handed to a kernel that overwrites it.  So outputs are kept until the compute stream
+	has waited for their copies: at the end of the step, or when another one starts and ``KEPT_BYTES`` of them would lie about.  (No event per
+	copy: three Engines in turn took 24.4 ms a step with those, 16.9 without.)"""
+
+	KEPT_BYTES = 4 << 30
+
+	def __init__(self, stream):
+		self.stream = stream
+		self._kept, self._bytes, self._any = [], 0, False
+
+	def start(self, output):
+		"""The output's copy on the host, which is there once the stream has come to it."""
+		compute, nbytes = torch.cuda.current_stream(), output.untyped_storage().nbytes()
+		if self._kept and self._bytes + nbytes > self.KEPT_BYTES:
+			compute.wait_stream(self.stream)
+			self._kept, self._bytes = [], 0
+		self.stream.wait_stream(compute)
+		with torch.cuda.stream(self.stream), torch.no_grad():
+			copy = output.to("cpu", non_blocking=True)
+		self._kept.append(output)
+		self._bytes += nbytes
+		self._any = True
+		return copy
+
+	def finish(self):
+		"""Behind the step's last copy; whether there was any."""
+		torch.cuda.current_stream().wait_stream(self.stream)
+		self._kept, self._bytes = [], 0
+		return self._any
+
+
 def preallocate_pool(blocks):
 	"""``ELF_PREALLOCATE_POOL="bf16:8,f32:1"`` (GiB per dtype, elf/execution/engine.py:71-93) grows the
 	pinned-host memory of activation offload before the first step.  The reference has one pool per
@@ -175,7 +208,7 @@ class Engine:
 		memories, peak_memories = OrderedDict(), OrderedDict()
 		T = OperationType
 		on_gpu = _GPU()
-		copies_outputs = False
+		copies = _OutputCopies(self.offload_stream)
 		if not _capturing():
 			# The host stays at most two steps ahead of the copies of a step's outputs to pinned memory: every step in flight holds
 			# its own set of them (823 MB of logits for 8 x 1024 tokens and 50257 words), and with five or more steps queued a
@@ -249,10 +282,7 @@ class Engine:
 				with _timed(block, f"backward({block.id}:{op.mb_id})"):
 					grads = grad_fns.popleft()()
 				if self.offload_stream is not None and not _capturing():  # a captured step keeps its outputs on the GPU
-					copies_outputs = True
-					self.offload_stream.wait_stream(torch.cuda.current_stream())
-					with torch.cuda.stream(self.offload_stream), torch.no_grad():
-						result[op.mb_id] = result[op.mb_id].to("cpu", non_blocking=True)
+					result[op.mb_id] = copies.start(result[op.mb_id])
 				for grad, var in zip(grads, block.output_variables):
 					for dst in var:
 						dst.set(dst.to_process, op.mb_id, _fake_p2p(grad))
@@ -306,8 +336,7 @@ class Engine:
 		for block in self.blocks:
 			block.compute_time.clear()
 		if self.offload_stream is not None and not _capturing():
-			torch.cuda.current_stream().wait_stream(self.offload_stream)
-			if copies_outputs:
+			if copies.finish():
 				self._output_copies.append(self.offload_stream.record_event())
 		for off in offloaders.values():
 			off.release()

@@ -1,10 +1,12 @@
 """Host logic of the Engine with stand-in blocks (no GPU): dispatch order, slot hand-offs
 between same-rank blocks, loss scaling, statistics surface, error paths of the Variable slots."""
 
+from types import SimpleNamespace
+
 import pytest
 import torch
 
-from elf_amd.execution import Engine, Variable, compute_loss
+from elf_amd.execution import Engine, Variable, compute_loss, engine as engine_module
 from elf_amd.partitioners.utils import sequential_signatures
 from elf_amd.registry import COMM_SCHEDULERS, SCHEDULERS
 from elf_amd.scheduling import OperationType as T, add_comms
@@ -200,3 +202,53 @@ def test_sequential_order_reports_a_schedule_that_cannot_run():
 		sequential_order(stuck, sigs)
 	with pytest.raises(AssertionError):
 		Engine([FakeBlock(0, [0, 1]), FakeBlock(1, [0, 1])])  # two ranks without all_ranks
+
+
+class _FakeStream:
+	"""The order of what a stream was asked: its own work as numbers, waits as what it waited for."""
+
+	def __init__(self):
+		self.enqueued, self.waited = 0, {}
+
+	def record_event(self):
+		return self, self.enqueued
+
+	def wait_event(self, event):
+		other, upto = event
+		self.waited[other] = max(self.waited.get(other, 0), upto)
+
+	def wait_stream(self, other):
+		self.wait_event((other, other.enqueued))
+
+
+@pytest.mark.parametrize("n,nbytes,kept", [(1, 1 << 30, 4), (4, 1 << 30, 4), (9, 1 << 30, 4), (3, 5 << 30, 1), (50, 1 << 20, 50)])
+def test_outputs_are_kept_until_the_compute_stream_has_waited_for_their_copies(monkeypatch, n, nbytes, kept):
+	"""An output that goes back to the allocator is handed to the compute stream's next kernel: its copy must not be reading it by then."""
+	import contextlib
+	import weakref
+
+	compute, side = _FakeStream(), _FakeStream()
+	monkeypatch.setattr(torch.cuda, "current_stream", lambda: compute)
+	monkeypatch.setattr(torch.cuda, "stream", lambda s: contextlib.nullcontext())
+	gone = {}
+
+	class Output:
+		def untyped_storage(self):
+			return SimpleNamespace(nbytes=lambda: nbytes)
+
+		def to(self, device, non_blocking):
+			assert device == "cpu" and non_blocking and side.waited.get(compute, 0) == compute.enqueued
+			side.enqueued += 1
+			return f"copy {side.enqueued}"
+
+	copies = engine_module._OutputCopies(side)
+	for i in range(1, n + 1):
+		compute.enqueued += 1  # the output's own kernel
+		out = Output()
+		weakref.finalize(out, lambda i=i: gone.setdefault(i, compute.waited.get(side, 0)))
+		assert copies.start(out) == f"copy {i}"
+		del out
+		assert len(gone) == (i - 1) // kept * kept
+	assert copies.finish()
+	assert sorted(gone) == list(range(1, n + 1)) and all(waited >= i for i, waited in gone.items())
+	assert not engine_module._OutputCopies(side).finish()

@@ -167,3 +167,32 @@ def test_steps_in_a_row_hand_over_their_own_outputs():
 	torch.cuda.synchronize()
 	for (out, loss), (want, want_loss) in zip(got, alone):
 		assert all(o.device.type == "cpu" and torch.equal(o, w) for o, w in zip(out, want)) and float(loss) == want_loss
+
+
+@pytest.mark.parametrize("sched,n_stages,d,V", [("afab", 1, 256, 16384), ("full_remat", 1, 256, 16384), ("afab", 2, 1024, 1024), ("full_remat", 2, 1024, 1024)])
+def test_every_micro_batch_hands_over_its_own_logits(sched, n_stages, d, V):
+	"""Six micro-batches whose logits take longer to the host than the kernels in between: each one's are those it gives in a step of its own.
+	While a copy waits its turn nothing else is written where it reads: not the next logits (one stage), not the gradient that the last
+	stage's backward makes right behind (two, of the logits' size)."""
+	from elf_amd import losses
+	from elf_amd.models import EndStage, StageModule, TransformerBlock
+	from elf_amd.pipeline import Pipeline
+
+	S, n = 256, 6
+	torch.manual_seed(5)
+	with torch.device("cuda"):
+		stages = [EndStage(StageModule([TransformerBlock(d, d // 64, 4 * d)], S), vocab_in=V if i == 0 else None, vocab_out=V if i == n_stages - 1 else None) for i in range(n_stages)]
+	stages = [st.to(torch.bfloat16) for st in stages]
+	ids = torch.randint(0, V, (4 * n, S + 1), generator=torch.Generator().manual_seed(6)).cuda()
+	x, t = ids[:, :-1].contiguous(), ids[:, 1:].contiguous()
+	pipe = Pipeline(stages, scheduler=sched, partitioner=False, placement=[0] * n_stages, mb_size=4)
+	alone = []
+	for i in range(n):
+		logits, _ = pipe(x[4 * i : 4 * i + 4], t[4 * i : 4 * i + 4], losses.cross_entropy, split_size=4)
+		torch.cuda.synchronize()
+		alone.append(logits[0].clone())
+	for _ in range(3):
+		pipe.zero_grad()
+		logits, _ = pipe(x, t, losses.cross_entropy, split_size=4)
+		torch.cuda.synchronize()
+		assert len(logits) == n and all(torch.equal(a, b) for a, b in zip(logits, alone))
